@@ -5,7 +5,7 @@ Products (all in-tree, git-ignored):
   hacapk-magma_amd/lib/libhmvgen.so  CPU input generator   (C ABI: include/hmvgen.h)
   oracle/liboracle.so                CPU oracle (test infrastructure)
   oracle/_ref/libhacapk_ref.so       reference entry-function sources compiled with
-                                     flang (only where /root/reference exists)
+                                     flang (only where /root/reference has files)
   oracle/_ref/ref_layout_*.txt       flang's layout of the reference's container types
   oracle/_ref/ref_driver             Fortran caller of libhmv.so with those types
 
@@ -93,8 +93,9 @@ def build_oracle():
 
 def build_ref():
     script = os.path.join(ORACLE, "ref_build.sh")
-    if not os.path.isdir("/root/reference"):
-        return None
+    ref = "/root/reference"
+    if not os.path.isdir(ref) or not os.listdir(ref):
+        return None  # no reference sources on this machine
     run(["bash", script])
     return os.path.join(ORACLE, "_ref", "libhacapk_ref.so")
 
