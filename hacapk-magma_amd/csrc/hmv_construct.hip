@@ -10,13 +10,14 @@
 // workgroup per block, all of its lanes on the block's rows/columns, the
 // scalar steps of ACA+ in the same order and arithmetic as the host
 // restatement (the cross updates, the pivot searches with their first-index
-// ties, and the overflow-safe norm, which stays sequential because its
-// scaling depends on the order).  Floating-point contraction is off in this
-// file, so entries and updates round as the host's do.
+// ties; only the norms, which are compared with thresholds and enter no
+// factor, are summed in another order).  Floating-point contraction is off
+// in this file, so entries and updates round as the host's do.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -33,7 +34,20 @@
 namespace {
 
 constexpr int kT = 256;
-constexpr int kCapFirst = 64;  // factor columns reserved per block in the first pass
+// Factor columns reserved per block in the first pass: ranks grow with the
+// digits asked for (at 163,840 unknowns at most 16 for 1e-5, 14 for 1e-4); a
+// block that needs more runs again with its full bound.
+int first_columns(double eps) {
+  const double digits = eps > 0.0 && eps < 1.0 ? std::ceil(-std::log10(eps)) : 0.0;
+  return std::max(16, std::min(64, 10 + 3 * (int)std::min(digits, 100.0)));
+}
+// Bytes of reserved columns in use at a time.  The blocks run in batches of
+// this size and each batch's factors are packed behind it, so that a
+// construction allocates little more than the factors: memory given back is
+// cleared at some 40 GB/s before it can be had again, and with 64 columns for
+// every block at once (7.2 GB at 81,920 unknowns for 0.9 GB of factors) every
+// few constructions waited 0.3 to 3 s for it.
+constexpr size_t kAcaBatchBytes = (size_t)1 << 30;
 
 // ---- entry function --------------------------------------------------------
 
@@ -111,16 +125,19 @@ __device__ double triangle_potential_sum(const double xs[3], const double ys[3],
   return sum;
 }
 
+// The centroid kernel off the diagonal (0-based faces).
+__device__ inline double centroid_entry(const Geo &g, int fi, int fj) {
+  const double dx = g.cent[3 * fi] - g.cent[3 * fj];
+  const double dy = g.cent[3 * fi + 1] - g.cent[3 * fj + 1];
+  const double dz = g.cent[3 * fi + 2] - g.cent[3 * fj + 2];
+  return g.area[fj] / (4.0 * M_PI * sqrt(dx * dx + dy * dy + dz * dz));
+}
+
 // HACApK_entry_ij(i, j) for 1-based original indices: collocation at the
 // centroid of face i, source face j (m_ppohBEM_matrix_element_ij.f90:49-76).
 __device__ double entry(const Geo &g, int i, int j) {
   const int fi = i - 1, fj = j - 1;
-  if (g.kernel == kKernelCentroid && fi != fj) {
-    const double dx = g.cent[3 * fi] - g.cent[3 * fj];
-    const double dy = g.cent[3 * fi + 1] - g.cent[3 * fj + 1];
-    const double dz = g.cent[3 * fi + 2] - g.cent[3 * fj + 2];
-    return g.area[fj] / (4.0 * M_PI * sqrt(dx * dx + dy * dy + dz * dz));
-  }
+  if (g.kernel == kKernelCentroid && fi != fj) return centroid_entry(g, fi, fj);
   double xs[3], ys[3], zs[3];
   for (int a = 0; a < 3; ++a) {
     const int nn = g.faces[3 * fj + a];
@@ -138,7 +155,7 @@ __device__ double entry(const Geo &g, int i, int j) {
 
 struct CLeaf {
   int ltmtx, nstrtl, ndl, nstrtt, ndt;
-  int cap;        // low rank: factor columns reserved at base
+  int cap;        // low rank: factor columns held (reserved) at base
   double *base;   // dense: A (ndl rows of ndt); low rank: V (ndt x cap), then U (ndl x cap)
   double *pa;     // low rank scratch: reference column (ndl), then reference row (ndt)
   int *msk;       // low rank scratch: row mask (ndl), then column mask (ndt)
@@ -151,9 +168,8 @@ struct AcaParams {
 
 enum { kAcaOk = 0, kAcaOverflow = 1 };
 
-__global__ __launch_bounds__(kT) void k_dense(const CLeaf *__restrict__ lv,
-                                              const int *__restrict__ ids, Geo g) {
-  const CLeaf L = lv[ids[blockIdx.x]];
+__global__ __launch_bounds__(kT) void k_dense(const CLeaf *__restrict__ lv, Geo g) {
+  const CLeaf L = lv[blockIdx.x];
   const int64_t n = (int64_t)L.ndl * L.ndt;
   for (int64_t e = threadIdx.x; e < n; e += kT) {
     const int il = (int)(e / L.ndt), it = (int)(e % L.ndt);
@@ -161,156 +177,217 @@ __global__ __launch_bounds__(kT) void k_dense(const CLeaf *__restrict__ lv,
   }
 }
 
-// ACA+ runs one wave per block: the block's scalar steps are sequential, so
-// a wave keeps them cheap (reductions by lane shuffles, no workgroup
-// barrier between waves) and many blocks run at once.
-constexpr int kA = 64;
+// ACA+ runs one workgroup per block.  Its scalar steps are sequential and
+// every vector pass of a step ends in a reduction that the next one needs, so
+// a block's time is its passes: their memory round trips for a short block,
+// its vectors over the workgroup's lanes for a long one.  Hence
+//  - one wave for short blocks (reductions by lane shuffles; most blocks are
+//    short, and many run at once), NT = 256 or 1024 threads for longer ones
+//    (aca_class);
+//  - three passes a step: the pivot column or row with its largest entry, the
+//    other one with the scaling and the update of its reference vector, the
+//    update of the other reference vector; each also forms the norms and the
+//    largest entries that the step reads from what it just wrote.
+// 163,840 unknowns, two spheres (blocks up to 41,088 x 41,088): 173 ms with
+// one wave per block and a pass per operation, 9.1 ms now; one sphere of
+// 81,920: 21.4 ms, 3.9 ms now; the factors are the same bits.
 
-// Helpers called by every lane with the same arguments; each returns the
-// same value in every lane, and ends with the lanes' writes visible.
-
-__device__ inline void wave_sync() { __syncthreads(); }
-
-// First index (1-based) of the largest (want_max) or smallest |vec|, as
-// HACApK_maxabsvalloc_d / HACApK_minabsvalloc_d scan.
-__device__ void abs_loc(const double *vec, int n, bool want_max, double &val, int &idx) {
-  double bv = 0.0;
-  int bi = n;  // none
-  for (int a = threadIdx.x; a < n; a += kA) {
-    const double x = fabs(vec[a]);
-    if (bi == n || (want_max ? x > bv : x < bv)) {
-      bv = x;
-      bi = a;
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    const double ov = __shfl_xor(bv, off, 64);
-    const int oi = __shfl_xor(bi, off, 64);
-    const bool take =
-        oi != n && (bi == n || (want_max ? ov > bv : ov < bv) || (ov == bv && oi < bi));
-    if (take) {
-      bv = ov;
-      bi = oi;
-    }
-  }
-  val = bv;
-  idx = bi + 1;
-}
-
-// HACApK_unrm_d, bit for bit.  Its running scale zscl is the prefix maximum
-// of the |entries| (those below 1e-30 skipped), so every entry's ratio
-// (zscl/zza or zza/zscl) comes from a wave-wide prefix-max scan and is formed
-// by the entry's own lane; only the accumulation of zzz, whose rounding order
-// matters, runs entry by entry (uniformly in every lane).
-__device__ inline double lane_double(double v, int l) {
+// A value that is the same in every lane, in scalar registers.
+__device__ inline double uniform(double v) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-__device__ double unrm(const double *za, int nd) {
-  const int lane = threadIdx.x;
-  double zscl = 0.0, zzz = 1.0;  // same value in every lane
-  for (int c0 = 0; c0 < nd; c0 += 64) {
-    const int i = c0 + lane;
-    const double a = i < nd ? fabs(za[i]) : 0.0;
-    const bool skip = i >= nd || a < 1.0e-30;
-    double incl = skip ? 0.0 : a;  // inclusive prefix max within the chunk
-    for (int off = 1; off < 64; off <<= 1) {
-      const double o = __shfl_up(incl, off, 64);
-      if (lane >= off && o > incl) incl = o;
+// Largest |entry| with its first index, and the sum of squares, of the
+// entries one thread has seen (HACApK_maxabsvalloc_d, HACApK_unrm_d).
+// Entries below 1e-30 do not count in the norm, as there.
+struct VecStat {
+  double mx = 0.0;
+  int ix = -1;  // none yet
+  double ss = 0.0;
+  __device__ void add(double v, int a) {
+    const double x = fabs(v);
+    if (ix < 0 || x > mx) {
+      mx = x;
+      ix = a;
     }
-    double excl = __shfl_up(incl, 1, 64);
-    if (lane == 0) excl = 0.0;
-    const double m = excl > zscl ? excl : zscl;  // zscl before entry i
-    const bool isnew = !skip && m < a;
-    const double q = skip ? 0.0 : (isnew ? m / a : a / m);
-    const unsigned long long newm = __ballot(isnew), skipm = __ballot(skip);
-    const int nl = min(64, nd - c0);
-    for (int l = 0; l < nl; ++l) {
-      if ((skipm >> l) & 1ull) continue;
-      const double ql = lane_double(q, l);
-      if ((newm >> l) & 1ull)
-        zzz = 1.0 + zzz * ql * ql;
-      else
-        zzz = zzz + ql * ql;
-    }
-    const double cm = lane_double(incl, nl - 1);
-    if (cm > zscl) zscl = cm;
+    if (!(x < 1.0e-30)) ss = ss + x * x;
   }
-  return zscl * sqrt(zzz);
-}
+  __device__ void merge(double omx, int oix, double oss) {
+    if (oix >= 0 && (ix < 0 || omx > mx || (omx == mx && oix < ix))) {
+      mx = omx;
+      ix = oix;
+    }
+    ss = ss + oss;
+  }
+};
 
-// Residual column (col = true: ndl entries of column ip) or row (ndt entries
-// of row ip) of a block after k crosses (HACApK_calc_vec): the entries of
-// unmasked positions, minus the accumulated cross products (summed in cross
-// order before the subtraction), masked positions zero once k > 0.
-__device__ void calc_vec(const CLeaf &L, const Geo &g, bool col, int k, int ip, double *vec,
-                         const double *U, const double *V) {
-  const int n = col ? L.ndl : L.ndt;
-  const int *m = col ? L.msk : L.msk + L.ndl;
-  for (int a = threadIdx.x; a < n; a += kA) {
-    double e;
-    if (m[a] == 0)
-      e = col ? entry(g, g.lod[a + L.nstrtl - 1], g.lod[ip + L.nstrtt - 2])
-              : entry(g, g.lod[ip + L.nstrtl - 2], g.lod[a + L.nstrtt - 1]);
-    else
-      e = vec[a];
-    if (k > 0) {
-      double t = 0.0;
-      for (int it = 0; it < k; ++it) {
-        const double x = col ? U[(size_t)it * L.ndl + a] : V[(size_t)it * L.ndt + a];
-        const double y = col ? V[(size_t)it * L.ndt + (ip - 1)] : U[(size_t)it * L.ndl + (ip - 1)];
-        t = t + x * y;
+// LDS of a workgroup's reductions: two buffers in turn, so that one barrier
+// per reduction is enough (a buffer is written again only after the next
+// reduction's barrier, which every reader has passed).
+template <int NT>
+struct AcaShared {
+  double mx[2][2][NT / 64], ss[2][2][NT / 64];
+  int ix[2][2][NT / 64];
+};
+
+// Reductions over the workgroup; every thread gets the same values, and the
+// barrier makes what the threads wrote before it visible to all of them.
+template <int NT>
+struct Aca {
+  AcaShared<NT> &sh;
+  int turn = 0;
+  __device__ explicit Aca(AcaShared<NT> &s) : sh(s) {}
+
+  __device__ static void wave_merge(VecStat &s, int from = 32) {
+#pragma unroll 1
+    for (int off = from; off > 0; off >>= 1) {
+      const double omx = __shfl_xor(s.mx, off, 64), oss = __shfl_xor(s.ss, off, 64);
+      const int oix = __shfl_xor(s.ix, off, 64);
+      s.merge(omx, oix, oss);
+    }
+    settle(s);
+  }
+  // the first lane's statistics (with entries that are no numbers the lanes
+  // may disagree), in scalar registers
+  __device__ static void settle(VecStat &s) {
+    s.mx = uniform(s.mx);
+    s.ss = uniform(s.ss);
+    s.ix = __builtin_amdgcn_readfirstlane(s.ix);
+  }
+  // the waves' statistics of this turn, merged by every wave alike
+  __device__ void gather(VecStat &s, int which) {
+    const int v = threadIdx.x & (NT / 64 - 1);
+    s.mx = sh.mx[turn][which][v];
+    s.ss = sh.ss[turn][which][v];
+    s.ix = sh.ix[turn][which][v];
+    wave_merge(s, NT / 128);
+  }
+  // Two statistics at once (`both`), or one.
+  __device__ void reduce(VecStat &p, VecStat &q, bool both) {
+    wave_merge(p);
+    if (both) wave_merge(q);
+    if constexpr (NT > 64) {
+      const int w = threadIdx.x >> 6;
+      if ((threadIdx.x & 63) == 0) {
+        sh.mx[turn][0][w] = p.mx;
+        sh.ss[turn][0][w] = p.ss;
+        sh.ix[turn][0][w] = p.ix;
+        if (both) {
+          sh.mx[turn][1][w] = q.mx;
+          sh.ss[turn][1][w] = q.ss;
+          sh.ix[turn][1][w] = q.ix;
+        }
       }
-      e = e - t;
-      if (m[a] == 1) e = 0.0;
+      __syncthreads();
+      gather(p, 0);
+      if (both) gather(q, 1);
+      turn ^= 1;
+    } else {
+      __syncthreads();
     }
-    vec[a] = e;
   }
-  wave_sync();
+  __device__ void reduce(VecStat &p) {
+    VecStat none;
+    reduce(p, none, false);
+  }
+  // ||vec|| from its statistics.  The squares are safe up to 1e150; past
+  // that (or with an infinity) the entries are scaled by the largest.  The
+  // reference accumulates in entry order; here the order is the reduction's,
+  // which moves the last bits of a number that is only compared with
+  // thresholds (no factor entry depends on them).
+  __device__ double norm(const VecStat &s, const double *vec, int n) {
+    if (!(s.mx > 1.0e150)) return sqrt(s.ss);
+    VecStat t;
+    for (int a = threadIdx.x; a < n; a += NT) t.add(vec[a] / s.mx, a);
+    reduce(t);
+    return s.mx * sqrt(t.ss);
+  }
+};
+
+// Entry a of the residual column ip (col) or row ip of a block after k
+// crosses (HACApK_calc_vec): the matrix entry minus the cross products
+// (summed in cross order before the subtraction); zero at a masked position
+// (there are none before the first cross).
+template <bool CENT>
+__device__ inline double residual(const CLeaf &L, const Geo &g, bool col, int k, int ip, int a,
+                                  const double *U, const double *V) {
+  if (L.msk[col ? a : L.ndl + a] != 0) return 0.0;
+  const int i = g.lod[col ? a + L.nstrtl - 1 : ip + L.nstrtl - 2];
+  const int j = g.lod[col ? ip + L.nstrtt - 2 : a + L.nstrtt - 1];
+  const double e = CENT ? centroid_entry(g, i - 1, j - 1) : entry(g, i, j);
+  if (k == 0) return e;
+  const int sx = col ? L.ndl : L.ndt, sy = col ? L.ndt : L.ndl;
+  const double *px = (col ? U : V) + a, *py = (col ? V : U) + (ip - 1);
+  double t = 0.0;
+  int it = 0;
+#pragma unroll 1
+  for (; it + 4 <= k; it += 4) {  // four crosses' loads together
+    double x[4], y[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      x[q] = px[(size_t)(it + q) * sx];
+      y[q] = py[(size_t)(it + q) * sy];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) t = t + x[q] * y[q];
+  }
+#pragma unroll 1
+  for (; it < k; ++it) t = t + px[(size_t)it * sx] * py[(size_t)it * sy];
+  return e - t;
 }
 
-__device__ void copy_vec(double *dst, const double *src, int n) {
-  for (int a = threadIdx.x; a < n; a += kA) dst[a] = src[a];
-  wave_sync();
+// A thread's entries tid, tid + nt, ... of that column or row into vec, with
+// their statistics.
+template <bool CENT>
+__device__ inline VecStat residual_loop(const CLeaf &L, const Geo &g, bool col, int k, int ip,
+                                        double *vec, const double *U, const double *V, int nt) {
+  VecStat s;
+  const int n = col ? L.ndl : L.ndt;
+#pragma unroll 1
+  for (int a = threadIdx.x; a < n; a += nt) {
+    const double e = residual<CENT>(L, g, col, k, ip, a, U, V);
+    vec[a] = e;
+    s.add(e, a);
+  }
+  return s;
 }
-
-__device__ void scale_vec(double *v, int n, double s) {
-  for (int a = threadIdx.x; a < n; a += kA) v[a] = v[a] * s;
-  wave_sync();
+// With the analytic entry, a call of its own: one copy of that code.
+__device__ __attribute__((noinline)) VecStat residual_any(const CLeaf &L, const Geo &g, bool col,
+                                                          int k, int ip, double *vec,
+                                                          const double *U, const double *V,
+                                                          int nt) {
+  return residual_loop<false>(L, g, col, k, ip, vec, U, V, nt);
 }
-
-// y += x * s
-__device__ void axpy_vec(double *y, const double *x, int n, double s) {
-  for (int a = threadIdx.x; a < n; a += kA) y[a] = y[a] + x[a] * s;
-  wave_sync();
-}
-
-__device__ void set_mask(int *m, int i1) {
-  if (threadIdx.x == 0) m[i1 - 1] = 1;
-  wave_sync();
+template <bool CENT>
+__device__ inline VecStat residual_part(const CLeaf &L, const Geo &g, bool col, int k, int ip,
+                                        double *vec, const double *U, const double *V, int nt) {
+  if constexpr (CENT)
+    return residual_loop<true>(L, g, col, k, ip, vec, U, V, nt);
+  else
+    return residual_any(L, g, col, k, ip, vec, U, V, nt);
 }
 
 // HACApK_acaplus (m_HACApK_base.f90:783-975) with param(61) = 1, for one
-// block per workgroup; restates the host fill's ACA+ step for step.
-__global__ __launch_bounds__(kA) void k_aca(const CLeaf *__restrict__ lv,
-                                            const int *__restrict__ ids, Geo g, AcaParams p,
+// block per workgroup; restates the host fill's ACA+ step for step.  CENT:
+// the centroid kernel on blocks that hold no diagonal entry.
+template <int NT, bool CENT>
+__global__ __launch_bounds__(NT) void k_aca(const CLeaf *__restrict__ lv, Geo g, AcaParams p,
                                             int *__restrict__ kt_out, int *__restrict__ status) {
-  const int id = ids[blockIdx.x];
+  __shared__ AcaShared<NT> shared;
+  Aca<NT> R(shared);
+  const int id = blockIdx.x;
   const CLeaf L = lv[id];
-  const int ndl = L.ndl, ndt = L.ndt, cap = L.cap;
+  const int ndl = L.ndl, ndt = L.ndt, cap = L.cap, tid = threadIdx.x;
   double *V = L.base;                    // zab(ndt, cap)
   double *U = L.base + (size_t)ndt * cap;  // zaa(ndl, cap)
   double *pa_ref = L.pa, *pb_ref = L.pa + ndl;
   int *lrow_msk = L.msk, *lcol_msk = L.msk + ndl;
-  auto ucol = [&](int k1) { return U + (size_t)(k1 - 1) * ndl; };
-  auto vcol = [&](int k1) { return V + (size_t)(k1 - 1) * ndt; };
 
-  for (int a = threadIdx.x; a < ndl + ndt; a += kA) L.msk[a] = 0;
-  for (int a = threadIdx.x; a < ndl + ndt; a += kA) L.pa[a] = 0.0;
-  wave_sync();
+  for (int a = tid; a < ndl + ndt; a += NT) L.msk[a] = 0;
+  __syncthreads();
 
   const double eps = p.eps;
   const double ACA_EPS = p.eps_factor * eps;
@@ -320,76 +397,134 @@ __global__ __launch_bounds__(kA) void k_aca(const CLeaf *__restrict__ lv,
   int k = 0;
   int st = kAcaOk;
 
+  // the residual column (row) ip after kk crosses into vec, with its statistics
+  auto calc = [&](bool col, int kk, int ip, double *vec) {
+    VecStat s = residual_part<CENT>(L, g, col, kk, ip, vec, U, V, NT);
+    R.reduce(s);
+    return s;
+  };
+  // y += x s, with y's statistics
+  auto axpy = [&](double *y, const double *x, int n, double s) {
+    VecStat t;
+    for (int a = tid; a < n; a += NT) {
+      const double v = y[a] + x[a] * s;
+      y[a] = v;
+      t.add(v, a);
+    }
+    R.reduce(t);
+    return t;
+  };
+  auto set_mask = [&](int *m, int i1) {
+    if (tid == 0) m[i1 - 1] = 1;
+  };
+
   int j_ref = 1;
-  calc_vec(L, g, true, k, j_ref, pa_ref, U, V);
-  double colnorm = unrm(pa_ref, ndl);
-  double rownorm;
+  VecStat sa = calc(true, k, j_ref, pa_ref);  // of pa_ref, as it is now
+  double colnorm = R.norm(sa, pa_ref, ndl);
   int i_ref;
-  abs_loc(pa_ref, ndl, false, rownorm, i_ref);
-  calc_vec(L, g, false, k, i_ref, pb_ref, U, V);
-  rownorm = unrm(pb_ref, ndt);
+  {
+    // first index of the smallest |entry|: the largest of their negatives
+    VecStat s;
+    for (int a = tid; a < ndl; a += NT) {
+      const double x = fabs(pa_ref[a]);
+      if (s.ix < 0 || x < -s.mx) {
+        s.mx = -x;
+        s.ix = a;
+      }
+    }
+    R.reduce(s);
+    i_ref = s.ix + 1;
+  }
+  VecStat sb = calc(false, k, i_ref, pb_ref);  // of pb_ref, as it is now
+  double rownorm = R.norm(sb, pb_ref, ndt);
 
   double apxnorm = 0.0;
   int lstop_aca = 0;
   int i = 0, j = 0;
-  double col_maxval, row_maxval;
   while ((k < p.kmax) && (ntries_row > 0 || ntries_col > 0) && (ntries > 0)) {
     ntries = ntries - 1;
     if (k + 1 > cap) {
       st = kAcaOverflow;
       break;
     }
-    double *pcol = ucol(k + 1);
-    double *prow = vcol(k + 1);
-    abs_loc(pa_ref, ndl, true, col_maxval, i);
-    abs_loc(pb_ref, ndt, true, row_maxval, j);
-
-    if (row_maxval > col_maxval) {
-      if (j != j_ref)
-        calc_vec(L, g, true, k, j, pcol, U, V);
-      else
-        copy_vec(pcol, pa_ref, ndl);
-      abs_loc(pcol, ndl, true, col_maxval, i);
-      if (col_maxval < ACA_EPS && k >= p.kmin) {
-        lstop_aca = 1;
-      } else {
-        calc_vec(L, g, false, k, i, prow, U, V);
-        const double piv = pcol[i - 1];
-        wave_sync();  // every lane has the pivot before the column is scaled
-        if (fabs(piv) > piv_min) {
-          scale_vec(pcol, ndl, 1.0 / piv);
-        } else {
-          k = max(k - 1, 0);
-          break;
-        }
-      }
+    double *pcol = U + (size_t)k * ndl;
+    double *prow = V + (size_t)k * ndt;
+    i = sa.ix + 1;
+    j = sb.ix + 1;
+    // The cross: the reference vector with the larger entry gives the first
+    // of column j and row i (its own copy when that is the reference's), its
+    // largest entry the pivot and the other index; the first is scaled by
+    // the pivot.  Then pb_ref -= prow pcol(i_ref), pa_ref -= pcol prow(j_ref).
+    const bool colfirst = sb.mx > sa.mx;
+    const int n1 = colfirst ? ndl : ndt, n2 = colfirst ? ndt : ndl;
+    double *v1 = colfirst ? pcol : prow, *v2 = colfirst ? prow : pcol;
+    VecStat s1;
+    if (colfirst ? j != j_ref : i != i_ref) {
+      s1 = calc(colfirst, k, colfirst ? j : i, v1);
     } else {
-      if (i != i_ref)
-        calc_vec(L, g, false, k, i, prow, U, V);
-      else
-        copy_vec(prow, pb_ref, ndt);
-      abs_loc(prow, ndt, true, row_maxval, j);
-      if (row_maxval < ACA_EPS && k >= p.kmin) {
-        lstop_aca = 1;
-      } else {
-        calc_vec(L, g, true, k, j, pcol, U, V);
-        const double piv = prow[j - 1];
-        wave_sync();  // every lane has the pivot before the row is scaled
-        if (fabs(piv) > piv_min) {
-          scale_vec(prow, ndt, 1.0 / piv);
+      const double *src = colfirst ? pa_ref : pb_ref;
+      for (int a = tid; a < n1; a += NT) v1[a] = src[a];
+      s1 = colfirst ? sa : sb;
+      __syncthreads();
+    }
+    if (colfirst)
+      i = s1.ix + 1;
+    else
+      j = s1.ix + 1;
+    VecStat q1, q2;  // of the scaled v1 and of v2 (norms)
+    bool a_done = false, b_done = false;
+    if (s1.mx < ACA_EPS && k >= p.kmin) {
+      lstop_aca = 1;
+      // the other one is not formed; the step may still count it (below), as
+      // zeros
+      for (int a = tid; a < n2; a += NT) v2[a] = 0.0;
+    } else {
+      // entries of v1 that other threads are about to scale
+      const double piv = uniform(v1[(colfirst ? i : j) - 1]);
+      const double at_ref = uniform(v1[(colfirst ? i_ref : j_ref) - 1]);
+      __syncthreads();
+      if (!(fabs(piv) > piv_min)) {
+        k = max(k - 1, 0);
+        break;
+      }
+      const double inv = 1.0 / piv;
+      // v2 and, when its reference vector is another one, that vector's
+      // update by v2 times the scaled v1's entry at the reference
+      const bool upd = colfirst ? i != i_ref : j != j_ref;
+      const double zinv = -(at_ref * inv);
+      double *ref2 = colfirst ? pb_ref : pa_ref;
+      VecStat sr;
+      q2 = residual_part<CENT>(L, g, !colfirst, k, colfirst ? i : j, v2, U, V, NT);
+      if (upd)
+        for (int a = tid; a < n2; a += NT) {
+          const double v = ref2[a] + v2[a] * zinv;
+          ref2[a] = v;
+          sr.add(v, a);
+        }
+      for (int a = tid; a < n1; a += NT) {
+        const double e = v1[a] * inv;
+        v1[a] = e;
+        q1.add(e, a);
+      }
+      R.reduce(q1, q2, true);
+      if (upd) {
+        R.reduce(sr);
+        if (colfirst) {
+          sb = sr;
+          b_done = true;
         } else {
-          k = max(k - 1, 0);
-          break;
+          sa = sr;
+          a_done = true;
         }
       }
     }
     set_mask(lrow_msk, i);
     set_mask(lcol_msk, j);
+    __syncthreads();
 
     if (i != i_ref) {
-      const double zinv = -pcol[i_ref - 1];
-      axpy_vec(pb_ref, prow, ndt, zinv);
-      rownorm = unrm(pb_ref, ndt);
+      if (!b_done) sb = axpy(pb_ref, prow, ndt, -uniform(pcol[i_ref - 1]));
+      rownorm = R.norm(sb, pb_ref, ndt);
     }
     if (i == i_ref || rownorm < ACA_EPS) {
       if (i == i_ref) ntries_row = ntries_row + 1;
@@ -397,14 +532,15 @@ __global__ __launch_bounds__(kA) void k_aca(const CLeaf *__restrict__ lv,
         rownorm = 0.0;
         i = i_ref;
         while (i != ((i_ref + ndl - 2) % ndl) + 1 && rownorm < za_ACA_EPS && ntries_row > 0) {
-          if (lrow_msk[i - 1] == 0) {
+          if (__builtin_amdgcn_readfirstlane(lrow_msk[i - 1]) == 0) {
             if (k + 1 > cap) {
               st = kAcaOverflow;
               break;
             }
-            calc_vec(L, g, false, k + 1, i, pb_ref, U, V);
-            rownorm = unrm(pb_ref, ndt);
+            sb = calc(false, k + 1, i, pb_ref);
+            rownorm = R.norm(sb, pb_ref, ndt);
             if (rownorm < ACA_EPS) set_mask(lrow_msk, i);
+            __syncthreads();
             ntries_row = ntries_row - 1;
           } else {
             rownorm = 0.0;
@@ -417,9 +553,8 @@ __global__ __launch_bounds__(kA) void k_aca(const CLeaf *__restrict__ lv,
     }
 
     if (j != j_ref) {
-      const double zinv = -prow[j_ref - 1];
-      axpy_vec(pa_ref, pcol, ndl, zinv);
-      colnorm = unrm(pa_ref, ndl);
+      if (!a_done) sa = axpy(pa_ref, pcol, ndl, -uniform(prow[j_ref - 1]));
+      colnorm = R.norm(sa, pa_ref, ndl);
     }
     if (j == j_ref || colnorm < ACA_EPS) {
       if (j == j_ref) ntries_col = ntries_col + 1;
@@ -427,14 +562,15 @@ __global__ __launch_bounds__(kA) void k_aca(const CLeaf *__restrict__ lv,
         colnorm = 0.0;
         j = j_ref;
         while (j != ((j_ref + ndt - 2) % ndt) + 1 && colnorm < za_ACA_EPS && ntries_col > 0) {
-          if (lcol_msk[j - 1] == 0) {
+          if (__builtin_amdgcn_readfirstlane(lcol_msk[j - 1]) == 0) {
             if (k + 1 > cap) {
               st = kAcaOverflow;
               break;
             }
-            calc_vec(L, g, true, k + 1, j, pa_ref, U, V);
-            colnorm = unrm(pa_ref, ndl);
+            sa = calc(true, k + 1, j, pa_ref);
+            colnorm = R.norm(sa, pa_ref, ndl);
             if (colnorm < ACA_EPS) set_mask(lcol_msk, j);
+            __syncthreads();
             ntries_col = ntries_col - 1;
           } else {
             colnorm = 0.0;
@@ -451,7 +587,7 @@ __global__ __launch_bounds__(kA) void k_aca(const CLeaf *__restrict__ lv,
       k = k + 1;
     }
     if (lstop_aca == 0) {
-      const double blknorm = unrm(pcol, ndl) * unrm(prow, ndt);
+      const double blknorm = R.norm(q1, v1, n1) * R.norm(q2, v2, n2);
       if (k == 0) {
         apxnorm = blknorm;
       } else {
@@ -464,10 +600,27 @@ __global__ __launch_bounds__(kA) void k_aca(const CLeaf *__restrict__ lv,
     k = k + 1;
   }
   if (st == kAcaOk && k > cap) st = kAcaOverflow;
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     kt_out[id] = k;
     status[id] = st;
   }
+}
+
+// The kt factor columns of a block (V, then U) from its reserved columns to
+// dst[blockIdx.x], V and U next to each other (null: none to copy); gridDim.y
+// workgroups share a block.
+__global__ __launch_bounds__(1024) void k_pack(const CLeaf *__restrict__ lv,
+                                               const int *__restrict__ kt,
+                                               double *const *__restrict__ dst) {
+  const CLeaf L = lv[blockIdx.x];
+  double *o = dst[blockIdx.x];
+  if (!o) return;
+  const int64_t k = kt[blockIdx.x], nv = k * L.ndt, nu = k * L.ndl;
+  const double *u = L.base + (int64_t)L.ndt * L.cap;
+  const int64_t t0 = blockIdx.y * (int64_t)blockDim.x + threadIdx.x;
+  const int64_t step = (int64_t)gridDim.y * blockDim.x;
+  for (int64_t e = t0; e < nv; e += step) o[e] = L.base[e];
+  for (int64_t e = t0; e < nu; e += step) o[nv + e] = u[e];
 }
 
 // ---- arena fill from device factors ----------------------------------------
@@ -496,15 +649,6 @@ __global__ __launch_bounds__(kT) void k_fill(const HmvFillOp *__restrict__ ops, 
     else
       reinterpret_cast<uint16_t *>(dst)[i] = to_bf16(v);
   }
-}
-
-template <typename T>
-hipError_t upload(T **dst, const T *src, size_t n) {
-  *dst = nullptr;
-  if (n == 0) return hipSuccess;
-  hipError_t e = hipMalloc((void **)dst, sizeof(T) * n);
-  if (e != hipSuccess) return e;
-  return hipMemcpy(*dst, src, sizeof(T) * n, hipMemcpyHostToDevice);
 }
 
 }  // namespace
@@ -538,7 +682,7 @@ hipError_t launch_fill(const FillOps &ops, char *arena) {
 struct hmv_dleaves_s {
   int nd = 0, nlf = 0;
   std::vector<CLeaf> lv;           // host copy of the device leaf table
-  std::vector<int> kt, status;     // per leaf
+  std::vector<int> kt;             // per leaf
   std::vector<hmv::RefLeaf> rec;   // leaf records with device factor pointers
   std::vector<void *> allocs;      // device allocations to free
   double seconds = 0.0;            // device fill time
@@ -555,22 +699,154 @@ hipError_t dalloc(hmv_dleaves_s *d, void **p, size_t bytes) {
   return e;
 }
 
-// Runs ACA+ on the listed low-rank leaves with the capacities in d->lv.
-hipError_t run_aca(hmv_dleaves_s *d, const std::vector<int> &ids, const Geo &g,
-                   const AcaParams &p, int *d_kt, int *d_st, CLeaf *d_lv) {
-  if (ids.empty()) return hipSuccess;
-  int *d_ids = nullptr;
-  hipError_t e = upload(&d_ids, ids.data(), ids.size());
-  if (e == hipSuccess &&
-      (e = hipMemcpy(d_lv, d->lv.data(), sizeof(CLeaf) * d->lv.size(), hipMemcpyHostToDevice)) ==
-          hipSuccess) {
-    hipLaunchKernelGGL(k_aca, dim3((unsigned)ids.size()), dim3(kA), 0, nullptr, d_lv, d_ids, g, p,
+// Threads per block of ACA+, by the longer side: one wave up to kAcaShort
+// entries (at most four per lane: the passes are round trips, and barriers
+// between waves would only add to them), 256 threads up to kAcaLong, else
+// 1024 (at 2,592 rows a block's 256 threads already make 11 trips a pass).
+constexpr int kAcaShort = 256, kAcaLong = 2048;
+
+template <int NT, bool CENT>
+void launch_aca_class(int n, const CLeaf *d_lv, const Geo &g, const AcaParams &p, int *d_kt,
+                      int *d_st) {
+  if (n > 0)
+    hipLaunchKernelGGL((k_aca<NT, CENT>), dim3((unsigned)n), dim3(NT), 0, nullptr, d_lv, g, p,
                        d_kt, d_st);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipDeviceSynchronize();
+}
+// The blocks of one batch, in the order of their classes (n of each).
+template <bool CENT>
+void launch_aca(const int (&n)[3], const CLeaf *d_lv, const Geo &g, const AcaParams &p, int *d_kt,
+                int *d_st) {
+  launch_aca_class<1024, CENT>(n[0], d_lv, g, p, d_kt, d_st);
+  launch_aca_class<256, CENT>(n[1], d_lv + n[0], g, p, d_kt + n[0], d_st + n[0]);
+  launch_aca_class<64, CENT>(n[2], d_lv + n[0] + n[1], g, p, d_kt + n[0] + n[1],
+                             d_st + n[0] + n[1]);
+}
+
+int aca_class(const CLeaf &L) {
+  const int len = std::max(L.ndl, L.ndt);
+  return len > kAcaLong ? 0 : len > kAcaShort ? 1 : 2;
+}
+
+// Runs ACA+ on the listed low-rank leaves (longest first) with at most
+// `columns` factor columns each, in batches; packs their factors into
+// allocations of d, and sets their records' base and cap and d->kt.  `again`
+// receives the leaves that need more columns.
+hipError_t run_aca(hmv_dleaves_s *d, const std::vector<int> &ids, const Geo &g,
+                   const AcaParams &p, int columns, std::vector<int> &again) {
+  if (ids.empty()) return hipSuccess;
+  // the analytic entry is needed with its kernel and on a diagonal
+  bool cent = g.kernel == kKernelCentroid;
+  size_t most = 0, total = 0;  // bytes of the largest block and of all
+  auto cap_of = [&](const CLeaf &L) {
+    return std::min(columns, std::min(p.kmax, std::min(L.ndl, L.ndt)) + 1);
+  };
+  auto bytes_of = [&](const CLeaf &L) {
+    return sizeof(double) * ((size_t)L.ndl + L.ndt) * (size_t)cap_of(L);
+  };
+  for (int i : ids) {
+    const CLeaf &L = d->lv[i];
+    cent = cent && (L.nstrtl + L.ndl <= L.nstrtt || L.nstrtt + L.ndt <= L.nstrtl);
+    most = std::max(most, bytes_of(L));
+    total += bytes_of(L);
   }
-  (void)hipFree(d_ids);
-  return e;
+  const size_t limit = std::min(total, std::max(most, kAcaBatchBytes));
+  // batches [first, last) of ids; the largest one's vectors and blocks
+  std::vector<size_t> ends;
+  size_t used = 0, len = 0, count = 0, len_most = 0, count_most = 0;
+  for (size_t q = 0; q < ids.size(); ++q) {
+    const CLeaf &L = d->lv[ids[q]];
+    if (used > 0 && used + bytes_of(L) > limit) {
+      ends.push_back(q);
+      used = len = count = 0;
+    }
+    used += bytes_of(L);
+    len += (size_t)L.ndl + L.ndt;
+    ++count;
+    len_most = std::max(len_most, len);
+    count_most = std::max(count_most, count);
+  }
+  ends.push_back(ids.size());
+  struct Buf {  // freed on every exit
+    char *p = nullptr;
+    ~Buf() { (void)hipFree(p); }
+  } buf;
+  const size_t o_pa = limit, o_lv = o_pa + sizeof(double) * len_most,
+               o_dst = o_lv + sizeof(CLeaf) * count_most,
+               o_msk = o_dst + sizeof(double *) * count_most,
+               o_kt = o_msk + sizeof(int) * len_most, o_st = o_kt + sizeof(int) * count_most,
+               bytes = o_st + sizeof(int) * count_most;
+  hipError_t e = hipMalloc((void **)&buf.p, bytes);
+  if (e != hipSuccess) return e;
+  CLeaf *d_lv = (CLeaf *)(buf.p + o_lv);
+  double **d_dst = (double **)(buf.p + o_dst);
+  int *d_kt = (int *)(buf.p + o_kt), *d_st = (int *)(buf.p + o_st);
+  std::vector<int> batch;
+  std::vector<CLeaf> lv;
+  std::vector<int> kt, st;
+  std::vector<double *> dst;
+  size_t first = 0;
+  for (size_t last : ends) {
+    batch.clear();
+    lv.clear();
+    int n[3] = {0, 0, 0};
+    size_t o_b = 0, o_v = 0;
+    for (int c = 0; c < 3; ++c)
+      for (size_t q = first; q < last; ++q) {
+        CLeaf L = d->lv[ids[q]];
+        if (aca_class(L) != c) continue;
+        L.cap = cap_of(L);
+        L.base = (double *)(buf.p + o_b);
+        L.pa = (double *)(buf.p + o_pa) + o_v;
+        L.msk = (int *)(buf.p + o_msk) + o_v;
+        o_b += bytes_of(L);
+        o_v += (size_t)L.ndl + L.ndt;
+        batch.push_back(ids[q]);
+        lv.push_back(L);
+        ++n[c];
+      }
+    first = last;
+    const size_t nb = batch.size();
+    kt.resize(nb);
+    st.resize(nb);
+    dst.assign(nb, nullptr);
+    if ((e = hipMemcpy(d_lv, lv.data(), sizeof(CLeaf) * nb, hipMemcpyHostToDevice)) != hipSuccess)
+      return e;
+    if (cent)
+      launch_aca<true>(n, d_lv, g, p, d_kt, d_st);
+    else
+      launch_aca<false>(n, d_lv, g, p, d_kt, d_st);
+    if ((e = hipGetLastError()) != hipSuccess ||
+        (e = hipMemcpy(kt.data(), d_kt, sizeof(int) * nb, hipMemcpyDeviceToHost)) != hipSuccess ||
+        (e = hipMemcpy(st.data(), d_st, sizeof(int) * nb, hipMemcpyDeviceToHost)) != hipSuccess)
+      return e;
+    size_t pool = 0;
+    for (size_t q = 0; q < nb; ++q)
+      if (st[q] == kAcaOk) pool += ((size_t)lv[q].ndl + lv[q].ndt) * (size_t)kt[q];
+    double *d_pool = nullptr;
+    if ((e = dalloc(d, (void **)&d_pool, sizeof(double) * pool)) != hipSuccess) return e;
+    size_t o = 0;
+    for (size_t q = 0; q < nb; ++q) {
+      if (st[q] != kAcaOk) {
+        again.push_back(batch[q]);
+        continue;
+      }
+      CLeaf &L = d->lv[batch[q]];
+      dst[q] = L.base = d_pool + o;
+      L.cap = d->kt[batch[q]] = kt[q];
+      o += ((size_t)L.ndl + L.ndt) * (size_t)kt[q];
+    }
+    if ((e = hipMemcpy(d_dst, dst.data(), sizeof(double *) * nb, hipMemcpyHostToDevice)) !=
+        hipSuccess)
+      return e;
+    // threads per block by its class, as for ACA+
+    const int threads[3] = {1024, 256, 64}, parts[3] = {8, 1, 1};
+    for (int c = 0, at = 0; c < 3; at += n[c++])
+      if (n[c] > 0)
+        hipLaunchKernelGGL(k_pack, dim3((unsigned)n[c], parts[c]), dim3(threads[c]), 0, nullptr,
+                           d_lv + at, d_kt + at, d_dst + at);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  return hipDeviceSynchronize();
 }
 
 }  // namespace
@@ -603,13 +879,15 @@ int hmv_construct(int nnode, const double *nodes, int nface, const int *faces, c
   d->nlf = nlf;
   d->lv.resize(nlf);
   d->kt.assign(nlf, 0);
-  d->status.assign(nlf, 0);
-  std::vector<int> lr_ids, dense_ids;
-  size_t pool = 0, scr = 0, msk = 0;
+  std::vector<int> lr_ids;
+  std::vector<CLeaf> dense;
+  std::vector<int> dense_ids;
+  size_t pool = 0;
   for (int i = 0; i < nlf; ++i) {
     const auto *r = reinterpret_cast<const hmv::RefLeaf *>(static_cast<const char *>(specs) +
                                                           (size_t)stride * i);
     CLeaf &L = d->lv[i];
+    L = CLeaf{};
     L.ltmtx = r->ltmtx;
     L.nstrtl = r->nstrtl;
     L.ndl = r->ndl;
@@ -622,133 +900,73 @@ int hmv_construct(int nnode, const double *nodes, int nface, const int *faces, c
       return HMV_ERR_ARG;
     }
     if (L.ltmtx == 1) {
-      L.cap = std::min(kCapFirst, std::min(cp->kmax, std::min(L.ndl, L.ndt)) + 1);
-      pool += (size_t)(L.ndl + L.ndt) * L.cap;
-      scr += (size_t)(L.ndl + L.ndt);
-      msk += (size_t)(L.ndl + L.ndt);
       lr_ids.push_back(i);
     } else {
-      L.cap = 0;
       pool += (size_t)L.ndl * L.ndt;
       dense_ids.push_back(i);
     }
   }
+  // device copies for the fill: geometry, then the dense leaf list
   hipError_t e;
-  double *d_pool = nullptr, *d_scr = nullptr, *d_geo = nullptr;
-  int *d_msk = nullptr, *d_faces = nullptr, *d_lod = nullptr, *d_kt = nullptr, *d_st = nullptr;
-  CLeaf *d_lv = nullptr;
-  const size_t geo_n = 3 * (size_t)nface + nface + 3 * (size_t)nnode;
+  struct Buf {  // freed on every exit
+    char *p = nullptr;
+    ~Buf() { (void)hipFree(p); }
+  } geo;
+  const size_t o_area = sizeof(double) * 3 * (size_t)nface,
+               o_nodes = o_area + sizeof(double) * (size_t)nface,
+               o_dense = o_nodes + sizeof(double) * 3 * (size_t)nnode,
+               o_faces = o_dense + sizeof(CLeaf) * dense_ids.size(),
+               o_lod = o_faces + sizeof(int) * 3 * (size_t)nface,
+               geo_bytes = o_lod + sizeof(int) * (size_t)nface;
+  double *d_pool = nullptr;
   if ((e = dalloc(d.get(), (void **)&d_pool, sizeof(double) * pool)) != hipSuccess ||
-      (e = hipMalloc((void **)&d_scr, sizeof(double) * std::max<size_t>(scr, 1))) != hipSuccess ||
-      (e = hipMalloc((void **)&d_msk, sizeof(int) * std::max<size_t>(msk, 1))) != hipSuccess ||
-      (e = hipMalloc((void **)&d_geo, sizeof(double) * geo_n)) != hipSuccess ||
-      (e = hipMalloc((void **)&d_faces, sizeof(int) * 3 * (size_t)nface)) != hipSuccess ||
-      (e = hipMalloc((void **)&d_lod, sizeof(int) * (size_t)nface)) != hipSuccess ||
-      (e = hipMalloc((void **)&d_kt, sizeof(int) * std::max(nlf, 1))) != hipSuccess ||
-      (e = hipMalloc((void **)&d_st, sizeof(int) * std::max(nlf, 1))) != hipSuccess ||
-      (e = hipMalloc((void **)&d_lv, sizeof(CLeaf) * std::max(nlf, 1))) != hipSuccess) {
-    (void)hipFree(d_scr);
-    (void)hipFree(d_msk);
-    (void)hipFree(d_geo);
-    (void)hipFree(d_faces);
-    (void)hipFree(d_lod);
-    (void)hipFree(d_kt);
-    (void)hipFree(d_st);
-    (void)hipFree(d_lv);
-    return hmv::hip_fail(e, "hmv_construct: device memory");
-  }
-  struct Tmp {  // freed on every exit
-    std::vector<void *> p;
-    ~Tmp() {
-      for (void *q : p) (void)hipFree(q);
-    }
-  } tmp;
-  tmp.p = {d_scr, d_msk, d_geo, d_faces, d_lod, d_kt, d_st, d_lv};
-  if ((e = hipMemset(d_kt, 0, sizeof(int) * std::max(nlf, 1))) != hipSuccess ||
-      (e = hipMemset(d_st, 0, sizeof(int) * std::max(nlf, 1))) != hipSuccess)
+      (e = hipMalloc((void **)&geo.p, geo_bytes)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_construct: device memory");
   auto t0 = std::chrono::steady_clock::now();
+  dense.reserve(dense_ids.size());
   {
-    size_t po = 0, so = 0, mo = 0;
-    for (CLeaf &L : d->lv) {
+    size_t po = 0;
+    for (int i : dense_ids) {
+      CLeaf &L = d->lv[i];
       L.base = d_pool + po;
-      if (L.ltmtx == 1) {
-        po += (size_t)(L.ndl + L.ndt) * L.cap;
-        L.pa = d_scr + so;
-        L.msk = d_msk + mo;
-        so += (size_t)(L.ndl + L.ndt);
-        mo += (size_t)(L.ndl + L.ndt);
-      } else {
-        po += (size_t)L.ndl * L.ndt;
-        L.pa = nullptr;
-        L.msk = nullptr;
-      }
+      po += (size_t)L.ndl * L.ndt;
+      dense.push_back(L);
     }
   }
-  if ((e = hipMemcpy(d_geo, cent, sizeof(double) * 3 * (size_t)nface, hipMemcpyHostToDevice)) !=
-          hipSuccess ||
-      (e = hipMemcpy(d_geo + 3 * (size_t)nface, area, sizeof(double) * nface,
-                     hipMemcpyHostToDevice)) != hipSuccess ||
-      (e = hipMemcpy(d_geo + 4 * (size_t)nface, nodes, sizeof(double) * 3 * (size_t)nnode,
-                     hipMemcpyHostToDevice)) != hipSuccess ||
-      (e = hipMemcpy(d_faces, faces, sizeof(int) * 3 * (size_t)nface, hipMemcpyHostToDevice)) !=
-          hipSuccess ||
-      (e = hipMemcpy(d_lod, lod, sizeof(int) * (size_t)nface, hipMemcpyHostToDevice)) != hipSuccess ||
-      (e = hipMemcpy(d_lv, d->lv.data(), sizeof(CLeaf) * d->lv.size(), hipMemcpyHostToDevice)) !=
-          hipSuccess)
-    return hmv::hip_fail(e, "hmv_construct: upload");
-  Geo g{d_geo, d_geo + 3 * (size_t)nface, d_geo + 4 * (size_t)nface, d_faces, d_lod, cp->kernel};
+  auto up = [&](size_t at, const void *src, size_t bytes) {
+    if (e == hipSuccess && bytes > 0) e = hipMemcpy(geo.p + at, src, bytes, hipMemcpyHostToDevice);
+  };
+  up(0, cent, sizeof(double) * 3 * (size_t)nface);
+  up(o_area, area, sizeof(double) * (size_t)nface);
+  up(o_nodes, nodes, sizeof(double) * 3 * (size_t)nnode);
+  up(o_dense, dense.data(), sizeof(CLeaf) * dense.size());
+  up(o_faces, faces, sizeof(int) * 3 * (size_t)nface);
+  up(o_lod, lod, sizeof(int) * (size_t)nface);
+  if (e != hipSuccess) return hmv::hip_fail(e, "hmv_construct: upload");
+  Geo g{(double *)geo.p,          (double *)(geo.p + o_area), (double *)(geo.p + o_nodes),
+        (int *)(geo.p + o_faces), (int *)(geo.p + o_lod),     cp->kernel};
   AcaParams ap{cp->aca_eps, cp->aca_eps_factor, cp->kmax, cp->kmin};
   // dense leaves
-  if (!dense_ids.empty()) {
-    int *d_ids = nullptr;
-    if ((e = upload(&d_ids, dense_ids.data(), dense_ids.size())) == hipSuccess) {
-      hipLaunchKernelGGL(k_dense, dim3((unsigned)dense_ids.size()), dim3(kT), 0, nullptr, d_lv,
-                         d_ids, g);
-      e = hipGetLastError();
-      if (e == hipSuccess) e = hipDeviceSynchronize();
-    }
-    (void)hipFree(d_ids);
-    if (e != hipSuccess) return hmv::hip_fail(e, "hmv_construct: dense fill");
+  if (!dense.empty()) {
+    hipLaunchKernelGGL(k_dense, dim3((unsigned)dense.size()), dim3(kT), 0, nullptr,
+                       (const CLeaf *)(geo.p + o_dense), g);
+    if ((e = hipGetLastError()) != hipSuccess)
+      return hmv::hip_fail(e, "hmv_construct: dense fill");
   }
   // low-rank leaves, largest first; then the ones that needed more columns
   std::sort(lr_ids.begin(), lr_ids.end(), [&](int a, int b) {
     const int64_t sa = (int64_t)d->lv[a].ndl + d->lv[a].ndt, sb = (int64_t)d->lv[b].ndl + d->lv[b].ndt;
     return sa != sb ? sa > sb : a < b;
   });
-  if ((e = run_aca(d.get(), lr_ids, g, ap, d_kt, d_st, d_lv)) != hipSuccess ||
-      (e = hipMemcpy(d->kt.data(), d_kt, sizeof(int) * nlf, hipMemcpyDeviceToHost)) != hipSuccess ||
-      (e = hipMemcpy(d->status.data(), d_st, sizeof(int) * nlf, hipMemcpyDeviceToHost)) != hipSuccess)
+  std::vector<int> again, failed;
+  if ((e = run_aca(d.get(), lr_ids, g, ap, first_columns(cp->aca_eps), again)) != hipSuccess ||
+      (e = run_aca(d.get(), again, g, ap, INT_MAX, failed)) != hipSuccess ||
+      (e = hipDeviceSynchronize()) != hipSuccess)  // the dense fill, if nothing followed it
     return hmv::hip_fail(e, "hmv_construct: ACA+");
-  std::vector<int> again;
-  size_t pool2 = 0;
-  for (int i : lr_ids)
-    if (d->status[i] == kAcaOverflow) {
-      CLeaf &L = d->lv[i];
-      L.cap = std::min(cp->kmax, std::min(L.ndl, L.ndt)) + 1;
-      pool2 += (size_t)(L.ndl + L.ndt) * L.cap;
-      again.push_back(i);
-    }
-  if (!again.empty()) {
-    double *d_pool2 = nullptr;
-    if ((e = dalloc(d.get(), (void **)&d_pool2, sizeof(double) * pool2)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_construct: device memory");
-    size_t po = 0;
-    for (int i : again) {
-      d->lv[i].base = d_pool2 + po;
-      po += (size_t)(d->lv[i].ndl + d->lv[i].ndt) * d->lv[i].cap;
-    }
-    if ((e = run_aca(d.get(), again, g, ap, d_kt, d_st, d_lv)) != hipSuccess ||
-        (e = hipMemcpy(d->kt.data(), d_kt, sizeof(int) * nlf, hipMemcpyDeviceToHost)) != hipSuccess ||
-        (e = hipMemcpy(d->status.data(), d_st, sizeof(int) * nlf, hipMemcpyDeviceToHost)) !=
-            hipSuccess)
-      return hmv::hip_fail(e, "hmv_construct: ACA+");
-    for (int i : again)
-      if (d->status[i] != kAcaOk) {
-        hmv::set_error("hmv_construct: ACA+ of leaf " + std::to_string(i + 1) +
-                       " exceeded its rank bound");
-        return HMV_ERR_STATE;
-      }
+  if (!failed.empty()) {
+    hmv::set_error("hmv_construct: ACA+ of leaf " + std::to_string(failed[0] + 1) +
+                   " exceeded its rank bound");
+    return HMV_ERR_STATE;
   }
   auto t1 = std::chrono::steady_clock::now();
   d->seconds = std::chrono::duration<double>(t1 - t0).count();

@@ -116,3 +116,85 @@ def test_arena_from_device_factors(gpu, O, H, tmp_path, prec):
     a.free()
     b.free()
     dev.free()
+
+
+def _construct_blocks(H, nodes, faces, blocks, eps):
+    """hmv_construct on low-rank blocks (first row, rows, first column,
+    columns; 0-based, faces in their own order): [U V^T] per block and the
+    dense matrix's entry function as an array of rows."""
+    import ctypes as C
+    rec = (H.LeafRec * len(blocks))()
+    for r, (l0, ndl, t0, ndt) in zip(rec, blocks):
+        r.ltmtx, r.nstrtl, r.ndl, r.nstrtt, r.ndt = 1, l0 + 1, ndl, t0 + 1, ndt
+    tri = nodes[faces]
+    cent = np.ascontiguousarray((tri[:, 0] + tri[:, 1] + tri[:, 2]) / 3.0)
+    area = 0.5 * np.linalg.norm(np.cross(tri[:, 1] - tri[:, 0], tri[:, 2] - tri[:, 0]), axis=1)
+    lod = np.arange(1, len(faces) + 1, dtype=np.int32)
+    cp = H._ConstructParams(kernel=H.KERNEL["centroid"], kmax=50, kmin=1, aca_eps=eps,
+                            aca_eps_factor=H.baseline_params(aca_eps=eps)["aca_eps_factor"])
+    I = C.POINTER(C.c_int)
+    D = C.POINTER(C.c_double)
+    d = C.c_void_p()
+    L = H.hmv_lib()
+    faces = np.ascontiguousarray(faces, np.int32)
+    assert L.hmv_construct(len(nodes), nodes.ctypes.data_as(D), len(faces), faces.ctypes.data_as(I),
+                           cent.ctypes.data_as(D), np.ascontiguousarray(area).ctypes.data_as(D),
+                           lod.ctypes.data_as(I), len(blocks), C.addressof(rec), C.sizeof(H.LeafRec),
+                           C.byref(cp), C.byref(d)) == 0, L.hmv_last_error()
+    kt = np.zeros(len(blocks), np.int32)
+    assert L.hmv_dleaves_info(d, None, kt.ctypes.data_as(I), None) == 0
+    out = []
+    for i, ((l0, ndl, t0, ndt), k) in enumerate(zip(blocks, kt)):
+        buf = np.zeros((ndl + ndt) * max(int(k), 1))
+        assert L.hmv_dleaves_download(d, i, buf.ctypes.data_as(D)) == 0
+        V, U = buf[:ndt * k].reshape(k, ndt), buf[ndt * k:(ndt + ndl) * k].reshape(k, ndl)
+        diff = cent[l0:l0 + ndl, None] - cent[None, t0:t0 + ndt]
+        with np.errstate(divide="ignore"):
+            A = area[None, t0:t0 + ndt] / (4 * np.pi * np.linalg.norm(diff, axis=2))
+        out.append((U.T @ V, A, int(k)))
+    L.hmv_dleaves_free(d)
+    return out
+
+
+@pytest.mark.parametrize("a,b", [(22, 300), (63, 65), (256, 257), (255, 1000), (2048, 257),
+                                 (2049, 2048), (5120, 4097)])
+def test_aca_workgroup_sizes(gpu, H, a, b):
+    """ACA+ takes 64, 256 or 1024 threads by a block's longer side (up to 256,
+    up to 2048, more).  Two far patches of a and b triangles, whose coupling is
+    one block each way: ranks and factors of all leaves equal the host fill's
+    bit for bit, as above."""
+    n1, f1 = H.icosphere(4)
+    n2, f2 = H.icosphere(4, 1.0, (30.0, 0.0, 0.0))
+    nodes, faces = H.merge((n1, f1[:a]), (n2, f2[:b]))
+    p = H.baseline_params(aca_eps=1e-6)
+    host = H.HMatrix(nodes, faces, p)
+    dev = H.DeviceHMatrix(nodes, faces, p)
+    t = host.leaf_table()
+    assert ((t[:, 0] == 1) & (t[:, 3] == a) & (t[:, 5] == b)).any()
+    assert np.array_equal(dev.table, t)
+    got = dev.download()
+    for (kind, x, _), (_, y, _) in zip(_leaf_values(host, host.lod), _leaf_values(got, host.lod)):
+        if kind == 1:
+            assert np.array_equal(x, y)
+    dev.free()
+
+
+def test_aca_block_on_the_diagonal(gpu, H):
+    """A block that holds diagonal entries evaluates them analytically (the
+    kernel that knows no diagonal is for the other blocks): at full rank
+    U V^T is the block, its diagonal the closed form of the self term."""
+    nodes, faces = H.icosphere(1)
+    n = 24
+    (uv, A, k), = _construct_blocks(H, nodes, faces, [(0, n, 0, n)], 1e-15)
+    tri = nodes[faces[:n]]
+    cent = tri.mean(axis=1)
+    self_term = np.zeros(n)
+    for i in range(3):
+        a, b = tri[:, i] - cent, tri[:, (i + 1) % 3] - cent
+        e = (b - a) / np.linalg.norm(b - a, axis=1)[:, None]
+        ta, tb = (a * e).sum(1), (b * e).sum(1)
+        h = np.linalg.norm(a - ta[:, None] * e, axis=1)
+        self_term += h * np.log((np.linalg.norm(b, axis=1) + tb) / (np.linalg.norm(a, axis=1) + ta))
+    A[np.arange(n), np.arange(n)] = self_term / (4 * np.pi)
+    print("rank", k, "error %.2e" % (np.linalg.norm(uv - A) / np.linalg.norm(A)), flush=True)
+    assert np.linalg.norm(uv - A) / np.linalg.norm(A) < 1e-10
