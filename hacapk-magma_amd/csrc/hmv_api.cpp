@@ -108,7 +108,7 @@ class HostPool {
 };
 
 int ensure_tk(hmv_arena_s *a, int k) {
-  const int64_t need = std::max<int64_t>(1, a->tpart_size) * k;
+  const int64_t need = (std::max<int64_t>(1, a->tpart_size) + a->launch.nyp) * k;
   if (need <= a->tk_cap) return HMV_OK;
   (void)hipFree(a->d_tk);
   a->d_tk = nullptr;
@@ -135,7 +135,8 @@ hipError_t enqueue_apply_block(hmv_arena_s *a, int k, const double *x, double *y
                                const int *skip, hipStream_t s) {
   HmvUnits u;
   fill_units(a, u);
-  return hmv_launch_block(&a->launch, &u, k, x, a->d_tk, y, beta, skip, s);
+  return hmv_launch_block(&a->launch, &u, k, x, a->d_tk,
+                          a->d_tk + std::max<int64_t>(1, a->tpart_size) * k, y, beta, skip, s);
 }
 
 hipError_t enqueue_apply(hmv_arena_s *a, const double *x, double *y, double beta, const int *skip,
@@ -176,6 +177,9 @@ void release(hmv_arena_s *a) {
   (void)hipFree(a->d_arena);
   (void)hipFree(a->d_work1);
   (void)hipFree(a->d_work2);
+  (void)hipFree(a->d_work2x);
+  (void)hipFree(a->d_yfin);
+  (void)hipFree(a->d_yp);
   (void)hipFree(a->d_tfin);
   (void)hipFree(a->d_winst1);
   (void)hipFree(a->d_winst2);
@@ -270,6 +274,15 @@ int first_input(const hmv::Plan &P, const HmvWork &w) {
   return z.kind == HMV_Z_X ? z.src : -1 - z.src;
 }
 
+// First y row of phase-2 item w, which may be a piece of a wide item.
+int first_row(const hmv::WideSplit &ws, const HmvWork &w) {
+  if (w.out_base >= 0) return w.out_base;
+  const int at = -1 - w.out_base;  // yfin's bases ascend
+  auto f = std::upper_bound(ws.yfin.begin(), ws.yfin.end(), at,
+                            [](int v, const HmvYFin &y) { return v < y.base; });
+  return (f - 1)->row;
+}
+
 // H-matmat units of group width tw: (work item, up to tw consecutive
 // 16-row tiles).  The items are sorted by locality (phase 1: first input
 // column; phase 2: first row) and the units cut into G contiguous ranges,
@@ -277,11 +290,12 @@ int first_input(const hmv::Plan &P, const HmvWork &w) {
 // the hardware sends to XCD p % G, runs a unit of range p % G.  Each XCD
 // then walks neighbouring items together, and the k inputs of the columns
 // they share stay in its L2.
-std::vector<int2> matmat_units(const hmv::Plan &P, const std::vector<HmvWork> &wl, bool phase1,
-                               int tw) {
+std::vector<int2> matmat_units(const hmv::Plan &P, const hmv::WideSplit &ws,
+                               const std::vector<HmvWork> &wl, bool phase1, int tw) {
   std::vector<std::pair<int64_t, int>> key(wl.size());
   for (size_t i = 0; i < wl.size(); ++i)
-    key[i] = {phase1 ? (int64_t)first_input(P, wl[i]) : (int64_t)wl[i].out_base, (int)i};
+    key[i] = {phase1 ? (int64_t)first_input(P, wl[i]) : (int64_t)first_row(ws, wl[i]),
+              (int)i};
   std::stable_sort(key.begin(), key.end(),
                    [](const std::pair<int64_t, int> &x, const std::pair<int64_t, int> &y) {
                      return x.first < y.first;
@@ -319,6 +333,14 @@ int upload_plan(hmv::Plan &P, hmv_arena *out, std::chrono::steady_clock::time_po
   a->nwork1 = (int)P.work1.size();
   a->nwork2 = (int)P.work2.size();
   a->ntfin = (int)P.tfin.size();
+  hmv::WideSplit ws;
+  const bool wide = hmv::split_wide(P, ws);
+  const std::vector<HmvWork> &work2 = wide ? ws.work2 : P.work2;  // as launched
+  std::vector<HmvZSeg> zseg_x;  // the plan's input runs with the pieces'
+  if (wide) {
+    zseg_x = P.zseg;
+    zseg_x.insert(zseg_x.end(), ws.zseg.begin(), ws.zseg.end());
+  }
   hipError_t e;
   if ((e = hipMalloc(&a->d_arena, P.arena_size)) != hipSuccess ||
       (e = P.arena ? hipMemcpy(a->d_arena, P.arena.get(), P.arena_size, hipMemcpyHostToDevice)
@@ -327,9 +349,12 @@ int upload_plan(hmv::Plan &P, hmv_arena *out, std::chrono::steady_clock::time_po
       (e = upload(&a->d_work1, P.work1)) != hipSuccess ||
       (e = upload(&a->d_work2, P.work2)) != hipSuccess ||
       (e = upload(&a->d_tfin, P.tfin)) != hipSuccess ||
-      (e = upload(&a->d_zseg, P.zseg)) != hipSuccess ||
+      (e = upload(&a->d_zseg, wide ? zseg_x : P.zseg)) != hipSuccess ||
       (e = upload(&a->d_outidx, P.outidx)) != hipSuccess ||
-      (e = upload(&a->d_codes, P.codes)) != hipSuccess) {
+      (e = upload(&a->d_codes, P.codes)) != hipSuccess ||
+      (e = upload(&a->d_work2x, ws.work2)) != hipSuccess ||
+      (e = upload(&a->d_yfin, ws.yfin)) != hipSuccess ||
+      (wide && (e = hipMalloc((void **)&a->d_yp, sizeof(double) * ws.nyp)) != hipSuccess)) {
     release(a);
     return hip_fail(e, "hmv_arena_build: upload");
   }
@@ -339,9 +364,9 @@ int upload_plan(hmv::Plan &P, hmv_arena *out, std::chrono::steady_clock::time_po
     auto inst_of = [&](int row) {
       return (int)(std::upper_bound(seg->begin(), seg->end(), row) - seg->begin()) - 1;
     };
-    std::vector<int> w1(P.work1.size()), w2(P.work2.size());
+    std::vector<int> w1(P.work1.size()), w2(work2.size());
     for (size_t i = 0; i < P.work1.size(); ++i) w1[i] = inst_of(first_input(P, P.work1[i]));
-    for (size_t i = 0; i < P.work2.size(); ++i) w2[i] = inst_of(P.work2[i].out_base);
+    for (size_t i = 0; i < work2.size(); ++i) w2[i] = inst_of(first_row(ws, work2[i]));
     if ((e = upload(&a->d_winst1, w1)) != hipSuccess ||
         (e = upload(&a->d_winst2, w2)) != hipSuccess) {
       release(a);
@@ -350,7 +375,7 @@ int upload_plan(hmv::Plan &P, hmv_arena *out, std::chrono::steady_clock::time_po
   }
   for (int ph = 0; ph < 2; ++ph)
     for (int w = 0; w < HMV_MM_WIDTHS; ++w) {
-      const std::vector<int2> u = matmat_units(P, ph == 0 ? P.work1 : P.work2, ph == 0, 1 << w);
+      const std::vector<int2> u = matmat_units(P, ws, ph == 0 ? P.work1 : work2, ph == 0, 1 << w);
       a->nunits[ph][w] = (int)u.size();
       if ((e = upload(&a->d_units[ph][w], u)) != hipSuccess) {
         release(a);
@@ -375,9 +400,13 @@ int upload_plan(hmv::Plan &P, hmv_arena *out, std::chrono::steady_clock::time_po
   L.nt1_small = P.nt1_small;
   L.tfin = a->d_tfin;
   L.ntfin = a->ntfin;
-  L.work2 = a->d_work2;
-  L.nwork2 = a->nwork2;
-  L.nwork2_small = P.nwork2_small;
+  L.work2 = wide ? a->d_work2x : a->d_work2;
+  L.nwork2 = (int)work2.size();
+  L.nwork2_small = wide ? ws.nwork2_small : P.nwork2_small;
+  L.yfin = a->d_yfin;
+  L.nyfin = (int)ws.yfin.size();
+  L.nyp = ws.nyp;
+  L.yp = a->d_yp;
   L.nt2_small = P.nt2_small;
   L.zseg = a->d_zseg;
   L.outidx = a->d_outidx;

@@ -45,10 +45,16 @@ struct hmv_arena_s {
   HmvZSeg *d_zseg = nullptr;
   int *d_outidx = nullptr, *d_codes = nullptr;
   double *d_t = nullptr;   // t slots + chunk partials (FP64 in every mode)
+  // phase 2 as it is launched when the plan has wide items: the work list
+  // with those in pieces (its input runs follow the plan's in d_zseg), and
+  // the pieces' partial rows
+  HmvWork *d_work2x = nullptr;
+  HmvYFin *d_yfin = nullptr;
+  double *d_yp = nullptr;
   HmvLaunch launch{};      // device tables of one apply
   int2 *d_units[2][HMV_MM_WIDTHS] = {};  // H-matmat units per phase and tile-group width
   int nunits[2][HMV_MM_WIDTHS] = {};
-  double *d_tk = nullptr;  // t buffer of the H-matmat (tpart_size * k doubles)
+  double *d_tk = nullptr;  // t buffer of the H-matmat ((tpart_size + partial rows) * k doubles)
   int64_t tk_cap = 0;      // its capacity in doubles
   int bt_vec[4] = {1, 1, 1, 1};      // H-matmat path choices (HmvUnits::vec, log_tw)
   int bt_log_tw[4] = {-1, -1, -1, -1};
@@ -112,10 +118,11 @@ extern "C" hipError_t hmv_launch_apply(const HmvLaunch *L, int phases, const dou
 #define HMV_KSTREAM_MAX_F64 8
 #define HMV_KSTREAM_MAX_NARROW 4
 extern "C" hipError_t hmv_launch_kstream(const HmvLaunch *L, int phase, int k, const double *x,
-                                         double *t, double *y, double beta, const int *skip,
-                                         hipStream_t stream);
+                                         double *t, double *yp, double *y, double beta,
+                                         const int *skip, hipStream_t stream);
+// t: tpart_size * k doubles; yp: the arena's partial rows * k doubles.
 extern "C" hipError_t hmv_launch_block(const HmvLaunch *L, const HmvUnits *units, int k,
-                                       const double *x, double *t, double *y, double beta,
-                                       const int *skip, hipStream_t stream);
+                                       const double *x, double *t, double *yp, double *y,
+                                       double beta, const int *skip, hipStream_t stream);
 
 #endif

@@ -66,7 +66,8 @@ struct HmvWork {
   short dt0, dt1;   // HMV_DT_*
   int zseg_begin;   // input sources [zseg_begin, zseg_end), in column order
   int zseg_end;
-  int out_base;     // phase 1: offset into outidx; phase 2: first y row
+  int out_base;     // phase 1: offset into outidx; phase 2: first y row, or
+                    // -1 - first partial row for a piece of a wide item
 };
 
 // t[slot] = t[base] + t[base + 1] + ... + t[base + np - 1]  (np >= 2; the
@@ -78,6 +79,22 @@ struct HmvTFin {
   int pad;
 };
 
+// Rows of a wide phase-2 item whose columns run as np pieces: y[row + r] =
+// sum over p of partial row base + p*rows + r, in piece order.
+struct HmvYFin {
+  int row, rows;
+  int base, np;
+  int inst;  // instance (multi-instance arenas)
+  int pad;
+};
+// Columns of a phase-2 item from which it runs in pieces, the most columns of
+// a piece, and the most partial rows of one arena.  A sphere's items hold up
+// to some 2,100 columns (mean 1,000) and stay whole: the pieces' own launch
+// costs 2 us, more than such an item holds the others up.
+#define HMV_WIDE_COLS 3072
+#define HMV_WIDE_PIECE 1024
+#define HMV_PARTIAL_ROWS 65536
+
 // Everything one apply launches over (device pointers).  Each phase's work
 // list holds its short blocks first (nwork_small of them, run with nt_small
 // threads per workgroup), then the rest (256 threads).
@@ -88,12 +105,15 @@ struct HmvLaunch {
   int nwork1, nwork1_small, nt1_small;
   const struct HmvTFin *tfin;
   int ntfin;
-  const struct HmvWork *work2;
+  const struct HmvWork *work2;  // wide items in pieces
   int nwork2, nwork2_small, nt2_small;
+  const struct HmvYFin *yfin;   // the wide items' rows
+  int nyfin, nyp;               // and their partial rows
   const struct HmvZSeg *zseg;
   const int *outidx;
   const int *codes;
   double *t;
+  double *yp;                   // partial rows of the single-vector product
   const int *winst1, *winst2;  // instance of each work item (multi-instance arenas; else null)
 };
 #define HMV_PHASE1 1  // phase 1 and the chunk-partial sums

@@ -109,7 +109,7 @@ __device__ inline void stream_item(
     const HmvWork &w, Acc *__restrict__ z, int *__restrict__ runs, const char *__restrict__ arena,
     const HmvZSeg *__restrict__ zsegs, const double *__restrict__ x, const int *__restrict__ codes,
     const double *__restrict__ t_in, const int *__restrict__ outidx, double *__restrict__ t_out,
-    double *__restrict__ y, double beta) {
+    double *__restrict__ yp, double *__restrict__ y, double beta) {
   constexpr int ZCH = zchunk<Acc, NT>();
   const int tid = threadIdx.x;
   constexpr int vr = rows_per_lane<PHASE, DT0>();
@@ -173,8 +173,12 @@ __device__ inline void stream_item(
     if constexpr (PHASE == 1) {
       t_out[outidx[w.out_base + r]] = (double)s;
     } else {
-      const int row = w.out_base + r;
       const double v = (double)s;
+      if (w.out_base < 0) {  // a piece of a wide item
+        yp[r - 1 - w.out_base] = v;
+        continue;
+      }
+      const int row = w.out_base + r;
       y[row] = beta == 0.0 ? v : __builtin_fma(beta, y[row], v);
     }
   }
@@ -186,7 +190,7 @@ hmv_stream_kernel(
     const char *__restrict__ arena, const HmvWork *__restrict__ works,
     const HmvZSeg *__restrict__ zsegs, const double *__restrict__ x, const int *__restrict__ codes,
     const double *__restrict__ t_in, const int *__restrict__ outidx, double *__restrict__ t_out,
-    double *__restrict__ y, double beta, const int *__restrict__ skip,
+    double *__restrict__ yp, double *__restrict__ y, double beta, const int *__restrict__ skip,
     const int *__restrict__ winst, const int *__restrict__ inst_done) {
   if (skip && *skip) return;
   // a finished instance of a multi-instance solve needs no more products
@@ -194,7 +198,7 @@ hmv_stream_kernel(
   __shared__ __attribute__((aligned(16))) Acc z[zchunk<Acc, NT>() + 4];
   __shared__ int runs[2 * HMV_RUN_MAX];
   stream_item<Acc, PHASE, DT0, DT1, NT>(works[blockIdx.x], z, runs, arena, zsegs, x, codes, t_in,
-                                        outidx, t_out, y, beta);
+                                        outidx, t_out, yp, y, beta);
 }
 
 // t[slot] = sum of the chunk partials t[base + p], p = 0 .. np-1, in order.
@@ -216,6 +220,24 @@ __global__ __launch_bounds__(HMV_WG_THREADS) void hmv_tfinal_kernel(
   t[f.slot] = s;
 }
 
+// Rows of the wide items: y = sum of the pieces' partial rows in piece order
+// + beta y (one workgroup per item).
+__global__ __launch_bounds__(64) void hmv_yfinal_kernel(const HmvYFin *__restrict__ fin,
+                                                        const double *__restrict__ yp,
+                                                        double *__restrict__ y, double beta,
+                                                        const int *__restrict__ skip,
+                                                        const int *__restrict__ inst_done) {
+  if (skip && *skip) return;
+  const HmvYFin f = fin[blockIdx.x];
+  if (inst_done && inst_done[f.inst]) return;
+  for (int r = threadIdx.x; r < f.rows; r += 64) {
+    const double *p = yp + f.base + r;
+    double s = p[0];
+    for (int q = 1; q < f.np; ++q) s += p[(size_t)q * f.rows];
+    y[f.row + r] = beta == 0.0 ? s : __builtin_fma(beta, y[f.row + r], s);
+  }
+}
+
 template <typename Acc, int PHASE, int DT0, int DT1>
 void launch_list(const HmvLaunch &L, const HmvWork *work, int n, int nsmall, int nt_small,
                  const double *x, double *y, double beta, const int *skip,
@@ -227,17 +249,17 @@ void launch_list(const HmvLaunch &L, const HmvWork *work, int n, int nsmall, int
   if (nsmall > 0) {
     if (nt_small == 64)
       hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1, 64>), dim3(nsmall), dim3(64), 0,
-                         stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, y, beta,
+                         stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, L.yp, y, beta,
                          skip, winst, inst_done);
     else
       hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1, 128>), dim3(nsmall), dim3(128), 0,
-                         stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, y, beta,
+                         stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, L.yp, y, beta,
                          skip, winst, inst_done);
   }
   if (n > nsmall)
     hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1>), dim3(n - nsmall),
                        dim3(HMV_WG_THREADS), 0, stream, L.arena, work + nsmall, L.zseg, x, L.codes,
-                       t_in, L.outidx, t_out, y, beta, skip, winst ? winst + nsmall : nullptr,
+                       t_in, L.outidx, t_out, L.yp, y, beta, skip, winst ? winst + nsmall : nullptr,
                        inst_done);
 }
 
@@ -252,9 +274,13 @@ void launch_mode(const HmvLaunch &L, int phases, const double *x, double *y, dou
       hipLaunchKernelGGL(hmv_tfinal_kernel, dim3((L.ntfin + HMV_WG_THREADS - 1) / HMV_WG_THREADS),
                          dim3(HMV_WG_THREADS), 0, stream, L.tfin, L.ntfin, L.t, skip);
   }
-  if (phases & HMV_PHASE2)
+  if (phases & HMV_PHASE2) {
     launch_list<Acc, 2, DT0, DT1>(L, L.work2, L.nwork2, L.nwork2_small, L.nt2_small, x, y, beta,
                                   skip, inst_done, stream);
+    if (L.nyfin > 0)
+      hipLaunchKernelGGL(hmv_yfinal_kernel, dim3(L.nyfin), dim3(64), 0, stream, L.yfin, L.yp, y,
+                         beta, skip, L.winst2 ? inst_done : nullptr);
+  }
 }
 
 // Plain streaming kernels of known traffic, for bandwidth calibration.

@@ -214,7 +214,8 @@ __device__ inline void kstream_item(const HmvWork &w, Acc *__restrict__ z, int *
                                     const double *__restrict__ x, const int *__restrict__ codes,
                                     const double *__restrict__ t_in,
                                     const int *__restrict__ outidx, double *__restrict__ t_out,
-                                    double *__restrict__ y, int k, double beta) {
+                                    double *__restrict__ yp, double *__restrict__ y, int k,
+                                    double beta) {
   constexpr int vr = rows_per_lane<PHASE, DT0>();
   constexpr int ZC = kcols<Acc, NT, vr, K>();
   const int tid = threadIdx.x;
@@ -281,8 +282,12 @@ __device__ inline void kstream_item(const HmvWork &w, Acc *__restrict__ z, int *
     if constexpr (PHASE == 1) {
       t_out[(size_t)outidx[w.out_base + r] * k + j] = (double)s;
     } else {
-      double *py = y + (size_t)(w.out_base + r) * k + j;
       const double v = (double)s;
+      if (w.out_base < 0) {  // a piece of a wide item
+        yp[(size_t)(r - 1 - w.out_base) * k + j] = v;
+        continue;
+      }
+      double *py = y + (size_t)(w.out_base + r) * k + j;
       *py = beta == 0.0 ? v : __builtin_fma(beta, *py, v);
     }
   }
@@ -298,18 +303,20 @@ hmv_kstream_kernel(const char *__restrict__ arena, const HmvWork *__restrict__ w
                    const HmvZSeg *__restrict__ zsegs, const double *__restrict__ x,
                    const int *__restrict__ codes, const double *__restrict__ t_in,
                    const int *__restrict__ outidx, double *__restrict__ t_out,
-                   double *__restrict__ y, int k, double beta, const int *__restrict__ skip) {
+                   double *__restrict__ yp, double *__restrict__ y, int k, double beta,
+                   const int *__restrict__ skip) {
   if (skip && *skip) return;
   constexpr int vr = rows_per_lane<PHASE, DT0>();
   __shared__ __attribute__((aligned(16))) Acc z[kbuf_elems<Acc, NT, vr, K>()];
   __shared__ int runs[2 * HMV_RUN_MAX];
   kstream_item<Acc, PHASE, DT0, DT1, NT, K, PAIRS>(works[blockIdx.x], z, runs, arena, zsegs, x,
-                                                   codes, t_in, outidx, t_out, y, k, beta);
+                                                   codes, t_in, outidx, t_out, yp, y, k, beta);
 }
 
 template <typename Acc, int PHASE, int DT0, int DT1, int K, bool PAIRS>
 void klaunch_list2(const HmvLaunch &L, const HmvWork *work, int n, int nsmall, int nt_small,
-                   const double *x, double *t, double *y, int k, double beta, const int *skip,
+                   const double *x, double *t, double *yp, double *y, int k, double beta,
+                   const int *skip,
                    hipStream_t s) {
   const double *t_in = PHASE == 2 ? t : nullptr;
   double *t_out = PHASE == 1 ? t : nullptr;
@@ -317,60 +324,61 @@ void klaunch_list2(const HmvLaunch &L, const HmvWork *work, int n, int nsmall, i
     if (nt_small == 64)
       hipLaunchKernelGGL((hmv_kstream_kernel<Acc, PHASE, DT0, DT1, 64, K, PAIRS>), dim3(nsmall),
                          dim3(64), 0, s, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out,
-                         y, k, beta, skip);
+                         yp, y, k, beta, skip);
     else
       hipLaunchKernelGGL((hmv_kstream_kernel<Acc, PHASE, DT0, DT1, 128, K, PAIRS>), dim3(nsmall),
                          dim3(128), 0, s, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out,
-                         y, k, beta, skip);
+                         yp, y, k, beta, skip);
   }
   if (n > nsmall)
     hipLaunchKernelGGL((hmv_kstream_kernel<Acc, PHASE, DT0, DT1, HMV_WG_THREADS, K, PAIRS>),
                        dim3(n - nsmall), dim3(HMV_WG_THREADS), 0, s, L.arena, work + nsmall, L.zseg,
-                       x, L.codes, t_in, L.outidx, t_out, y, k, beta, skip);
+                       x, L.codes, t_in, L.outidx, t_out, yp, y, k, beta, skip);
 }
 
 // Paired staging (kstage_pairs) for the FP64 column-cooperative staging
 // when k is even and x and t are 16-byte aligned.
 template <typename Acc, int PHASE, int DT0, int DT1, int K>
 void klaunch_list(const HmvLaunch &L, const HmvWork *work, int n, int nsmall, int nt_small,
-                  const double *x, double *t, double *y, int k, double beta, const int *skip,
+                  const double *x, double *t, double *yp, double *y, int k, double beta,
+                   const int *skip,
                   hipStream_t s) {
   constexpr int vr = rows_per_lane<PHASE, DT0>();
   if constexpr (sizeof(Acc) == 8 && kstage_batch<Acc, vr, K>() > 0) {
     if (k % 2 == 0 && ((uintptr_t)x | (uintptr_t)t) % 16 == 0) {
-      klaunch_list2<Acc, PHASE, DT0, DT1, K, true>(L, work, n, nsmall, nt_small, x, t, y, k, beta,
+      klaunch_list2<Acc, PHASE, DT0, DT1, K, true>(L, work, n, nsmall, nt_small, x, t, yp, y, k, beta,
                                                    skip, s);
       return;
     }
   }
-  klaunch_list2<Acc, PHASE, DT0, DT1, K, false>(L, work, n, nsmall, nt_small, x, t, y, k, beta,
+  klaunch_list2<Acc, PHASE, DT0, DT1, K, false>(L, work, n, nsmall, nt_small, x, t, yp, y, k, beta,
                                                 skip, s);
 }
 
 template <typename Acc, int DT0, int DT1, int K>
-void klaunch_phase(const HmvLaunch &L, int phase, const double *x, double *t, double *y, int k,
-                   double beta, const int *skip, hipStream_t s) {
+void klaunch_phase(const HmvLaunch &L, int phase, const double *x, double *t, double *yp, double *y,
+                   int k, double beta, const int *skip, hipStream_t s) {
   if (phase == 1)  // phase 1 reads only low-rank factors: both parts use DT1's type
     klaunch_list<Acc, 1, DT1, DT1, K>(L, L.work1, L.nwork1, L.nwork1_small, L.nt1_small, x, t,
-                                      nullptr, k, 0.0, skip, s);
+                                      nullptr, nullptr, k, 0.0, skip, s);
   else
-    klaunch_list<Acc, 2, DT0, DT1, K>(L, L.work2, L.nwork2, L.nwork2_small, L.nt2_small, x, t, y,
-                                      k, beta, skip, s);
+    klaunch_list<Acc, 2, DT0, DT1, K>(L, L.work2, L.nwork2, L.nwork2_small, L.nt2_small, x, t, yp,
+                                      y, k, beta, skip, s);
 }
 
 template <int K>
-void klaunch_mode(const HmvLaunch &L, int phase, const double *x, double *t, double *y, int k,
-                  double beta, const int *skip, hipStream_t s) {
+void klaunch_mode(const HmvLaunch &L, int phase, const double *x, double *t, double *yp, double *y,
+                  int k, double beta, const int *skip, hipStream_t s) {
   if (L.mode == 0)
-    klaunch_phase<double, HMV_DT_F64, HMV_DT_F64, K>(L, phase, x, t, y, k, beta, skip, s);
+    klaunch_phase<double, HMV_DT_F64, HMV_DT_F64, K>(L, phase, x, t, yp, y, k, beta, skip, s);
   else if constexpr (K > HMV_KSTREAM_MAX_NARROW)
     return;  // not instantiated: hmv_launch_kstream rejects these k
   else if (L.mode == 1)
-    klaunch_phase<float, HMV_DT_F32, HMV_DT_F32, K>(L, phase, x, t, y, k, beta, skip, s);
+    klaunch_phase<float, HMV_DT_F32, HMV_DT_F32, K>(L, phase, x, t, yp, y, k, beta, skip, s);
   else if (L.mode == 2)
-    klaunch_phase<float, HMV_DT_F32, HMV_DT_BF16, K>(L, phase, x, t, y, k, beta, skip, s);
+    klaunch_phase<float, HMV_DT_F32, HMV_DT_BF16, K>(L, phase, x, t, yp, y, k, beta, skip, s);
   else
-    klaunch_phase<float, HMV_DT_BF16, HMV_DT_BF16, K>(L, phase, x, t, y, k, beta, skip, s);
+    klaunch_phase<float, HMV_DT_BF16, HMV_DT_BF16, K>(L, phase, x, t, yp, y, k, beta, skip, s);
 }
 
 }  // namespace
@@ -378,17 +386,17 @@ void klaunch_mode(const HmvLaunch &L, int phase, const double *x, double *t, dou
 // One phase (1: t = V^T X into the t buffer; 2: Y = [A|U][X;T] + beta Y) of
 // the H-matmat for 1 <= k <= 8 right-hand sides.
 extern "C" hipError_t hmv_launch_kstream(const HmvLaunch *L, int phase, int k, const double *x,
-                                         double *t, double *y, double beta, const int *skip,
-                                         hipStream_t stream) {
+                                         double *t, double *yp, double *y, double beta,
+                                         const int *skip, hipStream_t stream) {
   if (k < 1 || k > (L->mode == 0 ? HMV_KSTREAM_MAX_F64 : HMV_KSTREAM_MAX_NARROW))
     return hipErrorInvalidValue;
   if (k <= 1)
-    klaunch_mode<1>(*L, phase, x, t, y, k, beta, skip, stream);
+    klaunch_mode<1>(*L, phase, x, t, yp, y, k, beta, skip, stream);
   else if (k <= 2)
-    klaunch_mode<2>(*L, phase, x, t, y, k, beta, skip, stream);
+    klaunch_mode<2>(*L, phase, x, t, yp, y, k, beta, skip, stream);
   else if (k <= 4)
-    klaunch_mode<4>(*L, phase, x, t, y, k, beta, skip, stream);
+    klaunch_mode<4>(*L, phase, x, t, yp, y, k, beta, skip, stream);
   else
-    klaunch_mode<8>(*L, phase, x, t, y, k, beta, skip, stream);
+    klaunch_mode<8>(*L, phase, x, t, yp, y, k, beta, skip, stream);
   return hipGetLastError();
 }

@@ -317,7 +317,8 @@ __global__ __launch_bounds__(64) void hmv_matmat_kernel(
     const char *__restrict__ arena, const HmvWork *__restrict__ works, const int2 *__restrict__ units,
     const HmvZSeg *__restrict__ zsegs, const double *__restrict__ x, const int *__restrict__ codes,
     const double *__restrict__ t_in, const int *__restrict__ outidx, double *__restrict__ t_out,
-    double *__restrict__ y, int k, double beta, const int *__restrict__ skip) {
+    double *__restrict__ yp, double *__restrict__ y, int k, double beta,
+    const int *__restrict__ skip) {
   if (skip && *skip) return;
   static_assert(TW == 1 || TW == 2 || TW == 4, "tiles per unit");
   __shared__ int runs[2 * HMV_RUN_MAX];
@@ -376,6 +377,10 @@ __global__ __launch_bounds__(64) void hmv_matmat_kernel(
         if constexpr (PHASE == 1) {
           t_out[(size_t)outidx[w.out_base + row] * k + j] = v;
         } else {
+          if (w.out_base < 0) {  // a piece of a wide item
+            yp[(size_t)(row - 1 - w.out_base) * k + j] = v;
+            continue;
+          }
           double *py = y + (size_t)(w.out_base + row) * k + j;
           *py = beta == 0.0 ? v : __builtin_fma(beta, *py, v);
         }
@@ -399,10 +404,28 @@ __global__ __launch_bounds__(256) void hmv_tfinal_block_kernel(const HmvTFin *__
   t[(size_t)f.slot * k + j] = s;
 }
 
+// Rows of the wide items: y = sum of the pieces' partial rows in piece order
+// + beta y (one workgroup per item, k columns interleaved).
+__global__ __launch_bounds__(256) void hmv_yfinal_block_kernel(const HmvYFin *__restrict__ fin, int k,
+                                                               const double *__restrict__ yp,
+                                                               double *__restrict__ y, double beta,
+                                                               const int *__restrict__ skip) {
+  if (skip && *skip) return;
+  const HmvYFin f = fin[blockIdx.x];
+  const size_t n = (size_t)f.rows * k;
+  double *py = y + (size_t)f.row * k;
+  for (size_t e = threadIdx.x; e < n; e += 256) {
+    const double *p = yp + (size_t)f.base * k + e;
+    double s = p[0];
+    for (int q = 1; q < f.np; ++q) s += p[(size_t)q * n];
+    py[e] = beta == 0.0 ? s : __builtin_fma(beta, py[e], s);
+  }
+}
+
 template <typename Acc, int PHASE, int DT0, int DT1>
 void launch_units(int kt, const HmvLaunch &L, const HmvUnits &U, const HmvWork *works,
-                  const double *x, double *t, double *y, int k, double beta, const int *skip,
-                  hipStream_t s) {
+                  const double *x, double *t, double *yp, double *y, int k, double beta,
+                  const int *skip, hipStream_t s) {
   const double *t_in = PHASE == 2 ? t : nullptr;
   double *t_out = PHASE == 1 ? t : nullptr;
   // EXACT reads the inputs in 16-byte pairs: x and t must be 16-byte aligned
@@ -411,7 +434,7 @@ void launch_units(int kt, const HmvLaunch &L, const HmvUnits &U, const HmvWork *
 #define HMV_MM_GO(KT, TW, EX)                                                                  \
   hipLaunchKernelGGL((hmv_matmat_kernel<Acc, PHASE, DT0, DT1, KT, TW, EX>), dim3(n), dim3(64), 0, \
                      s, L.arena, works, U.u[PHASE - 1][w], L.zseg, x, L.codes, t_in, L.outidx,      \
-                     t_out, y, k, beta, skip)
+                     t_out, yp, y, k, beta, skip)
 #define HMV_MM_LAUNCH(KT, TW)                                      \
   do {                                                             \
     const int w = TW == 4 ? 2 : TW == 2 ? 1 : 0, n = U.n[PHASE - 1][w]; \
@@ -452,42 +475,45 @@ void launch_units(int kt, const HmvLaunch &L, const HmvUnits &U, const HmvWork *
 
 template <typename Acc, int DT0, int DT1>
 void launch_block(const HmvLaunch &L, const HmvUnits &U, int k, const double *x, double *t,
-                  double *y, double beta, const int *skip, hipStream_t s) {
+                  double *yp, double *y, double beta, const int *skip, hipStream_t s) {
   const int kt = (k + 15) / 16;
   // few right-hand sides stream on the vector units (hmv_kstream.hip) unless
   // the arena's tuning sends their class to MFMA
   const bool vec = k <= (L.mode == 0 ? HMV_KSTREAM_MAX_F64 : HMV_KSTREAM_MAX_NARROW) &&
                    U.vec[k <= 1 ? 0 : k <= 2 ? 1 : k <= 4 ? 2 : 3];
   if (vec)
-    (void)hmv_launch_kstream(&L, 1, k, x, t, nullptr, 0.0, skip, s);
+    (void)hmv_launch_kstream(&L, 1, k, x, t, nullptr, nullptr, 0.0, skip, s);
   else
-    launch_units<Acc, 1, DT1, DT1>(kt, L, U, L.work1, x, t, nullptr, k, 0.0, skip, s);
+    launch_units<Acc, 1, DT1, DT1>(kt, L, U, L.work1, x, t, nullptr, nullptr, k, 0.0, skip, s);
   if (L.ntfin > 0) {
     const int64_t n = (int64_t)L.ntfin * k;
     hipLaunchKernelGGL(hmv_tfinal_block_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
                        L.tfin, L.ntfin, k, t, skip);
   }
   if (vec)
-    (void)hmv_launch_kstream(&L, 2, k, x, t, y, beta, skip, s);
+    (void)hmv_launch_kstream(&L, 2, k, x, t, yp, y, beta, skip, s);
   else
-    launch_units<Acc, 2, DT0, DT1>(kt, L, U, L.work2, x, t, y, k, beta, skip, s);
+    launch_units<Acc, 2, DT0, DT1>(kt, L, U, L.work2, x, t, yp, y, k, beta, skip, s);
+  if (L.nyfin > 0)
+    hipLaunchKernelGGL(hmv_yfinal_block_kernel, dim3(L.nyfin), dim3(256), 0, s, L.yfin, k, yp, y,
+                       beta, skip);
 }
 
 }  // namespace
 
 // Y = H X + beta*Y for k (1..128) interleaved right-hand sides; t holds
-// tpart_size * k doubles.
+// tpart_size * k doubles, yp the partial rows * k.
 extern "C" hipError_t hmv_launch_block(const HmvLaunch *L, const HmvUnits *units, int k,
-                                       const double *x, double *t, double *y, double beta,
-                                       const int *skip, hipStream_t stream) {
+                                       const double *x, double *t, double *yp, double *y,
+                                       double beta, const int *skip, hipStream_t stream) {
   if (L->mode == 0)
-    launch_block<double, HMV_DT_F64, HMV_DT_F64>(*L, *units, k, x, t, y, beta, skip, stream);
+    launch_block<double, HMV_DT_F64, HMV_DT_F64>(*L, *units, k, x, t, yp, y, beta, skip, stream);
   else if (L->mode == 1)
-    launch_block<float, HMV_DT_F32, HMV_DT_F32>(*L, *units, k, x, t, y, beta, skip, stream);
+    launch_block<float, HMV_DT_F32, HMV_DT_F32>(*L, *units, k, x, t, yp, y, beta, skip, stream);
   else if (L->mode == 2)
-    launch_block<float, HMV_DT_F32, HMV_DT_BF16>(*L, *units, k, x, t, y, beta, skip, stream);
+    launch_block<float, HMV_DT_F32, HMV_DT_BF16>(*L, *units, k, x, t, yp, y, beta, skip, stream);
   else
-    launch_block<float, HMV_DT_BF16, HMV_DT_BF16>(*L, *units, k, x, t, y, beta, skip, stream);
+    launch_block<float, HMV_DT_BF16, HMV_DT_BF16>(*L, *units, k, x, t, yp, y, beta, skip, stream);
   return hipGetLastError();
 }
 
@@ -502,7 +528,9 @@ extern "C" hipError_t hmv_launch_block(const HmvLaunch *L, const HmvUnits *units
 // Nothing in it needs clearing between calls: phase 1 writes every t slot
 // and chunk partial that the finalize and phase 2 read.  Calls that overlap
 // on one device share the array and race.
-static __device__ __align__(256) double scratch[HMV_STATIC_SCRATCH_BYTES / sizeof(double)];
+// Behind it, the partial rows of the wide items (at most HMV_PARTIAL_ROWS).
+constexpr size_t kStaticT = HMV_STATIC_SCRATCH_BYTES / sizeof(double);
+static __device__ __align__(256) double scratch[kStaticT + (size_t)HMV_PARTIAL_ROWS * HMV_MAX_RHS];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -564,7 +592,7 @@ extern "C" int hmv_apply_block_static(hmv_arena a, int k, const double *x, doubl
   if (rc) return rc;
   HmvUnits u;
   hmv::fill_units(a, u);
-  e = hmv_launch_block(&a->launch, &u, k, x, t, y, beta, nullptr, (hipStream_t)stream);
+  e = hmv_launch_block(&a->launch, &u, k, x, t, t + kStaticT, y, beta, nullptr, (hipStream_t)stream);
   if (e != hipSuccess) return hmv::hip_fail(e, "hmv_apply_block_static: launch");
   return HMV_OK;
 }

@@ -721,4 +721,72 @@ bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const 
 }
 }  // namespace
 
+bool split_wide(const Plan &P, WideSplit &out) {
+  out = WideSplit();
+  auto pieces = [&](const HmvWork &w) {
+    const int n = w.ncol0 + w.ncol1;
+    return n < HMV_WIDE_COLS ? 1 : (n + HMV_WIDE_PIECE - 1) / HMV_WIDE_PIECE;
+  };
+  // the widest first, as long as their partial rows fit
+  std::vector<int> wide;
+  for (size_t i = 0; i < P.work2.size(); ++i)
+    if (pieces(P.work2[i]) > 1) wide.push_back((int)i);
+  if (wide.empty()) return false;
+  std::stable_sort(wide.begin(), wide.end(), [&](int a, int b) {
+    return P.work2[a].ncol0 + P.work2[a].ncol1 > P.work2[b].ncol0 + P.work2[b].ncol1;
+  });
+  std::vector<int> at(P.work2.size(), -1);  // wide item -> its HmvYFin
+  for (int i : wide) {
+    const HmvWork &w = P.work2[i];
+    const int np = pieces(w);
+    if ((int64_t)out.nyp + (int64_t)np * w.rows > HMV_PARTIAL_ROWS) continue;
+    int inst = 0;
+    while (inst + 2 < (int)P.seg.size() && w.out_base >= P.seg[inst + 1]) ++inst;
+    at[i] = (int)out.yfin.size();
+    out.yfin.push_back(HmvYFin{w.out_base, w.rows, out.nyp, np, inst, 0});
+    out.nyp += np * w.rows;
+  }
+  if (out.yfin.empty()) return false;
+  const int nz = (int)P.zseg.size();
+  auto piece = [&](const HmvWork &w, const HmvYFin &f, int p) {
+    const int n = w.ncol0 + w.ncol1;
+    const int lo = (int)((int64_t)n * p / f.np), hi = (int)((int64_t)n * (p + 1) / f.np);
+    HmvWork o = w;
+    const int lo0 = std::min(lo, w.ncol0), hi0 = std::min(hi, w.ncol0);
+    const int lo1 = std::max(lo - w.ncol0, 0), hi1 = std::max(hi - w.ncol0, 0);
+    o.ncol0 = hi0 - lo0;
+    o.ncol1 = hi1 - lo1;
+    if (w.off0 >= 0) o.off0 = w.off0 + (int64_t)lo0 * w.rows_p * dtype_size(w.dt0);
+    if (w.off1 >= 0) o.off1 = w.off1 + (int64_t)lo1 * w.rows_p * dtype_size(w.dt1);
+    o.out_base = -1 - (f.base + p * w.rows);
+    o.zseg_begin = nz + (int)out.zseg.size();
+    for (int z = w.zseg_begin; z < w.zseg_end; ++z) {
+      const HmvZSeg &s = P.zseg[z];
+      const int a = std::max(lo, s.col), b = std::min(hi, s.col + s.ncols);
+      if (a < b) out.zseg.push_back(HmvZSeg{s.kind, b - a, s.src + (a - s.col), a - lo});
+    }
+    o.zseg_end = nz + (int)out.zseg.size();
+    return o;
+  };
+  // one workgroup class of the list: items in place, further pieces last
+  auto part = [&](size_t b, size_t e) {
+    std::vector<HmvWork> more;
+    for (size_t i = b; i < e; ++i) {
+      const HmvWork &w = P.work2[i];
+      if (at[i] < 0) {
+        out.work2.push_back(w);
+        continue;
+      }
+      const HmvYFin &f = out.yfin[at[i]];
+      out.work2.push_back(piece(w, f, 0));
+      for (int p = 1; p < f.np; ++p) more.push_back(piece(w, f, p));
+    }
+    out.work2.insert(out.work2.end(), more.begin(), more.end());
+  };
+  part(0, P.nwork2_small);
+  out.nwork2_small = (int)out.work2.size();
+  part(P.nwork2_small, P.work2.size());
+  return true;
+}
+
 }  // namespace hmv

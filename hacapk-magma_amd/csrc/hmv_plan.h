@@ -113,6 +113,24 @@ bool build_plan(int nd, int nlf, const void *leaves, int stride, int prec,
 bool build_plan_device(int nd, int nlf, const void *leaves, int stride, int prec,
                        const PlanTuning &tune, Plan &out, std::string &err);
 
+// Phase 2's work list with its wide items (HMV_WIDE_COLS columns or more) in
+// pieces: a workgroup's time is its columns, and a row atom facing a large
+// cluster without an admissible block holds tens of thousands (on two spheres
+// of 20,480 unknowns, one of 1,280: 40,973, where the median is 816; there
+// the 19-column H-matmat took 1,368 us with it whole, 265 us in pieces, and
+// single products of such meshes half their time).  The
+// first piece takes the item's place; the others end the item's workgroup
+// class.  `zseg` receives the pieces' input runs, indexed behind the plan's.
+struct WideSplit {
+  std::vector<HmvWork> work2;
+  int nwork2_small = 0;
+  std::vector<HmvZSeg> zseg;
+  std::vector<HmvYFin> yfin;
+  int nyp = 0;  // partial rows
+};
+// False when there is no wide item (out stays empty).
+bool split_wide(const Plan &P, WideSplit &out);
+
 // Checks every index of a plan against the buffers it addresses (work
 // blocks inside the arena image, input runs, codes and outputs inside x, t
 // and y, partial sums inside t), so that a plan read from a file cannot make
