@@ -54,12 +54,20 @@ __device__ inline void stage(Acc *__restrict__ z, const Inputs &in, int c0, int 
 // z[zb + j*m].  Loads go in batches of U issued together; the last, partial
 // batch gives its missing columns the out-of-range offset (they load zero)
 // and the zero slot z[zmax] as input.
-template <typename Acc, int DT, int VR, int U>
+template <typename Acc, int DT, int VR, int U, bool DEEP>
 __device__ inline void accumulate(__amdgpu_buffer_rsrc_t rs, uint32_t vb, int step, int n,
                                   const Acc *__restrict__ z, int zb, int m, int zmax,
                                   Acc (&a)[VR]) {
   using LN = Lane<DT, VR>;
   int j = 0;
+  if constexpr (DEEP)
+    for (; j + 2 * U <= n; j += 2 * U) {
+      typename LN::raw v[2 * U];
+#pragma unroll
+      for (int k = 0; k < 2 * U; ++k) v[k] = LN::load(rs, vb, (j + k) * step);
+#pragma unroll
+      for (int k = 0; k < 2 * U; ++k) LN::fma(v[k], z[zb + (j + k) * m], a);
+    }
   for (; j + U <= n; j += U) {
     typename LN::raw v[U];
 #pragma unroll
@@ -78,15 +86,17 @@ __device__ inline void accumulate(__amdgpu_buffer_rsrc_t rs, uint32_t vb, int st
 
 // Lane's columns of local range [lo, hi) of a part: local column cg + j*m,
 // j in [ceil((lo-cg)/m), ceil((hi-cg)/m)); zshift maps a local column to its
-// staged slot (slot = local column + zshift).
-template <typename Acc, int DT, int VR>
+// staged slot (slot = local column + zshift).  DEEP: two batches' loads together
+// while two are left.
+template <typename Acc, int DT, int VR, bool DEEP>
 __device__ inline void run_cols(const Part<DT, VR> &P, int lo, int hi, int cg, int m, int zshift,
                                 int zmax, const Acc *__restrict__ z, Acc (&a)[VR]) {
   const int j0 = lo > cg ? (lo - cg + m - 1) / m : 0;
   const int j1 = hi > cg ? (hi - cg + m - 1) / m : 0;
   if (j1 > j0)
-    accumulate<Acc, DT, VR, batch_loads<DT, VR>()>(P.rs, P.voff + (uint32_t)(j0 * P.step), P.step,
-                                                   j1 - j0, z, cg + j0 * m + zshift, m, zmax, a);
+    accumulate<Acc, DT, VR, batch_loads<DT, VR>(), DEEP>(P.rs, P.voff + (uint32_t)(j0 * P.step),
+                                                         P.step, j1 - j0, z,
+                                                         cg + j0 * m + zshift, m, zmax, a);
 }
 
 // PHASE 1: t[outidx[out_base + r]] = row sums.
@@ -104,7 +114,7 @@ constexpr int zchunk() {
   return HMV_ZCHUNK * NT / HMV_WG_THREADS * (sizeof(Acc) == 4 && NT < HMV_WG_THREADS ? 2 : 1);
 }
 
-template <typename Acc, int PHASE, int DT0, int DT1, int NT>
+template <typename Acc, int PHASE, int DT0, int DT1, int NT, bool DEEP>
 __device__ inline void stream_item(
     const HmvWork &w, Acc *__restrict__ z, int *__restrict__ runs, const char *__restrict__ arena,
     const HmvZSeg *__restrict__ zsegs, const double *__restrict__ x, const int *__restrict__ codes,
@@ -149,12 +159,12 @@ __device__ inline void stream_item(
         lo0 = npf == PF ? lo0 : cw;   // a lane with fewer than PF columns here has none left
       }
       const int hi0 = min(c0 + cw, w.ncol0);
-      if (lo0 < hi0) run_cols<Acc, DT0, vr>(P0, lo0, hi0, cg, m, -c0, cw, z, a);
+      if (lo0 < hi0) run_cols<Acc, DT0, vr, DEEP>(P0, lo0, hi0, cg, m, -c0, cw, z, a);
       // an item stored with one type has one part (ncol1 == 0)
       if constexpr (DT0 != DT1) {
         if (w.ncol1 > 0 && c0 + cw > w.ncol0) {
           const Part<DT1, vr> P1(arena + w.off1, w.rows_p, w.ncol1, rq, cg, m);
-          run_cols<Acc, DT1, vr>(P1, max(c0, w.ncol0) - w.ncol0, c0 + cw - w.ncol0, cg, m,
+          run_cols<Acc, DT1, vr, DEEP>(P1, max(c0, w.ncol0) - w.ncol0, c0 + cw - w.ncol0, cg, m,
                                  w.ncol0 - c0, cw, z, a);
         }
       }
@@ -184,7 +194,7 @@ __device__ inline void stream_item(
   }
 }
 
-template <typename Acc, int PHASE, int DT0, int DT1, int NT = HMV_WG_THREADS>
+template <typename Acc, int PHASE, int DT0, int DT1, int NT, bool DEEP>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
 hmv_stream_kernel(
     const char *__restrict__ arena, const HmvWork *__restrict__ works,
@@ -197,7 +207,7 @@ hmv_stream_kernel(
   if (inst_done && inst_done[winst[blockIdx.x]]) return;
   __shared__ __attribute__((aligned(16))) Acc z[zchunk<Acc, NT>() + 4];
   __shared__ int runs[2 * HMV_RUN_MAX];
-  stream_item<Acc, PHASE, DT0, DT1, NT>(works[blockIdx.x], z, runs, arena, zsegs, x, codes, t_in,
+  stream_item<Acc, PHASE, DT0, DT1, NT, DEEP>(works[blockIdx.x], z, runs, arena, zsegs, x, codes, t_in,
                                         outidx, t_out, yp, y, beta);
 }
 
@@ -238,29 +248,53 @@ __global__ __launch_bounds__(64) void hmv_yfinal_kernel(const HmvYFin *__restric
   }
 }
 
+// Launches of kDeepMin to kDeepMax items with 8-byte lane loads take twice the
+// loads per batch (DEEP; the sums keep their order).  With a few workgroups
+// per CU the time is one item's chain of round trips, and eight loads halve
+// it: at 5,120 unknowns (400 items a phase, FP64) a product takes 19.1 us
+// against 21.1, at 20,480 (1,600 items) 40.8 against 45.8.  Below, the lanes
+// have too few columns for a longer batch (1,280 unknowns: 12.1 against
+// 11.0 us); above, the other workgroups cover the trips and the longer
+// batches only delay the ends (81,920: 182.4 against 182.2; 327,680: 1.4%
+// slower).
+constexpr int kDeepMin = 256, kDeepMax = 2560;
+
+template <typename Acc, int PHASE, int DT0, int DT1, int NT>
+void launch_items(const HmvLaunch &L, const HmvWork *work, int n, const int *winst, bool deep,
+                  const double *x, double *y, double beta, const int *skip, const int *inst_done,
+                  hipStream_t stream) {
+  if (n <= 0) return;
+  const double *t_in = PHASE == 2 ? L.t : nullptr;
+  double *t_out = PHASE == 1 ? L.t : nullptr;
+  if constexpr (DT0 == DT1 && DT0 != HMV_DT_BF16) {
+    if (deep) {
+      hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1, NT, true>), dim3(n), dim3(NT), 0,
+                         stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, L.yp, y,
+                         beta, skip, winst, inst_done);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1, NT, false>), dim3(n), dim3(NT), 0,
+                     stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, L.yp, y,
+                     beta, skip, winst, inst_done);
+}
+
 template <typename Acc, int PHASE, int DT0, int DT1>
 void launch_list(const HmvLaunch &L, const HmvWork *work, int n, int nsmall, int nt_small,
                  const double *x, double *y, double beta, const int *skip,
                  const int *inst_done, hipStream_t stream) {
-  const double *t_in = PHASE == 2 ? L.t : nullptr;
-  double *t_out = PHASE == 1 ? L.t : nullptr;
   const int *winst = PHASE == 1 ? L.winst1 : L.winst2;
   if (!winst) inst_done = nullptr;
-  if (nsmall > 0) {
-    if (nt_small == 64)
-      hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1, 64>), dim3(nsmall), dim3(64), 0,
-                         stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, L.yp, y, beta,
-                         skip, winst, inst_done);
-    else
-      hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1, 128>), dim3(nsmall), dim3(128), 0,
-                         stream, L.arena, work, L.zseg, x, L.codes, t_in, L.outidx, t_out, L.yp, y, beta,
-                         skip, winst, inst_done);
-  }
-  if (n > nsmall)
-    hipLaunchKernelGGL((hmv_stream_kernel<Acc, PHASE, DT0, DT1>), dim3(n - nsmall),
-                       dim3(HMV_WG_THREADS), 0, stream, L.arena, work + nsmall, L.zseg, x, L.codes,
-                       t_in, L.outidx, t_out, L.yp, y, beta, skip, winst ? winst + nsmall : nullptr,
-                       inst_done);
+  const bool deep = n >= kDeepMin && n <= kDeepMax;
+  if (nt_small == 64)
+    launch_items<Acc, PHASE, DT0, DT1, 64>(L, work, nsmall, winst, deep, x, y, beta, skip,
+                                           inst_done, stream);
+  else
+    launch_items<Acc, PHASE, DT0, DT1, 128>(L, work, nsmall, winst, deep, x, y, beta, skip,
+                                            inst_done, stream);
+  launch_items<Acc, PHASE, DT0, DT1, HMV_WG_THREADS>(L, work + nsmall, n - nsmall,
+                                                     winst ? winst + nsmall : nullptr, deep, x, y,
+                                                     beta, skip, inst_done, stream);
 }
 
 template <typename Acc, int DT0, int DT1>

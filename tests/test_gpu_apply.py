@@ -283,3 +283,25 @@ def test_calibration_kernels(gpu):
     assert 0 < nbytes / ms_read / 1e6 < 8000 and 0 < 2 * nbytes / ms_copy / 1e6 < 8000
     assert 1.0 < tf < 78.6
 
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16", "bf16_all"])
+@pytest.mark.parametrize("n", [255, 256, 1000, 2560, 2561])
+def test_launches_around_the_longer_batches(gpu, O, prec, n):
+    """Launches of 256 to 2,560 items take longer load batches: n phase-2 items
+    whose lanes hold from one column up to a few more than three batches, and
+    n phase-1 items."""
+    from synthetic_leaves import LeafSet
+    rows, nd = 4, 4 * n + 400
+    lv = []
+    for i in range(n):
+        nc = 1 + (37 * i) % 380
+        lv.append(("dense", rows * i, rows, (11 * i) % (nd - 400), nc, 0))
+        lv.append(("lowrank", rows * i, rows, rows * i, 7, 3))
+    hm = LeafSet(gpu, nd, lv, n)
+    a = gpu.Arena(hm, prec)
+    assert a.stats["nwork_phase1"] == n and a.stats["nwork_phase2"] >= n
+    x = gpu.uniform(3, nd)
+    err = _rel(a.matvec(x), O.adot_body_lfmtx(hm, x))
+    assert err <= {"f64": TOL64, "f32": 1e-5, "bf16": 2e-2, "bf16_all": 2e-2}[prec]
+    a.free()
