@@ -207,9 +207,9 @@ hmv_tuning to_public(const hmv::PlanTuning &t) {
   return o;
 }
 
-// Public tuning (0 = the precision's default) -> plan tuning.
-hmv::PlanTuning from_public(int prec, const hmv_tuning *t) {
-  hmv::PlanTuning p = hmv::default_tuning(prec);
+// Public tuning (0 = the default for the problem's size) -> plan tuning.
+hmv::PlanTuning from_public(const hmv_tuning *t) {
+  hmv::PlanTuning p = hmv::auto_tuning();
   if (!t) return p;
   if (t->p1_target_bytes != 0) p.p1_target_bytes = t->p1_target_bytes;
   if (t->p1_row_tile != 0) p.p1_row_tile = t->p1_row_tile;
@@ -256,7 +256,7 @@ int build_from_device_leaves(int nd, int nlf, const void *leaves, int stride, in
   auto t0 = std::chrono::steady_clock::now();
   hmv::Plan P;
   std::string err;
-  if (!hmv::build_plan_device(nd, nlf, leaves, stride, prec, from_public(prec, tuning), P, err)) {
+  if (!hmv::build_plan_device(nd, nlf, leaves, stride, prec, from_public(tuning), P, err)) {
     set_error("hmv_arena_build_dleaves: " + err);
     return HMV_ERR_ARG;
   }
@@ -526,11 +526,13 @@ int autotune_search(const char *who, int nd, int precision, int reps, Make make,
       (e = hipEventCreate(&e0)) != hipSuccess || (e = hipEventCreate(&e1)) != hipSuccess) {
     rc = hip_fail(e, (std::string(who) + ": setup").c_str());
   }
-  // time per apply of an arena built with t (the arena lives only for the measurement)
-  auto measure = [&](const hmv::PlanTuning &t, double *ms) -> int {
+  // time per apply of an arena built with t (the arena lives only for the
+  // measurement); t's open fields become what the arena was built with
+  auto measure = [&](hmv::PlanTuning &t, double *ms) -> int {
     hmv_arena a = nullptr;
     int r = make(t, &a);
     if (r) return r;
+    t = from_public(&a->tuning);
     hipError_t he = hipSuccess;
     for (int i = 0; i < 2 && he == hipSuccess; ++i) he = hmv::enqueue_apply(a, dx, dy, 0.0, nullptr, s);
     if (he == hipSuccess) he = hipEventRecord(e0, s);
@@ -550,7 +552,7 @@ int autotune_search(const char *who, int nd, int precision, int reps, Make make,
            a.p2_max_rows == b.p2_max_rows && a.p1_small_threads == b.p1_small_threads &&
            a.p2_small_threads == b.p2_small_threads;
   };
-  hmv::PlanTuning cur = hmv::default_tuning(precision);
+  hmv::PlanTuning cur = hmv::auto_tuning();
   double cur_ms = 0.0;
   if (!rc) rc = measure(cur, &cur_ms);
   if (!rc && default_ms) *default_ms = cur_ms;
@@ -570,7 +572,8 @@ int autotune_search(const char *who, int nd, int precision, int reps, Make make,
   };
   search([](hmv::PlanTuning &t, int64_t v) { t.p1_small_threads = (int)v; }, {-1, 64, 128});
   search([](hmv::PlanTuning &t, int64_t v) { t.p2_small_threads = (int)v; }, {-1, 64, 128});
-  search([](hmv::PlanTuning &t, int64_t v) { t.p1_target_bytes = v; }, {48 << 10, 96 << 10, 192 << 10});
+  search([](hmv::PlanTuning &t, int64_t v) { t.p1_target_bytes = v; },
+         {32 << 10, 48 << 10, 96 << 10, 192 << 10});
   search([](hmv::PlanTuning &t, int64_t v) { t.p2_max_rows = (int)v; }, {128, 256});
   search([](hmv::PlanTuning &t, int64_t v) { t.p1_row_tile = (int)v; }, {128, 256});
   if (e1) (void)hipEventDestroy(e1);
@@ -603,7 +606,7 @@ int hmv_init(int device) {
 
 int hmv_arena_build(int nd, int nlf, const void *leaves, int leaf_stride, int precision,
                     hmv_arena *out) {
-  int rc = build(nd, nlf, leaves, leaf_stride, precision, from_public(precision, nullptr), out);
+  int rc = build(nd, nlf, leaves, leaf_stride, precision, from_public(nullptr), out);
   if (!rc) (*out)->seg = {0, nd};
   return rc;
 }
@@ -620,7 +623,7 @@ int hmv_arena_build_multi(int ninst, const int *nd, const int *nlf, const void *
   if (!concat_instances("hmv_arena_build_multi", ninst, nd, nlf, leaves, leaf_stride, seg, all))
     return HMV_ERR_ARG;
   return build(seg[ninst], (int)all.size(), all.data(), (int)sizeof(hmv::RefLeaf), precision,
-               from_public(precision, tuning), out, &seg);
+               from_public(tuning), out, &seg);
 }
 
 int hmv_arena_segments(hmv_arena a, int *offsets, int cap) {
@@ -645,7 +648,7 @@ int hmv_default_tuning(int precision, hmv_tuning *t) {
 
 int hmv_arena_build_tuned(int nd, int nlf, const void *leaves, int leaf_stride, int precision,
                           const hmv_tuning *tuning, hmv_arena *out) {
-  int rc = build(nd, nlf, leaves, leaf_stride, precision, from_public(precision, tuning), out);
+  int rc = build(nd, nlf, leaves, leaf_stride, precision, from_public(tuning), out);
   if (!rc) (*out)->seg = {0, nd};
   return rc;
 }
@@ -1055,7 +1058,7 @@ int hmv_plan_create_tuned(int nd, int nlf, const void *leaves, int leaf_stride, 
   *out = nullptr;
   hmv_plan p = new hmv_plan_s();
   std::string err;
-  if (!hmv::build_plan(nd, nlf, leaves, leaf_stride, precision, from_public(precision, tuning),
+  if (!hmv::build_plan(nd, nlf, leaves, leaf_stride, precision, from_public(tuning),
                        p->P, err)) {
     delete p;
     set_error("hmv_plan_create: " + err);

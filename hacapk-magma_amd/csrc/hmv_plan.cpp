@@ -86,6 +86,13 @@ PlanTuning default_tuning(int prec) {
   return t;
 }
 
+PlanTuning auto_tuning() {
+  PlanTuning t;
+  t.p1_target_bytes = 0;
+  t.p1_small_threads = t.p2_small_threads = 0;
+  return t;
+}
+
 namespace {
 bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const PlanTuning &tune,
                Plan &P, std::string &err, bool device);
@@ -102,10 +109,31 @@ bool build_plan_device(int nd, int nlf, const void *leaves, int stride, int prec
 }
 
 namespace {
-bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const PlanTuning &tune,
+// Phase-1 bytes per workgroup of a problem whose V factors take `bytes`: 512
+// workgroups or more (two per CU), each of 32 to 96 KiB.  FP64 products: 5,120
+// unknowns (12 MB of V) 26.9 us at 96 KiB and 20.8 at 32; 20,480 (70 MB) 46.7
+// and 48.6.  All-BF16, 25,597 unknowns (22 MB): 31.9 and 25.4.
+int64_t target_bytes(int64_t bytes) {
+  return std::min<int64_t>(96 << 10, std::max<int64_t>(32 << 10, bytes / 512));
+}
+
+// Small workgroups for a phase's short blocks (nt threads, the precision's
+// default) once its items fill the chip's wave slots twice over; before that
+// they only lengthen each item's chain.  BF16 products with 128 threads in
+// phase 1 and 64 in phase 2, against 256 in both: 81,920 unknowns (6,340 and
+// 5,674 items) 110 and 76 us, 163,840 (12,840 and 11,348) 151 and 147,
+// 327,680 (26,152 and 22,855) 272 and 286.
+int small_threads(int nt, size_t items) {
+  constexpr int kWaveSlots = 256 * 32;  // 256 CUs
+  return nt > 0 && items < (size_t)(2 * kWaveSlots / (nt / 64)) ? -1 : nt;
+}
+
+bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const PlanTuning &tuning,
                Plan &P, std::string &err, bool device) {
   P = Plan();
-  auto nt_ok = [](int v) { return v == -1 || v == 64 || v == 128; };
+  PlanTuning tune = tuning;  // fields at 0 are chosen as the sizes become known
+  const PlanTuning large = default_tuning(prec);
+  auto nt_ok = [](int v) { return v == -1 || v == 0 || v == 64 || v == 128; };
   if (!nt_ok(tune.p1_small_threads) || !nt_ok(tune.p2_small_threads)) {
     err = "invalid tuning: small-workgroup threads must be -1, 64 or 128";
     return false;
@@ -120,11 +148,6 @@ bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const 
   };
   P.nd = nd;
   P.prec = prec;
-  P.tune.p1_target_bytes = tune.p1_target_bytes;
-  P.tune.p1_row_tile = tune.p1_row_tile;
-  P.tune.p2_max_rows = tune.p2_max_rows;
-  P.tune.p1_small_threads = tune.p1_small_threads;
-  P.tune.p2_small_threads = tune.p2_small_threads;
   P.seg = {0, nd};
   if (nd <= 0) {
     err = "nd must be positive";
@@ -142,7 +165,7 @@ bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const 
     err = "unknown precision";
     return false;
   }
-  if (tune.p1_target_bytes < 1024 || tune.p1_row_tile < 1 || tune.p1_row_tile > HMV_MAX_ROWS ||
+  if ((tune.p1_target_bytes != 0 && tune.p1_target_bytes < 1024) || tune.p1_row_tile < 1 || tune.p1_row_tile > HMV_MAX_ROWS ||
       tune.p2_max_rows < 1 || tune.p2_max_rows > HMV_MAX_ROWS) {
     err = "invalid tuning parameters";
     return false;
@@ -252,6 +275,11 @@ bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const 
       cg[c].lr.push_back(i);
       cg[c].r += l->kt;
     }
+  }
+  if (tune.p1_target_bytes == 0) {
+    int64_t v = 0;
+    for (const ColGroup &g : cg) v += (int64_t)g.r * g.n * es_l;
+    tune.p1_target_bytes = target_bytes(v);
   }
   st.row_groups = (int64_t)rg.size();
   st.col_groups = (int64_t)cg.size();
@@ -714,6 +742,15 @@ bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const 
     }
     order(items, out);
   };
+  if (tune.p1_small_threads == 0)
+    tune.p1_small_threads = small_threads(large.p1_small_threads, it1.size());
+  if (tune.p2_small_threads == 0)
+    tune.p2_small_threads = small_threads(large.p2_small_threads, it2.size());
+  P.tune.p1_target_bytes = tune.p1_target_bytes;
+  P.tune.p1_row_tile = tune.p1_row_tile;
+  P.tune.p2_max_rows = tune.p2_max_rows;
+  P.tune.p1_small_threads = tune.p1_small_threads;
+  P.tune.p2_small_threads = tune.p2_small_threads;
   order_split(it1, tune.p1_small_threads, vr, P.work1, P.nwork1_small, P.nt1_small);
   order_split(it2, tune.p2_small_threads, vr2, P.work2, P.nwork2_small, P.nt2_small);
   lap("order");

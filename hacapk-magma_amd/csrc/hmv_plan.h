@@ -100,9 +100,13 @@ struct PlanTuning {
   int p2_small_threads = -1;            // same for phase 2; -1: off
   int xcd_groups = 8;                   // dispatcher round-robin width (XCDs)
 };
-// Defaults of a storage precision (measured on MI355X: the narrow types
-// gain from more, smaller workgroups on short blocks; FP64 does not).
+// Defaults of a storage precision for large problems (measured on MI355X: the
+// narrow types gain from more, smaller workgroups on short blocks; FP64 does
+// not).
 PlanTuning default_tuning(int prec);
+// Fields left to the plan (0): phase-1 bytes and small-workgroup threads by
+// the problem's size, the others at their defaults.
+PlanTuning auto_tuning();
 
 // Builds the plan.  `leaves` points at nlf records spaced `stride` bytes.
 // Returns false and fills `err` on invalid input.

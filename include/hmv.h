@@ -87,7 +87,9 @@ int hmv_arena_build(int nd, int nlf, const void *leaves, int leaf_stride, int pr
                     hmv_arena *out);
 
 /* Repack tunables for hmv_arena_build_tuned (used by the autotuner); 0 in a
- * field = the precision's default (96 KiB, 256, 256, and per precision).
+ * field = the default: 256 and 256 rows; 32 to 96 KiB by the problem's size;
+ * small workgroups as the precision's once the problem's blocks fill the chip
+ * twice over, else -1.
  *   p1_target_bytes   arena bytes per phase-1 workgroup (rank-vector rows x columns)
  *   p1_row_tile       most rank vectors per phase-1 workgroup
  *   p2_max_rows       most rows per phase-2 workgroup
@@ -102,7 +104,8 @@ typedef struct {
   int p1_small_threads;
   int p2_small_threads;
 } hmv_tuning;
-/* Defaults of a precision (what hmv_arena_build uses). */
+/* Defaults of a precision for large problems (what hmv_arena_build uses from
+ * some 330,000 unknowns on; smaller ones: hmv_arena_tuning_get). */
 int hmv_default_tuning(int precision, hmv_tuning *t);
 int hmv_arena_build_tuned(int nd, int nlf, const void *leaves, int leaf_stride, int precision,
                           const hmv_tuning *tuning, hmv_arena *out);

@@ -136,3 +136,24 @@ def test_plan_rejects_bad_input(H, sphere3):
         H.plan_tables(sphere3, "f64", {"p1_small_threads": 96})
     with pytest.raises(H.HmvError, match="tuning"):
         H.plan_tables(sphere3, "f64", {"p2_max_rows": 1000})
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16", "bf16_all"])
+def test_small_problems_take_more_and_whole_workgroups(H, O, sphere4, prec):
+    """Without a tuning, phase-1 blocks hold 32 KiB on a small problem (not 96)
+    and no block runs in a small workgroup; the emulated apply equals the
+    oracle.  Given values hold at every size."""
+    T = H.plan_tables(sphere4, prec)
+    assert T["nt1_small"] == 0 and T["nt2_small"] == 0
+    es = {"f64": 8, "f32": 4}.get(prec, 2)
+    w = T["work1"]
+    one_row = w["ncol0"] * es  # a rank vector longer than the target is a block by itself
+    assert np.all((w["rows"] * one_row <= 32 << 10) | (w["rows"] <= 16))
+    x = H.uniform(6, sphere4.nd)
+    _, y = PE.run(T, x, sphere4.nd)
+    y_ref = O.adot_body_lfmtx(sphere4, x)
+    assert np.linalg.norm(y - y_ref) / np.linalg.norm(y_ref) < TOL[prec]
+    G = H.plan_tables(sphere4, prec, H.default_tuning(prec))
+    g = G["work1"]
+    assert (g["rows"] * g["ncol0"] * es).max() > 32 << 10
+    assert G["nt1_small"] == max(0, H.default_tuning(prec)["p1_small_threads"])
