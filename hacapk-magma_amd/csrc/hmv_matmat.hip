@@ -4,7 +4,8 @@
 // N x k row-major); t likewise (slot s's k values at t[s*k]).  The apply runs
 // over the same arena and work lists as the single-vector kernel, one wave
 // (64 threads) per unit: a work item and a group of up to TW of its 16-row
-// tiles.
+// tiles.  Launches of few units give each NW waves, which take the unit's
+// column groups in turn and add their accumulators in wave order at the end.
 //
 // The wave walks the item's columns four at a time.  Per column quad, one
 // 8-byte (or 4/2-byte) load per lane and tile gives the 16 x 4 A fragment
@@ -184,7 +185,7 @@ __device__ inline void load_group(Group<DT, KT, NT, U> &g, __amdgpu_buffer_rsrc_
                                  uint32_t r_es, int q0, const BSrc &src, int k,
                                  const BLane<KT> &bl) {
   using E = Entry<DT>;
-  const int cq = threadIdx.x >> 4;
+  const int cq = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int col = q0 + 4 * u + cq;
@@ -226,11 +227,12 @@ __device__ inline void mma_group(typename Mfma<Acc>::acc (&acc)[TW][KT],
 
 // Tables the input pointers of part columns [w0, w1) (item columns cbase +
 // ...) at tbl[0 ..), and zeros for the kPad entries that follow.
+template <int NW>
 __device__ inline void fill_window(gdouble **__restrict__ tbl, const Inputs &in,
                                    const int *__restrict__ codes, int cbase, int w0, int w1,
                                    const double *__restrict__ x, const double *__restrict__ t,
                                    int k) {
-  for (int i = (int)threadIdx.x; i < w1 - w0 + kPad; i += 64) {
+  for (int i = (int)threadIdx.x; i < w1 - w0 + kPad; i += 64 * NW) {
     const double *p = g_zero_inputs;
     if (i < w1 - w0) {
       const int code = input_code(in, codes, cbase + w0 + i);
@@ -240,16 +242,22 @@ __device__ inline void fill_window(gdouble **__restrict__ tbl, const Inputs &in,
   }
 }
 
-// Multiplies part columns [lo, hi) into the accumulators, U quads at a
-// time, the next group's loads in flight while the current one multiplies.
-template <typename Acc, bool EXACT, bool RUN, int DT, int KT, int TW, int NT>
+// Multiplies this wave's groups of part columns [lo, hi) into the
+// accumulators (U quads a group, every NW-th group of the workgroup's NW
+// waves), the next group's loads in flight while the current one multiplies.
+template <typename Acc, bool EXACT, bool RUN, int DT, int KT, int TW, int NT, int NW>
 __device__ inline void run_columns(typename Mfma<Acc>::acc (&acc)[TW][KT],
                                    __amdgpu_buffer_rsrc_t rs, uint32_t cs, uint32_t r_es, int lo,
                                    int hi, const BSrc &src, int k, const BLane<KT> &bl) {
   constexpr int U = group_quads<KT, NT>();
-  constexpr int S = 4 * U;  // columns per group
-  static_assert(S <= kPad, "a group past the window reads zero entries");
+  constexpr int SG = 4 * U;   // columns per group
+  constexpr int S = SG * NW;  // columns between a wave's groups
+  static_assert(SG <= kPad, "a group past the window reads zero entries");
   Group<DT, KT, NT, U> g0, g1;
+  if constexpr (NW > 1) {
+    lo += SG * (int)(threadIdx.x >> 6);
+    if (lo >= hi) return;
+  }
   load_group<EXACT, RUN>(g0, rs, cs, r_es, lo, src, k, bl);
   int q0 = lo;
   for (; q0 + 2 * S < hi; q0 += 2 * S) {  // g0 holds group q0; two more follow
@@ -268,7 +276,7 @@ __device__ inline void run_columns(typename Mfma<Acc>::acc (&acc)[TW][KT],
 // with DT at rs, item columns cbase + [0, ncolp)).  Inputs of one x run
 // (phase 1) are addressed directly; otherwise kWin columns at a time, the
 // window's input pointers tabled in LDS first.
-template <typename Acc, bool EXACT, bool RUN, int DT, int KT, int TW, int NT>
+template <typename Acc, bool EXACT, bool RUN, int DT, int KT, int TW, int NT, int NW>
 __device__ inline void part_mma(typename Mfma<Acc>::acc (&acc)[TW][KT], __amdgpu_buffer_rsrc_t rs,
                                 int rows_p, int tile0, int ncolp, int cbase, const Inputs &in,
                                 const int *__restrict__ codes, gdouble **__restrict__ tbl,
@@ -280,15 +288,15 @@ __device__ inline void part_mma(typename Mfma<Acc>::acc (&acc)[TW][KT], __amdgpu
   if constexpr (RUN) {
     const BSrc src{nullptr, 0, (gdouble *)(x + (size_t)(in.z0.src + cbase) * k) + bl.jl,
                    (gdouble *)g_zero_inputs + bl.jl, ncolp};
-    run_columns<Acc, EXACT, true, DT, KT, TW, NT>(acc, rs, cs, r_es, 0, ncolp, src, k, bl);
+    run_columns<Acc, EXACT, true, DT, KT, TW, NT, NW>(acc, rs, cs, r_es, 0, ncolp, src, k, bl);
   } else {
     for (int w0 = 0; w0 < ncolp; w0 += kWin) {
       const int w1 = min(ncolp, w0 + kWin);
       __syncthreads();  // the table's previous contents are read
-      fill_window(tbl, in, codes, cbase, w0, w1, x, t, k);
+      fill_window<NW>(tbl, in, codes, cbase, w0, w1, x, t, k);
       __syncthreads();
       const BSrc src{tbl, w0, nullptr, nullptr, w1};
-      run_columns<Acc, EXACT, false, DT, KT, TW, NT>(acc, rs, cs, r_es, w0, w1, src, k, bl);
+      run_columns<Acc, EXACT, false, DT, KT, TW, NT, NW>(acc, rs, cs, r_es, w0, w1, src, k, bl);
     }
   }
 }
@@ -296,24 +304,24 @@ __device__ inline void part_mma(typename Mfma<Acc>::acc (&acc)[TW][KT], __amdgpu
 // Both parts of the item for NT tiles (the unit's tile count, fixed at
 // compile time so that the accumulators stay in place); an item stored
 // with one type has one part.
-template <typename Acc, bool EXACT, bool RUN, int DT0, int DT1, int KT, int TW, int NT>
+template <typename Acc, bool EXACT, bool RUN, int DT0, int DT1, int KT, int TW, int NT, int NW>
 __device__ inline void unit_mma(typename Mfma<Acc>::acc (&acc)[TW][KT], const HmvWork &w,
                                 __amdgpu_buffer_rsrc_t rs0, __amdgpu_buffer_rsrc_t rs1, int tile0,
                                 const Inputs &in, const int *__restrict__ codes,
                                 gdouble **__restrict__ tbl, const double *__restrict__ x,
                                 const double *__restrict__ t, int k, const BLane<KT> &bl) {
-  part_mma<Acc, EXACT, RUN, DT0, KT, TW, NT>(acc, rs0, w.rows_p, tile0, w.ncol0, 0, in, codes,
+  part_mma<Acc, EXACT, RUN, DT0, KT, TW, NT, NW>(acc, rs0, w.rows_p, tile0, w.ncol0, 0, in, codes,
                                              tbl, x, t, k, bl);
   if constexpr (DT0 != DT1)
-    part_mma<Acc, EXACT, RUN, DT1, KT, TW, NT>(acc, rs1, w.rows_p, tile0, w.ncol1, w.ncol0, in,
+    part_mma<Acc, EXACT, RUN, DT1, KT, TW, NT, NW>(acc, rs1, w.rows_p, tile0, w.ncol1, w.ncol0, in,
                                                codes, tbl, x, t, k, bl);
 }
 
-// One wave per unit {item, tile0 << 8 | nt}: tiles tile0 .. tile0+nt-1 of
+// NW waves per unit {item, tile0 << 8 | nt}: tiles tile0 .. tile0+nt-1 of
 // the item.  PHASE 1: t[outidx[out_base + row] * k + j];  PHASE 2:
 // y[(out_base + row) * k + j].
-template <typename Acc, int PHASE, int DT0, int DT1, int KT, int TW, bool EXACT>
-__global__ __launch_bounds__(64) void hmv_matmat_kernel(
+template <typename Acc, int PHASE, int DT0, int DT1, int KT, int TW, bool EXACT, int NW>
+__global__ __launch_bounds__(64 * NW) void hmv_matmat_kernel(
     const char *__restrict__ arena, const HmvWork *__restrict__ works, const int2 *__restrict__ units,
     const HmvZSeg *__restrict__ zsegs, const double *__restrict__ x, const int *__restrict__ codes,
     const double *__restrict__ t_in, const int *__restrict__ outidx, double *__restrict__ t_out,
@@ -326,13 +334,13 @@ __global__ __launch_bounds__(64) void hmv_matmat_kernel(
   const int2 unit = units[blockIdx.x];
   const HmvWork w = works[unit.x];
   const int tile0 = unit.y >> 8, nt = unit.y & 255;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   BLane<KT> bl;
   bl.j0 = lane & 15;
   bl.jl = bcol<KT>(0, bl.j0);
 #pragma unroll
   for (int tt = 0; tt < KT; ++tt) bl.jd[tt] = min(bcol<KT>(tt, bl.j0), k - 1) - bl.jl;
-  const Inputs in = load_inputs<64>(w, zsegs, runs);
+  const Inputs in = load_inputs<64 * NW>(w, zsegs, runs);
   const __amdgpu_buffer_rsrc_t rs0 =
       rsrc(arena + w.off0, (uint32_t)((size_t)w.rows_p * w.ncol0 * Entry<DT0>::es));
   const __amdgpu_buffer_rsrc_t rs1 =
@@ -344,21 +352,39 @@ __global__ __launch_bounds__(64) void hmv_matmat_kernel(
 #pragma unroll
     for (int tt = 0; tt < KT; ++tt) acc[m][tt] = typename Mfma<Acc>::acc{0, 0, 0, 0};
   if (nt >= TW)
-    unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, TW>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in, k,
+    unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, TW, NW>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in, k,
                                                bl);
   else if constexpr (TW == 2)
-    unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 1>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in, k,
+    unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 1, NW>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in, k,
                                               bl);
   else if constexpr (TW == 4) {
     if (nt == 1)
-      unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 1>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in,
+      unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 1, NW>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in,
                                                 k, bl);
     else if (nt == 2)
-      unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 2>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in,
+      unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 2, NW>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in,
                                                 k, bl);
     else
-      unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 3>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in,
+      unit_mma<Acc, EXACT, PHASE == 1, DT0, DT1, KT, TW, 3, NW>(acc, w, rs0, rs1, tile0, in, codes, tbl, x, t_in,
                                                 k, bl);
+  }
+  if constexpr (NW > 1) {
+    // the waves' accumulators, summed in wave order by wave 0
+    __shared__ typename Mfma<Acc>::acc sums[NW - 1][64];
+    const int wv = threadIdx.x >> 6;
+#pragma unroll
+    for (int m = 0; m < TW; ++m) {
+      if (m >= nt) continue;
+#pragma unroll
+      for (int tt = 0; tt < KT; ++tt) {
+        __syncthreads();  // the previous tile's sums are read
+        if (wv > 0) sums[wv - 1][lane] = acc[m][tt];
+        __syncthreads();
+        if (wv == 0)
+          for (int q = 0; q < NW - 1; ++q) acc[m][tt] += sums[q][lane];
+      }
+    }
+    if (wv > 0) return;
   }
   // lane holds rows Mfma::row(lane, i), column lane%16 of each 16 x 16 tile
   const int j0 = lane & 15;
@@ -422,6 +448,21 @@ __global__ __launch_bounds__(256) void hmv_yfinal_block_kernel(const HmvYFin *__
   }
 }
 
+// Up to this many units (two fills of the chip at four waves per SIMD), a
+// unit's columns are shared by several waves: one wave per unit leaves SIMDs
+// idle or with a lone last unit, and a unit's time is its column groups' round
+// trips.  Phase 2 (some 1,000 columns an item): four waves; 5,120 unknowns (356
+// units), k = 16 / 32 / 128: 29 / 34 / 65 -> 16 / 22 / 38 us; 42,235 (3,113),
+// k = 19 / 40: 136 / 232 -> 116 / 200 us; 81,920 (5,674), k = 32: 266 -> 230 us.
+// At 327,680 (22,855 units) k = 16 loses 10% and k = 32 gains 1%: one wave.
+// Phase 1 (median 50 to 80 columns): two; 42,235 unknowns (7,876 units) 101 ->
+// 90 and 189 -> 161 us; from 12,756 units on 3% faster to 19% slower.
+constexpr int kFewUnits = 8192;
+template <int PHASE>
+constexpr int few_waves() {
+  return PHASE == 1 ? 2 : 4;
+}
+
 template <typename Acc, int PHASE, int DT0, int DT1>
 void launch_units(int kt, const HmvLaunch &L, const HmvUnits &U, const HmvWork *works,
                   const double *x, double *t, double *yp, double *y, int k, double beta,
@@ -431,18 +472,23 @@ void launch_units(int kt, const HmvLaunch &L, const HmvUnits &U, const HmvWork *
   // EXACT reads the inputs in 16-byte pairs: x and t must be 16-byte aligned
   // (a caller's x may start anywhere; t is allocated by the engine)
   const bool exact = ((uintptr_t)x % 16 == 0) && ((uintptr_t)t % 16 == 0);
-#define HMV_MM_GO(KT, TW, EX)                                                                  \
-  hipLaunchKernelGGL((hmv_matmat_kernel<Acc, PHASE, DT0, DT1, KT, TW, EX>), dim3(n), dim3(64), 0, \
-                     s, L.arena, works, U.u[PHASE - 1][w], L.zseg, x, L.codes, t_in, L.outidx,      \
-                     t_out, yp, y, k, beta, skip)
+#define HMV_MM_GO(KT, TW, EX, NW)                                                              \
+  hipLaunchKernelGGL((hmv_matmat_kernel<Acc, PHASE, DT0, DT1, KT, TW, EX, NW>), dim3(n),       \
+                     dim3(64 * NW), 0, s, L.arena, works, U.u[PHASE - 1][w], L.zseg, x, L.codes, \
+                     t_in, L.outidx, t_out, yp, y, k, beta, skip)
 #define HMV_MM_LAUNCH(KT, TW)                                      \
   do {                                                             \
     const int w = TW == 4 ? 2 : TW == 2 ? 1 : 0, n = U.n[PHASE - 1][w]; \
+    const bool few = n <= kFewUnits, ex = exact && k == 16 * KT;   \
     if (n > 0) {                                                   \
-      if (exact && k == 16 * KT)                                   \
-        HMV_MM_GO(KT, TW, true);                                   \
+      if (few && ex)                                               \
+        HMV_MM_GO(KT, TW, true, few_waves<PHASE>());               \
+      else if (few)                                                \
+        HMV_MM_GO(KT, TW, false, few_waves<PHASE>());              \
+      else if (ex)                                                 \
+        HMV_MM_GO(KT, TW, true, 1);                                \
       else                                                         \
-        HMV_MM_GO(KT, TW, false);                                  \
+        HMV_MM_GO(KT, TW, false, 1);                               \
     }                                                              \
   } while (0)
   // tiles per unit: the tuned choice of the KT class when it is one of the

@@ -214,3 +214,32 @@ def test_block_refinement(gpu, O, sphere4, prec, inner):
         assert _rel(U[:, j], u1) < bound
     a64.free()
     alow.free()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16", "bf16_all"])
+@pytest.mark.parametrize("k", [9, 16, 32, 40, 64, 128])
+def test_matmat_waves_sharing_a_unit(gpu, O, prec, k):
+    """Launches of few units share each unit's columns among several waves:
+    blocks from one column to a few past two windows of 1,024, and of one to
+    several 16-row tiles, against the oracle."""
+    from synthetic_leaves import LeafSet
+    nd = 5000
+    cols = [1, 3, 4, 15, 16, 17, 31, 33, 63, 64, 65, 127, 129, 255, 500, 1023, 1024, 1025, 1040,
+            1088, 2047, 2048, 2049, 2113]
+    lv, r = [], 0
+    for i, nc in enumerate(cols):
+        rows = [1, 15, 16, 17, 33, 48, 70][i % 7]
+        lv.append(("dense", r, rows, 7 * i, nc, 0))
+        if i % 3 == 0:
+            lv.append(("lowrank", r, rows, 100 + i, 10 + 40 * i, 1 + i))
+        r += rows
+    hm = LeafSet(gpu, nd, lv, 4)
+    a = gpu.Arena(hm, prec)
+    X = np.stack([gpu.uniform(60 + j, nd) for j in range(k)], axis=1)
+    Y = a.matmat(X)
+    tol = {"f64": 1e-12, "f32": 1e-5, "bf16": 2e-2, "bf16_all": 2e-2}[prec]
+    for j in sorted({0, k // 2, k - 1}):
+        ref = O.adot_body_lfmtx(hm, X[:, j])
+        assert np.linalg.norm(Y[:, j] - ref) / np.linalg.norm(ref) <= tol
+    assert np.array_equal(a.matmat(X), Y)
+    a.free()
