@@ -202,12 +202,18 @@ hmv_stream_kernel(
     const double *__restrict__ t_in, const int *__restrict__ outidx, double *__restrict__ t_out,
     double *__restrict__ yp, double *__restrict__ y, double beta, const int *__restrict__ skip,
     const int *__restrict__ winst, const int *__restrict__ inst_done) {
-  if (skip && *skip) return;
+  // the flag and the work record are read together, one round trip instead of
+  // two (also the record's own start without a flag): 1,280 unknowns 11.5 ->
+  // 11.0 us a product, 20,480 42.0 -> 41.1 us
+  const int stop = skip ? *skip : 0;
+  const HmvWork w = works[blockIdx.x];
+  asm volatile("" : : "s"(stop), "s"(w.off0), "s"(w.rows), "s"(w.ncol0), "s"(w.zseg_begin));
+  if (stop) return;
   // a finished instance of a multi-instance solve needs no more products
   if (inst_done && inst_done[winst[blockIdx.x]]) return;
   __shared__ __attribute__((aligned(16))) Acc z[zchunk<Acc, NT>() + 4];
   __shared__ int runs[2 * HMV_RUN_MAX];
-  stream_item<Acc, PHASE, DT0, DT1, NT, DEEP>(works[blockIdx.x], z, runs, arena, zsegs, x, codes, t_in,
+  stream_item<Acc, PHASE, DT0, DT1, NT, DEEP>(w, z, runs, arena, zsegs, x, codes, t_in,
                                         outidx, t_out, yp, y, beta);
 }
 
