@@ -590,7 +590,7 @@ extern "C" int hmv_block_bicgstab_ir(hmv_arena a64, hmv_arena alow, int k, const
 // vector kernels run over a table of blocks that never cross a segment
 // (block b covers [beg, end) of segment seg), so a block reads its
 // instance's scalars once and its dot partials belong to one instance; the
-// partials of an instance are summed in block order.
+// partials of an instance are summed in a fixed order.
 
 namespace {
 
@@ -629,8 +629,16 @@ __global__ __launch_bounds__(kT) void ks_dots(const SegBlock *__restrict__ tb,
   }
 }
 
-// One thread per instance: its blocks [bstart[s], bstart[s+1]) summed in order.
-__global__ __launch_bounds__(kT) void ks_final(int nseg, const int *__restrict__ bstart,
+// Sum over the group of `lanes` consecutive lanes (a power of two <= 64),
+// every lane of which is active: a fixed tree, the same in each lane.
+__device__ inline double group_sum(double v, int lanes) {
+  for (int off = lanes / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// `lanes` threads per instance sum its blocks [bstart[s], bstart[s+1]) in a
+// fixed order; the first of them takes the instance's step.
+__global__ __launch_bounds__(kT) void ks_final(int nseg, int lanes, const int *__restrict__ bstart,
                                                const double *__restrict__ part,
                                                ColState *__restrict__ cs, BlockState *bs,
                                                int stage, int *__restrict__ done_flags) {
@@ -638,12 +646,17 @@ __global__ __launch_bounds__(kT) void ks_final(int nseg, const int *__restrict__
   __shared__ int sdone;
   if (threadIdx.x == 0) sdone = 1;
   __syncthreads();
-  for (int s = threadIdx.x; s < nseg; s += kT) {
+  const int sub = threadIdx.x & (lanes - 1);
+  for (int s = threadIdx.x / lanes; s < nseg; s += kT / lanes) {
     double d0 = 0.0, d1 = 0.0;
-    for (int b = bstart[s]; b < bstart[s + 1]; ++b) {
+    const int b1 = bstart[s + 1];
+    for (int b = bstart[s] + sub; b < b1; b += lanes) {
       d0 += part[2 * b];
       d1 += part[2 * b + 1];
     }
+    d0 = group_sum(d0, lanes);
+    d1 = group_sum(d1, lanes);
+    if (sub != 0) continue;
     ColState c = cs[s];
     col_step(c, d0, d1, bs, stage);
     cs[s] = c;
@@ -715,6 +728,7 @@ __global__ __launch_bounds__(kT) void ks_update_ur(
 
 struct SegWork {
   int nseg = 0, nblk = 0;
+  int lanes = 1;  // threads that sum the blocks of one instance
   int64_t n = 0;
   hipStream_t s = nullptr;
   SegBlock *tb = nullptr;
@@ -771,34 +785,43 @@ hipError_t seg_iteration(hmv_arena_s *a, SegWork &w, double *u) {
   hipLaunchKernelGGL(ks_dots, dim3(nb), dim3(kT), 0, w.s, w.tb, w.rhat, w.v,
                      (const double *)nullptr, (const double *)nullptr, w.part,
                      (const BlockState *)w.bs);
-  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.bstart, w.part, w.cs, w.bs, 1,
+  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 1,
                      w.flags);
   hipLaunchKernelGGL(ks_update_t, dim3(nb), dim3(kT), 0, w.s, w.tb, w.r, w.v, w.t, w.cs, w.bs);
   if ((e = hmv::enqueue_apply(a, w.t, w.sv, 0.0, skip, w.s, w.flags)) != hipSuccess) return e;
   hipLaunchKernelGGL(ks_dots, dim3(nb), dim3(kT), 0, w.s, w.tb, w.sv, w.t, w.sv, w.sv, w.part,
                      (const BlockState *)w.bs);
-  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.bstart, w.part, w.cs, w.bs, 2,
+  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 2,
                      w.flags);
   hipLaunchKernelGGL(ks_update_ur, dim3(nb), dim3(kT), 0, w.s, w.tb, w.p, w.t, w.sv, w.rhat, u,
                      w.r, w.part, w.cs, w.bs);
-  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.bstart, w.part, w.cs, w.bs, 3,
+  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 3,
                      w.flags);
   return hipGetLastError();
 }
 
 // Tables and buffers of the per-instance solver over arena a's segments:
-// a block table whose blocks hold at most 16 elements per thread and never
-// cross an instance; bstart[s] = first block of instance s.
+// a block table whose blocks never cross an instance; bstart[s] = first block
+// of instance s.  A block holds one element per thread until that fills the
+// chip eight times over (kSegBlocks), then up to 16.  The vector passes are
+// bound by latency: at 16 elements per thread, 8 instances of 320 to 20,480
+// unknowns are 19 blocks on 256 CUs, and a direction update over 30 slots
+// took 37 us; in 232 blocks their whole solve takes 11.5 ms instead of 18.3.  An
+// instance's partials are summed by one lane for each 4 blocks.
 int seg_setup(hmv_arena_s *a, SegWork &w, std::vector<int> &bstart, const char *who) {
   w.nseg = (int)a->seg.size() - 1;
   w.n = a->nd;
-  constexpr int kChunk = 16 * kT;
+  constexpr int kSegBlocks = 2048;
+  const int64_t per = (w.n + (int64_t)kT * kSegBlocks - 1) / ((int64_t)kT * kSegBlocks);
+  const int chunk = kT * (int)std::clamp<int64_t>(per, 1, 16);
   std::vector<SegBlock> tb;
   bstart.assign(w.nseg + 1, 0);
   for (int sgi = 0; sgi < w.nseg; ++sgi) {
     bstart[sgi] = (int)tb.size();
-    for (int i = a->seg[sgi]; i < a->seg[sgi + 1]; i += kChunk)
-      tb.push_back(SegBlock{sgi, i, std::min(a->seg[sgi + 1], i + kChunk), 0});
+    const int end = a->seg[sgi + 1];
+    for (int64_t i = a->seg[sgi]; i < end; i += chunk)
+      tb.push_back(SegBlock{sgi, (int)i, (int)std::min<int64_t>(end, i + chunk), 0});
+    while (w.lanes < 64 && 4 * w.lanes < (int)tb.size() - bstart[sgi]) w.lanes *= 2;
   }
   bstart[w.nseg] = (int)tb.size();
   w.nblk = (int)tb.size();
@@ -850,7 +873,7 @@ int seg_solve(hmv_arena_s *a, SegWork &w, const double *b, double *u, double eps
   hipLaunchKernelGGL(kb_init, dim3(g), dim3(kT), 0, w.s, w.n, b, w.r, w.rhat, w.p, w.v);
   hipLaunchKernelGGL(ks_dots, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, w.r, w.r, b, b, w.part,
                      (const BlockState *)nullptr);
-  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.bstart, w.part, w.cs, w.bs, 0,
+  hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 0,
                      w.flags);
   if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
     return hmv::hip_fail(e, (name + ": setup").c_str());
@@ -1125,15 +1148,6 @@ struct SgGlobal {
   int step, ik, ikn, m, maxit, all_done, pad;
 };
 
-// Fixed-order sum over the blocks [b0, b1) of part[stride * b + off]: thread
-// t takes blocks b0 + t, b0 + t + kT, ..., then the block sum.
-__device__ inline double inst_sum(const double *__restrict__ part, int b0, int b1, int stride,
-                                  int off, double *sh) {
-  double s = 0.0;
-  for (int b = b0 + (int)threadIdx.x; b < b1; b += kT) s += part[(size_t)stride * b + off];
-  return blk_sum(s, sh);
-}
-
 // r = b, p_0 = b (zero initial guess)
 __global__ __launch_bounds__(kT) void sg_init(int64_t n, const double *__restrict__ b,
                                               double *__restrict__ r, double *__restrict__ p) {
@@ -1183,8 +1197,18 @@ __global__ __launch_bounds__(kT) void sg_update_ur(const SegBlock *__restrict__ 
   const int s = B.seg;
   if (inst[s].done) return;  // the stage-2 pass skips stopped instances
   const int b0 = bstart[s], b1 = bstart[s + 1];
-  const double d0 = inst_sum(apart, b0, b1, 2, 0, sh), d1 = inst_sum(apart, b0, b1, 2, 1, sh);
   const int ik = gs->ikn;  // the slot of this step
+  const double *pk = p + (size_t)ik * n, *q = ap + (size_t)ik * n;
+  // the first elements are under way while the partials are summed
+  int i = B.beg + threadIdx.x;
+  const int i0 = min(i, B.end - 1);
+  double uv = u[i0], pv = pk[i0], rv = r[i0], qv = q[i0];
+  double t0 = 0.0, t1 = 0.0;
+  for (int b = b0 + (int)threadIdx.x; b < b1; b += kT) {
+    t0 += apart[2 * (size_t)b];
+    t1 += apart[2 * (size_t)b + 1];
+  }
+  const double d0 = blk_sum(t0, sh), d1 = blk_sum(t1, sh);
   const double alpha = d0 / d1;
   const bool bad = d1 == 0.0 || !isfinite(alpha);
   if ((int)blockIdx.x == b0 && threadIdx.x == 0) {
@@ -1196,13 +1220,19 @@ __global__ __launch_bounds__(kT) void sg_update_ur(const SegBlock *__restrict__ 
     }
   }
   if (bad) return;
-  const double *pk = p + (size_t)ik * n, *q = ap + (size_t)ik * n;
   double s2 = 0.0;
-  for (int i = B.beg + threadIdx.x; i < B.end; i += kT) {
-    u[i] = u[i] + alpha * pk[i];
-    const double ri = r[i] - alpha * q[i];
+  while (i < B.end) {
+    const double ri = rv - alpha * qv;
+    u[i] = uv + alpha * pv;
     r[i] = ri;
     s2 = __builtin_fma(ri, ri, s2);
+    i += kT;
+    if (i < B.end) {
+      uv = u[i];
+      pv = pk[i];
+      rv = r[i];
+      qv = q[i];
+    }
   }
   const double r0 = blk_sum(s2, sh);
   if (threadIdx.x == 0) rpart[blockIdx.x] = r0;
@@ -1242,15 +1272,33 @@ __global__ __launch_bounds__(kT) void sg_dots_beta(const SegBlock *__restrict__ 
   }
 }
 
-// Per-instance scalar stages, one thread per instance (its blocks summed in
-// block order):
+// beta_l = -(A p_l, A r) / capap_l for the slots l <= ik of the running
+// instances: `lanes` threads per instance and slot sum the instance's blocks
+// in a fixed order.
+__global__ __launch_bounds__(kT) void sg_betas(int nseg, int lanes,
+                                               const int *__restrict__ bstart,
+                                               const double *__restrict__ part, SgInst *inst,
+                                               const SgGlobal *gs) {
+  if (gs->all_done) return;
+  const int nl = gs->ik + 1, e = (int)((blockIdx.x * kT + threadIdx.x) / lanes);
+  if (e >= nseg * nl) return;
+  const int s = e / nl, l = e % nl, sub = threadIdx.x & (lanes - 1);
+  const double cap = inst[s].capap[l];
+  const bool done = inst[s].done;
+  double v = 0.0;
+  const int b1 = bstart[s + 1];
+  for (int b = bstart[s] + sub; b < b1; b += lanes) v += part[(size_t)b * kGcrM + l];
+  v = group_sum(v, lanes);
+  if (sub == 0 && !done) inst[s].beta[l] = -v / cap;
+}
+
+// Per-instance scalar stages, `lanes` threads per instance summing its blocks
+// in a fixed order:
 //   0: setup from the (r, r), (b, b) pairs;
 //   2: ||r|| from the (r, r) partials, the step and stopping tests, then the
-//      common slots (ik = the slot just used, ikn = the next one);
-//   3: beta_l = -(A p_l, A r) / capap_l for l <= ik (one thread per
-//      instance and slot).
+//      common slots (ik = the slot just used, ikn = the next one).
 // done_flags mirrors each instance's done flag for the H-matvec.
-__global__ __launch_bounds__(kT) void sg_final(int nseg, const int *__restrict__ bstart,
+__global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *__restrict__ bstart,
                                                const double *__restrict__ part, SgInst *inst,
                                                SgGlobal *gs, int stage,
                                                int *__restrict__ done_flags) {
@@ -1258,25 +1306,19 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, const int *__restrict__
   __shared__ int sdone;
   if (threadIdx.x == 0) sdone = 1;
   __syncthreads();
-  if (stage == 3) {
-    const int ik = gs->ik;
-    for (int e = threadIdx.x; e < nseg * (ik + 1); e += kT) {
-      const int s = e / (ik + 1), l = e % (ik + 1);
-      if (inst[s].done) continue;
-      double v = 0.0;
-      for (int b = bstart[s]; b < bstart[s + 1]; ++b) v += part[(size_t)b * kGcrM + l];
-      inst[s].beta[l] = -v / inst[s].capap[l];
-    }
-    return;
-  }
-  for (int s = threadIdx.x; s < nseg; s += kT) {
+  const int sub = threadIdx.x & (lanes - 1), np = stage == 0 ? 2 : 1;
+  for (int s = threadIdx.x / lanes; s < nseg; s += kT / lanes) {
     SgInst &c = inst[s];
+    double d0 = 0.0, d1 = 0.0;
+    const int b1 = bstart[s + 1];
+    for (int b = bstart[s] + sub; b < b1; b += lanes) {
+      d0 += part[(size_t)np * b];
+      if (stage == 0) d1 += part[2 * (size_t)b + 1];
+    }
+    d0 = group_sum(d0, lanes);
+    d1 = group_sum(d1, lanes);
+    if (sub != 0) continue;
     if (stage == 0) {
-      double d0 = 0.0, d1 = 0.0;
-      for (int b = bstart[s]; b < bstart[s + 1]; ++b) {
-        d0 += part[2 * b];
-        d1 += part[2 * b + 1];
-      }
       c.rnorm = sqrt(d0);
       c.bnorm = sqrt(d1);
       c.alpha = 0.0;
@@ -1293,8 +1335,6 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, const int *__restrict__
         c.done = 1;
       }
     } else if (!c.done) {
-      double d0 = 0.0;
-      for (int b = bstart[s]; b < bstart[s + 1]; ++b) d0 += part[b];
       c.step += 1;
       c.rnorm = sqrt(d0);
       if (!isfinite(c.rnorm)) {
@@ -1328,7 +1368,9 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, const int *__restrict__
 
 // p_ikn = c0 r + sum_{l <= ik, l != ikn} beta_l p_l and ap_ikn likewise with
 // ar (c0 = 1 + beta_ikn when the slot is reused, else 1), per instance, and
-// the next step's alpha partials (ap_ikn, r), (ap_ikn, ap_ikn).
+// the next step's alpha partials (ap_ikn, r), (ap_ikn, ap_ikn).  An element's
+// slots are loaded kDir at a time (one at a time is a chain of m loads).
+constexpr int kDir = 8;
 __global__ __launch_bounds__(kT) void sg_update_dir(const SegBlock *__restrict__ tb, int64_t n,
                                                     const double *__restrict__ r,
                                                     const double *__restrict__ ar,
@@ -1349,11 +1391,21 @@ __global__ __launch_bounds__(kT) void sg_update_dir(const SegBlock *__restrict__
   for (int i = B.beg + threadIdx.x; i < B.end; i += kT) {
     const double ri = r[i];
     double pv = c0 * ri, av = c0 * ar[i];
-    for (int l = 0; l <= ik; ++l) {
-      if (l == ikn) continue;
-      const double bl = c.beta[l];
-      pv = __builtin_fma(bl, p[(size_t)l * n + i], pv);
-      av = __builtin_fma(bl, ap[(size_t)l * n + i], av);
+    for (int l0 = 0; l0 <= ik; l0 += kDir) {
+      double pl[kDir], al[kDir];
+#pragma unroll
+      for (int j = 0; j < kDir; ++j) {
+        const size_t at = (size_t)min(l0 + j, ik) * n + i;
+        pl[j] = p[at];
+        al[j] = ap[at];
+      }
+#pragma unroll
+      for (int j = 0; j < kDir; ++j) {
+        if (l0 + j > ik || l0 + j == ikn) continue;
+        const double bl = c.beta[l0 + j];
+        pv = __builtin_fma(bl, pl[j], pv);
+        av = __builtin_fma(bl, al[j], av);
+      }
     }
     pn[i] = pv;
     apn[i] = av;
@@ -1405,14 +1457,15 @@ hipError_t sg_iteration(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, double
   double *rpart = gw.part + 2 * (size_t)nb;
   hipLaunchKernelGGL(sg_update_ur, dim3(nb), dim3(kT), 0, w.s, w.tb, w.bstart, w.n, gw.p, gw.ap,
                      u, gw.r, (const double *)gw.part, rpart, gw.inst, (const SgGlobal *)gw.gs);
-  hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.bstart, (const double *)rpart,
-                     gw.inst, gw.gs, 2, w.flags);
+  hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
+                     (const double *)rpart, gw.inst, gw.gs, 2, w.flags);
   hipError_t e = hmv::enqueue_apply(a, gw.r, gw.ar, 0.0, skip, w.s, w.flags);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(sg_dots_beta, dim3(nb, (gw.m + kGroup - 1) / kGroup), dim3(kT), 0, w.s, w.tb,
                      w.n, gw.ap, gw.ar, gw.part, (const SgInst *)gw.inst, (const SgGlobal *)gw.gs);
-  hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.bstart, (const double *)gw.part,
-                     gw.inst, gw.gs, 3, w.flags);
+  const int nbeta = (int)(((int64_t)w.nseg * gw.m * w.lanes + kT - 1) / kT);
+  hipLaunchKernelGGL(sg_betas, dim3(nbeta), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
+                     (const double *)gw.part, gw.inst, (const SgGlobal *)gw.gs);
   hipLaunchKernelGGL(sg_update_dir, dim3(nb), dim3(kT), 0, w.s, w.tb, w.n, gw.r, gw.ar, gw.p,
                      gw.ap, gw.part, (const SgInst *)gw.inst, (const SgGlobal *)gw.gs);
   return hipGetLastError();
@@ -1436,7 +1489,7 @@ int sg_solve(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, const double *b, 
   hipLaunchKernelGGL(sg_init, dim3(g), dim3(kT), 0, w.s, w.n, b, gw.r, gw.p);
   hipLaunchKernelGGL(ks_dots, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, gw.r, gw.r, b, b, gw.part,
                      (const BlockState *)nullptr);
-  hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.bstart,
+  hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
                      (const double *)gw.part, gw.inst, gw.gs, 0, w.flags);
   // ap_0 = A p_0 (the stopped instances' workgroups return) and the first
   // step's alpha partials

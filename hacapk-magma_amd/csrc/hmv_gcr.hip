@@ -107,8 +107,13 @@ __global__ __launch_bounds__(kT) void g_update_ur(int n, int nb, const double *_
     s0 += apart[2 * b];
     s1 += apart[2 * b + 1];
   }
-  const double d0 = blk_sum(s0, sh), d1 = blk_sum(s1, sh);
   const int ik = st->ikn;  // the slot of this step
+  const double *pk = p + (size_t)ik * n, *q = ap + (size_t)ik * n;
+  // the first elements are under way while the partials are summed
+  int i = blockIdx.x * kT + threadIdx.x;
+  const int i0 = min(i, n - 1);
+  double uv = u[i0], pv = pk[i0], rv = r[i0], qv = q[i0];
+  const double d0 = blk_sum(s0, sh), d1 = blk_sum(s1, sh);
   const double alpha = d0 / d1;
   const bool bad = d1 == 0.0 || !isfinite(alpha);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -121,13 +126,19 @@ __global__ __launch_bounds__(kT) void g_update_ur(int n, int nb, const double *_
     }
   }
   if (bad) return;
-  const double *pk = p + (size_t)ik * n, *q = ap + (size_t)ik * n;
   double s2 = 0.0;
-  for (int i = blockIdx.x * kT + threadIdx.x; i < n; i += gridDim.x * kT) {
-    u[i] = u[i] + alpha * pk[i];
-    const double ri = r[i] - alpha * q[i];
+  while (i < n) {
+    const double ri = rv - alpha * qv;
+    u[i] = uv + alpha * pv;
     r[i] = ri;
     s2 = __builtin_fma(ri, ri, s2);
+    i += gridDim.x * kT;
+    if (i < n) {
+      uv = u[i];
+      pv = pk[i];
+      rv = r[i];
+      qv = q[i];
+    }
   }
   const double r0 = blk_sum(s2, sh);
   if (threadIdx.x == 0) rpart[blockIdx.x] = r0;
@@ -245,6 +256,10 @@ __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__
 // ... and the next step's alpha partials (ap_ikn, r), (ap_ikn, ap_ikn) into
 // part[2*blk + {0,1}], in g_dots_alpha's order (same grid, same per-thread
 // sequence), so that the step needs no separate dot pass.
+// An element's slots are loaded kDir at a time: one at a time leaves a chain
+// of up to m loads per thread, which is what the pass takes at a few
+// elements per thread.
+constexpr int kDir = 8;
 __global__ __launch_bounds__(kT) void g_update_dir(int n, const double *__restrict__ r,
                                                    const double *__restrict__ ar,
                                                    double *__restrict__ p, double *__restrict__ ap,
@@ -258,11 +273,21 @@ __global__ __launch_bounds__(kT) void g_update_dir(int n, const double *__restri
   for (int i = blockIdx.x * kT + threadIdx.x; i < n; i += gridDim.x * kT) {
     const double ri = r[i];
     double pv = c0 * ri, av = c0 * ar[i];
-    for (int l = 0; l <= ik; ++l) {
-      if (l == ikn) continue;
-      const double bl = st->beta[l];
-      pv = __builtin_fma(bl, p[(size_t)l * n + i], pv);
-      av = __builtin_fma(bl, ap[(size_t)l * n + i], av);
+    for (int l0 = 0; l0 <= ik; l0 += kDir) {
+      double pl[kDir], al[kDir];
+#pragma unroll
+      for (int j = 0; j < kDir; ++j) {
+        const size_t at = (size_t)min(l0 + j, ik) * n + i;
+        pl[j] = p[at];
+        al[j] = ap[at];
+      }
+#pragma unroll
+      for (int j = 0; j < kDir; ++j) {
+        if (l0 + j > ik || l0 + j == ikn) continue;
+        const double bl = st->beta[l0 + j];
+        pv = __builtin_fma(bl, pl[j], pv);
+        av = __builtin_fma(bl, al[j], av);
+      }
     }
     pn[i] = pv;
     apn[i] = av;

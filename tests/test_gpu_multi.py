@@ -197,3 +197,64 @@ def test_multi_autotune(gpu, O, instances):
         lo, hi = m.offsets[i], m.offsets[i + 1]
         assert _rel(y[lo:hi], O.adot_body_lfmtx(hm, x[lo:hi])) <= 2e-2
     m.free()
+
+
+def _diagonal_blocks(H, nd, seed, width=32):
+    """2 I + E on the diagonal blocks of `width` unknowns, E uniform in
+    [-0.1, 0.1]: well conditioned, cheap at any size.  Returns the leaves and
+    x -> A x."""
+    from synthetic_leaves import LeafSet
+    sizes = [min(width, nd - r) for r in range(0, nd, width)]
+    lv = LeafSet(H, nd, [("dense", i * width, m, i * width, m, 0) for i, m in enumerate(sizes)],
+                 seed)
+    mats = []
+    for buf, m in zip(lv._bufs, sizes):
+        M = buf.reshape(m, m)
+        M *= 0.1
+        M += 2.0 * np.eye(m)
+        mats.append(M)
+    full = len(sizes) if sizes[-1] == width else len(sizes) - 1
+    stack = np.stack(mats[:full]) if full else np.zeros((0, width, width))
+
+    def mul(x):
+        y = np.matmul(stack, x[:full * width].reshape(full, width, 1)).reshape(-1)
+        return y if full == len(sizes) else np.concatenate([y, mats[-1] @ x[full * width:]])
+
+    return lv, mul
+
+
+# blocks of 256 rows: one per instance; 2, 1 and 67 of them (an instance's
+# partials summed by 1 and by 32 lanes); blocks of 512 rows, 79 and 1,094
+@pytest.mark.parametrize("sizes", [(256, 40), (257, 33, 17000), (300, 40000, 560000)])
+def test_multi_solvers_block_sizes(gpu, sizes):
+    """Every instance's true residual, recomputed here, is below the stopping
+    bound whatever the number of blocks its dots are summed over (the FP64
+    residual and this one differ by rounding; 1e-3 of the bound is 1,000 times the
+    unit round-off), and the solvers take the steps of the single-instance
+    ones, give or take the 3 that the other groupings of the dots allow."""
+    inst = [_diagonal_blocks(gpu, n, 3 + i) for i, n in enumerate(sizes)]
+    m64 = gpu.MultiArena([lv for lv, _ in inst], "f64")
+    mlow = gpu.MultiArena([lv for lv, _ in inst], "f32")
+    b = gpu.uniform(60, m64.nd)
+    runs = {
+        "bicgstab": m64.bicgstab_multi(b, eps=1e-10, maxit=100),
+        "bicgstab_ir": gpu.multi_bicgstab_ir(m64, mlow, b, eps=1e-10, inner_eps=1e-3),
+        "gcr_ir": gpu.multi_gcr_ir(m64, mlow, b, eps=1e-10, inner_eps=1e-3, m=5),
+    }
+    for name, (u, cols, _, info) in runs.items():
+        assert info["status_name"] == "converged", name
+        for i, (lv, mul) in enumerate(inst):
+            lo, hi = m64.offsets[i], m64.offsets[i + 1]
+            bar = 1.5e-10 if name == "bicgstab" else 1.001e-10
+            assert _rel(mul(u[lo:hi]), b[lo:hi]) < bar, (name, i)
+    for i, (lv, _) in enumerate(inst):
+        lo, hi = m64.offsets[i], m64.offsets[i + 1]
+        a64, alow = gpu.Arena(lv, "f64"), gpu.Arena(lv, "f32")
+        _, one, _ = gpu.gcr_ir(a64, alow, b[lo:hi], eps=1e-10, inner_eps=1e-3, m=5)
+        assert abs(one["inner_total"] - runs["gcr_ir"][1][i]["nstp"]) <= 3
+        _, one, _ = a64.bicgstab(b[lo:hi], eps=1e-10, maxit=100)
+        assert abs(one["nstp"] - runs["bicgstab"][1][i]["nstp"]) <= 3
+        a64.free()
+        alow.free()
+    m64.free()
+    mlow.free()
