@@ -1122,8 +1122,8 @@ def autotune(hm, precision="f64", reps=20):
 
 def bicgstab_ir(a64, alow, b, u0=None, eps=1e-8, inner_eps=1e-4, max_outer=30, max_inner=1000,
                 check_every=8):
-    """Mixed-precision refinement (FP64 residual, low-precision inner BiCGSTAB;
-    the inner solver reads its residual every `check_every` iterations)."""
+    """Mixed-precision refinement (FP64 residual, low-precision inner
+    BiCGSTAB; hmv_bicgstab_ir)."""
     b = np.ascontiguousarray(b, np.float64)
     u0 = np.zeros_like(b) if u0 is None else np.ascontiguousarray(u0, np.float64)
     db, du = DeviceBuffer.from_array(b), DeviceBuffer.from_array(u0)

@@ -8,9 +8,9 @@
 // (element i belongs to column i % k), k a power of two <= 128, so each
 // thread of a 256-thread block stays on one column through its grid-stride
 // loop; per-column dot products reduce in a fixed order (deterministic).  One
-// iteration (two H-matmats and the fused vector kernels) is captured as a
-// hipGraph; a device flag set when every column has stopped turns the
-// remaining launched iterations into no-ops.
+// iteration is two H-matmats and the fused vector kernels; the host feeds the
+// iterations (hmv_feed.h), and a device flag set when every column has stopped
+// turns those launched after it into no-ops.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -21,6 +21,7 @@
 
 #include "hmv.h"
 #include "hmv_engine.h"
+#include "hmv_feed.h"
 
 namespace {
 
@@ -37,7 +38,7 @@ struct BlockState {
   int maxit;
   int all_done;  // every column stopped
   int iter;      // iterations launched and not skipped
-  int pad;
+  int ticks;     // iterations ended, skipped ones included
 };
 
 // Sums v over the threads of the block that share a column (tid % k);
@@ -71,6 +72,17 @@ __global__ __launch_bounds__(kT) void kb_dots(int64_t n, int k, const double *__
     part[2 * ((size_t)blockIdx.x * k + threadIdx.x)] = r0;
     part[2 * ((size_t)blockIdx.x * k + threadIdx.x) + 1] = r1;
   }
+}
+
+// End of a scalar stage: the iteration counts and the word the host watches.
+__device__ inline void block_tick(BlockState *bs, int stage, int all_done, HmvSolveHost *h) {
+  if (stage == 0) bs->iter = bs->ticks = 0;
+  if (stage == 3) {
+    bs->iter += 1;
+    bs->ticks += 1;
+  }
+  bs->all_done = all_done;
+  if (stage == 0 || stage == 3) hmv::publish(h, bs->ticks, all_done);
 }
 
 // Scalar step of one system (column or instance) from its reduced dots:
@@ -139,8 +151,11 @@ __device__ inline void col_step(ColState &c, double d0, double d1, const BlockSt
 // every load is coalesced, then the G group sums are added in order.
 __global__ __launch_bounds__(kT) void kb_final(int nb, int k, const double *__restrict__ part,
                                                ColState *__restrict__ cs, BlockState *bs,
-                                               int stage) {
-  if (bs->all_done && stage != 0) return;
+                                               int stage, HmvSolveHost *h) {
+  if (bs->all_done && stage != 0) {
+    if (stage == 3 && threadIdx.x == 0) hmv::publish(h, bs->ticks += 1, 1);
+    return;
+  }
   __shared__ double red[kT];
   __shared__ int sdone;
   const int tid = threadIdx.x, nv = 2 * k, G = kT / nv;  // k is a power of two <= 128
@@ -165,9 +180,7 @@ __global__ __launch_bounds__(kT) void kb_final(int nb, int k, const double *__re
   }
   __syncthreads();
   if (tid == 0) {
-    if (stage == 0) bs->iter = 0;
-    if (stage == 3) bs->iter += 1;
-    bs->all_done = sdone;
+    block_tick(bs, stage, sdone, h);
   }
 }
 
@@ -261,12 +274,8 @@ struct BlockWork {
   double *part = nullptr;
   ColState *cs = nullptr;
   BlockState *bs = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  const double *graph_u = nullptr;  // the iterate the captured graph updates
+  HmvSolveHost *h = nullptr;  // the arena's
   ~BlockWork() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
     if (s) (void)hipStreamDestroy(s);
     for (double *q : {r, rhat, p, v, t, sv, part}) (void)hipFree(q);
     (void)hipFree(cs);
@@ -283,15 +292,15 @@ hipError_t enqueue_iteration(hmv_arena_s *a, BlockWork &w, double *u) {
   hipLaunchKernelGGL(kb_dots, dim3(g), dim3(kT), 0, w.s, w.n, k, w.rhat, w.v,
                      (const double *)nullptr, (const double *)nullptr, w.part,
                      (const BlockState *)w.bs);
-  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 1);
+  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 1, w.h);
   hipLaunchKernelGGL(kb_update_t, dim3(g), dim3(kT), 0, w.s, w.n, k, w.r, w.v, w.t, w.cs, w.bs);
   if ((e = hmv::enqueue_apply_block(a, k, w.t, w.sv, 0.0, skip, w.s)) != hipSuccess) return e;
   hipLaunchKernelGGL(kb_dots, dim3(g), dim3(kT), 0, w.s, w.n, k, w.sv, w.t, w.sv, w.sv, w.part,
                      (const BlockState *)w.bs);
-  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 2);
+  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 2, w.h);
   hipLaunchKernelGGL(kb_update_ur, dim3(g), dim3(kT), 0, w.s, w.n, k, w.p, w.t, w.sv, w.rhat, u,
                      w.r, w.part, w.cs, w.bs);
-  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 3);
+  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 3, w.h);
   return hipGetLastError();
 }
 
@@ -365,17 +374,19 @@ int block_setup(hmv_arena_s *a, BlockWork &w, int k, const char *who) {
 // k BiCGSTABs sharing one H-matmat per step, from u (zero_guess: u = 0 and
 // r = b without a product), until every column has stopped or maxit
 // iterations ran; cs receives the columns' final states, iters the
-// iterations run.  The iteration graph is captured on the first call with a
-// given u and reused by later calls.
+// iterations run.
 int block_solve(hmv_arena_s *a, BlockWork &w, const double *b, double *u, double eps, int maxit,
-                int check_every, bool zero_guess, std::vector<ColState> &cs, int &iters,
+                bool zero_guess, std::vector<ColState> &cs, int &iters,
                 const char *who) {
   const std::string name(who);
   const int g = grid_of(w.n), k = w.k;
   BlockState init{};
   init.eps = eps;
   init.maxit = maxit;
-  hipError_t e = hipMemcpyAsync(w.bs, &init, sizeof(init), hipMemcpyHostToDevice, w.s);
+  hipError_t e;
+  if ((e = hmv::solve_host(a, w.s, w.h)) != hipSuccess)
+    return hmv::hip_fail(e, (name + ": setup").c_str());
+  e = hipMemcpyAsync(w.bs, &init, sizeof(init), hipMemcpyHostToDevice, w.s);
   if (e != hipSuccess) return hmv::hip_fail(e, (name + ": setup").c_str());
   if (zero_guess)
     hipLaunchKernelGGL(kb_fill_n, dim3(g), dim3(kT), 0, w.s, w.n, w.r, 0.0);
@@ -384,37 +395,14 @@ int block_solve(hmv_arena_s *a, BlockWork &w, const double *b, double *u, double
   hipLaunchKernelGGL(kb_init, dim3(g), dim3(kT), 0, w.s, w.n, b, w.r, w.rhat, w.p, w.v);
   hipLaunchKernelGGL(kb_dots, dim3(g), dim3(kT), 0, w.s, w.n, k, w.r, w.r, b, b, w.part,
                      (const BlockState *)nullptr);
-  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 0);
-  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
+  hipLaunchKernelGGL(kb_final, dim3(1), dim3(kT), 0, w.s, g, k, w.part, w.cs, w.bs, 0, w.h);
+  if ((e = hipGetLastError()) != hipSuccess)
     return hmv::hip_fail(e, (name + ": setup").c_str());
-  if (!w.exec || w.graph_u != u) {
-    if (w.exec) (void)hipGraphExecDestroy(w.exec);
-    if (w.graph) (void)hipGraphDestroy(w.graph);
-    w.exec = nullptr;
-    w.graph = nullptr;
-    if ((e = hipStreamBeginCapture(w.s, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": capture").c_str());
-    hipError_t ec = enqueue_iteration(a, w, u);
-    e = hipStreamEndCapture(w.s, &w.graph);
-    if (ec != hipSuccess) return hmv::hip_fail(ec, (name + ": capture").c_str());
-    if (e != hipSuccess ||
-        (e = hipGraphInstantiate(&w.exec, w.graph, nullptr, nullptr, 0)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": graph").c_str());
-    w.graph_u = u;
-  }
   BlockState host{};
   int launched = 0;
-  while (launched < maxit) {
-    const int burst = std::min(check_every, maxit - launched);
-    for (int i = 0; i < burst; ++i)
-      if ((e = hipGraphLaunch(w.exec, w.s)) != hipSuccess)
-        return hmv::hip_fail(e, (name + ": launch").c_str());
-    launched += burst;
-    if ((e = hipMemcpyAsync(&host, w.bs, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess ||
-        (e = hipStreamSynchronize(w.s)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": state").c_str());
-    if (host.all_done) break;
-  }
+  if ((e = hmv::feed(w.h, w.s, launched, maxit,
+                     [&] { return enqueue_iteration(a, w, u); })) != hipSuccess)
+    return hmv::hip_fail(e, (name + ": iterations").c_str());
   if ((e = hipMemcpyAsync(&host, w.bs, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess ||
       (e = hipStreamSynchronize(w.s)) != hipSuccess)
     return hmv::hip_fail(e, (name + ": state").c_str());
@@ -428,13 +416,12 @@ int block_solve(hmv_arena_s *a, BlockWork &w, const double *b, double *u, double
 }  // namespace
 
 extern "C" int hmv_block_bicgstab(hmv_arena a, int k, const double *b, double *u, double eps,
-                                  int maxit, int check_every, hmv_column_info *cols,
+                                  int maxit, int /*check_every*/, hmv_column_info *cols,
                                   hmv_solve_info *info) {
   if (!a || !b || !u || k < 1 || k > HMV_MAX_RHS || (k & (k - 1)) != 0 || maxit < 0) {
     hmv::set_error("hmv_block_bicgstab: invalid argument (k must be a power of two <= 128)");
     return HMV_ERR_ARG;
   }
-  if (check_every < 1) check_every = 1;
   const char *who = "hmv_block_bicgstab";
   BlockWork w;
   int rc = block_setup(a, w, k, who);
@@ -442,7 +429,7 @@ extern "C" int hmv_block_bicgstab(hmv_arena a, int k, const double *b, double *u
   auto t0 = std::chrono::steady_clock::now();
   std::vector<ColState> cs;
   int iters = 0;
-  if ((rc = block_solve(a, w, b, u, eps, maxit, check_every, false, cs, iters, who))) return rc;
+  if ((rc = block_solve(a, w, b, u, eps, maxit, false, cs, iters, who))) return rc;
   auto t1 = std::chrono::steady_clock::now();
   std::vector<double> rel;
   if ((rc = block_residual(a, w, b, u, w.r, rel)) != HMV_OK) return rc;
@@ -474,7 +461,7 @@ extern "C" int hmv_block_bicgstab(hmv_arena a, int k, const double *b, double *u
 
 extern "C" int hmv_block_bicgstab_ir(hmv_arena a64, hmv_arena alow, int k, const double *b,
                                      double *u, double eps, double inner_eps, int max_outer,
-                                     int max_inner, int check_every, hmv_column_info *cols,
+                                     int max_inner, int /*check_every*/, hmv_column_info *cols,
                                      hmv_solve_info *info) {
   const char *who = "hmv_block_bicgstab_ir";
   if (!a64 || !alow || !b || !u || k < 1 || k > HMV_MAX_RHS || (k & (k - 1)) != 0 ||
@@ -484,7 +471,6 @@ extern "C" int hmv_block_bicgstab_ir(hmv_arena a64, hmv_arena alow, int k, const
                    "two <= 128, 0 < inner_eps < 1)");
     return HMV_ERR_ARG;
   }
-  if (check_every < 1) check_every = 1;
   int rc = hmv::ensure_tk(a64, k);
   if (rc) return rc;
   BlockWork w;  // inner solves over the low-precision arena
@@ -535,7 +521,7 @@ extern "C" int hmv_block_bicgstab_ir(hmv_arena a64, hmv_arena alow, int k, const
     hipLaunchKernelGGL(kb_zero_cols, dim3(g), dim3(kT), 0, w.s, w.n, k, buf.r2, buf.stopped);
     hipLaunchKernelGGL(kb_fill_n, dim3(g), dim3(kT), 0, w.s, w.n, buf.d, 0.0);
     int iters = 0;
-    if ((rc = block_solve(alow, w, buf.r2, buf.d, inner_eps, max_inner, check_every, true, cs, iters,
+    if ((rc = block_solve(alow, w, buf.r2, buf.d, inner_eps, max_inner, true, cs, iters,
                           who)))
       return rc;
     inner_total += iters;
@@ -641,8 +627,12 @@ __device__ inline double group_sum(double v, int lanes) {
 __global__ __launch_bounds__(kT) void ks_final(int nseg, int lanes, const int *__restrict__ bstart,
                                                const double *__restrict__ part,
                                                ColState *__restrict__ cs, BlockState *bs,
-                                               int stage, int *__restrict__ done_flags) {
-  if (bs->all_done && stage != 0) return;
+                                               int stage, int *__restrict__ done_flags,
+                                               HmvSolveHost *h) {
+  if (bs->all_done && stage != 0) {
+    if (stage == 3 && threadIdx.x == 0) hmv::publish(h, bs->ticks += 1, 1);
+    return;
+  }
   __shared__ int sdone;
   if (threadIdx.x == 0) sdone = 1;
   __syncthreads();
@@ -665,9 +655,7 @@ __global__ __launch_bounds__(kT) void ks_final(int nseg, int lanes, const int *_
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    if (stage == 0) bs->iter = 0;
-    if (stage == 3) bs->iter += 1;
-    bs->all_done = sdone;
+    block_tick(bs, stage, sdone, h);
   }
 }
 
@@ -738,13 +726,9 @@ struct SegWork {
   ColState *cs = nullptr;
   BlockState *bs = nullptr;
   int *flags = nullptr;  // per-instance done flags read by the H-matvec
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  const double *graph_u = nullptr;  // the iterate the captured graph updates
+  HmvSolveHost *h = nullptr;  // the arena's
   ~SegWork() {
     (void)hipFree(flags);
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
     if (s) (void)hipStreamDestroy(s);
     for (double *q : {r, rhat, p, v, t, sv, part}) (void)hipFree(q);
     (void)hipFree(tb);
@@ -786,17 +770,17 @@ hipError_t seg_iteration(hmv_arena_s *a, SegWork &w, double *u) {
                      (const double *)nullptr, (const double *)nullptr, w.part,
                      (const BlockState *)w.bs);
   hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 1,
-                     w.flags);
+                     w.flags, w.h);
   hipLaunchKernelGGL(ks_update_t, dim3(nb), dim3(kT), 0, w.s, w.tb, w.r, w.v, w.t, w.cs, w.bs);
   if ((e = hmv::enqueue_apply(a, w.t, w.sv, 0.0, skip, w.s, w.flags)) != hipSuccess) return e;
   hipLaunchKernelGGL(ks_dots, dim3(nb), dim3(kT), 0, w.s, w.tb, w.sv, w.t, w.sv, w.sv, w.part,
                      (const BlockState *)w.bs);
   hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 2,
-                     w.flags);
+                     w.flags, w.h);
   hipLaunchKernelGGL(ks_update_ur, dim3(nb), dim3(kT), 0, w.s, w.tb, w.p, w.t, w.sv, w.rhat, u,
                      w.r, w.part, w.cs, w.bs);
   hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 3,
-                     w.flags);
+                     w.flags, w.h);
   return hipGetLastError();
 }
 
@@ -806,7 +790,7 @@ hipError_t seg_iteration(hmv_arena_s *a, SegWork &w, double *u) {
 // chip eight times over (kSegBlocks), then up to 16.  The vector passes are
 // bound by latency: at 16 elements per thread, 8 instances of 320 to 20,480
 // unknowns are 19 blocks on 256 CUs, and a direction update over 30 slots
-// took 37 us; in 232 blocks their whole solve takes 11.5 ms instead of 18.3.  An
+// took 37 us; 232 blocks brought their whole solve from 18.3 to 11.5 ms.  An
 // instance's partials are summed by one lane for each 4 blocks.
 int seg_setup(hmv_arena_s *a, SegWork &w, std::vector<int> &bstart, const char *who) {
   w.nseg = (int)a->seg.size() - 1;
@@ -852,9 +836,8 @@ double seconds_since(std::chrono::steady_clock::time_point t0) {
 // One BiCGSTAB per instance from u (zero_guess: u = 0, and r = b without a
 // product), in lockstep until every instance has stopped or maxit
 // iterations ran.  cs receives the instances' final states; done_at (may be
-// null) the time since t0 at which each instance was first seen stopped;
-// iters the iterations run.  The iteration graph is captured on the first
-// call with a given u and reused by later calls.
+// null) the time since t0 at which each instance was first seen stopped, looked
+// at every check_every iterations; iters the iterations run.
 int seg_solve(hmv_arena_s *a, SegWork &w, const double *b, double *u, double eps, int maxit,
               int check_every, bool zero_guess, std::chrono::steady_clock::time_point t0,
               std::vector<ColState> &cs, std::vector<double> *done_at, int &iters,
@@ -864,7 +847,9 @@ int seg_solve(hmv_arena_s *a, SegWork &w, const double *b, double *u, double eps
   init.eps = eps;
   init.maxit = maxit;
   const int g = grid_of(w.n);
-  hipError_t e = hipMemcpyAsync(w.bs, &init, sizeof(init), hipMemcpyHostToDevice, w.s);
+  hipError_t e = hmv::solve_host(a, w.s, w.h);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(w.bs, &init, sizeof(init), hipMemcpyHostToDevice, w.s);
   if (e != hipSuccess) return hmv::hip_fail(e, (name + ": setup").c_str());
   if (zero_guess)
     hipLaunchKernelGGL(kb_fill, dim3(g), dim3(kT), 0, w.s, w.n, w.r, 0.0);
@@ -874,24 +859,9 @@ int seg_solve(hmv_arena_s *a, SegWork &w, const double *b, double *u, double eps
   hipLaunchKernelGGL(ks_dots, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, w.r, w.r, b, b, w.part,
                      (const BlockState *)nullptr);
   hipLaunchKernelGGL(ks_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart, w.part, w.cs, w.bs, 0,
-                     w.flags);
-  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
+                     w.flags, w.h);
+  if ((e = hipGetLastError()) != hipSuccess)
     return hmv::hip_fail(e, (name + ": setup").c_str());
-  if (!w.exec || w.graph_u != u) {
-    if (w.exec) (void)hipGraphExecDestroy(w.exec);
-    if (w.graph) (void)hipGraphDestroy(w.graph);
-    w.exec = nullptr;
-    w.graph = nullptr;
-    if ((e = hipStreamBeginCapture(w.s, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": capture").c_str());
-    hipError_t ec = seg_iteration(a, w, u);
-    e = hipStreamEndCapture(w.s, &w.graph);
-    if (ec != hipSuccess) return hmv::hip_fail(ec, (name + ": capture").c_str());
-    if (e != hipSuccess ||
-        (e = hipGraphInstantiate(&w.exec, w.graph, nullptr, nullptr, 0)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": graph").c_str());
-    w.graph_u = u;
-  }
   cs.resize(w.nseg);
   auto poll = [&]() -> hipError_t {
     hipError_t pe = hipMemcpyAsync(cs.data(), w.cs, sizeof(ColState) * w.nseg,
@@ -904,15 +874,16 @@ int seg_solve(hmv_arena_s *a, SegWork &w, const double *b, double *u, double eps
     }
     return pe;
   };
-  if ((e = poll()) != hipSuccess) return hmv::hip_fail(e, (name + ": state").c_str());
+  if ((done_at || maxit < 1) && (e = poll()) != hipSuccess)
+    return hmv::hip_fail(e, (name + ": state").c_str());
   BlockState host{};
   int launched = 0;
   while (launched < maxit) {
-    const int burst = std::min(check_every, maxit - launched);
-    for (int i = 0; i < burst; ++i)
-      if ((e = hipGraphLaunch(w.exec, w.s)) != hipSuccess)
-        return hmv::hip_fail(e, (name + ": launch").c_str());
-    launched += burst;
+    // the states are read along the way only for the times in done_at
+    const int burst = done_at ? std::min(check_every, maxit - launched) : maxit;
+    if ((e = hmv::feed(w.h, w.s, launched, launched + burst,
+                       [&] { return seg_iteration(a, w, u); })) != hipSuccess)
+      return hmv::hip_fail(e, (name + ": iterations").c_str());
     if ((e = hipMemcpyAsync(&host, w.bs, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess ||
         (e = poll()) != hipSuccess)
       return hmv::hip_fail(e, (name + ": state").c_str());
@@ -1145,7 +1116,8 @@ struct SgInst {
 
 struct SgGlobal {
   double eps;
-  int step, ik, ikn, m, maxit, all_done, pad;
+  int step, ik, ikn, m, maxit, all_done;
+  int ticks;  // steps ended, with those that found every instance stopped
 };
 
 // r = b, p_0 = b (zero initial guess)
@@ -1301,8 +1273,11 @@ __global__ __launch_bounds__(kT) void sg_betas(int nseg, int lanes,
 __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *__restrict__ bstart,
                                                const double *__restrict__ part, SgInst *inst,
                                                SgGlobal *gs, int stage,
-                                               int *__restrict__ done_flags) {
-  if (gs->all_done && stage != 0) return;
+                                               int *__restrict__ done_flags, HmvSolveHost *h) {
+  if (gs->all_done && stage != 0) {
+    if (threadIdx.x == 0) hmv::publish(h, gs->ticks += 1, 1);
+    return;
+  }
   __shared__ int sdone;
   if (threadIdx.x == 0) sdone = 1;
   __syncthreads();
@@ -1354,15 +1329,17 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
   __syncthreads();
   if (threadIdx.x == 0) {
     if (stage == 0) {
-      gs->step = 0;
+      gs->step = gs->ticks = 0;
       gs->ik = 0;
       gs->ikn = 0;
     } else {
       gs->ik = gs->ikn;
       gs->step += 1;
+      gs->ticks += 1;
       gs->ikn = gs->step % gs->m;
     }
     gs->all_done = sdone;
+    hmv::publish(h, gs->ticks, sdone);
   }
 }
 
@@ -1424,12 +1401,7 @@ struct SegGcrWork {
   double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr, *part = nullptr;
   SgInst *inst = nullptr;
   SgGlobal *gs = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  const double *graph_u = nullptr;
   ~SegGcrWork() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
     for (double *q : {r, ar, p, ap, part}) (void)hipFree(q);
     (void)hipFree(inst);
     (void)hipFree(gs);
@@ -1458,7 +1430,7 @@ hipError_t sg_iteration(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, double
   hipLaunchKernelGGL(sg_update_ur, dim3(nb), dim3(kT), 0, w.s, w.tb, w.bstart, w.n, gw.p, gw.ap,
                      u, gw.r, (const double *)gw.part, rpart, gw.inst, (const SgGlobal *)gw.gs);
   hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
-                     (const double *)rpart, gw.inst, gw.gs, 2, w.flags);
+                     (const double *)rpart, gw.inst, gw.gs, 2, w.flags, w.h);
   hipError_t e = hmv::enqueue_apply(a, gw.r, gw.ar, 0.0, skip, w.s, w.flags);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(sg_dots_beta, dim3(nb, (gw.m + kGroup - 1) / kGroup), dim3(kT), 0, w.s, w.tb,
@@ -1473,10 +1445,9 @@ hipError_t sg_iteration(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, double
 
 // One GCR(m) per instance for A d = b from d = 0 (the caller zeroes d), in
 // lockstep until every instance has stopped or maxit steps ran.  inst
-// receives the instances' final states, iters the steps run.  The
-// iteration graph is captured on the first call with a given d.
-int sg_solve(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, const double *b, double *d,
-             double eps, int maxit, int check_every, std::vector<SgInst> &inst, int &iters,
+// receives the instances' final states, iters the steps run.
+int sg_solve(hmv_arena_s *a, SegWork &w, SegGcrWork &gw, const double *b, double *d,
+             double eps, int maxit, std::vector<SgInst> &inst, int &iters,
              const char *who) {
   const std::string name(who);
   SgGlobal init{};
@@ -1484,49 +1455,29 @@ int sg_solve(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, const double *b, 
   init.m = gw.m;
   init.maxit = maxit;
   const int g = grid_of(w.n);
-  hipError_t e = hipMemcpyAsync(gw.gs, &init, sizeof(init), hipMemcpyHostToDevice, w.s);
+  hipError_t e = hmv::solve_host(a, w.s, w.h);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(gw.gs, &init, sizeof(init), hipMemcpyHostToDevice, w.s);
   if (e != hipSuccess) return hmv::hip_fail(e, (name + ": setup").c_str());
   hipLaunchKernelGGL(sg_init, dim3(g), dim3(kT), 0, w.s, w.n, b, gw.r, gw.p);
   hipLaunchKernelGGL(ks_dots, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, gw.r, gw.r, b, b, gw.part,
                      (const BlockState *)nullptr);
   hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
-                     (const double *)gw.part, gw.inst, gw.gs, 0, w.flags);
+                     (const double *)gw.part, gw.inst, gw.gs, 0, w.flags, w.h);
   // ap_0 = A p_0 (the stopped instances' workgroups return) and the first
   // step's alpha partials
   if ((e = hmv::enqueue_apply(a, gw.p, gw.ap, 0.0, &gw.gs->all_done, w.s, w.flags)) != hipSuccess)
     return hmv::hip_fail(e, (name + ": setup").c_str());
   hipLaunchKernelGGL(sg_dots_alpha, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, w.n, gw.ap, gw.r,
                      gw.part, (const SgGlobal *)gw.gs);
-  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
+  if ((e = hipGetLastError()) != hipSuccess)
     return hmv::hip_fail(e, (name + ": setup").c_str());
-  if (!gw.exec || gw.graph_u != d) {
-    if (gw.exec) (void)hipGraphExecDestroy(gw.exec);
-    if (gw.graph) (void)hipGraphDestroy(gw.graph);
-    gw.exec = nullptr;
-    gw.graph = nullptr;
-    if ((e = hipStreamBeginCapture(w.s, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": capture").c_str());
-    hipError_t ec = sg_iteration(a, w, gw, d);
-    e = hipStreamEndCapture(w.s, &gw.graph);
-    if (ec != hipSuccess) return hmv::hip_fail(ec, (name + ": capture").c_str());
-    if (e != hipSuccess ||
-        (e = hipGraphInstantiate(&gw.exec, gw.graph, nullptr, nullptr, 0)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": graph").c_str());
-    gw.graph_u = d;
-  }
   SgGlobal host{};
   int launched = 0;
-  for (;;) {
-    if ((e = hipMemcpyAsync(&host, gw.gs, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess ||
-        (e = hipStreamSynchronize(w.s)) != hipSuccess)
-      return hmv::hip_fail(e, (name + ": state").c_str());
-    if (host.all_done || launched >= maxit) break;
-    const int burst = std::min(check_every, maxit - launched);
-    for (int i = 0; i < burst; ++i)
-      if ((e = hipGraphLaunch(gw.exec, w.s)) != hipSuccess)
-        return hmv::hip_fail(e, (name + ": launch").c_str());
-    launched += burst;
-  }
+  if ((e = hmv::feed(w.h, w.s, launched, maxit,
+                     [&] { return sg_iteration(a, w, gw, d); })) != hipSuccess ||
+      (e = hipMemcpyAsync(&host, gw.gs, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess)
+    return hmv::hip_fail(e, (name + ": iterations").c_str());
   inst.resize(w.nseg);
   if ((e = hipMemcpyAsync(inst.data(), gw.inst, sizeof(SgInst) * w.nseg, hipMemcpyDeviceToHost,
                           w.s)) != hipSuccess ||
@@ -1540,7 +1491,7 @@ int sg_solve(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, const double *b, 
 
 extern "C" int hmv_multi_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, double *u,
                                 double eps, double inner_eps, int m, int max_outer, int max_inner,
-                                int check_every, hmv_column_info *inst, double *inst_seconds,
+                                int /*check_every*/, hmv_column_info *inst, double *inst_seconds,
                                 hmv_solve_info *info) {
   const char *who = "hmv_multi_gcr_ir";
   if (!a64 || !alow || !b || !u || max_outer < 1 || max_inner < 1 || m < 1 || m > kGcrM ||
@@ -1550,7 +1501,6 @@ extern "C" int hmv_multi_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, 
                    "1 <= m <= 32, 0 < inner_eps < 1)");
     return HMV_ERR_ARG;
   }
-  if (check_every < 1) check_every = 1;
   SegWork w;  // block table, stream and FP64 residuals
   std::vector<int> bstart;
   int rc = seg_setup(alow, w, bstart, who);
@@ -1606,7 +1556,7 @@ extern "C" int hmv_multi_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, 
     hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, buf.r2, buf.stopped);
     hipLaunchKernelGGL(kb_fill, dim3(g), dim3(kT), 0, w.s, w.n, buf.d, 0.0);
     int iters = 0;
-    if ((rc = sg_solve(alow, w, gw, buf.r2, buf.d, inner_eps, max_inner, check_every, cs, iters,
+    if ((rc = sg_solve(alow, w, gw, buf.r2, buf.d, inner_eps, max_inner, cs, iters,
                        who)))
       return rc;
     inner_total += iters;

@@ -12,6 +12,7 @@
 #include "hmv_plan.h"
 
 struct HmvSolveWork;
+struct HmvSolveHost;
 
 // H-matmat work units: one wave per (work item, group of up to 1 << w
 // consecutive 16-row tiles), unit = {item, first tile << 8 | tiles}; one
@@ -68,6 +69,7 @@ struct hmv_arena_s {
   hipStream_t hstream = nullptr;
   HmvSolveWork *solve = nullptr;             // solver workspace (lazy)
   struct HmvGcrWork *gcr = nullptr;          // GCR(m) workspace (lazy)
+  HmvSolveHost *solve_host = nullptr;        // pinned memory of the solvers (hmv_feed.h)
   hmv_arena_stats stats{};
   // what a saved arena file needs besides the device tables
   int64_t nzseg = 0, noutidx = 0, ncodes = 0;

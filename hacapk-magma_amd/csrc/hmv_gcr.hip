@@ -13,8 +13,8 @@
 // overwritten, so its beta is -(ar, ar)/capap_1 and it scales the new
 // direction by (1 + beta_1), as in the reference.  All betas use the
 // unmodified ar, so one pass computes them and one fused pass applies them.
-// One iteration is captured as a hipGraph; a device flag set on convergence
-// turns the remaining launched iterations into no-ops.
+// The host feeds the iterations (hmv_feed.h); a device flag set on
+// convergence turns those launched after it into no-ops.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,11 +24,12 @@
 
 #include "hmv.h"
 #include "hmv_engine.h"
+#include "hmv_feed.h"
 
 namespace {
 
 constexpr int kT = 256;
-constexpr int kMaxB = 512;
+constexpr int kMaxB = kSolveMaxBlocks;
 constexpr int kMaxM = HMV_GCR_MAX_M;
 static_assert(kMaxM >= 3, "the partial buffer holds the alpha pairs and the (r, r) partials");
 
@@ -39,7 +40,8 @@ struct GcrState {
   int step;  // completed steps (the reference's in)
   int ik;    // slot of the current direction (0-based)
   int ikn;   // slot of the next direction (0-based)
-  int m, maxit, done, status, pad;
+  int m, maxit, done, status;
+  int ticks;  // iterations ended, with those that found the solve stopped
 };
 
 __device__ inline double blk_sum(double v, double *sh) {
@@ -179,9 +181,26 @@ __global__ __launch_bounds__(kT) void g_dots_beta(int n, const double *__restric
 // (nb partials), step, stop; 3: betas from the per-slot partials, one wave
 // per slot (lanes sum the blocks in a fixed order, then a fixed shuffle
 // tree: deterministic)
+__device__ inline void g_publish(HmvSolveHost *h, const GcrState *st) {
+  if (st->done) {
+    h->step = st->step;
+    h->status = st->status;
+    h->rnorm = st->rnorm;
+    h->bnorm = st->bnorm;
+  }
+  hmv::publish(h, st->ticks, st->done);
+}
+
 __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__ part,
-                                              GcrState *st, int stage, double *__restrict__ hist) {
-  if (st->done && stage != 0) return;
+                                              GcrState *st, int stage, double *__restrict__ hist,
+                                              HmvSolveHost *h) {
+  if (st->done && stage != 0) {
+    if (stage == 2 && threadIdx.x == 0) {
+      st->ticks += 1;
+      g_publish(h, st);
+    }
+    return;
+  }
   __shared__ double sh[4];
   if (stage == 3) {
     // wave w takes slots w, w + 4, ...; all their loads go out together
@@ -233,6 +252,7 @@ __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__
     } else if (st->maxit <= 0) {
       st->done = 1;
     }
+    st->ticks = 0;
   } else {
     st->step += 1;
     st->rnorm = sqrt(d0);
@@ -248,7 +268,9 @@ __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__
       st->status = HMV_SOLVE_MAXITER;
       st->done = 1;
     }
+    st->ticks += 1;
   }
+  g_publish(h, st);
 }
 
 // p_ikn = c0 r + sum_{il <= ik, il != ikn} beta_il p_il;  ap_ikn likewise
@@ -318,28 +340,17 @@ int grid_of(int n) {
 
 }  // namespace
 
-// GCR workspace, kept with the arena between calls (the iteration graph is
-// re-captured only when m, the history capacity or the solution vector change).
+// GCR workspace, kept with the arena between calls.
 struct HmvGcrWork {
   int m = 0;
   size_t hist_cap = 0;
   hipStream_t s = nullptr;
   double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr, *part = nullptr, *hist = nullptr;
   GcrState *st = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  double *g_u = nullptr;  // solution vector the graph was captured with
-  void drop_graph() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    exec = nullptr;
-    graph = nullptr;
-    g_u = nullptr;
-  }
+  double *ir_r = nullptr, *ir_d = nullptr;  // refinement: outer residual, correction
   ~HmvGcrWork() {
-    drop_graph();
     if (s) (void)hipStreamDestroy(s);
-    for (double *q : {r, ar, p, ap, part, hist}) (void)hipFree(q);
+    for (double *q : {r, ar, p, ap, part, hist, ir_r, ir_d}) (void)hipFree(q);
     (void)hipFree(st);
   }
 };
@@ -384,7 +395,7 @@ int gcr_work(hmv_arena_s *a, int m, int maxit, GcrWork *&out) {
   return HMV_OK;
 }
 
-hipError_t gcr_iteration(hmv_arena_s *a, GcrWork &w, int n, int m, double *u) {
+hipError_t gcr_iteration(hmv_arena_s *a, GcrWork &w, int n, int m, double *u, HmvSolveHost *h) {
   const int g = grid_of(n);
   const int *skip = &w.st->done;
   // (r, r) partials at [2g, 3g) of the g * kMaxM partials, apart from the
@@ -394,13 +405,14 @@ hipError_t gcr_iteration(hmv_arena_s *a, GcrWork &w, int n, int m, double *u) {
   // g_update_dir (or, for the first step, from the setup's g_dots_alpha)
   hipLaunchKernelGGL(g_update_ur, dim3(g), dim3(kT), 0, w.s, n, g, w.p, w.ap, u, w.r,
                      (const double *)w.part, rpart, w.st);
-  hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, (const double *)rpart, w.st, 2, w.hist);
+  hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, (const double *)rpart, w.st, 2, w.hist,
+                     h);
   hipError_t e = hmv::enqueue_apply(a, w.r, w.ar, 0.0, skip, w.s);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(g_dots_beta, dim3(g, (m + kGroup - 1) / kGroup), dim3(kT), 0, w.s, n, w.ap,
                      w.ar, w.part,
                      (const GcrState *)w.st);
-  hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 3, w.hist);
+  hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 3, w.hist, h);
   hipLaunchKernelGGL(g_update_dir, dim3(g), dim3(kT), 0, w.s, n, w.r, w.ar, w.p, w.ap, w.part,
                      (const GcrState *)w.st);
   return hipGetLastError();
@@ -410,32 +422,34 @@ hipError_t gcr_iteration(hmv_arena_s *a, GcrWork &w, int n, int m, double *u) {
 
 namespace {
 int gcrm_run(hmv_arena a, const double *b, double *u, double eps, int maxit, int m,
-             int check_every, double *hist, hmv_solve_info *info, bool true_res,
+             double *hist, hmv_solve_info *info, bool true_res,
              bool zero_guess = false);
 }
 
 extern "C" int hmv_gcrm(hmv_arena a, const double *b, double *u, double eps, int maxit, int m,
-                        int check_every, double *hist, hmv_solve_info *info) {
-  return gcrm_run(a, b, u, eps, maxit, m, check_every, hist, info, true);
+                        int /*check_every*/, double *hist, hmv_solve_info *info) {
+  return gcrm_run(a, b, u, eps, maxit, m, hist, info, true);
 }
 
 namespace {
 // true_res: recompute ||b - A u|| / ||b|| at the end (one more product).
 // zero_guess: u is known to be zero, so r = b without the product A u.
 int gcrm_run(hmv_arena a, const double *b, double *u, double eps, int maxit, int m,
-             int check_every, double *hist, hmv_solve_info *info, bool true_res,
+             double *hist, hmv_solve_info *info, bool true_res,
              bool zero_guess) {
   if (!a || !b || !u || maxit < 0 || m < 1 || m > kMaxM) {
     hmv::set_error("hmv_gcrm: invalid argument (1 <= m <= 32)");
     return HMV_ERR_ARG;
   }
-  if (check_every < 1) check_every = 1;
   const int n = a->nd, g = grid_of(n);
   GcrWork *wp = nullptr;
   int rc = gcr_work(a, m, maxit, wp);
   if (rc) return rc;
   GcrWork &w = *wp;
   hipError_t e;
+  HmvSolveHost *h = nullptr;
+  if ((e = hmv::solve_host(a, w.s, h)) != hipSuccess)
+    return hmv::hip_fail(e, "hmv_gcrm: workspace");
   auto t0 = std::chrono::steady_clock::now();
   GcrState init{};
   init.eps = eps;
@@ -447,44 +461,24 @@ int gcrm_run(hmv_arena a, const double *b, double *u, double eps, int maxit, int
   hipLaunchKernelGGL(g_init, dim3(g), dim3(kT), 0, w.s, n, b, zero_guess ? nullptr : w.ar, w.r,
                      w.p);
   hipLaunchKernelGGL(g_dots2, dim3(g), dim3(kT), 0, w.s, n, w.r, w.r, b, b, w.part);
-  hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 0, w.hist);
+  hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 0, w.hist, h);
   // ap_1 = A p_1 (skipped when already converged) and the first step's
   // alpha partials
   if ((e = hmv::enqueue_apply(a, w.p, w.ap, 0.0, &w.st->done, w.s)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_gcrm: setup");
   hipLaunchKernelGGL(g_dots_alpha, dim3(g), dim3(kT), 0, w.s, n, w.ap, w.r, w.part,
                      (const GcrState *)w.st);
-  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
-    return hmv::hip_fail(e, "hmv_gcrm: setup");
-  if (!w.exec || w.g_u != u) {
-    w.drop_graph();
-    if ((e = hipStreamBeginCapture(w.s, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_gcrm: capture");
-    hipError_t ec = gcr_iteration(a, w, n, m, u);
-    e = hipStreamEndCapture(w.s, &w.graph);
-    if (ec != hipSuccess) return hmv::hip_fail(ec, "hmv_gcrm: capture");
-    if (e != hipSuccess ||
-        (e = hipGraphInstantiate(&w.exec, w.graph, nullptr, nullptr, 0)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_gcrm: graph");
-    w.g_u = u;
-  }
-  GcrState host{};
+  if ((e = hipGetLastError()) != hipSuccess) return hmv::hip_fail(e, "hmv_gcrm: setup");
   int launched = 0;
-  for (;;) {
-    if ((e = hipMemcpyAsync(&host, w.st, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess ||
-        (e = hipStreamSynchronize(w.s)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_gcrm: state");
-    if (host.done || launched >= maxit) break;
-    const int burst = std::min(check_every, maxit - launched);
-    for (int i = 0; i < burst; ++i)
-      if ((e = hipGraphLaunch(w.exec, w.s)) != hipSuccess)
-        return hmv::hip_fail(e, "hmv_gcrm: launch");
-    launched += burst;
-  }
+  e = hmv::feed(h, w.s, launched, maxit,
+                [&] { return gcr_iteration(a, w, n, m, u, h); });
+  // the refinement goes on on the same stream; a caller's u is complete here
+  if (e == hipSuccess && (true_res || !hmv::stopped(h))) e = hipStreamSynchronize(w.s);
+  if (e != hipSuccess) return hmv::hip_fail(e, "hmv_gcrm: iterations");
   auto t1 = std::chrono::steady_clock::now();
   if (hist) {
     std::fill(hist, hist + maxit + 1, NAN);
-    if ((e = hipMemcpy(hist, w.hist, sizeof(double) * ((size_t)host.step + 1),
+    if ((e = hipMemcpy(hist, w.hist, sizeof(double) * ((size_t)h->step + 1),
                        hipMemcpyDeviceToHost)) != hipSuccess)
       return hmv::hip_fail(e, "hmv_gcrm: history");
   }
@@ -494,27 +488,24 @@ int gcrm_run(hmv_arena a, const double *b, double *u, double eps, int maxit, int
     if ((e = hmv::enqueue_apply(a, u, w.ar, 0.0, nullptr, w.s)) != hipSuccess)
       return hmv::hip_fail(e, "hmv_gcrm: true residual");
     hipLaunchKernelGGL(g_init, dim3(g), dim3(kT), 0, w.s, n, b, w.ar, w.r, w.p);
-    hipLaunchKernelGGL(g_dots2, dim3(g), dim3(kT), 0, w.s, n, w.r, w.r, b, b, w.part);
-    std::vector<double> part(2 * (size_t)g);
-    if ((e = hipMemcpyAsync(part.data(), w.part, sizeof(double) * part.size(), hipMemcpyDeviceToHost,
-                            w.s)) != hipSuccess ||
-        (e = hipStreamSynchronize(w.s)) != hipSuccess)
+    hipLaunchKernelGGL(g_dots2, dim3(g), dim3(kT), 0, w.s, n, w.r, w.r, b, b, h->part);
+    if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
       return hmv::hip_fail(e, "hmv_gcrm: true residual");
     double rr = 0.0, bb = 0.0;
     for (int i = 0; i < g; ++i) {
-      rr += part[2 * i];
-      bb += part[2 * i + 1];
+      rr += h->part[2 * i];
+      bb += h->part[2 * i + 1];
     }
     tr = std::sqrt(rr) / std::sqrt(bb);
   }
   if (info) {
-    info->nstp = host.step;
-    info->status = host.done ? host.status : HMV_SOLVE_MAXITER;
-    info->relres = host.rnorm / host.bnorm;
+    info->nstp = h->step;
+    info->status = h->status;
+    info->relres = h->rnorm / h->bnorm;
     info->true_relres = tr;
     info->seconds = std::chrono::duration<double>(t1 - t0).count();
     info->outer = 0;
-    info->inner_total = host.step;
+    info->inner_total = h->step;
   }
   return HMV_OK;
 }
@@ -538,32 +529,22 @@ __global__ __launch_bounds__(kT) void g_add_clear(int n, double *__restrict__ u,
   }
 }
 
-struct IrBufs {
-  double *r = nullptr, *d = nullptr, *v = nullptr, *part = nullptr;
-  hipStream_t s = nullptr;
-  ~IrBufs() {
-    for (double *q : {r, d, v, part}) (void)hipFree(q);
-    if (s) (void)hipStreamDestroy(s);
-  }
-};
-
-// r = b - A u and ||r|| / ||b|| (A: the arena a)
-int residual(hmv_arena_s *a, IrBufs &w, const double *b, const double *u, double *rel) {
+// r = b - A u and ||r|| / ||b|| (A: the arena a) on stream s; the partial
+// dots go to h
+int residual(hmv_arena_s *a, hipStream_t s, HmvSolveHost *h, const double *b, const double *u,
+             double *v, double *r, double *rel) {
   const int n = a->nd, g = grid_of(n);
   hipError_t e;
-  if ((e = hmv::enqueue_apply(a, u, w.v, 0.0, nullptr, w.s)) != hipSuccess)
+  if ((e = hmv::enqueue_apply(a, u, v, 0.0, nullptr, s)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_gcr_ir: residual");
-  hipLaunchKernelGGL(g_residual, dim3(g), dim3(kT), 0, w.s, n, b, w.v, w.r);
-  hipLaunchKernelGGL(g_dots2, dim3(g), dim3(kT), 0, w.s, n, w.r, w.r, b, b, w.part);
-  std::vector<double> part(2 * (size_t)g);
-  if ((e = hipMemcpyAsync(part.data(), w.part, sizeof(double) * part.size(), hipMemcpyDeviceToHost,
-                          w.s)) != hipSuccess ||
-      (e = hipStreamSynchronize(w.s)) != hipSuccess)
+  hipLaunchKernelGGL(g_residual, dim3(g), dim3(kT), 0, s, n, b, v, r);
+  hipLaunchKernelGGL(g_dots2, dim3(g), dim3(kT), 0, s, n, r, r, b, b, h->part);
+  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(s)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_gcr_ir: residual");
   double rr = 0.0, bb = 0.0;
   for (int i = 0; i < g; ++i) {
-    rr += part[2 * i];
-    bb += part[2 * i + 1];
+    rr += h->part[2 * i];
+    bb += h->part[2 * i + 1];
   }
   *rel = std::sqrt(rr) / std::sqrt(bb);
   return HMV_OK;
@@ -572,7 +553,7 @@ int residual(hmv_arena_s *a, IrBufs &w, const double *b, const double *u, double
 }  // namespace
 
 extern "C" int hmv_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, double *u, double eps,
-                          double inner_eps, int m, int max_outer, int max_inner, int check_every,
+                          double inner_eps, int m, int max_outer, int max_inner, int /*check_every*/,
                           double *hist, hmv_solve_info *info) {
   if (!a64 || !alow || !b || !u || a64->nd != alow->nd || m < 1 || m > kMaxM || max_outer < 0 ||
       max_inner < 0) {
@@ -581,17 +562,22 @@ extern "C" int hmv_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, double
   }
   const int n = a64->nd, g = grid_of(n);
   const size_t nb = sizeof(double) * (size_t)n;
-  IrBufs w;
+  // everything runs on the stream of the low-precision arena's workspace,
+  // whose ar holds A64 u between the inner solves
+  GcrWork *wp = nullptr;
+  int rc = gcr_work(alow, m, max_inner, wp);
+  if (rc) return rc;
+  GcrWork &w = *wp;
+  HmvSolveHost *h = nullptr;
   hipError_t e;
-  if ((e = hipStreamCreateWithFlags(&w.s, hipStreamNonBlocking)) != hipSuccess ||
-      (e = hipMalloc(&w.r, nb)) != hipSuccess || (e = hipMalloc(&w.d, nb)) != hipSuccess ||
-      (e = hipMalloc(&w.v, nb)) != hipSuccess ||
-      (e = hipMalloc(&w.part, sizeof(double) * 2 * (size_t)g)) != hipSuccess ||
-      (e = hipMemsetAsync(w.d, 0, nb, w.s)) != hipSuccess)
+  if ((!w.ir_r && (e = hipMalloc(&w.ir_r, nb)) != hipSuccess) ||
+      (!w.ir_d && (e = hipMalloc(&w.ir_d, nb)) != hipSuccess) ||
+      (e = hmv::solve_host(alow, w.s, h)) != hipSuccess ||
+      (e = hipMemsetAsync(w.ir_d, 0, nb, w.s)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_gcr_ir: workspace");
   auto t0 = std::chrono::steady_clock::now();
   double rel = 0.0;
-  int rc = residual(a64, w, b, u, &rel);
+  rc = residual(a64, w.s, h, b, u, w.ar, w.ir_r, &rel);
   if (rc) return rc;
   if (hist) hist[0] = rel;
   int outer = 0, inner_total = 0, status = HMV_SOLVE_MAXITER;
@@ -599,13 +585,13 @@ extern "C" int hmv_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, double
   while (status == HMV_SOLVE_MAXITER && rel >= eps && outer < max_outer) {
     // solve Alow d = r to inner_eps with GCR(m), d starting at zero
     hmv_solve_info in{};
-    rc = gcrm_run(alow, w.r, w.d, inner_eps, max_inner, m, check_every, nullptr, &in, false, true);
+    rc = gcrm_run(alow, w.ir_r, w.ir_d, inner_eps, max_inner, m, nullptr, &in, false, true);
     if (rc) return rc;
     inner_total += in.nstp;
     if (in.status == HMV_SOLVE_NONFINITE) status = HMV_SOLVE_NONFINITE;
-    hipLaunchKernelGGL(g_add_clear, dim3(g), dim3(kT), 0, w.s, n, u, w.d);
+    hipLaunchKernelGGL(g_add_clear, dim3(g), dim3(kT), 0, w.s, n, u, w.ir_d);
     ++outer;
-    rc = residual(a64, w, b, u, &rel);
+    rc = residual(a64, w.s, h, b, u, w.ar, w.ir_r, &rel);
     if (rc) return rc;
     if (hist) hist[outer] = rel;
     if (!std::isfinite(rel)) status = HMV_SOLVE_NONFINITE;

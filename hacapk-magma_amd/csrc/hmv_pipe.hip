@@ -16,8 +16,8 @@
 // nor returns (it hands back the initial guess, :188,483-484,595); here the
 // iterate starts at u and is returned in u.  Each step is two fused vector
 // kernels (with their dot products), two one-block scalar kernels and two
-// H-matvecs, captured as one hipGraph; a device flag set on convergence turns
-// the remaining launched steps into no-ops.
+// H-matvecs; the host feeds the steps (hmv_feed.h) and a device flag set on
+// convergence turns those launched after it into no-ops.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,6 +27,7 @@
 
 #include "hmv.h"
 #include "hmv_engine.h"
+#include "hmv_feed.h"
 
 namespace {
 
@@ -37,6 +38,7 @@ constexpr int kND = 5;  // dot products per partial record
 struct PipeState {
   double alpha, beta, zeta, znorm, bnorm, rnorm, eps;
   int step, maxit, done, status;
+  int ticks;  // steps ended, with those that found the solve stopped
 };
 
 __device__ inline double blk_sum(double v, double *sh) {
@@ -149,8 +151,12 @@ __global__ __launch_bounds__(kT) void p_update2(
 
 // stage 0: setup;  1: zeta;  2: beta, alpha, ||r||, step, stop
 __global__ __launch_bounds__(kT) void p_final(int nb, const double *__restrict__ part, PipeState *st,
-                                              int stage, double *__restrict__ hist) {
-  if (st->done && stage != 0) return;
+                                              int stage, double *__restrict__ hist,
+                                              HmvSolveHost *h) {
+  if (st->done && stage != 0) {
+    if (stage == 2 && threadIdx.x == 0) hmv::publish(h, st->ticks += 1, 1);
+    return;
+  }
   __shared__ double sh[4];
   double d[kND];
   const int nd = stage == 0 ? 3 : stage == 1 ? 2 : kND;
@@ -169,6 +175,7 @@ __global__ __launch_bounds__(kT) void p_final(int nb, const double *__restrict__
     st->rnorm = sqrt(d[0]);
     st->bnorm = sqrt(d[2]);
     st->step = 0;
+    st->ticks = 0;
     st->done = 0;
     st->status = HMV_SOLVE_MAXITER;
     if (hist) hist[0] = st->rnorm / st->bnorm;
@@ -184,6 +191,7 @@ __global__ __launch_bounds__(kT) void p_final(int nb, const double *__restrict__
       st->status = HMV_SOLVE_BREAKDOWN;
       st->done = 1;
     }
+    hmv::publish(h, 0, st->done);
   } else if (stage == 1) {
     // both dots zero: the half step (zeta = 0) is taken and stage 2 reports
     // convergence, or breakdown through beta = alpha / zeta
@@ -216,6 +224,7 @@ __global__ __launch_bounds__(kT) void p_final(int nb, const double *__restrict__
       st->status = HMV_SOLVE_BREAKDOWN;
       st->done = 1;
     }
+    hmv::publish(h, st->ticks += 1, st->done);
   }
 }
 
@@ -240,11 +249,7 @@ struct PipeWork {
   double *r = nullptr, *r0 = nullptr, *w = nullptr, *t = nullptr, *v = nullptr, *p = nullptr,
          *sv = nullptr, *z = nullptr, *q = nullptr, *y = nullptr;
   PipeState *st = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
   ~PipeWork() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
     if (s) (void)hipStreamDestroy(s);
     (void)hipFree(mem);
     (void)hipFree(part);
@@ -253,18 +258,18 @@ struct PipeWork {
   }
 };
 
-hipError_t pipe_step(hmv_arena_s *a, PipeWork &w, int n, double *x) {
+hipError_t pipe_step(hmv_arena_s *a, PipeWork &w, int n, double *x, HmvSolveHost *h) {
   const int g = grid_of(n);
   const int *skip = &w.st->done;
   const PipeState *cst = w.st;
   hipLaunchKernelGGL(p_update1, dim3(g), dim3(kT), 0, w.s, n, w.r, w.w, w.t, w.v, w.p, w.sv, w.z,
                      w.q, w.y, w.part, cst);
-  hipLaunchKernelGGL(p_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 1, w.hist);
+  hipLaunchKernelGGL(p_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 1, w.hist, h);
   hipError_t e = hmv::enqueue_apply(a, w.z, w.v, 0.0, skip, w.s);  // v = A z
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(p_update2, dim3(g), dim3(kT), 0, w.s, n, w.p, w.q, w.y, w.t, w.v, w.sv, w.z,
                      w.r0, x, w.r, w.w, w.part, cst);
-  hipLaunchKernelGGL(p_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 2, w.hist);
+  hipLaunchKernelGGL(p_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 2, w.hist, h);
   e = hmv::enqueue_apply(a, w.w, w.t, 0.0, skip, w.s);  // t = A w
   if (e != hipSuccess) return e;
   return hipGetLastError();
@@ -273,21 +278,22 @@ hipError_t pipe_step(hmv_arena_s *a, PipeWork &w, int n, double *x) {
 }  // namespace
 
 extern "C" int hmv_bicgstab_pipe(hmv_arena a, const double *b, double *u, double eps, int maxit,
-                                 int check_every, double *hist, hmv_solve_info *info) {
+                                 int /*check_every*/, double *hist, hmv_solve_info *info) {
   if (!a || !b || !u || maxit < 0) {
     hmv::set_error("hmv_bicgstab_pipe: invalid argument");
     return HMV_ERR_ARG;
   }
-  if (check_every < 1) check_every = 1;
   const int n = a->nd, g = grid_of(n);
   PipeWork w;
+  HmvSolveHost *h = nullptr;
   const size_t nb = sizeof(double) * (size_t)n;
   hipError_t e;
   if ((e = hipStreamCreateWithFlags(&w.s, hipStreamNonBlocking)) != hipSuccess ||
       (e = hipMalloc(&w.mem, nb * 10)) != hipSuccess ||
       (e = hipMalloc(&w.part, sizeof(double) * (size_t)g * kND)) != hipSuccess ||
       (e = hipMalloc(&w.hist, sizeof(double) * ((size_t)maxit + 1))) != hipSuccess ||
-      (e = hipMalloc(&w.st, sizeof(PipeState))) != hipSuccess)
+      (e = hipMalloc(&w.st, sizeof(PipeState))) != hipSuccess ||
+      (e = hmv::solve_host(a, w.s, h)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_bicgstab_pipe: workspace");
   double *m = w.mem;
   w.r = m;
@@ -312,28 +318,15 @@ extern "C" int hmv_bicgstab_pipe(hmv_arena a, const double *b, double *u, double
       (e = hmv::enqueue_apply(a, w.w, w.t, 0.0, nullptr, w.s)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_bicgstab_pipe: setup");
   hipLaunchKernelGGL(p_dots_setup, dim3(g), dim3(kT), 0, w.s, n, w.r, w.w, b, w.part);
-  hipLaunchKernelGGL(p_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 0, w.hist);
-  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess ||
-      (e = hipStreamBeginCapture(w.s, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-    return hmv::hip_fail(e, "hmv_bicgstab_pipe: setup");
-  hipError_t ec = pipe_step(a, w, n, u);
-  e = hipStreamEndCapture(w.s, &w.graph);
-  if (ec != hipSuccess) return hmv::hip_fail(ec, "hmv_bicgstab_pipe: capture");
-  if (e != hipSuccess || (e = hipGraphInstantiate(&w.exec, w.graph, nullptr, nullptr, 0)) != hipSuccess)
-    return hmv::hip_fail(e, "hmv_bicgstab_pipe: graph");
+  hipLaunchKernelGGL(p_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 0, w.hist, h);
+  if ((e = hipGetLastError()) != hipSuccess) return hmv::hip_fail(e, "hmv_bicgstab_pipe: setup");
   PipeState host{};
   int launched = 0;
-  for (;;) {
-    if ((e = hipMemcpyAsync(&host, w.st, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess ||
-        (e = hipStreamSynchronize(w.s)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_bicgstab_pipe: state");
-    if (host.done || launched >= maxit) break;
-    const int burst = std::min(check_every, maxit - launched);
-    for (int i = 0; i < burst; ++i)
-      if ((e = hipGraphLaunch(w.exec, w.s)) != hipSuccess)
-        return hmv::hip_fail(e, "hmv_bicgstab_pipe: launch");
-    launched += burst;
-  }
+  if ((e = hmv::feed(h, w.s, launched, maxit,
+                     [&] { return pipe_step(a, w, n, u, h); })) != hipSuccess ||
+      (e = hipMemcpyAsync(&host, w.st, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess ||
+      (e = hipStreamSynchronize(w.s)) != hipSuccess)
+    return hmv::hip_fail(e, "hmv_bicgstab_pipe: steps");
   auto t1 = std::chrono::steady_clock::now();
   if (hist) {
     std::fill(hist, hist + maxit + 1, NAN);

@@ -8,11 +8,10 @@
 //   u += alpha p + zeta t;  r = t - zeta s;  beta = alpha/zeta (r^,r_new)/(r^,r)
 // The reference copies p->kp and t->kt (no preconditioner) and returns every
 // dot product to the host; here the scalars stay on the device, dots are
-// fused (two per pass, deterministic two-level reduction), one iteration is
-// captured as a hipGraph, and the host reads the residual every
-// `check_every` iterations.  A device flag set on convergence turns the
-// remaining launched iterations into no-ops, so the result equals stopping
-// at the first converged iteration.
+// fused (two per pass, deterministic two-level reduction), and the host feeds
+// the iterations (hmv_feed.h).  A device flag set on convergence turns those
+// launched after it into no-ops, so the result equals stopping at the first
+// converged iteration.
 #include <hip/hip_runtime.h>
 
 #include <chrono>
@@ -22,11 +21,12 @@
 
 #include "hmv.h"
 #include "hmv_engine.h"
+#include "hmv_feed.h"
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kMaxBlocks = 512;
+constexpr int kMaxBlocks = kSolveMaxBlocks;
 
 struct SolveState {
   double alpha, beta, zeta;
@@ -39,6 +39,7 @@ struct SolveState {
   int done;       // 1 once converged / stopped
   int status;     // HMV_SOLVE_*
   int maxit;
+  int ticks;      // iterations ended, with those that found the solve stopped
 };
 
 __device__ inline double block_sum(double v, double *sh) {
@@ -102,12 +103,28 @@ __device__ inline void reduce_parts(int nb, const double *part, SolveState *st, 
 
 __device__ inline bool finite(double v) { return isfinite(v); }
 
-// stage: 0 setup (d0 = (r,r), d1 = (b,b)), 1 alpha, 2 zeta, 3 beta,
+__device__ inline void publish(HmvSolveHost *h, const SolveState *st) {
+  if (st->done) {
+    h->step = st->step;
+    h->status = st->status;
+    h->rnorm = st->rnorm;
+    h->bnorm = st->bnorm;
+  }
+  hmv::publish(h, st->ticks, st->done);
+}
+
+// stage: 0 setup (d0 = (r,r), d1 = (b,b)), 3 beta and the stopping test,
 // 4 residual replacement (d0 = (r^, r), d1 = (r, r) of the true residual)
 __global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__restrict__ part,
                                                     SolveState *st, int stage,
-                                                    double *__restrict__ hist) {
-  if (st->done && stage != 0 && stage != 4) return;
+                                                    double *__restrict__ hist, HmvSolveHost *h) {
+  if (st->done && stage != 0 && stage != 4) {
+    if (threadIdx.x == 0) {
+      st->ticks += 1;
+      publish(h, st);
+    }
+    return;
+  }
   __shared__ double sh[4];
   reduce_parts(nb, part, st, sh);
   if (threadIdx.x != 0) return;
@@ -117,6 +134,7 @@ __global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__rest
     st->rnorm = sqrt(st->d0);
     st->bnorm = sqrt(st->d1);
     st->step = 0;
+    st->ticks = 0;
     st->alpha = 0.0;
     st->beta = 0.0;
     st->zeta = 0.0;
@@ -130,23 +148,6 @@ __global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__rest
       st->status = HMV_SOLVE_CONVERGED;
       st->done = 1;
     } else if (st->maxit <= 0) {
-      st->done = 1;
-    }
-  } else if (stage == 1) {
-    const double zden = st->d0;
-    st->alpha = st->rr / zden;
-    if (zden == 0.0 || !finite(st->alpha)) {
-      st->status = finite(zden) ? HMV_SOLVE_BREAKDOWN : HMV_SOLVE_NONFINITE;
-      st->done = 1;
-    }
-  } else if (stage == 2) {
-    const double znom = st->d0, zden = st->d1;
-    // s = A t = 0 (both dots zero): t is the residual of u + alpha p; zeta = 0
-    // takes that half step and stage 3 decides (converged, else breakdown)
-    const bool half = zden == 0.0 && znom == 0.0;
-    st->zeta = half ? 0.0 : znom / zden;
-    if (!half && (zden == 0.0 || !finite(st->zeta))) {
-      st->status = finite(zden) ? HMV_SOLVE_BREAKDOWN : HMV_SOLVE_NONFINITE;
       st->done = 1;
     }
   } else if (stage == 4) {
@@ -174,6 +175,7 @@ __global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__rest
     st->rr = rr_new;
     st->rnorm = sqrt(st->d1);
     st->step += 1;
+    st->ticks += 1;
     if (hist) hist[st->step] = st->rnorm / st->bnorm;
     if (!finite(st->rnorm)) {
       st->status = HMV_SOLVE_NONFINITE;
@@ -190,6 +192,7 @@ __global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__rest
       st->done = 1;
     }
   }
+  publish(h, st);
 }
 
 // p = r + beta (p - zeta v)
@@ -333,12 +336,6 @@ struct HmvSolveWork {
   double *hist = nullptr;
   int hist_cap = 0;
   SolveState *st = nullptr;
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
-  const double *g_b = nullptr;  // vectors the graph was captured with
-  double *g_u = nullptr;
-  hmv_arena_s *g_arena = nullptr;
-  double *g_hist = nullptr;
 };
 
 namespace hmv {
@@ -346,8 +343,6 @@ namespace hmv {
 void free_solve_work(hmv_arena_s *a) {
   HmvSolveWork *w = a->solve;
   if (!w) return;
-  if (w->exec) (void)hipGraphExecDestroy(w->exec);
-  if (w->graph) (void)hipGraphDestroy(w->graph);
   if (w->stream) (void)hipStreamDestroy(w->stream);
   (void)hipFree(w->r);
   (void)hipFree(w->rhat);
@@ -394,18 +389,12 @@ int ensure_work(hmv_arena_s *a, int hist_need) {
     if ((e = hipMalloc(&w->hist, sizeof(double) * hist_need)) != hipSuccess)
       return hmv::hip_fail(e, "solver history");
     w->hist_cap = hist_need;
-    if (w->exec) {
-      (void)hipGraphExecDestroy(w->exec);
-      (void)hipGraphDestroy(w->graph);
-      w->exec = nullptr;
-      w->graph = nullptr;
-    }
   }
   return HMV_OK;
 }
 
 // Enqueues one BiCGSTAB iteration on w->stream.
-hipError_t enqueue_iteration(hmv_arena_s *a, HmvSolveWork *w, double *u) {
+hipError_t enqueue_iteration(hmv_arena_s *a, HmvSolveWork *w, double *u, HmvSolveHost *h) {
   const int n = w->n, g = grid_for(n);
   hipStream_t s = w->stream;
   const int *skip = &w->st->done;
@@ -425,29 +414,31 @@ hipError_t enqueue_iteration(hmv_arena_s *a, HmvSolveWork *w, double *u) {
   hipLaunchKernelGGL(k_update_ur, dim3(g), dim3(kThreads), 0, s, n, g, w->p, w->t, w->s, w->rhat,
                      u, w->r, (const double *)w->part, part2, w->st);
   hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, (const double *)part2, w->st, 3,
-                     w->hist);
+                     w->hist, h);
   return hipGetLastError();
 }
 
 // Core BiCGSTAB; b, u device vectors.  hist_host may be null.
 // zero_guess: u is known to be zero, so r = b without the product A u.
+// drain: wait for the stream at the end (else iterations that found the
+// solve stopped may still be on it).
 int run_bicgstab(hmv_arena_s *a, const double *b, double *u, double eps, int maxit,
-                 int check_every, double *hist_host, hmv_solve_info *info, bool use_graph,
-                 bool zero_guess) {
+                 double *hist_host, hmv_solve_info *info, bool zero_guess, bool drain) {
   int rc = ensure_work(a, maxit + 1);
   if (rc) return rc;
   HmvSolveWork *w = a->solve;
   const int n = w->n, g = grid_for(n);
   hipStream_t s = w->stream;
   hipError_t e;
-  if (check_every < 1) check_every = 1;
   auto t0 = std::chrono::steady_clock::now();
 
   // r = b - A u; r^ = r; p = v = 0; rr = (r,r), bnorm = sqrt((b,b)) on device
   SolveState init{};
   init.eps = eps;
   init.maxit = maxit;
-  SolveState host{};
+  HmvSolveHost *h = nullptr;
+  if ((e = hmv::solve_host(a, s, h)) != hipSuccess)
+    return hmv::hip_fail(e, "bicgstab: workspace");
   if ((e = hipMemcpyAsync(w->st, &init, sizeof(init), hipMemcpyHostToDevice, s)) != hipSuccess)
     return hmv::hip_fail(e, "bicgstab: state upload");
   if (!zero_guess && (e = hmv::enqueue_apply(a, u, w->r, 0.0, nullptr, s)) != hipSuccess)
@@ -456,87 +447,50 @@ int run_bicgstab(hmv_arena_s *a, const double *b, double *u, double eps, int max
                      zero_guess ? 1 : 0);
   hipLaunchKernelGGL(k_dots, dim3(g), dim3(kThreads), 0, s, n, w->r, w->r, b, b, w->part,
                      (const SolveState *)nullptr);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 0, w->hist);
+  hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 0, w->hist,
+                     h);
   if ((e = hipGetLastError()) != hipSuccess) return hmv::hip_fail(e, "bicgstab: setup launch");
 
-  // graph of one iteration (re-captured when the vectors or arena change)
-  if (use_graph && (w->g_u != u || w->g_arena != a || !w->exec)) {
-    if (w->exec) {
-      (void)hipGraphExecDestroy(w->exec);
-      (void)hipGraphDestroy(w->graph);
-      w->exec = nullptr;
-      w->graph = nullptr;
-    }
-    if ((e = hipStreamSynchronize(s)) != hipSuccess) return hmv::hip_fail(e, "bicgstab: sync");
-    if ((e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-      return hmv::hip_fail(e, "bicgstab: begin capture");
-    hipError_t ec = enqueue_iteration(a, w, u);
-    hipGraph_t graph = nullptr;
-    e = hipStreamEndCapture(s, &graph);
-    if (ec != hipSuccess) return hmv::hip_fail(ec, "bicgstab: capture");
-    if (e != hipSuccess) return hmv::hip_fail(e, "bicgstab: end capture");
-    w->graph = graph;
-    if ((e = hipGraphInstantiate(&w->exec, graph, nullptr, nullptr, 0)) != hipSuccess)
-      return hmv::hip_fail(e, "bicgstab: instantiate");
-    w->g_u = u;
-    w->g_arena = a;
-  }
-
   int launched = 0;
-  while (launched < maxit) {
-    const int burst = std::min(check_every, maxit - launched);
-    for (int k = 0; k < burst; ++k) {
-      if (use_graph)
-        e = hipGraphLaunch(w->exec, s);
-      else
-        e = enqueue_iteration(a, w, u);
-      if (e != hipSuccess) return hmv::hip_fail(e, "bicgstab: iteration launch");
-    }
-    launched += burst;
-    if ((e = hipMemcpyAsync(&host, w->st, sizeof(host), hipMemcpyDeviceToHost, s)) != hipSuccess ||
-        (e = hipStreamSynchronize(s)) != hipSuccess)
-      return hmv::hip_fail(e, "bicgstab: state read");
-    if (host.done) break;
-  }
-  if ((e = hipMemcpyAsync(&host, w->st, sizeof(host), hipMemcpyDeviceToHost, s)) != hipSuccess ||
-      (e = hipStreamSynchronize(s)) != hipSuccess)
-    return hmv::hip_fail(e, "bicgstab: state read");
+  e = hmv::feed(h, s, launched, maxit,
+                [&] { return enqueue_iteration(a, w, u, h); });
+  if (e == hipSuccess && (drain || !hmv::stopped(h))) e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return hmv::hip_fail(e, "bicgstab: iterations");
   auto t1 = std::chrono::steady_clock::now();
 
   if (hist_host) {
     std::vector<double> hh(maxit + 1, NAN);
-    if ((e = hipMemcpy(hh.data(), w->hist, sizeof(double) * (host.step + 1), hipMemcpyDeviceToHost)) !=
+    if ((e = hipMemcpy(hh.data(), w->hist, sizeof(double) * (h->step + 1), hipMemcpyDeviceToHost)) !=
         hipSuccess)
       return hmv::hip_fail(e, "bicgstab: history");
     std::memcpy(hist_host, hh.data(), sizeof(double) * (maxit + 1));
   }
   if (info) {
-    info->nstp = host.step;
-    info->status = host.done ? host.status : HMV_SOLVE_MAXITER;
-    info->relres = host.rnorm / host.bnorm;
+    info->nstp = h->step;
+    info->status = h->status;
+    info->relres = h->rnorm / h->bnorm;
     info->seconds = std::chrono::duration<double>(t1 - t0).count();
     info->outer = 0;
-    info->inner_total = host.step;
+    info->inner_total = h->step;
   }
   return HMV_OK;
 }
 
-// ||b - A u|| / ||b|| with the arena `a` (device vectors), using w->r2.
-int true_relres(hmv_arena_s *a, const double *b, const double *u, double *out) {
+// ||b - A u|| / ||b|| with the arena `a` (device vectors) on stream s, using
+// a's r2; the partial dots go to h.
+int true_relres(hmv_arena_s *a, const double *b, const double *u, double *out, hipStream_t s,
+                HmvSolveHost *h) {
   HmvSolveWork *w = a->solve;
   const int n = w->n, g = grid_for(n);
-  hipStream_t s = w->stream;
   hipError_t e;
   if ((e = hmv::enqueue_apply(a, u, w->r2, 0.0, nullptr, s)) != hipSuccess)
     return hmv::hip_fail(e, "true residual apply");
   hipLaunchKernelGGL(k_residual, dim3(g), dim3(kThreads), 0, s, n, b, w->r2);
-  hipLaunchKernelGGL(k_dots, dim3(g), dim3(kThreads), 0, s, n, w->r2, w->r2, b, b, w->part,
+  hipLaunchKernelGGL(k_dots, dim3(g), dim3(kThreads), 0, s, n, w->r2, w->r2, b, b, h->part,
                      (const SolveState *)nullptr);
-  std::vector<double> part(2 * g);
-  if ((e = hipMemcpyAsync(part.data(), w->part, sizeof(double) * 2 * g, hipMemcpyDeviceToHost, s)) !=
-          hipSuccess ||
-      (e = hipStreamSynchronize(s)) != hipSuccess)
+  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(s)) != hipSuccess)
     return hmv::hip_fail(e, "true residual");
+  const double *part = h->part;
   double rr = 0.0, bb = 0.0;
   for (int i = 0; i < g; ++i) {
     rr += part[2 * i];
@@ -550,8 +504,8 @@ int true_relres(hmv_arena_s *a, const double *b, const double *u, double *out) {
 
 extern "C" {
 
-int hmv_bicgstab(hmv_arena a, const double *b, double *u, double eps, int maxit, int check_every,
-                 double *hist, hmv_solve_info *info) {
+int hmv_bicgstab(hmv_arena a, const double *b, double *u, double eps, int maxit,
+                 int /*check_every*/, double *hist, hmv_solve_info *info) {
   if (!a || !b || !u) {
     hmv::set_error("hmv_bicgstab: null argument");
     return HMV_ERR_ARG;
@@ -561,16 +515,16 @@ int hmv_bicgstab(hmv_arena a, const double *b, double *u, double eps, int maxit,
     return HMV_ERR_ARG;
   }
   hmv_solve_info loc{};
-  int rc = run_bicgstab(a, b, u, eps, maxit, check_every, hist, &loc, true, false);
+  int rc = run_bicgstab(a, b, u, eps, maxit, hist, &loc, false, true);
   if (rc) return rc;
-  rc = true_relres(a, b, u, &loc.true_relres);
+  rc = true_relres(a, b, u, &loc.true_relres, a->solve->stream, a->solve_host);
   if (rc) return rc;
   if (info) *info = loc;
   return HMV_OK;
 }
 
 int hmv_bicgstab_ir(hmv_arena a64, hmv_arena alow, const double *b, double *u, double eps,
-                    double inner_eps, int max_outer, int max_inner, int check_every, double *hist,
+                    double inner_eps, int max_outer, int max_inner, int /*check_every*/, double *hist,
                     hmv_solve_info *info) {
   if (!a64 || !alow || !b || !u || a64->nd != alow->nd) {
     hmv::set_error("hmv_bicgstab_ir: invalid arguments");
@@ -583,36 +537,35 @@ int hmv_bicgstab_ir(hmv_arena a64, hmv_arena alow, const double *b, double *u, d
   HmvSolveWork *w64 = a64->solve;
   HmvSolveWork *wl = alow->solve;
   const int n = a64->nd, g = grid_for(n);
+  hipStream_t s = wl->stream;  // of the residuals too
+  HmvSolveHost *h = nullptr;
   hipError_t e;
+  if ((e = hmv::solve_host(alow, s, h)) != hipSuccess) return hmv::hip_fail(e, "ir: workspace");
   auto t0 = std::chrono::steady_clock::now();
   double rel = 0.0;
   // outer residual r2 = b - A64 u (in w64->r2), relres
-  rc = true_relres(a64, b, u, &rel);
+  rc = true_relres(a64, b, u, &rel, s, h);
   if (rc) return rc;
   if (hist) hist[0] = rel;
   int outer = 0, inner_total = 0, status = HMV_SOLVE_MAXITER;
   if (!std::isfinite(rel)) status = HMV_SOLVE_NONFINITE;
   while (status == HMV_SOLVE_MAXITER && rel >= eps && outer < max_outer) {
     // correction d (wl->x2) = 0; solve Alow d = r2 with the inner BiCGSTAB
-    if ((e = hipStreamSynchronize(w64->stream)) != hipSuccess)
-      return hmv::hip_fail(e, "ir: sync");
-    hipLaunchKernelGGL(k_fill, dim3(g), dim3(kThreads), 0, wl->stream, n, wl->x2, 0.0);
+    hipLaunchKernelGGL(k_fill, dim3(g), dim3(kThreads), 0, s, n, wl->x2, 0.0);
     hmv_solve_info in{};
-    rc = run_bicgstab(alow, w64->r2, wl->x2, inner_eps, max_inner, check_every, nullptr, &in, true,
-                      true);
+    rc = run_bicgstab(alow, w64->r2, wl->x2, inner_eps, max_inner, nullptr, &in, true,
+                      false);
     if (rc) return rc;
     inner_total += in.nstp;
-    if ((e = hipStreamSynchronize(wl->stream)) != hipSuccess) return hmv::hip_fail(e, "ir: sync");
-    hipLaunchKernelGGL(k_add_clear, dim3(g), dim3(kThreads), 0, w64->stream, n, u, wl->x2);
+    hipLaunchKernelGGL(k_add_clear, dim3(g), dim3(kThreads), 0, s, n, u, wl->x2);
     ++outer;
-    rc = true_relres(a64, b, u, &rel);
+    rc = true_relres(a64, b, u, &rel, s, h);
     if (rc) return rc;
     if (hist) hist[outer] = rel;
     if (!std::isfinite(rel)) status = HMV_SOLVE_NONFINITE;
     if (in.status == HMV_SOLVE_NONFINITE) status = HMV_SOLVE_NONFINITE;
   }
   if (status == HMV_SOLVE_MAXITER && rel < eps) status = HMV_SOLVE_CONVERGED;
-  if ((e = hipStreamSynchronize(w64->stream)) != hipSuccess) return hmv::hip_fail(e, "ir: sync");
   auto t1 = std::chrono::steady_clock::now();
   if (info) {
     info->nstp = inner_total;
@@ -652,7 +605,9 @@ int hmv_bicgstab_ru(hmv_arena a64, hmv_arena alow, const double *b, double *u, d
   SolveState init{};
   init.eps = eps;
   init.maxit = maxit;
-  SolveState host{};
+  HmvSolveHost *h = nullptr;
+  if ((e = hmv::solve_host(alow, s, h)) != hipSuccess)
+    return hmv::hip_fail(e, "bicgstab_ru: workspace");
   // r = b - A64 u, r^ = r, p = v = 0
   if ((e = hipMemcpyAsync(w->st, &init, sizeof(init), hipMemcpyHostToDevice, s)) != hipSuccess ||
       (e = hmv::enqueue_apply(a64, u, w->r, 0.0, nullptr, s)) != hipSuccess)
@@ -660,41 +615,22 @@ int hmv_bicgstab_ru(hmv_arena a64, hmv_arena alow, const double *b, double *u, d
   hipLaunchKernelGGL(k_init, dim3(g), dim3(kThreads), 0, s, n, b, w->r, w->rhat, w->p, w->v, 0);
   hipLaunchKernelGGL(k_dots, dim3(g), dim3(kThreads), 0, s, n, w->r, w->r, b, b, w->part,
                      (const SolveState *)nullptr);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 0, w->hist);
+  hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 0, w->hist,
+                     h);
   if ((e = hipGetLastError()) != hipSuccess) return hmv::hip_fail(e, "bicgstab_ru: setup");
-  if (w->g_u != u || w->g_arena != alow || !w->exec) {
-    if (w->exec) {
-      (void)hipGraphExecDestroy(w->exec);
-      (void)hipGraphDestroy(w->graph);
-      w->exec = nullptr;
-      w->graph = nullptr;
-    }
-    if ((e = hipStreamSynchronize(s)) != hipSuccess ||
-        (e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-      return hmv::hip_fail(e, "bicgstab_ru: capture");
-    hipError_t ec = enqueue_iteration(alow, w, u);
-    hipGraph_t graph = nullptr;
-    e = hipStreamEndCapture(s, &graph);
-    if (ec != hipSuccess) return hmv::hip_fail(ec, "bicgstab_ru: capture");
-    if (e != hipSuccess) return hmv::hip_fail(e, "bicgstab_ru: end capture");
-    w->graph = graph;
-    if ((e = hipGraphInstantiate(&w->exec, graph, nullptr, nullptr, 0)) != hipSuccess)
-      return hmv::hip_fail(e, "bicgstab_ru: instantiate");
-    w->g_u = u;
-    w->g_arena = alow;
-  }
+  SolveState host{};
   auto read_state = [&]() -> hipError_t {
     hipError_t re = hipMemcpyAsync(&host, w->st, sizeof(host), hipMemcpyDeviceToHost, s);
     return re == hipSuccess ? hipStreamSynchronize(s) : re;
   };
   if ((e = read_state()) != hipSuccess) return hmv::hip_fail(e, "bicgstab_ru: state");
   double r_last = host.rnorm;
-  int updates = 0;
+  int updates = 0, launched = 0;
   while (!host.done) {  // done: converged on the true residual, or stopped
     const int burst = std::min(check_every, std::max(1, maxit - host.step));
-    for (int k = 0; k < burst; ++k)
-      if ((e = hipGraphLaunch(w->exec, s)) != hipSuccess)
-        return hmv::hip_fail(e, "bicgstab_ru: iteration launch");
+    if ((e = hmv::feed(h, s, launched, launched + burst,
+                       [&] { return enqueue_iteration(alow, w, u, h); })) != hipSuccess)
+      return hmv::hip_fail(e, "bicgstab_ru: iterations");
     if ((e = read_state()) != hipSuccess) return hmv::hip_fail(e, "bicgstab_ru: state");
     const bool sloppy_done = host.done && host.status == HMV_SOLVE_CONVERGED;
     if (host.done && !sloppy_done) break;  // breakdown, non-finite or out of steps
@@ -705,7 +641,8 @@ int hmv_bicgstab_ru(hmv_arena a64, hmv_arena alow, const double *b, double *u, d
       hipLaunchKernelGGL(k_residual, dim3(g), dim3(kThreads), 0, s, n, b, w->r);
       hipLaunchKernelGGL(k_dots, dim3(g), dim3(kThreads), 0, s, n, w->rhat, w->r, w->r, w->r,
                          w->part, (const SolveState *)nullptr);
-      hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 4, w->hist);
+      hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 4, w->hist,
+                         h);
       if ((e = read_state()) != hipSuccess) return hmv::hip_fail(e, "bicgstab_ru: state");
       ++updates;
       r_last = host.rnorm;
@@ -720,7 +657,7 @@ int hmv_bicgstab_ru(hmv_arena a64, hmv_arena alow, const double *b, double *u, d
   loc.seconds = std::chrono::duration<double>(t1 - t0).count();
   loc.outer = updates;
   loc.inner_total = host.step;
-  rc = true_relres(a64, b, u, &loc.true_relres);
+  rc = true_relres(a64, b, u, &loc.true_relres, s, h);
   if (rc) return rc;
   if (loc.status == HMV_SOLVE_CONVERGED && !(loc.true_relres < eps)) loc.status = HMV_SOLVE_MAXITER;
   if (info) *info = loc;

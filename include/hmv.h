@@ -225,15 +225,16 @@ typedef struct {
 /* Unpreconditioned BiCGSTAB (m_HACApK_solve.f90:342-449) on device vectors:
  * u (initial guess in, solution out), b.  Stops when ||r||/||b|| < eps or
  * after maxit steps.  hist (host, may be NULL) receives maxit+1 relative
- * residuals (hist[0] initial).  check_every: residual read-back period in
- * iterations (1 = every iteration, like the reference). */
+ * residuals (hist[0] initial).  check_every: accepted for callers written
+ * for a read-back period; the host follows the stopping test of every
+ * iteration, and no value changes the result or the time. */
 int hmv_bicgstab(hmv_arena a, const double *b, double *u, double eps, int maxit, int check_every,
                  double *hist, hmv_solve_info *info);
 
 /* Mixed-precision iterative refinement: the FP64 residual r = b - A64 u, an
  * inner BiCGSTAB with the low-precision arena `alow` to inner_eps, u += d;
- * repeats until ||b - A64 u||/||b|| < eps or max_outer steps.  check_every:
- * residual read-back period of the inner solver.
+ * repeats until ||b - A64 u||/||b|| < eps or max_outer steps.  check_every as
+ * for hmv_bicgstab.
  * hist (host, may be NULL) receives max_outer+1 outer relative residuals. */
 int hmv_bicgstab_ir(hmv_arena a64, hmv_arena alow, const double *b, double *u, double eps,
                     double inner_eps, int max_outer, int max_inner, int check_every, double *hist,
@@ -254,7 +255,8 @@ int hmv_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, double *u, double
  * in FP64; whenever the iterated residual has fallen by `delta` (0..1) since
  * the last replacement, or the iteration reports convergence, the true
  * residual b - A64 u (FP64 arena) replaces it without restarting.  Stops on
- * ||b - A64 u|| / ||b|| < eps.  info->outer = number of replacements. */
+ * ||b - A64 u|| / ||b|| < eps; the residual is looked at every check_every
+ * iterations.  info->outer = number of replacements. */
 int hmv_bicgstab_ru(hmv_arena a64, hmv_arena alow, const double *b, double *u, double eps,
                     int maxit, int check_every, double delta, hmv_solve_info *info);
 
@@ -312,7 +314,7 @@ int hmv_block_bicgstab_ir(hmv_arena a64, hmv_arena alow, int k, const double *b,
 /* One BiCGSTAB per instance of a multi-instance arena (hmv_arena_build_multi),
  * all advancing together: one H-matvec launch per phase covers every
  * instance, scalars and stopping are per instance (a finished instance is
- * frozen), one hipGraph per iteration.  b, u: the instances' vectors
+ * frozen).  b, u: the instances' vectors
  * concatenated.  inst (ninst entries, may be NULL) receives per-instance
  * steps, status and residuals; inst_seconds (may be NULL) the wall time at
  * which each instance was seen finished (residual read-back every
@@ -327,7 +329,7 @@ int hmv_multi_bicgstab(hmv_arena a, const double *b, double *u, double eps, int 
  * residual r_i = b_i - A64_i u_i on a64; an instance with
  * ||r_i||/||b_i|| < eps stops (converged); the others solve A_low d = r by
  * one BiCGSTAB per instance in lockstep (hmv_multi_bicgstab's iteration,
- * one hipGraph per iteration, each instance to inner_eps, at most
+ * each instance to inner_eps, at most
  * max_inner iterations; stopped instances skip their products) and take
  * u += d.  At most max_outer steps.  inst receives per instance the inner
  * iterations summed over the outer steps, the status and the final FP64
@@ -342,9 +344,9 @@ int hmv_multi_bicgstab_ir(hmv_arena a64, hmv_arena alow, const double *b, double
 /* The same refinement per instance with GCR(m) inner solves (1 <= m <=
  * HMV_GCR_MAX_M): one GCR(m) per running instance in lockstep, the steps of
  * hmv_gcrm (m_HACApK_solve.f90:506-571) with each instance's own alpha,
- * betas and projections, one hipGraph per step, each instance to
- * inner_eps, at most max_inner steps.  inst's nstp counts the inner steps
- * (one product each).  No reference counterpart. */
+ * betas and projections, each instance to
+ * inner_eps, at most max_inner steps; check_every as for hmv_bicgstab.
+ * inst's nstp counts the inner steps (one product each).  No reference counterpart. */
 int hmv_multi_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, double *u, double eps,
                      double inner_eps, int m, int max_outer, int max_inner, int check_every,
                      hmv_column_info *inst, double *inst_seconds, hmv_solve_info *info);

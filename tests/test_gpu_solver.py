@@ -181,3 +181,55 @@ def test_reference_named_pipelined_bicgstab(gpu, O, sphere3, variant):
     A = O.dense(hm)
     assert lrtrn == 0 and nstp > 0
     assert np.linalg.norm(A @ u - b) / np.linalg.norm(b) < 5e-8
+
+
+def _solve_calls(H, a64, alow, m64, mlow, b, bm, maxit, ce):
+    """Every solver with maxit (inner) iterations: iterates, steps, states."""
+    B = np.stack([b, 2.0 * b[::-1]], axis=1)
+    kw = dict(eps=1e-9, check_every=ce)
+    ir = dict(kw, inner_eps=1e-3, max_outer=3, max_inner=maxit)
+    return {
+        "bicgstab": a64.bicgstab(b, maxit=maxit, **kw),
+        "pipe": a64.bicgstab_pipe(b, maxit=maxit, **kw),
+        "gcrm": a64.gcrm(b, maxit=maxit, mreset=3, **kw),
+        "block": a64.block_bicgstab(B, maxit=maxit, **kw),
+        "multi": m64.bicgstab_multi(bm, maxit=maxit, **kw),
+        "bicgstab_ir": H.bicgstab_ir(a64, alow, b, **ir),
+        "gcr_ir": H.gcr_ir(a64, alow, b, m=3, **ir),
+        "block_ir": H.block_bicgstab_ir(a64, alow, B, **ir),
+        "multi_bicgstab_ir": H.multi_bicgstab_ir(m64, mlow, bm, **ir),
+        "multi_gcr_ir": H.multi_gcr_ir(m64, mlow, bm, m=3, **ir),
+    }
+
+
+# one, two (the launches that go ahead of the last iteration seen to end)
+# and three iterations, and more than any of the solves needs
+@pytest.mark.parametrize("maxit", [1, 2, 3, 400])
+def test_fed_iterations(gpu, sphere3, maxit):
+    """The iterations launched ahead of the stop change nothing: iterates,
+    steps and states are the same bits for every check_every and call after
+    call, no solve takes more than maxit steps, and one cut off at maxit is
+    at the iterate that the longer solve had there (its history is a prefix
+    of that one's)."""
+    a64, alow = gpu.Arena(sphere3, "f64"), gpu.Arena(sphere3, "f32")
+    m64, mlow = gpu.MultiArena([sphere3, sphere3], "f64"), gpu.MultiArena([sphere3, sphere3], "f32")
+    b = gpu.uniform(31, sphere3.nd)
+    bm = np.concatenate([b, gpu.uniform(32, sphere3.nd)])
+    first = _solve_calls(gpu, a64, alow, m64, mlow, b, bm, maxit, 1)
+    for ce in (1, 2, 8):
+        again = _solve_calls(gpu, a64, alow, m64, mlow, b, bm, maxit, ce)
+        for name, r in again.items():
+            assert np.array_equal(r[0], first[name][0]), (name, ce)
+            i0, i1 = (next(v for v in t[::-1] if isinstance(v, dict)) for t in (first[name], r))
+            assert i0["nstp"] == i1["nstp"] and i0["status"] == i1["status"], (name, ce)
+            if not name.endswith("_ir"):
+                assert i1["nstp"] <= maxit and (maxit > 3 or i1["status_name"] == "maxiter")
+                assert maxit <= 3 or i1["status_name"] == "converged"
+    if maxit <= 3:
+        for name in ("bicgstab", "pipe", "gcrm"):
+            kw = dict(mreset=3) if name == "gcrm" else {}
+            long = {"bicgstab": a64.bicgstab, "pipe": a64.bicgstab_pipe, "gcrm": a64.gcrm}[name](
+                b, eps=1e-9, maxit=400, **kw)
+            assert np.array_equal(first[name][2], long[2][:maxit + 1]), name
+    for a in (a64, alow, m64, mlow):
+        a.free()
