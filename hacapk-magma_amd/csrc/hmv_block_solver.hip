@@ -716,6 +716,7 @@ __global__ __launch_bounds__(kT) void ks_update_ur(
 
 struct SegWork {
   int nseg = 0, nblk = 0;
+  int maxblk = 0;  // blocks of the instance with the most
   int lanes = 1;  // threads that sum the blocks of one instance
   int64_t n = 0;
   hipStream_t s = nullptr;
@@ -805,10 +806,11 @@ int seg_setup(hmv_arena_s *a, SegWork &w, std::vector<int> &bstart, const char *
     const int end = a->seg[sgi + 1];
     for (int64_t i = a->seg[sgi]; i < end; i += chunk)
       tb.push_back(SegBlock{sgi, (int)i, (int)std::min<int64_t>(end, i + chunk), 0});
-    while (w.lanes < 64 && 4 * w.lanes < (int)tb.size() - bstart[sgi]) w.lanes *= 2;
+    w.maxblk = std::max(w.maxblk, (int)tb.size() - bstart[sgi]);
   }
   bstart[w.nseg] = (int)tb.size();
   w.nblk = (int)tb.size();
+  while (w.lanes < 64 && 4 * w.lanes < w.maxblk) w.lanes *= 2;
   const size_t nbytes = sizeof(double) * (size_t)w.n;
   hipError_t e;
   if ((e = hipStreamCreateWithFlags(&w.s, hipStreamNonBlocking)) != hipSuccess ||
@@ -1106,11 +1108,13 @@ namespace {
 
 constexpr int kGcrM = HMV_GCR_MAX_M;
 constexpr int kGroup = 4;  // slots per block row of the beta dots
+constexpr int kMaxBetaB = 128;  // blocks of an instance whose partials every block may sum
+static_assert(kT == 8 * kGcrM, "8 threads sum the partials of a slot's beta");
 
 struct SgInst {
   double alpha, rnorm, bnorm;
   double capap[kGcrM];
-  double beta[kGcrM];
+  double beta[kGcrM];  // of instances with more than kMaxBetaB blocks (sg_betas)
   int step, done, status, pad;
 };
 
@@ -1163,18 +1167,20 @@ __global__ __launch_bounds__(kT) void sg_update_ur(const SegBlock *__restrict__ 
                                                    const double *__restrict__ apart,
                                                    double *__restrict__ rpart, SgInst *inst,
                                                    const SgGlobal *gs) {
-  if (gs->all_done) return;
   __shared__ double sh[4];
   const SegBlock B = tb[blockIdx.x];
+  const int all_done = gs->all_done, ik = gs->ikn;  // the slot of this step
+  hmv::together(B.seg | all_done | ik, 0.0, 0.0, 0.0);
+  if (all_done) return;
   const int s = B.seg;
-  if (inst[s].done) return;  // the stage-2 pass skips stopped instances
-  const int b0 = bstart[s], b1 = bstart[s + 1];
-  const int ik = gs->ikn;  // the slot of this step
+  const int done = inst[s].done, b0 = bstart[s], b1 = bstart[s + 1];
   const double *pk = p + (size_t)ik * n, *q = ap + (size_t)ik * n;
   // the first elements are under way while the partials are summed
   int i = B.beg + threadIdx.x;
   const int i0 = min(i, B.end - 1);
   double uv = u[i0], pv = pk[i0], rv = r[i0], qv = q[i0];
+  hmv::together(done | b0 | b1, uv, pv, rv, qv, 0.0, 0.0, 0.0);
+  if (done) return;  // the stage-2 pass skips stopped instances
   double t0 = 0.0, t1 = 0.0;
   for (int b = b0 + (int)threadIdx.x; b < b1; b += kT) {
     t0 += apart[2 * (size_t)b];
@@ -1219,11 +1225,13 @@ __global__ __launch_bounds__(kT) void sg_dots_beta(const SegBlock *__restrict__ 
                                                    double *__restrict__ part,
                                                    const SgInst *__restrict__ inst,
                                                    const SgGlobal *gs) {
-  if (gs->all_done) return;
   const SegBlock B = tb[blockIdx.x];
-  if (inst[B.seg].done) return;
-  const int ik = gs->ik, ikn = gs->ikn, l0 = blockIdx.y * kGroup;
-  if (l0 > ik) return;
+  const int all_done = gs->all_done, ik = gs->ik, ikn = gs->ikn, l0 = blockIdx.y * kGroup;
+  hmv::together(B.seg | all_done | ik | ikn, 0.0, 0.0, 0.0);
+  if (all_done || l0 > ik) return;
+  const int done = inst[B.seg].done;
+  int i = B.beg + threadIdx.x;
+  double a = ar[min(i, B.end - 1)];
   __shared__ double sh[4];
   const double *v[kGroup];
 #pragma unroll
@@ -1231,11 +1239,21 @@ __global__ __launch_bounds__(kT) void sg_dots_beta(const SegBlock *__restrict__ 
     const int l = min(l0 + j, ik);
     v[j] = l == ikn ? ar : ap + (size_t)l * n;
   }
-  double s[kGroup] = {0.0, 0.0, 0.0, 0.0};
-  for (int i = B.beg + threadIdx.x; i < B.end; i += kT) {
-    const double a = ar[i];
+  double x[kGroup];
 #pragma unroll
-    for (int j = 0; j < kGroup; ++j) s[j] = __builtin_fma(v[j][i], a, s[j]);
+  for (int j = 0; j < kGroup; ++j) x[j] = v[j][min(i, B.end - 1)];
+  hmv::together(done, a, x[0], x[1], x[2], x[3], 0.0, 0.0);
+  if (done) return;
+  double s[kGroup] = {0.0, 0.0, 0.0, 0.0};
+  while (i < B.end) {
+#pragma unroll
+    for (int j = 0; j < kGroup; ++j) s[j] = __builtin_fma(x[j], a, s[j]);
+    i += kT;
+    if (i < B.end) {
+      a = ar[i];
+#pragma unroll
+      for (int j = 0; j < kGroup; ++j) x[j] = v[j][i];
+    }
   }
 #pragma unroll
   for (int j = 0; j < kGroup; ++j) {
@@ -1245,7 +1263,8 @@ __global__ __launch_bounds__(kT) void sg_dots_beta(const SegBlock *__restrict__ 
 }
 
 // beta_l = -(A p_l, A r) / capap_l for the slots l <= ik of the running
-// instances: `lanes` threads per instance and slot sum the instance's blocks
+// instances, where an instance has more blocks than every block of
+// sg_update_dir should sum the partials of (kMaxBetaB): `lanes` threads per instance and slot sum the instance's blocks
 // in a fixed order.
 __global__ __launch_bounds__(kT) void sg_betas(int nseg, int lanes,
                                                const int *__restrict__ bstart,
@@ -1274,7 +1293,8 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
                                                const double *__restrict__ part, SgInst *inst,
                                                SgGlobal *gs, int stage,
                                                int *__restrict__ done_flags, HmvSolveHost *h) {
-  if (gs->all_done && stage != 0) {
+  const SgGlobal z = *gs;
+  if (z.all_done && stage != 0) {
     if (threadIdx.x == 0) hmv::publish(h, gs->ticks += 1, 1);
     return;
   }
@@ -1284,15 +1304,18 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
   const int sub = threadIdx.x & (lanes - 1), np = stage == 0 ? 2 : 1;
   for (int s = threadIdx.x / lanes; s < nseg; s += kT / lanes) {
     SgInst &c = inst[s];
+    const int b0 = bstart[s], b1 = bstart[s + 1], cdone = c.done, cstep = c.step;
+    const double cb = c.bnorm;
+    hmv::together(b0 | b1 | cdone | cstep, cb, 0.0, 0.0);
     double d0 = 0.0, d1 = 0.0;
-    const int b1 = bstart[s + 1];
-    for (int b = bstart[s] + sub; b < b1; b += lanes) {
+    for (int b = b0 + sub; b < b1; b += lanes) {
       d0 += part[(size_t)np * b];
       if (stage == 0) d1 += part[2 * (size_t)b + 1];
     }
     d0 = group_sum(d0, lanes);
     d1 = group_sum(d1, lanes);
     if (sub != 0) continue;
+    int stop;
     if (stage == 0) {
       c.rnorm = sqrt(d0);
       c.bnorm = sqrt(d1);
@@ -1309,22 +1332,28 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
       } else if (gs->maxit <= 0) {
         c.done = 1;
       }
-    } else if (!c.done) {
-      c.step += 1;
-      c.rnorm = sqrt(d0);
-      if (!isfinite(c.rnorm)) {
-        c.status = HMV_SOLVE_NONFINITE;
-        c.done = 1;
-      } else if (c.rnorm / c.bnorm < gs->eps) {
-        c.status = HMV_SOLVE_CONVERGED;
-        c.done = 1;
-      } else if (c.step >= gs->maxit) {
-        c.status = HMV_SOLVE_MAXITER;
+    } else if (!cdone) {
+      const double rnorm = sqrt(d0);
+      c.step = cstep + 1;
+      c.rnorm = rnorm;
+      int status = -1;
+      if (!isfinite(rnorm))
+        status = HMV_SOLVE_NONFINITE;
+      else if (rnorm / cb < z.eps)
+        status = HMV_SOLVE_CONVERGED;
+      else if (cstep + 1 >= z.maxit)
+        status = HMV_SOLVE_MAXITER;
+      if (status >= 0) {
+        c.status = status;
         c.done = 1;
       }
+      stop = status >= 0;
+    } else {
+      stop = 1;
     }
-    done_flags[s] = c.done;
-    if (!c.done) atomicAnd(&sdone, 0);
+    if (stage == 0) stop = c.done;
+    done_flags[s] = stop;
+    if (!stop) atomicAnd(&sdone, 0);
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1332,62 +1361,103 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
       gs->step = gs->ticks = 0;
       gs->ik = 0;
       gs->ikn = 0;
+      gs->all_done = sdone;
+      hmv::publish(h, 0, sdone);
     } else {
-      gs->ik = gs->ikn;
-      gs->step += 1;
-      gs->ticks += 1;
-      gs->ikn = gs->step % gs->m;
+      gs->ik = z.ikn;
+      gs->step = z.step + 1;
+      gs->ticks = z.ticks + 1;
+      gs->ikn = (z.step + 1) % z.m;
+      gs->all_done = sdone;
+      hmv::publish(h, z.ticks + 1, sdone);
     }
-    gs->all_done = sdone;
-    hmv::publish(h, gs->ticks, sdone);
   }
 }
 
 // p_ikn = c0 r + sum_{l <= ik, l != ikn} beta_l p_l and ap_ikn likewise with
 // ar (c0 = 1 + beta_ikn when the slot is reused, else 1), per instance, and
-// the next step's alpha partials (ap_ikn, r), (ap_ikn, ap_ikn).  An element's
-// slots are loaded kDir at a time (one at a time is a chain of m loads).
+// the next step's alpha partials (ap_ikn, r), (ap_ikn, ap_ikn).  With
+// `betas` the block first forms its instance's betas from the partials
+// bpart of sg_dots_beta, 8 threads a slot; a launch of its own for that is 4
+// of the 57 us of a step of 8 instances of up to 80 blocks.  An element's
+// slots are loaded kDir at a time, a group ahead of its sums and the first
+// one ahead of the betas (one at a time is a chain of m loads).
 constexpr int kDir = 8;
-__global__ __launch_bounds__(kT) void sg_update_dir(const SegBlock *__restrict__ tb, int64_t n,
+__global__ __launch_bounds__(kT) void sg_update_dir(const SegBlock *__restrict__ tb,
+                                                    const int *__restrict__ bstart, int64_t n,
                                                     const double *__restrict__ r,
                                                     const double *__restrict__ ar,
                                                     double *__restrict__ p,
                                                     double *__restrict__ ap,
+                                                    const double *__restrict__ bpart, int betas,
                                                     double *__restrict__ part,
                                                     const SgInst *__restrict__ inst,
                                                     const SgGlobal *gs) {
-  if (gs->all_done) return;
+  __shared__ double sh[4], sb[kGcrM];
   const SegBlock B = tb[blockIdx.x];
+  const int all_done = gs->all_done, ik = gs->ik, ikn = gs->ikn;
+  hmv::together(B.seg | all_done | ik | ikn, 0.0, 0.0, 0.0);
+  if (all_done) return;
   const SgInst &c = inst[B.seg];
-  if (c.done) return;
-  __shared__ double sh[4];
-  const int ik = gs->ik, ikn = gs->ikn;
-  const double c0 = ikn <= ik ? 1.0 + c.beta[ikn] : 1.0;
+  const int l = threadIdx.x >> 3, sub = threadIdx.x & 7, lc = min(l, ik);
+  const int done = c.done, b0 = bstart[B.seg], b1 = bstart[B.seg + 1];
+  const double scale = betas ? c.capap[lc] : c.beta[lc];
+  int i = B.beg + threadIdx.x;
+  const int i0 = min(i, B.end - 1);
+  double rv = r[i0], av0 = ar[i0];
+  double pl[kDir], al[kDir];
+  auto load = [&](int l0, int at) {
+#pragma unroll
+    for (int j = 0; j < kDir; ++j) {
+      pl[j] = p[(size_t)min(l0 + j, ik) * n + at];
+      al[j] = ap[(size_t)min(l0 + j, ik) * n + at];
+    }
+  };
+  load(0, i0);
+  hmv::together(done | b0 | b1, scale, rv, av0);
+  if (done) return;
+  if (betas) {
+    double v = 0.0;
+    for (int b = b0 + sub; b < b1; b += 8) v += bpart[(size_t)b * kGcrM + lc];
+    v = group_sum(v, 8);
+    if (sub == 0) sb[l] = -v / scale;
+  } else if (sub == 0) {
+    sb[l] = scale;
+  }
+  __syncthreads();
+  const double c0 = ikn <= ik ? 1.0 + sb[ikn] : 1.0;
   double *pn = p + (size_t)ikn * n, *apn = ap + (size_t)ikn * n;
   double s0 = 0.0, s1 = 0.0;
-  for (int i = B.beg + threadIdx.x; i < B.end; i += kT) {
-    const double ri = r[i];
-    double pv = c0 * ri, av = c0 * ar[i];
+  while (i < B.end) {
+    const double ri = rv;
+    double pv = c0 * ri, av = c0 * av0;
     for (int l0 = 0; l0 <= ik; l0 += kDir) {
-      double pl[kDir], al[kDir];
+      double pc[kDir], ac[kDir];
 #pragma unroll
       for (int j = 0; j < kDir; ++j) {
-        const size_t at = (size_t)min(l0 + j, ik) * n + i;
-        pl[j] = p[at];
-        al[j] = ap[at];
+        pc[j] = pl[j];
+        ac[j] = al[j];
+      }
+      if (l0 + kDir <= ik) {
+        load(l0 + kDir, i);
+      } else if (i + kT < B.end) {
+        rv = r[i + kT];
+        av0 = ar[i + kT];
+        load(0, i + kT);
       }
 #pragma unroll
       for (int j = 0; j < kDir; ++j) {
         if (l0 + j > ik || l0 + j == ikn) continue;
-        const double bl = c.beta[l0 + j];
-        pv = __builtin_fma(bl, pl[j], pv);
-        av = __builtin_fma(bl, al[j], av);
+        const double bl = sb[l0 + j];
+        pv = __builtin_fma(bl, pc[j], pv);
+        av = __builtin_fma(bl, ac[j], av);
       }
     }
     pn[i] = pv;
     apn[i] = av;
     s0 = __builtin_fma(av, ri, s0);
     s1 = __builtin_fma(av, av, s1);
+    i += kT;
   }
   const double r0 = blk_sum(s0, sh), r1 = blk_sum(s1, sh);
   if (threadIdx.x == 0) {
@@ -1398,11 +1468,12 @@ __global__ __launch_bounds__(kT) void sg_update_dir(const SegBlock *__restrict__
 
 struct SegGcrWork {
   int m = 0;
-  double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr, *part = nullptr;
+  double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr;
+  double *part = nullptr, *bpart = nullptr;  // 3 per block; one per block and slot
   SgInst *inst = nullptr;
   SgGlobal *gs = nullptr;
   ~SegGcrWork() {
-    for (double *q : {r, ar, p, ap, part}) (void)hipFree(q);
+    for (double *q : {r, ar, p, ap, part, bpart}) (void)hipFree(q);
     (void)hipFree(inst);
     (void)hipFree(gs);
   }
@@ -1414,7 +1485,8 @@ int sg_setup(const SegWork &w, SegGcrWork &gw, int m, const char *who) {
   hipError_t e;
   if ((e = hipMalloc(&gw.r, nb)) != hipSuccess || (e = hipMalloc(&gw.ar, nb)) != hipSuccess ||
       (e = hipMalloc(&gw.p, nb * m)) != hipSuccess || (e = hipMalloc(&gw.ap, nb * m)) != hipSuccess ||
-      (e = hipMalloc(&gw.part, sizeof(double) * (size_t)w.nblk * kGcrM)) != hipSuccess ||
+      (e = hipMalloc(&gw.part, sizeof(double) * 3 * (size_t)w.nblk)) != hipSuccess ||
+      (e = hipMalloc(&gw.bpart, sizeof(double) * (size_t)w.nblk * kGcrM)) != hipSuccess ||
       (e = hipMalloc(&gw.inst, sizeof(SgInst) * w.nseg)) != hipSuccess ||
       (e = hipMalloc(&gw.gs, sizeof(SgGlobal))) != hipSuccess)
     return hmv::hip_fail(e, (std::string(who) + ": GCR workspace").c_str());
@@ -1424,8 +1496,8 @@ int sg_setup(const SegWork &w, SegGcrWork &gw, int m, const char *who) {
 hipError_t sg_iteration(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, double *u) {
   const int nb = w.nblk;
   const int *skip = &gw.gs->all_done;
-  // (r, r) partials at [2 nb, 3 nb) of the nb * kGcrM partials, apart from the
-  // alpha pairs at [0, 2 nb) that sg_update_ur reads while writing them
+  // (r, r) partials at [2 nb, 3 nb), apart from the alpha pairs at [0, 2 nb)
+  // that sg_update_ur reads while writing them
   double *rpart = gw.part + 2 * (size_t)nb;
   hipLaunchKernelGGL(sg_update_ur, dim3(nb), dim3(kT), 0, w.s, w.tb, w.bstart, w.n, gw.p, gw.ap,
                      u, gw.r, (const double *)gw.part, rpart, gw.inst, (const SgGlobal *)gw.gs);
@@ -1434,12 +1506,16 @@ hipError_t sg_iteration(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, double
   hipError_t e = hmv::enqueue_apply(a, gw.r, gw.ar, 0.0, skip, w.s, w.flags);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(sg_dots_beta, dim3(nb, (gw.m + kGroup - 1) / kGroup), dim3(kT), 0, w.s, w.tb,
-                     w.n, gw.ap, gw.ar, gw.part, (const SgInst *)gw.inst, (const SgGlobal *)gw.gs);
-  const int nbeta = (int)(((int64_t)w.nseg * gw.m * w.lanes + kT - 1) / kT);
-  hipLaunchKernelGGL(sg_betas, dim3(nbeta), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
-                     (const double *)gw.part, gw.inst, (const SgGlobal *)gw.gs);
-  hipLaunchKernelGGL(sg_update_dir, dim3(nb), dim3(kT), 0, w.s, w.tb, w.n, gw.r, gw.ar, gw.p,
-                     gw.ap, gw.part, (const SgInst *)gw.inst, (const SgGlobal *)gw.gs);
+                     w.n, gw.ap, gw.ar, gw.bpart, (const SgInst *)gw.inst, (const SgGlobal *)gw.gs);
+  const int betas = w.maxblk <= kMaxBetaB;
+  if (!betas) {
+    const int nbeta = (int)(((int64_t)w.nseg * gw.m * w.lanes + kT - 1) / kT);
+    hipLaunchKernelGGL(sg_betas, dim3(nbeta), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
+                       (const double *)gw.bpart, gw.inst, (const SgGlobal *)gw.gs);
+  }
+  hipLaunchKernelGGL(sg_update_dir, dim3(nb), dim3(kT), 0, w.s, w.tb, w.bstart, w.n, gw.r, gw.ar,
+                     gw.p, gw.ap, (const double *)gw.bpart, betas, gw.part,
+                     (const SgInst *)gw.inst, (const SgGlobal *)gw.gs);
   return hipGetLastError();
 }
 

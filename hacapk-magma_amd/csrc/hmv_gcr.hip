@@ -31,12 +31,12 @@ namespace {
 constexpr int kT = 256;
 constexpr int kMaxB = kSolveMaxBlocks;
 constexpr int kMaxM = HMV_GCR_MAX_M;
-static_assert(kMaxM >= 3, "the partial buffer holds the alpha pairs and the (r, r) partials");
+constexpr int kMaxBetaB = 128;  // blocks of a beta dot
+static_assert(kT == 8 * kMaxM, "8 threads sum the partials of a slot's beta");
 
 struct GcrState {
   double alpha, bnorm, rnorm, eps;
   double capap[kMaxM];
-  double beta[kMaxM];
   int step;  // completed steps (the reference's in)
   int ik;    // slot of the current direction (0-based)
   int ikn;   // slot of the next direction (0-based)
@@ -102,19 +102,21 @@ __global__ __launch_bounds__(kT) void g_update_ur(int n, int nb, const double *_
                                                   double *__restrict__ u, double *__restrict__ r,
                                                   const double *__restrict__ apart,
                                                   double *__restrict__ rpart, GcrState *st) {
-  if (st->done) return;
   __shared__ double sh[4];
+  const int done = st->done, ik = st->ikn;  // the slot of this step
+  int i = blockIdx.x * kT + threadIdx.x;
+  const int i0 = min(i, n - 1);
+  double uv = u[i0], rv = r[i0];
   double s0 = 0.0, s1 = 0.0;
   for (int b = threadIdx.x; b < nb; b += kT) {
     s0 += apart[2 * b];
     s1 += apart[2 * b + 1];
   }
-  const int ik = st->ikn;  // the slot of this step
+  hmv::together(done | ik, uv, rv, s0, s1, 0.0, 0.0, 0.0);
+  if (done) return;
   const double *pk = p + (size_t)ik * n, *q = ap + (size_t)ik * n;
   // the first elements are under way while the partials are summed
-  int i = blockIdx.x * kT + threadIdx.x;
-  const int i0 = min(i, n - 1);
-  double uv = u[i0], pv = pk[i0], rv = r[i0], qv = q[i0];
+  double pv = pk[i0], qv = q[i0];
   const double d0 = blk_sum(s0, sh), d1 = blk_sum(s1, sh);
   const double alpha = d0 / d1;
   const bool bad = d1 == 0.0 || !isfinite(alpha);
@@ -154,9 +156,11 @@ constexpr int kGroup = 4;
 __global__ __launch_bounds__(kT) void g_dots_beta(int n, const double *__restrict__ ap,
                                                   const double *__restrict__ ar,
                                                   double *__restrict__ part, const GcrState *st) {
-  if (st->done) return;
-  const int ik = st->ik, ikn = st->ikn, l0 = blockIdx.y * kGroup;
-  if (l0 > ik) return;
+  const int done = st->done, ik = st->ik, ikn = st->ikn, l0 = blockIdx.y * kGroup;
+  int i = blockIdx.x * kT + threadIdx.x;
+  double a = ar[min(i, n - 1)];
+  hmv::together(done | ik | ikn, a, 0.0, 0.0);
+  if (done || l0 > ik) return;
   __shared__ double sh[4];
   const double *v[kGroup];
 #pragma unroll
@@ -165,10 +169,15 @@ __global__ __launch_bounds__(kT) void g_dots_beta(int n, const double *__restric
     v[j] = l == ikn ? ar : ap + (size_t)l * n;
   }
   double s[kGroup] = {0.0, 0.0, 0.0, 0.0};
-  for (int i = blockIdx.x * kT + threadIdx.x; i < n; i += gridDim.x * kT) {
-    const double a = ar[i];
+  while (i < n) {
+    double x[kGroup];
 #pragma unroll
-    for (int j = 0; j < kGroup; ++j) s[j] = __builtin_fma(v[j][i], a, s[j]);
+    for (int j = 0; j < kGroup; ++j) x[j] = v[j][i];
+    const double ai = a;
+    i += gridDim.x * kT;
+    if (i < n) a = ar[i];
+#pragma unroll
+    for (int j = 0; j < kGroup; ++j) s[j] = __builtin_fma(x[j], ai, s[j]);
   }
 #pragma unroll
   for (int j = 0; j < kGroup; ++j) {
@@ -178,9 +187,7 @@ __global__ __launch_bounds__(kT) void g_dots_beta(int n, const double *__restric
 }
 
 // stage 0: setup (d0 = (r,r), d1 = (b,b) from nb partial pairs); 2: ||r||
-// (nb partials), step, stop; 3: betas from the per-slot partials, one wave
-// per slot (lanes sum the blocks in a fixed order, then a fixed shuffle
-// tree: deterministic)
+// (nb partials), step, stop
 __device__ inline void g_publish(HmvSolveHost *h, const GcrState *st) {
   if (st->done) {
     h->step = st->step;
@@ -194,35 +201,7 @@ __device__ inline void g_publish(HmvSolveHost *h, const GcrState *st) {
 __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__ part,
                                               GcrState *st, int stage, double *__restrict__ hist,
                                               HmvSolveHost *h) {
-  if (st->done && stage != 0) {
-    if (stage == 2 && threadIdx.x == 0) {
-      st->ticks += 1;
-      g_publish(h, st);
-    }
-    return;
-  }
   __shared__ double sh[4];
-  if (stage == 3) {
-    // wave w takes slots w, w + 4, ...; all their loads go out together
-    constexpr int kW = kT / 64, kL = (kMaxM + kW - 1) / kW;
-    const int ik = st->ik, lane = threadIdx.x & 63, w0 = threadIdx.x >> 6;
-    double s[kL];
-#pragma unroll
-    for (int j = 0; j < kL; ++j) s[j] = 0.0;
-    for (int b = lane; b < nb; b += 64)
-#pragma unroll
-      for (int j = 0; j < kL; ++j)
-        if (w0 + j * kW <= ik) s[j] += part[(size_t)b * kMaxM + w0 + j * kW];
-#pragma unroll
-    for (int j = 0; j < kL; ++j) {
-      const int l = w0 + j * kW;
-      if (l > ik) break;
-      double v = s[j];
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-      if (lane == 0) st->beta[l] = -v / st->capap[l];
-    }
-    return;
-  }
   double s0 = 0.0, s1 = 0.0;
   if (stage == 0) {
     for (int b = threadIdx.x; b < nb; b += kT) {
@@ -231,6 +210,16 @@ __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__
     }
   } else {
     for (int b = threadIdx.x; b < nb; b += kT) s0 += part[b];
+  }
+  const int done = st->done, step = st->step, m = st->m, maxit = st->maxit, ticks = st->ticks;
+  const double bnorm = st->bnorm, eps = st->eps;
+  hmv::together(done | step | m | maxit | ticks, s0, bnorm, eps);
+  if (done && stage != 0) {
+    if (threadIdx.x == 0) {
+      st->ticks = ticks + 1;
+      g_publish(h, st);
+    }
+    return;
   }
   const double d0 = blk_sum(s0, sh), d1 = blk_sum(s1, sh);
   if (threadIdx.x != 0) return;
@@ -254,23 +243,41 @@ __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__
     }
     st->ticks = 0;
   } else {
-    st->step += 1;
-    st->rnorm = sqrt(d0);
-    st->ikn = st->step % st->m;
-    if (hist) hist[st->step] = st->rnorm / st->bnorm;
-    if (!isfinite(st->rnorm)) {
-      st->status = HMV_SOLVE_NONFINITE;
-      st->done = 1;
-    } else if (st->rnorm / st->bnorm < st->eps) {
-      st->status = HMV_SOLVE_CONVERGED;
-      st->done = 1;
-    } else if (st->step >= st->maxit) {
-      st->status = HMV_SOLVE_MAXITER;
-      st->done = 1;
+    const double rnorm = sqrt(d0), rel = rnorm / bnorm;
+    st->step = step + 1;
+    st->rnorm = rnorm;
+    st->ikn = (step + 1) % m;
+    st->ticks = ticks + 1;
+    if (hist) hist[step + 1] = rel;
+    int status = -1;
+    if (!isfinite(rnorm))
+      status = HMV_SOLVE_NONFINITE;
+    else if (rel < eps)
+      status = HMV_SOLVE_CONVERGED;
+    else if (step + 1 >= maxit)
+      status = HMV_SOLVE_MAXITER;
+    if (status < 0) {
+      hmv::publish(h, ticks + 1, 0);
+      return;
     }
-    st->ticks += 1;
+    st->status = status;
+    st->done = 1;
   }
   g_publish(h, st);
+}
+
+// beta_l = -(v_l, ar) / capap_l for the slots l <= ik, from the nbb partials
+// of g_dots_beta: every block sums them alike, 8 threads a slot, into sb.  A
+// launch of its own for this took 4.7 us of a step at 82k unknowns.
+__device__ inline void form_betas(int nbb, const double *__restrict__ bpart,
+                                  const double *__restrict__ capap, int ik, double *sb) {
+  const int l = threadIdx.x >> 3, sub = threadIdx.x & 7;
+  const double cap = capap[min(l, ik)];
+  double v = 0.0;
+  for (int b = sub; b < nbb; b += 8) v += bpart[(size_t)b * kMaxM + min(l, ik)];
+  for (int off = 4; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if (sub == 0) sb[l] = -v / cap;
+  __syncthreads();
 }
 
 // p_ikn = c0 r + sum_{il <= ik, il != ikn} beta_il p_il;  ap_ikn likewise
@@ -278,43 +285,66 @@ __global__ __launch_bounds__(kT) void g_final(int nb, const double *__restrict__
 // ... and the next step's alpha partials (ap_ikn, r), (ap_ikn, ap_ikn) into
 // part[2*blk + {0,1}], in g_dots_alpha's order (same grid, same per-thread
 // sequence), so that the step needs no separate dot pass.
-// An element's slots are loaded kDir at a time: one at a time leaves a chain
-// of up to m loads per thread, which is what the pass takes at a few
-// elements per thread.
+// An element's slots are loaded kDir at a time, a group ahead of its sums and
+// the first one ahead of the betas: one at a time leaves a chain of up to m
+// loads per thread, which is what the pass takes at a few elements each.
 constexpr int kDir = 8;
-__global__ __launch_bounds__(kT) void g_update_dir(int n, const double *__restrict__ r,
+__global__ __launch_bounds__(kT) void g_update_dir(int n, int nbb, const double *__restrict__ r,
                                                    const double *__restrict__ ar,
                                                    double *__restrict__ p, double *__restrict__ ap,
+                                                   const double *__restrict__ bpart,
                                                    double *__restrict__ part, const GcrState *st) {
-  if (st->done) return;
-  __shared__ double sh[4];
-  const int ik = st->ik, ikn = st->ikn;
-  const double c0 = ikn <= ik ? 1.0 + st->beta[ikn] : 1.0;
+  __shared__ double sh[4], sb[kMaxM];
+  const int done = st->done, ik = st->ik, ikn = st->ikn;
+  int i = blockIdx.x * kT + threadIdx.x;
+  const int i0 = min(i, n - 1);
+  double rv = r[i0], av0 = ar[i0];
+  hmv::together(done | ik | ikn, rv, av0, 0.0);
+  if (done) return;
+  double pl[kDir], al[kDir];
+  auto load = [&](int l0, int at) {
+#pragma unroll
+    for (int j = 0; j < kDir; ++j) {
+      pl[j] = p[(size_t)min(l0 + j, ik) * n + at];
+      al[j] = ap[(size_t)min(l0 + j, ik) * n + at];
+    }
+  };
+  load(0, i0);
+  form_betas(nbb, bpart, st->capap, ik, sb);
+  const double c0 = ikn <= ik ? 1.0 + sb[ikn] : 1.0;
   double *pn = p + (size_t)ikn * n, *apn = ap + (size_t)ikn * n;
   double s0 = 0.0, s1 = 0.0;
-  for (int i = blockIdx.x * kT + threadIdx.x; i < n; i += gridDim.x * kT) {
-    const double ri = r[i];
-    double pv = c0 * ri, av = c0 * ar[i];
+  const int stride = gridDim.x * kT;
+  while (i < n) {
+    const double ri = rv;
+    double pv = c0 * ri, av = c0 * av0;
     for (int l0 = 0; l0 <= ik; l0 += kDir) {
-      double pl[kDir], al[kDir];
+      double pc[kDir], ac[kDir];
 #pragma unroll
       for (int j = 0; j < kDir; ++j) {
-        const size_t at = (size_t)min(l0 + j, ik) * n + i;
-        pl[j] = p[at];
-        al[j] = ap[at];
+        pc[j] = pl[j];
+        ac[j] = al[j];
+      }
+      if (l0 + kDir <= ik) {
+        load(l0 + kDir, i);
+      } else if (i + stride < n) {
+        rv = r[i + stride];
+        av0 = ar[i + stride];
+        load(0, i + stride);
       }
 #pragma unroll
       for (int j = 0; j < kDir; ++j) {
         if (l0 + j > ik || l0 + j == ikn) continue;
-        const double bl = st->beta[l0 + j];
-        pv = __builtin_fma(bl, pl[j], pv);
-        av = __builtin_fma(bl, al[j], av);
+        const double bl = sb[l0 + j];
+        pv = __builtin_fma(bl, pc[j], pv);
+        av = __builtin_fma(bl, ac[j], av);
       }
     }
     pn[i] = pv;
     apn[i] = av;
     s0 = __builtin_fma(av, ri, s0);
     s1 = __builtin_fma(av, av, s1);
+    i += stride;
   }
   const double r0 = blk_sum(s0, sh), r1 = blk_sum(s1, sh);
   if (threadIdx.x == 0) {
@@ -338,6 +368,10 @@ int grid_of(int n) {
   return std::max(1, std::min((n + kT - 1) / kT, kMaxB));
 }
 
+// Blocks of a beta dot: 4 elements per thread, and few enough that every
+// block of g_update_dir can sum the partials of all of them.
+int beta_grid(int n) { return std::max(1, std::min((n + 4 * kT - 1) / (4 * kT), kMaxBetaB)); }
+
 }  // namespace
 
 // GCR workspace, kept with the arena between calls.
@@ -345,12 +379,13 @@ struct HmvGcrWork {
   int m = 0;
   size_t hist_cap = 0;
   hipStream_t s = nullptr;
-  double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr, *part = nullptr, *hist = nullptr;
+  double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr, *part = nullptr, *bpart = nullptr,
+         *hist = nullptr;
   GcrState *st = nullptr;
   double *ir_r = nullptr, *ir_d = nullptr;  // refinement: outer residual, correction
   ~HmvGcrWork() {
     if (s) (void)hipStreamDestroy(s);
-    for (double *q : {r, ar, p, ap, part, hist, ir_r, ir_d}) (void)hipFree(q);
+    for (double *q : {r, ar, p, ap, part, bpart, hist, ir_r, ir_d}) (void)hipFree(q);
     (void)hipFree(st);
   }
 };
@@ -384,7 +419,8 @@ int gcr_work(hmv_arena_s *a, int m, int maxit, GcrWork *&out) {
     if ((e = hipStreamCreateWithFlags(&w->s, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipMalloc(&w->r, nb)) != hipSuccess || (e = hipMalloc(&w->ar, nb)) != hipSuccess ||
         (e = hipMalloc(&w->p, nb * m)) != hipSuccess || (e = hipMalloc(&w->ap, nb * m)) != hipSuccess ||
-        (e = hipMalloc(&w->part, sizeof(double) * (size_t)g * kMaxM)) != hipSuccess ||
+        (e = hipMalloc(&w->part, sizeof(double) * 3 * (size_t)g)) != hipSuccess ||
+        (e = hipMalloc(&w->bpart, sizeof(double) * (size_t)beta_grid(n) * kMaxM)) != hipSuccess ||
         (e = hipMalloc(&w->hist, sizeof(double) * w->hist_cap)) != hipSuccess ||
         (e = hipMalloc(&w->st, sizeof(GcrState))) != hipSuccess) {
       hmv::free_gcr_work(a);
@@ -396,10 +432,10 @@ int gcr_work(hmv_arena_s *a, int m, int maxit, GcrWork *&out) {
 }
 
 hipError_t gcr_iteration(hmv_arena_s *a, GcrWork &w, int n, int m, double *u, HmvSolveHost *h) {
-  const int g = grid_of(n);
+  const int g = grid_of(n), gb = beta_grid(n);
   const int *skip = &w.st->done;
-  // (r, r) partials at [2g, 3g) of the g * kMaxM partials, apart from the
-  // alpha pairs at [0, 2g) that g_update_ur reads while writing them
+  // (r, r) partials at [2g, 3g) of the partials, apart from the alpha pairs
+  // at [0, 2g) that g_update_ur reads while writing them
   double *rpart = w.part + 2 * (size_t)g;
   // the alpha partials of this step come from the previous step's
   // g_update_dir (or, for the first step, from the setup's g_dots_alpha)
@@ -409,12 +445,10 @@ hipError_t gcr_iteration(hmv_arena_s *a, GcrWork &w, int n, int m, double *u, Hm
                      h);
   hipError_t e = hmv::enqueue_apply(a, w.r, w.ar, 0.0, skip, w.s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(g_dots_beta, dim3(g, (m + kGroup - 1) / kGroup), dim3(kT), 0, w.s, n, w.ap,
-                     w.ar, w.part,
-                     (const GcrState *)w.st);
-  hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 3, w.hist, h);
-  hipLaunchKernelGGL(g_update_dir, dim3(g), dim3(kT), 0, w.s, n, w.r, w.ar, w.p, w.ap, w.part,
-                     (const GcrState *)w.st);
+  hipLaunchKernelGGL(g_dots_beta, dim3(gb, (m + kGroup - 1) / kGroup), dim3(kT), 0, w.s, n, w.ap,
+                     w.ar, w.bpart, (const GcrState *)w.st);
+  hipLaunchKernelGGL(g_update_dir, dim3(g), dim3(kT), 0, w.s, n, gb, w.r, w.ar, w.p, w.ap,
+                     (const double *)w.bpart, w.part, (const GcrState *)w.st);
   return hipGetLastError();
 }
 

@@ -71,12 +71,26 @@ __global__ __launch_bounds__(kThreads) void k_dots(int n, const double *__restri
                                                     const double *__restrict__ d,
                                                     double *__restrict__ part,
                                                     const SolveState *st) {
-  if (st && st->done) return;
   __shared__ double sh[4];
+  int i = blockIdx.x * kThreads + threadIdx.x;
+  const int i0 = min(i, n - 1);
+  const int done = st ? st->done : 0;
+  double av = a[i0], bv = b[i0], cv = c ? c[i0] : 0.0, dv = c ? d[i0] : 0.0;
+  hmv::together(done, av, bv, cv, dv, 0.0, 0.0, 0.0);
+  if (done) return;
   double s0 = 0.0, s1 = 0.0;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
-    s0 = __builtin_fma(a[i], b[i], s0);
-    if (c) s1 = __builtin_fma(c[i], d[i], s1);
+  while (i < n) {
+    s0 = __builtin_fma(av, bv, s0);
+    s1 = __builtin_fma(cv, dv, s1);
+    i += gridDim.x * kThreads;
+    if (i < n) {
+      av = a[i];
+      bv = b[i];
+      if (c) {
+        cv = c[i];
+        dv = d[i];
+      }
+    }
   }
   double r0 = block_sum(s0, sh);
   double r1 = c ? block_sum(s1, sh) : 0.0;
@@ -86,13 +100,17 @@ __global__ __launch_bounds__(kThreads) void k_dots(int n, const double *__restri
   }
 }
 
-// Fixed-order sum of the partials into st->d0, st->d1.
-__device__ inline void reduce_parts(int nb, const double *part, SolveState *st, double *sh) {
-  double s0 = 0.0, s1 = 0.0;
+// A thread's share of the nb partial pairs.
+__device__ inline void part_pairs(int nb, const double *__restrict__ part, double &s0, double &s1) {
+  s0 = s1 = 0.0;
   for (int i = threadIdx.x; i < nb; i += kThreads) {
     s0 += part[2 * i];
     s1 += part[2 * i + 1];
   }
+}
+
+// Fixed-order sum of the threads' shares into st->d0, st->d1.
+__device__ inline void reduce_parts(double s0, double s1, SolveState *st, double *sh) {
   double r0 = block_sum(s0, sh);
   double r1 = block_sum(s1, sh);
   if (threadIdx.x == 0) {
@@ -113,21 +131,10 @@ __device__ inline void publish(HmvSolveHost *h, const SolveState *st) {
   hmv::publish(h, st->ticks, st->done);
 }
 
+// The scalar stages on the state z, d0 and d1 being the dots summed.
 // stage: 0 setup (d0 = (r,r), d1 = (b,b)), 3 beta and the stopping test,
 // 4 residual replacement (d0 = (r^, r), d1 = (r, r) of the true residual)
-__global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__restrict__ part,
-                                                    SolveState *st, int stage,
-                                                    double *__restrict__ hist, HmvSolveHost *h) {
-  if (st->done && stage != 0 && stage != 4) {
-    if (threadIdx.x == 0) {
-      st->ticks += 1;
-      publish(h, st);
-    }
-    return;
-  }
-  __shared__ double sh[4];
-  reduce_parts(nb, part, st, sh);
-  if (threadIdx.x != 0) return;
+__device__ inline void k_stage(SolveState *st, int stage, double *__restrict__ hist) {
   if (stage == 0) {
     // d0 = (r,r) (r^ = r initially), d1 = (b,b)
     st->rr = st->d0;
@@ -192,7 +199,28 @@ __global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__rest
       st->done = 1;
     }
   }
-  publish(h, st);
+}
+
+__global__ __launch_bounds__(kThreads) void k_final(int nb, const double *__restrict__ part,
+                                                    SolveState *st, int stage,
+                                                    double *__restrict__ hist, HmvSolveHost *h) {
+  __shared__ double sh[4];
+  double s0, s1;
+  part_pairs(nb, part, s0, s1);
+  SolveState z = *st;
+  hmv::together(z.done | z.step | z.maxit | z.ticks, s0, s1, z.alpha, z.zeta, z.rr, z.bnorm, z.eps);
+  if (z.done && stage != 0 && stage != 4) {
+    if (threadIdx.x == 0) {
+      st->ticks += 1;
+      publish(h, st);
+    }
+    return;
+  }
+  reduce_parts(s0, s1, &z, sh);
+  if (threadIdx.x != 0) return;
+  k_stage(&z, stage, hist);
+  *st = z;
+  publish(h, &z);
 }
 
 // p = r + beta (p - zeta v)
@@ -200,10 +228,21 @@ __global__ __launch_bounds__(kThreads) void k_update_p(int n, const double *__re
                                                         const double *__restrict__ v,
                                                         double *__restrict__ p,
                                                         const SolveState *st) {
-  if (st->done) return;
+  int i = blockIdx.x * kThreads + threadIdx.x;
+  const int i0 = min(i, n - 1), done = st->done;
   const double beta = st->beta, zeta = st->zeta;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads)
-    p[i] = r[i] + beta * (p[i] - zeta * v[i]);
+  double rv = r[i0], vv = v[i0], pv = p[i0];
+  hmv::together(done, beta, zeta, rv, vv, pv, 0.0, 0.0);
+  if (done) return;
+  while (i < n) {
+    p[i] = rv + beta * (pv - zeta * vv);
+    i += gridDim.x * kThreads;
+    if (i < n) {
+      rv = r[i];
+      vv = v[i];
+      pv = p[i];
+    }
+  }
 }
 
 // alpha = rr / (r^, v) from the nb partial pairs of k_dots, summed in
@@ -214,12 +253,16 @@ __global__ __launch_bounds__(kThreads) void k_update_t(int n, int nb, const doub
                                                         double *__restrict__ t,
                                                         const double *__restrict__ part,
                                                         SolveState *st) {
-  if (st->done) return;
   __shared__ double sh[4];
-  double s0 = 0.0;
-  for (int i = threadIdx.x; i < nb; i += kThreads) s0 += part[2 * i];
+  int i = blockIdx.x * kThreads + threadIdx.x;
+  const int i0 = min(i, n - 1), done = st->done;
+  const double rr = st->rr;
+  double rv = r[i0], vv = v[i0], s0, s1;
+  part_pairs(nb, part, s0, s1);
+  hmv::together(done, rr, rv, vv, s0, 0.0, 0.0, 0.0);
+  if (done) return;
   const double zden = block_sum_all(s0, sh);
-  const double alpha = st->rr / zden;
+  const double alpha = rr / zden;
   const bool bad = zden == 0.0 || !finite(alpha);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->d0 = zden;
@@ -230,8 +273,14 @@ __global__ __launch_bounds__(kThreads) void k_update_t(int n, int nb, const doub
     }
   }
   if (bad) return;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads)
-    t[i] = r[i] - alpha * v[i];
+  while (i < n) {
+    t[i] = rv - alpha * vv;
+    i += gridDim.x * kThreads;
+    if (i < n) {
+      rv = r[i];
+      vv = v[i];
+    }
+  }
 }
 
 // zeta = (s, t) / (s, s) from the nb partial pairs zpart of k_dots, summed
@@ -244,13 +293,14 @@ __global__ __launch_bounds__(kThreads) void k_update_ur(
     const double *__restrict__ s, const double *__restrict__ rhat, double *__restrict__ u,
     double *__restrict__ r, const double *__restrict__ zpart, double *__restrict__ part,
     SolveState *st) {
-  if (st->done) return;
   __shared__ double sh[4];
-  double z0 = 0.0, z1 = 0.0;
-  for (int i = threadIdx.x; i < nb; i += kThreads) {
-    z0 += zpart[2 * i];
-    z1 += zpart[2 * i + 1];
-  }
+  int i = blockIdx.x * kThreads + threadIdx.x;
+  const int i0 = min(i, n - 1), done = st->done;
+  const double alpha = st->alpha;
+  double uv = u[i0], pv = p[i0], tv = t[i0], sv = s[i0], qv = rhat[i0], z0, z1;
+  part_pairs(nb, zpart, z0, z1);
+  hmv::together(done, uv, pv, tv, sv, qv, z0, z1);
+  if (done) return;
   const double znom = block_sum_all(z0, sh), zden = block_sum_all(z1, sh);
   // s = A t = 0 (both dots zero): the half step u += alpha p, r = t is taken
   // with zeta = 0, and k_final's beta stage reports convergence or breakdown
@@ -267,14 +317,21 @@ __global__ __launch_bounds__(kThreads) void k_update_ur(
     }
   }
   if (bad) return;
-  const double alpha = st->alpha;
   double s0 = 0.0, s1 = 0.0;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
-    u[i] = (u[i] + alpha * p[i]) + zeta * t[i];
-    const double ri = t[i] - zeta * s[i];
+  while (i < n) {
+    u[i] = (uv + alpha * pv) + zeta * tv;
+    const double ri = tv - zeta * sv;
     r[i] = ri;
-    s0 = __builtin_fma(rhat[i], ri, s0);
+    s0 = __builtin_fma(qv, ri, s0);
     s1 = __builtin_fma(ri, ri, s1);
+    i += gridDim.x * kThreads;
+    if (i < n) {
+      uv = u[i];
+      pv = p[i];
+      tv = t[i];
+      sv = s[i];
+      qv = rhat[i];
+    }
   }
   double r0 = block_sum(s0, sh);
   double r1 = block_sum(s1, sh);
