@@ -174,6 +174,7 @@ void release(hmv_arena_s *a) {
   if (!a) return;
   hmv::free_solve_work(a);
   hmv::free_gcr_work(a);
+  hmv::free_multi_work(a);
   if (a->solve_host) (void)hipHostFree(a->solve_host);
   (void)hipFree(a->d_arena);
   (void)hipFree(a->d_work1);

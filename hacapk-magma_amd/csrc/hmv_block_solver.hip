@@ -727,17 +727,59 @@ struct SegWork {
   ColState *cs = nullptr;
   BlockState *bs = nullptr;
   int *flags = nullptr;  // per-instance done flags read by the H-matvec
+  double *r2 = nullptr, *d = nullptr;  // refinement: outer residual, correction
   HmvSolveHost *h = nullptr;  // the arena's
   ~SegWork() {
     (void)hipFree(flags);
     if (s) (void)hipStreamDestroy(s);
-    for (double *q : {r, rhat, p, v, t, sv, part}) (void)hipFree(q);
+    for (double *q : {r, rhat, p, v, t, sv, part, r2, d}) (void)hipFree(q);
     (void)hipFree(tb);
     (void)hipFree(bstart);
     (void)hipFree(cs);
     (void)hipFree(bs);
   }
 };
+
+struct SgInst;
+struct SgGlobal;
+
+struct SegGcrWork {
+  int m = 0;
+  double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr;
+  double *part = nullptr, *bpart = nullptr;  // 3 per block; one per block and slot
+  SgInst *inst = nullptr;
+  SgGlobal *gs = nullptr;
+  void free_all() {
+    for (double **q : {&r, &ar, &p, &ap, &part, &bpart}) {
+      (void)hipFree(*q);
+      *q = nullptr;
+    }
+    (void)hipFree(inst);
+    (void)hipFree(gs);
+    inst = nullptr;
+    gs = nullptr;
+    m = 0;
+  }
+  ~SegGcrWork() { free_all(); }
+};
+
+}  // namespace
+
+// Workspace of the per-instance solvers, kept with the arena whose products
+// they take between calls; the GCR part holds the m of its last call.
+struct HmvMultiWork {
+  SegWork w;
+  SegGcrWork gw;
+};
+
+namespace hmv {
+void free_multi_work(hmv_arena_s *a) {
+  delete a->multi;
+  a->multi = nullptr;
+}
+}  // namespace hmv
+
+namespace {
 
 __global__ __launch_bounds__(kT) void kb_fill(int64_t n, double *__restrict__ x, double v) {
   for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT)
@@ -755,9 +797,9 @@ __global__ __launch_bounds__(kT) void kb_add(int64_t n, double *__restrict__ u,
 // stops at its setup and their products are skipped)
 __global__ __launch_bounds__(kT) void ks_zero_stopped(const SegBlock *__restrict__ tb,
                                                       double *__restrict__ r,
-                                                      const int *__restrict__ stopped) {
+                                                      const HmvInstHost *hi) {
   const SegBlock B = tb[blockIdx.x];
-  if (!stopped[B.seg]) return;
+  if (!hi[B.seg].stopped) return;
   for (int i = B.beg + threadIdx.x; i < B.end; i += kT) r[i] = 0.0;
 }
 
@@ -793,14 +835,14 @@ hipError_t seg_iteration(hmv_arena_s *a, SegWork &w, double *u) {
 // unknowns are 19 blocks on 256 CUs, and a direction update over 30 slots
 // took 37 us; 232 blocks brought their whole solve from 18.3 to 11.5 ms.  An
 // instance's partials are summed by one lane for each 4 blocks.
-int seg_setup(hmv_arena_s *a, SegWork &w, std::vector<int> &bstart, const char *who) {
+int seg_setup(hmv_arena_s *a, SegWork &w, const char *who) {
   w.nseg = (int)a->seg.size() - 1;
   w.n = a->nd;
   constexpr int kSegBlocks = 2048;
   const int64_t per = (w.n + (int64_t)kT * kSegBlocks - 1) / ((int64_t)kT * kSegBlocks);
   const int chunk = kT * (int)std::clamp<int64_t>(per, 1, 16);
   std::vector<SegBlock> tb;
-  bstart.assign(w.nseg + 1, 0);
+  std::vector<int> bstart(w.nseg + 1, 0);
   for (int sgi = 0; sgi < w.nseg; ++sgi) {
     bstart[sgi] = (int)tb.size();
     const int end = a->seg[sgi + 1];
@@ -823,11 +865,38 @@ int seg_setup(hmv_arena_s *a, SegWork &w, std::vector<int> &bstart, const char *
       (e = hipMalloc(&w.cs, sizeof(ColState) * w.nseg)) != hipSuccess ||
       (e = hipMalloc(&w.bs, sizeof(BlockState))) != hipSuccess ||
       (e = hipMalloc(&w.flags, sizeof(int) * w.nseg)) != hipSuccess ||
+      (e = hipMalloc(&w.r2, nbytes)) != hipSuccess || (e = hipMalloc(&w.d, nbytes)) != hipSuccess ||
       (e = hipMemcpy(w.tb, tb.data(), sizeof(SegBlock) * tb.size(), hipMemcpyHostToDevice)) !=
           hipSuccess ||
       (e = hipMemcpy(w.bstart, bstart.data(), sizeof(int) * bstart.size(), hipMemcpyHostToDevice)) !=
           hipSuccess)
     return hmv::hip_fail(e, (std::string(who) + ": workspace").c_str());
+  return HMV_OK;
+}
+
+// Buffers of the GCR steps.
+int sg_setup(const SegWork &w, SegGcrWork &gw, int m, const char *who);
+
+// The arena's workspace, with the GCR part for m directions if m > 0.
+int multi_work(hmv_arena_s *a, int m, HmvMultiWork *&out, const char *who) {
+  int rc = HMV_OK;
+  if (!a->multi) {
+    a->multi = new HmvMultiWork();
+    rc = seg_setup(a, a->multi->w, who);
+  }
+  if (rc == HMV_OK && m > 0 && a->multi->gw.m != m) {
+    a->multi->gw.free_all();
+    rc = sg_setup(a->multi->w, a->multi->gw, m, who);
+  }
+  hipError_t e;
+  if (rc == HMV_OK &&
+      (e = hmv::solve_host(a, a->multi->w.s, a->multi->w.h)) != hipSuccess)
+    rc = hmv::hip_fail(e, (std::string(who) + ": workspace").c_str());
+  if (rc != HMV_OK) {
+    hmv::free_multi_work(a);
+    return rc;
+  }
+  out = a->multi;
   return HMV_OK;
 }
 
@@ -898,10 +967,28 @@ int seg_solve(hmv_arena_s *a, SegWork &w, const double *b, double *u, double eps
   return HMV_OK;
 }
 
-// Per-instance ||b - A u||^2 and ||b||^2 (r receives b - A u), each summed
-// over the instance's blocks in block order.
+// rr, bb of every instance from its blocks' pairs, to the host's records.
+__global__ __launch_bounds__(kT) void ks_sums(int nseg, int lanes, const int *__restrict__ bstart,
+                                              const double *__restrict__ part, HmvInstHost *hi) {
+  const int s = (int)((blockIdx.x * kT + threadIdx.x) / lanes), sub = threadIdx.x & (lanes - 1);
+  if (s >= nseg) return;
+  double d0 = 0.0, d1 = 0.0;
+  const int b1 = bstart[s + 1];
+  for (int b = bstart[s] + sub; b < b1; b += lanes) {
+    d0 += part[2 * b];
+    d1 += part[2 * b + 1];
+  }
+  d0 = group_sum(d0, lanes);
+  d1 = group_sum(d1, lanes);
+  if (sub == 0) {
+    hi[s].rr = d0;
+    hi[s].bb = d1;
+  }
+}
+
+// Per-instance ||b - A u||^2 and ||b||^2 (r receives b - A u) in the host's
+// records, each summed over the instance's blocks in a fixed order.
 int seg_residuals(hmv_arena_s *a, SegWork &w, const double *b, const double *u, double *r,
-                  const std::vector<int> &bstart, std::vector<double> &rr, std::vector<double> &bb,
                   const char *who) {
   const int g = grid_of(w.n);
   hipError_t e = hmv::enqueue_apply(a, u, r, 0.0, nullptr, w.s);
@@ -909,19 +996,11 @@ int seg_residuals(hmv_arena_s *a, SegWork &w, const double *b, const double *u, 
   hipLaunchKernelGGL(kb_residual, dim3(g), dim3(kT), 0, w.s, w.n, b, r);
   hipLaunchKernelGGL(ks_dots, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, r, r, b, b, w.part,
                      (const BlockState *)nullptr);
-  std::vector<double> part(2 * (size_t)w.nblk);
-  if ((e = hipGetLastError()) != hipSuccess ||
-      (e = hipMemcpyAsync(part.data(), w.part, sizeof(double) * part.size(), hipMemcpyDeviceToHost,
-                          w.s)) != hipSuccess ||
-      (e = hipStreamSynchronize(w.s)) != hipSuccess)
+  const int gs = (int)(((int64_t)w.nseg * w.lanes + kT - 1) / kT);
+  hipLaunchKernelGGL(ks_sums, dim3(gs), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
+                     (const double *)w.part, hmv::inst_host(w.h));
+  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
     return hmv::hip_fail(e, (std::string(who) + ": residual").c_str());
-  rr.assign(w.nseg, 0.0);
-  bb.assign(w.nseg, 0.0);
-  for (int sgi = 0; sgi < w.nseg; ++sgi)
-    for (int bi = bstart[sgi]; bi < bstart[sgi + 1]; ++bi) {
-      rr[sgi] += part[2 * bi];
-      bb[sgi] += part[2 * bi + 1];
-    }
   return HMV_OK;
 }
 
@@ -936,10 +1015,11 @@ extern "C" int hmv_multi_bicgstab(hmv_arena a, const double *b, double *u, doubl
   }
   if (check_every < 1) check_every = 1;
   const char *who = "hmv_multi_bicgstab";
-  SegWork w;
-  std::vector<int> bstart;
-  int rc = seg_setup(a, w, bstart, who);
+  HmvMultiWork *mw = nullptr;
+  int rc = multi_work(a, 0, mw, who);
   if (rc) return rc;
+  SegWork &w = mw->w;
+  const HmvInstHost *hi = hmv::inst_host(w.h);
   auto t0 = std::chrono::steady_clock::now();
   std::vector<ColState> cs;
   std::vector<double> done_at(w.nseg, -1.0);
@@ -948,12 +1028,11 @@ extern "C" int hmv_multi_bicgstab(hmv_arena a, const double *b, double *u, doubl
     return rc;
   const double total = seconds_since(t0);
   // true residuals per instance: r = b - A u
-  std::vector<double> rr, bb;
-  if ((rc = seg_residuals(a, w, b, u, w.r, bstart, rr, bb, who))) return rc;
+  if ((rc = seg_residuals(a, w, b, u, w.r, who))) return rc;
   int maxstep = 0, worst = HMV_SOLVE_CONVERGED;
   double maxrel = 0.0;
   for (int sgi = 0; sgi < w.nseg; ++sgi) {
-    const double rel = std::sqrt(rr[sgi]) / std::sqrt(bb[sgi]);
+    const double rel = std::sqrt(hi[sgi].rr) / std::sqrt(hi[sgi].bb);
     const int status = cs[sgi].done ? cs[sgi].status : HMV_SOLVE_MAXITER;
     if (inst) {
       inst[sgi].nstp = cs[sgi].step;
@@ -990,39 +1069,28 @@ extern "C" int hmv_multi_bicgstab_ir(hmv_arena a64, hmv_arena alow, const double
     return HMV_ERR_ARG;
   }
   if (check_every < 1) check_every = 1;
-  SegWork w;  // inner solves over the low-precision arena
-  std::vector<int> bstart;
-  int rc = seg_setup(alow, w, bstart, who);
+  HmvMultiWork *mw = nullptr;  // inner solves over the low-precision arena
+  int rc = multi_work(alow, 0, mw, who);
   if (rc) return rc;
+  SegWork &w = mw->w;
+  HmvInstHost *hi = hmv::inst_host(w.h);
   const int nseg = w.nseg;
-  struct Buf {
-    double *r2 = nullptr, *d = nullptr;
-    int *stopped = nullptr;
-    ~Buf() {
-      (void)hipFree(r2);
-      (void)hipFree(d);
-      (void)hipFree(stopped);
-    }
-  } buf;
-  const size_t nbytes = sizeof(double) * (size_t)w.n;
   hipError_t e;
-  if ((e = hipMalloc(&buf.r2, nbytes)) != hipSuccess || (e = hipMalloc(&buf.d, nbytes)) != hipSuccess ||
-      (e = hipMalloc(&buf.stopped, sizeof(int) * nseg)) != hipSuccess)
-    return hmv::hip_fail(e, "hmv_multi_bicgstab_ir: workspace");
   const int g = grid_of(w.n);
   auto t0 = std::chrono::steady_clock::now();
-  std::vector<int> status(nseg, HMV_SOLVE_MAXITER), stopped(nseg, 0), steps(nseg, 0);
-  std::vector<double> rel(nseg, 0.0), done_at(nseg, -1.0), rr, bb;
+  std::vector<int> status(nseg, HMV_SOLVE_MAXITER), steps(nseg, 0);
+  std::vector<double> rel(nseg, 0.0), done_at(nseg, -1.0);
   std::vector<ColState> cs;
   int outer = 0, inner_total = 0;
+  for (int s = 0; s < nseg; ++s) hi[s].stopped = 0;
   for (;;) {
     // FP64 residual of every instance on the FP64 arena
-    if ((rc = seg_residuals(a64, w, b, u, buf.r2, bstart, rr, bb, who))) return rc;
+    if ((rc = seg_residuals(a64, w, b, u, w.r2, who))) return rc;
     const double now = seconds_since(t0);
     bool all = true;
     for (int s = 0; s < nseg; ++s) {
-      if (stopped[s]) continue;
-      rel[s] = std::sqrt(rr[s]) / std::sqrt(bb[s]);
+      if (hi[s].stopped) continue;
+      rel[s] = std::sqrt(hi[s].rr) / std::sqrt(hi[s].bb);
       if (!std::isfinite(rel[s]))
         status[s] = HMV_SOLVE_NONFINITE;
       else if (rel[s] < eps)
@@ -1031,38 +1099,34 @@ extern "C" int hmv_multi_bicgstab_ir(hmv_arena a64, hmv_arena alow, const double
         all = false;
         continue;
       }
-      stopped[s] = 1;
+      hi[s].stopped = 1;
       done_at[s] = now;
     }
     if (all || outer >= max_outer) break;
     // inner solves A_low d = r on the instances still running
-    if ((e = hipMemcpyAsync(buf.stopped, stopped.data(), sizeof(int) * nseg, hipMemcpyHostToDevice,
-                            w.s)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_multi_bicgstab_ir: flags");
-    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, buf.r2, buf.stopped);
-    hipLaunchKernelGGL(kb_fill, dim3(g), dim3(kT), 0, w.s, w.n, buf.d, 0.0);
+    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, w.r2,
+                       (const HmvInstHost *)hi);
+    hipLaunchKernelGGL(kb_fill, dim3(g), dim3(kT), 0, w.s, w.n, w.d, 0.0);
     int iters = 0;
-    if ((rc = seg_solve(alow, w, buf.r2, buf.d, inner_eps, max_inner, check_every, true, t0, cs,
+    if ((rc = seg_solve(alow, w, w.r2, w.d, inner_eps, max_inner, check_every, true, t0, cs,
                         nullptr, iters, who)))
       return rc;
     inner_total += iters;
     for (int s = 0; s < nseg; ++s) {
-      if (stopped[s]) continue;
+      if (hi[s].stopped) continue;
       steps[s] += cs[s].step;
       if (cs[s].done && cs[s].status == HMV_SOLVE_NONFINITE) {
         // the correction of this instance is not usable: it stops here
         status[s] = HMV_SOLVE_NONFINITE;
-        stopped[s] = 1;
+        hi[s].stopped = 1;
         done_at[s] = seconds_since(t0);
       }
     }
     // u += d, with d = 0 on every stopped instance (those stopped before this
     // solve never updated d; one stopped just now may hold a non-finite d)
-    if ((e = hipMemcpyAsync(buf.stopped, stopped.data(), sizeof(int) * nseg, hipMemcpyHostToDevice,
-                            w.s)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_multi_bicgstab_ir: flags");
-    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, buf.d, buf.stopped);
-    hipLaunchKernelGGL(kb_add, dim3(g), dim3(kT), 0, w.s, w.n, u, buf.d);
+    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, w.d,
+                       (const HmvInstHost *)hi);
+    hipLaunchKernelGGL(kb_add, dim3(g), dim3(kT), 0, w.s, w.n, u, w.d);
     if ((e = hipGetLastError()) != hipSuccess)
       return hmv::hip_fail(e, "hmv_multi_bicgstab_ir: update");
     ++outer;
@@ -1124,9 +1188,15 @@ struct SgGlobal {
   int ticks;  // steps ended, with those that found every instance stopped
 };
 
-// r = b, p_0 = b (zero initial guess)
+// r = b, p_0 = b (zero initial guess); the solve's parameters
 __global__ __launch_bounds__(kT) void sg_init(int64_t n, const double *__restrict__ b,
-                                              double *__restrict__ r, double *__restrict__ p) {
+                                              double *__restrict__ r, double *__restrict__ p,
+                                              SgGlobal *gs, double eps, int m, int maxit) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    gs->eps = eps;
+    gs->m = m;
+    gs->maxit = maxit;
+  }
   for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT) {
     r[i] = b[i];
     p[i] = b[i];
@@ -1288,11 +1358,13 @@ __global__ __launch_bounds__(kT) void sg_betas(int nseg, int lanes,
 //   0: setup from the (r, r), (b, b) pairs;
 //   2: ||r|| from the (r, r) partials, the step and stopping tests, then the
 //      common slots (ik = the slot just used, ikn = the next one).
-// done_flags mirrors each instance's done flag for the H-matvec.
+// done_flags mirrors each instance's done flag for the H-matvec; an instance
+// that stops leaves its steps and status in the host's record.
 __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *__restrict__ bstart,
                                                const double *__restrict__ part, SgInst *inst,
                                                SgGlobal *gs, int stage,
                                                int *__restrict__ done_flags, HmvSolveHost *h) {
+  HmvInstHost *hi = hmv::inst_host(h);
   const SgGlobal z = *gs;
   if (z.all_done && stage != 0) {
     if (threadIdx.x == 0) hmv::publish(h, gs->ticks += 1, 1);
@@ -1305,8 +1377,9 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
   for (int s = threadIdx.x / lanes; s < nseg; s += kT / lanes) {
     SgInst &c = inst[s];
     const int b0 = bstart[s], b1 = bstart[s + 1], cdone = c.done, cstep = c.step;
+    const int seen = stage == 0 ? 0 : done_flags[s];
     const double cb = c.bnorm;
-    hmv::together(b0 | b1 | cdone | cstep, cb, 0.0, 0.0);
+    hmv::together(b0 | b1 | cdone | cstep | seen, cb, 0.0, 0.0);
     double d0 = 0.0, d1 = 0.0;
     for (int b = b0 + sub; b < b1; b += lanes) {
       d0 += part[(size_t)np * b];
@@ -1353,7 +1426,14 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
     }
     if (stage == 0) stop = c.done;
     done_flags[s] = stop;
-    if (!stop) atomicAnd(&sdone, 0);
+    if (!stop) {
+      atomicAnd(&sdone, 0);
+    } else if (!seen) {  // on the host before the word that says all have stopped
+      hi[s].step = c.step;
+      hi[s].done = c.done;
+      hi[s].status = c.status;
+      __threadfence_system();
+    }
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1362,6 +1442,7 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
       gs->ik = 0;
       gs->ikn = 0;
       gs->all_done = sdone;
+      h->step = 0;
       hmv::publish(h, 0, sdone);
     } else {
       gs->ik = z.ikn;
@@ -1369,6 +1450,7 @@ __global__ __launch_bounds__(kT) void sg_final(int nseg, int lanes, const int *_
       gs->ticks = z.ticks + 1;
       gs->ikn = (z.step + 1) % z.m;
       gs->all_done = sdone;
+      if (sdone) h->step = z.step + 1;
       hmv::publish(h, z.ticks + 1, sdone);
     }
   }
@@ -1466,21 +1548,7 @@ __global__ __launch_bounds__(kT) void sg_update_dir(const SegBlock *__restrict__
   }
 }
 
-struct SegGcrWork {
-  int m = 0;
-  double *r = nullptr, *ar = nullptr, *p = nullptr, *ap = nullptr;
-  double *part = nullptr, *bpart = nullptr;  // 3 per block; one per block and slot
-  SgInst *inst = nullptr;
-  SgGlobal *gs = nullptr;
-  ~SegGcrWork() {
-    for (double *q : {r, ar, p, ap, part, bpart}) (void)hipFree(q);
-    (void)hipFree(inst);
-    (void)hipFree(gs);
-  }
-};
-
 int sg_setup(const SegWork &w, SegGcrWork &gw, int m, const char *who) {
-  gw.m = m;
   const size_t nb = sizeof(double) * (size_t)w.n;
   hipError_t e;
   if ((e = hipMalloc(&gw.r, nb)) != hipSuccess || (e = hipMalloc(&gw.ar, nb)) != hipSuccess ||
@@ -1490,6 +1558,7 @@ int sg_setup(const SegWork &w, SegGcrWork &gw, int m, const char *who) {
       (e = hipMalloc(&gw.inst, sizeof(SgInst) * w.nseg)) != hipSuccess ||
       (e = hipMalloc(&gw.gs, sizeof(SgGlobal))) != hipSuccess)
     return hmv::hip_fail(e, (std::string(who) + ": GCR workspace").c_str());
+  gw.m = m;
   return HMV_OK;
 }
 
@@ -1520,22 +1589,17 @@ hipError_t sg_iteration(hmv_arena_s *a, const SegWork &w, SegGcrWork &gw, double
 }
 
 // One GCR(m) per instance for A d = b from d = 0 (the caller zeroes d), in
-// lockstep until every instance has stopped or maxit steps ran.  inst
-// receives the instances' final states, iters the steps run.
-int sg_solve(hmv_arena_s *a, SegWork &w, SegGcrWork &gw, const double *b, double *d,
-             double eps, int maxit, std::vector<SgInst> &inst, int &iters,
-             const char *who) {
+// lockstep until every instance has stopped or maxit (>= 1) steps ran.  The
+// host's records receive the instances' steps and states, iters the steps
+// run.
+int sg_solve(hmv_arena_s *a, SegWork &w, SegGcrWork &gw, const double *b, double *d, double eps,
+             int maxit, int &iters, const char *who) {
   const std::string name(who);
-  SgGlobal init{};
-  init.eps = eps;
-  init.m = gw.m;
-  init.maxit = maxit;
   const int g = grid_of(w.n);
   hipError_t e = hmv::solve_host(a, w.s, w.h);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(gw.gs, &init, sizeof(init), hipMemcpyHostToDevice, w.s);
   if (e != hipSuccess) return hmv::hip_fail(e, (name + ": setup").c_str());
-  hipLaunchKernelGGL(sg_init, dim3(g), dim3(kT), 0, w.s, w.n, b, gw.r, gw.p);
+  hipLaunchKernelGGL(sg_init, dim3(g), dim3(kT), 0, w.s, w.n, b, gw.r, gw.p, gw.gs, eps, gw.m,
+                     maxit);
   hipLaunchKernelGGL(ks_dots, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, gw.r, gw.r, b, b, gw.part,
                      (const BlockState *)nullptr);
   hipLaunchKernelGGL(sg_final, dim3(1), dim3(kT), 0, w.s, w.nseg, w.lanes, w.bstart,
@@ -1548,18 +1612,11 @@ int sg_solve(hmv_arena_s *a, SegWork &w, SegGcrWork &gw, const double *b, double
                      gw.part, (const SgGlobal *)gw.gs);
   if ((e = hipGetLastError()) != hipSuccess)
     return hmv::hip_fail(e, (name + ": setup").c_str());
-  SgGlobal host{};
   int launched = 0;
-  if ((e = hmv::feed(w.h, w.s, launched, maxit,
-                     [&] { return sg_iteration(a, w, gw, d); })) != hipSuccess ||
-      (e = hipMemcpyAsync(&host, gw.gs, sizeof(host), hipMemcpyDeviceToHost, w.s)) != hipSuccess)
-    return hmv::hip_fail(e, (name + ": iterations").c_str());
-  inst.resize(w.nseg);
-  if ((e = hipMemcpyAsync(inst.data(), gw.inst, sizeof(SgInst) * w.nseg, hipMemcpyDeviceToHost,
-                          w.s)) != hipSuccess ||
-      (e = hipStreamSynchronize(w.s)) != hipSuccess)
-    return hmv::hip_fail(e, (name + ": state").c_str());
-  iters = host.step;
+  e = hmv::feed(w.h, w.s, launched, maxit, [&] { return sg_iteration(a, w, gw, d); });
+  if (e == hipSuccess && !hmv::stopped(w.h)) e = hipStreamSynchronize(w.s);
+  if (e != hipSuccess) return hmv::hip_fail(e, (name + ": iterations").c_str());
+  iters = w.h->step;
   return HMV_OK;
 }
 
@@ -1577,41 +1634,28 @@ extern "C" int hmv_multi_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, 
                    "1 <= m <= 32, 0 < inner_eps < 1)");
     return HMV_ERR_ARG;
   }
-  SegWork w;  // block table, stream and FP64 residuals
-  std::vector<int> bstart;
-  int rc = seg_setup(alow, w, bstart, who);
+  HmvMultiWork *mw = nullptr;
+  int rc = multi_work(alow, m, mw, who);
   if (rc) return rc;
-  SegGcrWork gw;
-  if ((rc = sg_setup(w, gw, m, who))) return rc;
+  SegWork &w = mw->w;  // block table, stream and FP64 residuals
+  SegGcrWork &gw = mw->gw;
+  HmvInstHost *hi = hmv::inst_host(w.h);
   const int nseg = w.nseg;
-  struct Buf {
-    double *r2 = nullptr, *d = nullptr;
-    int *stopped = nullptr;
-    ~Buf() {
-      (void)hipFree(r2);
-      (void)hipFree(d);
-      (void)hipFree(stopped);
-    }
-  } buf;
-  const size_t nbytes = sizeof(double) * (size_t)w.n;
   hipError_t e;
-  if ((e = hipMalloc(&buf.r2, nbytes)) != hipSuccess || (e = hipMalloc(&buf.d, nbytes)) != hipSuccess ||
-      (e = hipMalloc(&buf.stopped, sizeof(int) * nseg)) != hipSuccess)
-    return hmv::hip_fail(e, "hmv_multi_gcr_ir: workspace");
   const int g = grid_of(w.n);
   auto t0 = std::chrono::steady_clock::now();
-  std::vector<int> status(nseg, HMV_SOLVE_MAXITER), stopped(nseg, 0), steps(nseg, 0);
-  std::vector<double> rel(nseg, 0.0), done_at(nseg, -1.0), rr, bb;
-  std::vector<SgInst> cs;
+  std::vector<int> status(nseg, HMV_SOLVE_MAXITER), steps(nseg, 0);
+  std::vector<double> rel(nseg, 0.0), done_at(nseg, -1.0);
   int outer = 0, inner_total = 0;
+  for (int s = 0; s < nseg; ++s) hi[s].stopped = 0;
   for (;;) {
     // FP64 residual of every instance on the FP64 arena
-    if ((rc = seg_residuals(a64, w, b, u, buf.r2, bstart, rr, bb, who))) return rc;
+    if ((rc = seg_residuals(a64, w, b, u, w.r2, who))) return rc;
     const double now = seconds_since(t0);
     bool all = true;
     for (int s = 0; s < nseg; ++s) {
-      if (stopped[s]) continue;
-      rel[s] = std::sqrt(rr[s]) / std::sqrt(bb[s]);
+      if (hi[s].stopped) continue;
+      rel[s] = std::sqrt(hi[s].rr) / std::sqrt(hi[s].bb);
       if (!std::isfinite(rel[s]))
         status[s] = HMV_SOLVE_NONFINITE;
       else if (rel[s] < eps)
@@ -1620,38 +1664,33 @@ extern "C" int hmv_multi_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, 
         all = false;
         continue;
       }
-      stopped[s] = 1;
+      hi[s].stopped = 1;
       done_at[s] = now;
     }
     if (all || outer >= max_outer) break;
     // inner solves A_low d = r on the instances still running (a stopped
     // instance's r is zero, so its inner solve stops at the setup)
-    if ((e = hipMemcpyAsync(buf.stopped, stopped.data(), sizeof(int) * nseg, hipMemcpyHostToDevice,
-                            w.s)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_multi_gcr_ir: flags");
-    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, buf.r2, buf.stopped);
-    hipLaunchKernelGGL(kb_fill, dim3(g), dim3(kT), 0, w.s, w.n, buf.d, 0.0);
+    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, w.r2,
+                       (const HmvInstHost *)hi);
+    hipLaunchKernelGGL(kb_fill, dim3(g), dim3(kT), 0, w.s, w.n, w.d, 0.0);
     int iters = 0;
-    if ((rc = sg_solve(alow, w, gw, buf.r2, buf.d, inner_eps, max_inner, cs, iters,
-                       who)))
+    if ((rc = sg_solve(alow, w, gw, w.r2, w.d, inner_eps, max_inner, iters, who)))
       return rc;
     inner_total += iters;
     for (int s = 0; s < nseg; ++s) {
-      if (stopped[s]) continue;
-      steps[s] += cs[s].step;
-      if (cs[s].done && cs[s].status == HMV_SOLVE_NONFINITE) {
+      if (hi[s].stopped) continue;
+      steps[s] += hi[s].step;
+      if (hi[s].done && hi[s].status == HMV_SOLVE_NONFINITE) {
         // the correction of this instance is not usable: it stops here
         status[s] = HMV_SOLVE_NONFINITE;
-        stopped[s] = 1;
+        hi[s].stopped = 1;
         done_at[s] = seconds_since(t0);
       }
     }
     // u += d, with d = 0 on every stopped instance
-    if ((e = hipMemcpyAsync(buf.stopped, stopped.data(), sizeof(int) * nseg, hipMemcpyHostToDevice,
-                            w.s)) != hipSuccess)
-      return hmv::hip_fail(e, "hmv_multi_gcr_ir: flags");
-    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, buf.d, buf.stopped);
-    hipLaunchKernelGGL(kb_add, dim3(g), dim3(kT), 0, w.s, w.n, u, buf.d);
+    hipLaunchKernelGGL(ks_zero_stopped, dim3(w.nblk), dim3(kT), 0, w.s, w.tb, w.d,
+                       (const HmvInstHost *)hi);
+    hipLaunchKernelGGL(kb_add, dim3(g), dim3(kT), 0, w.s, w.n, u, w.d);
     if ((e = hipGetLastError()) != hipSuccess)
       return hmv::hip_fail(e, "hmv_multi_gcr_ir: update");
     ++outer;

@@ -69,6 +69,7 @@ struct hmv_arena_s {
   hipStream_t hstream = nullptr;
   HmvSolveWork *solve = nullptr;             // solver workspace (lazy)
   struct HmvGcrWork *gcr = nullptr;          // GCR(m) workspace (lazy)
+  struct HmvMultiWork *multi = nullptr;      // per-instance solvers' workspace (lazy)
   HmvSolveHost *solve_host = nullptr;        // pinned memory of the solvers (hmv_feed.h)
   hmv_arena_stats stats{};
   // what a saved arena file needs besides the device tables
@@ -87,6 +88,7 @@ hipError_t enqueue_apply(hmv_arena_s *a, const double *x, double *y, double beta
                          hipStream_t s, const int *inst_done = nullptr);
 void free_solve_work(hmv_arena_s *a);
 void free_gcr_work(hmv_arena_s *a);
+void free_multi_work(hmv_arena_s *a);
 // The arena's H-matmat unit lists and path choices.
 void fill_units(const hmv_arena_s *a, HmvUnits &u);
 // Enqueues Y = H X + beta*Y for k interleaved right-hand sides (1..128).

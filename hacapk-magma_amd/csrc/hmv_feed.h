@@ -33,9 +33,20 @@ struct HmvSolveHost {
   double part[2 * kSolveMaxBlocks];  // partial dot products read on the host
 };
 
+// ... followed by one of these for each instance of a multi-instance arena.
+struct HmvInstHost {
+  double rr, bb;           // summed dots of its segment
+  int step, done, status;  // valid once stopped
+  int stopped;             // written by the host, read by the kernels
+};
+
 namespace hmv {
 
 constexpr int kFeedWindow = 2;
+
+__host__ __device__ inline HmvInstHost *inst_host(HmvSolveHost *h) {
+  return reinterpret_cast<HmvInstHost *>(h + 1);
+}
 
 // Has the values, loads still under way included, in registers here: the
 // loads above are issued together and waited for once.  The solvers' vector
@@ -64,7 +75,8 @@ __device__ inline void publish(HmvSolveHost *h, int ticks, int done) {
 inline hipError_t solve_host(hmv_arena_s *a, hipStream_t s, HmvSolveHost *&h) {
   hipError_t e;
   if (!a->solve_host &&
-      (e = hipHostMalloc((void **)&a->solve_host, sizeof(HmvSolveHost),
+      (e = hipHostMalloc((void **)&a->solve_host,
+                         sizeof(HmvSolveHost) + a->seg.size() * sizeof(HmvInstHost),
                          hipHostMallocMapped | hipHostMallocCoherent)) != hipSuccess) {
     a->solve_host = nullptr;
     return e;

@@ -353,10 +353,17 @@ __global__ __launch_bounds__(kT) void g_update_dir(int n, int nbb, const double 
   }
 }
 
-// r = b - ar (r = b when ar is null: a zero initial guess);  p_1 = r
+// r = b - ar (r = b when ar is null: a zero initial guess);  p_1 = r; the
+// state's parameters (st may be null)
 __global__ __launch_bounds__(kT) void g_init(int n, const double *__restrict__ b,
                                              const double *__restrict__ ar,
-                                             double *__restrict__ r, double *__restrict__ p) {
+                                             double *__restrict__ r, double *__restrict__ p,
+                                             GcrState *st, double eps, int m, int maxit) {
+  if (st && blockIdx.x == 0 && threadIdx.x == 0) {
+    st->eps = eps;
+    st->m = m;
+    st->maxit = maxit;
+  }
   for (int i = blockIdx.x * kT + threadIdx.x; i < n; i += gridDim.x * kT) {
     const double ri = ar ? b[i] - ar[i] : b[i];
     r[i] = ri;
@@ -485,15 +492,10 @@ int gcrm_run(hmv_arena a, const double *b, double *u, double eps, int maxit, int
   if ((e = hmv::solve_host(a, w.s, h)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_gcrm: workspace");
   auto t0 = std::chrono::steady_clock::now();
-  GcrState init{};
-  init.eps = eps;
-  init.m = m;
-  init.maxit = maxit;
-  if ((e = hipMemcpyAsync(w.st, &init, sizeof(init), hipMemcpyHostToDevice, w.s)) != hipSuccess ||
-      (!zero_guess && (e = hmv::enqueue_apply(a, u, w.ar, 0.0, nullptr, w.s)) != hipSuccess))
+  if (!zero_guess && (e = hmv::enqueue_apply(a, u, w.ar, 0.0, nullptr, w.s)) != hipSuccess)
     return hmv::hip_fail(e, "hmv_gcrm: setup");
   hipLaunchKernelGGL(g_init, dim3(g), dim3(kT), 0, w.s, n, b, zero_guess ? nullptr : w.ar, w.r,
-                     w.p);
+                     w.p, w.st, eps, m, maxit);
   hipLaunchKernelGGL(g_dots2, dim3(g), dim3(kT), 0, w.s, n, w.r, w.r, b, b, w.part);
   hipLaunchKernelGGL(g_final, dim3(1), dim3(kT), 0, w.s, g, w.part, w.st, 0, w.hist, h);
   // ap_1 = A p_1 (skipped when already converged) and the first step's
@@ -521,7 +523,8 @@ int gcrm_run(hmv_arena a, const double *b, double *u, double eps, int maxit, int
   if (true_res) {
     if ((e = hmv::enqueue_apply(a, u, w.ar, 0.0, nullptr, w.s)) != hipSuccess)
       return hmv::hip_fail(e, "hmv_gcrm: true residual");
-    hipLaunchKernelGGL(g_init, dim3(g), dim3(kT), 0, w.s, n, b, w.ar, w.r, w.p);
+    hipLaunchKernelGGL(g_init, dim3(g), dim3(kT), 0, w.s, n, b, w.ar, w.r, w.p,
+                       (GcrState *)nullptr, 0.0, 0, 0);
     hipLaunchKernelGGL(g_dots2, dim3(g), dim3(kT), 0, w.s, n, w.r, w.r, b, b, h->part);
     if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(w.s)) != hipSuccess)
       return hmv::hip_fail(e, "hmv_gcrm: true residual");

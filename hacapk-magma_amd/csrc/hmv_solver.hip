@@ -341,12 +341,18 @@ __global__ __launch_bounds__(kThreads) void k_update_ur(
   }
 }
 
-// r = b - Ab (in place: y holds A u on entry), rhat = r, p = v = 0
+// r = b - Ab (in place: y holds A u on entry), rhat = r, p = v = 0;
+// the state's parameters
 __global__ __launch_bounds__(kThreads) void k_init(int n, const double *__restrict__ b,
                                                     double *__restrict__ r,
                                                     double *__restrict__ rhat,
                                                     double *__restrict__ p,
-                                                    double *__restrict__ v, int zero_guess) {
+                                                    double *__restrict__ v, int zero_guess,
+                                                    SolveState *st, double eps, int maxit) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->eps = eps;
+    st->maxit = maxit;
+  }
   for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
     const double ri = zero_guess ? b[i] : b[i] - r[i];  // r holds A u unless u = 0
     r[i] = ri;
@@ -490,18 +496,13 @@ int run_bicgstab(hmv_arena_s *a, const double *b, double *u, double eps, int max
   auto t0 = std::chrono::steady_clock::now();
 
   // r = b - A u; r^ = r; p = v = 0; rr = (r,r), bnorm = sqrt((b,b)) on device
-  SolveState init{};
-  init.eps = eps;
-  init.maxit = maxit;
   HmvSolveHost *h = nullptr;
   if ((e = hmv::solve_host(a, s, h)) != hipSuccess)
     return hmv::hip_fail(e, "bicgstab: workspace");
-  if ((e = hipMemcpyAsync(w->st, &init, sizeof(init), hipMemcpyHostToDevice, s)) != hipSuccess)
-    return hmv::hip_fail(e, "bicgstab: state upload");
   if (!zero_guess && (e = hmv::enqueue_apply(a, u, w->r, 0.0, nullptr, s)) != hipSuccess)
     return hmv::hip_fail(e, "bicgstab: initial apply");
   hipLaunchKernelGGL(k_init, dim3(g), dim3(kThreads), 0, s, n, b, w->r, w->rhat, w->p, w->v,
-                     zero_guess ? 1 : 0);
+                     zero_guess ? 1 : 0, w->st, eps, maxit);
   hipLaunchKernelGGL(k_dots, dim3(g), dim3(kThreads), 0, s, n, w->r, w->r, b, b, w->part,
                      (const SolveState *)nullptr);
   hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 0, w->hist,
@@ -659,17 +660,14 @@ int hmv_bicgstab_ru(hmv_arena a64, hmv_arena alow, const double *b, double *u, d
   hipStream_t s = w->stream;
   hipError_t e;
   auto t0 = std::chrono::steady_clock::now();
-  SolveState init{};
-  init.eps = eps;
-  init.maxit = maxit;
   HmvSolveHost *h = nullptr;
   if ((e = hmv::solve_host(alow, s, h)) != hipSuccess)
     return hmv::hip_fail(e, "bicgstab_ru: workspace");
   // r = b - A64 u, r^ = r, p = v = 0
-  if ((e = hipMemcpyAsync(w->st, &init, sizeof(init), hipMemcpyHostToDevice, s)) != hipSuccess ||
-      (e = hmv::enqueue_apply(a64, u, w->r, 0.0, nullptr, s)) != hipSuccess)
+  if ((e = hmv::enqueue_apply(a64, u, w->r, 0.0, nullptr, s)) != hipSuccess)
     return hmv::hip_fail(e, "bicgstab_ru: setup");
-  hipLaunchKernelGGL(k_init, dim3(g), dim3(kThreads), 0, s, n, b, w->r, w->rhat, w->p, w->v, 0);
+  hipLaunchKernelGGL(k_init, dim3(g), dim3(kThreads), 0, s, n, b, w->r, w->rhat, w->p, w->v, 0,
+                     w->st, eps, maxit);
   hipLaunchKernelGGL(k_dots, dim3(g), dim3(kThreads), 0, s, n, w->r, w->r, b, b, w->part,
                      (const SolveState *)nullptr);
   hipLaunchKernelGGL(k_final, dim3(1), dim3(kThreads), 0, s, g, w->part, w->st, 0, w->hist,
