@@ -40,15 +40,20 @@ int hip_fail(hipError_t e, const char *what) {
 // process may use).  The workers sleep between calls and are joined at exit.
 class HostPool {
  public:
+  static constexpr size_t kPoolMin = 131072;
   static HostPool &get() {
     static HostPool pool;
     return pool;
   }
   // fn(lo, hi) over [0, n) in nparts() contiguous parts; the caller runs
-  // the first part itself.
+  // the first part itself.  Below kPoolMin the caller runs it all: waking
+  // the threads takes 20 us a pass, more than they save (a host product,
+  // with two passes, on one thread and on 8: 47 and 81 us at 6,400 unknowns,
+  // 213 and 238 at 81,920, 342 and 364 at 122,880, 416 and 415 at 163,840,
+  // 795 and 756 at 327,680).
   void parallel_for(size_t n, const std::function<void(size_t, size_t)> &fn) {
     const size_t parts = th_.size() + 1;
-    if (parts == 1 || n < 4096) {
+    if (parts == 1 || n < kPoolMin) {
       fn(0, n);
       return;
     }
@@ -855,11 +860,14 @@ int hmv_apply_host(hmv_arena a, const double *zu, double *zau) {
     set_error("hmv_apply_host: null argument");
     return HMV_ERR_ARG;
   }
+  constexpr size_t kUploadMax = 65536;
   hipError_t e;
   const size_t n = (size_t)a->nd, nb = sizeof(double) * n;
   if (!a->hstream) {  // created last: set only when every buffer exists
     if ((e = hipMalloc(&a->d_hx, nb)) != hipSuccess ||
-        (e = hipHostMalloc((void **)&a->h_x, nb, hipHostMallocDefault)) != hipSuccess ||
+        (e = hipHostMalloc((void **)&a->h_x, nb, hipHostMallocMapped | hipHostMallocCoherent)) !=
+            hipSuccess ||
+        (e = hipHostGetDevicePointer((void **)&a->h_x_dev, a->h_x, 0)) != hipSuccess ||
         (e = hipHostMalloc((void **)&a->h_y, nb, hipHostMallocDefault)) != hipSuccess ||
         (e = hipHostGetDevicePointer((void **)&a->h_y_dev, a->h_y, 0)) != hipSuccess ||
         (e = hipStreamCreateWithFlags(&a->hstream, hipStreamNonBlocking)) != hipSuccess) {
@@ -867,12 +875,12 @@ int hmv_apply_host(hmv_arena a, const double *zu, double *zau) {
       (void)hipFree(a->d_hx);
       (void)hipHostFree(a->h_x);
       (void)hipHostFree(a->h_y);
-      a->d_hx = a->h_x = a->h_y = a->h_y_dev = nullptr;
+      a->d_hx = a->h_x = a->h_x_dev = a->h_y = a->h_y_dev = nullptr;
       a->hstream = nullptr;
       return hip_fail(e, "hmv_apply_host: setup");
     }
   }
-  // one copy over PCIe, from pinned staging: zu up; the apply's phase 2
+  // one pass over PCIe, from pinned staging: zu up; the apply's phase 2
   // writes H zu straight into pinned host memory as its rows finish (0.48
   // against 0.52 ms with a download after the apply at 163,840 unknowns).
   // The CPU's passes over the caller's arrays (zu into staging, zau += H zu
@@ -882,7 +890,13 @@ int hmv_apply_host(hmv_arena a, const double *zu, double *zau) {
   pool.parallel_for(n, [&](size_t lo, size_t hi) {
     std::memcpy(hx + lo, zu + lo, sizeof(double) * (hi - lo));
   });
-  if ((e = hipMemcpyAsync(a->d_hx, hx, nb, hipMemcpyHostToDevice, a->hstream)) != hipSuccess)
+  // a kernel reads a short x over PCIe 5 us sooner than the copy engine has
+  // it there (a product of 6,400 unknowns 81 -> 77 us, of 26k 131 -> 125,
+  // of 42k 152 -> 148, of 82k 239 -> 237); a long one later (102k 297 -> 299,
+  // 123k 364 -> 369)
+  e = n <= kUploadMax ? hmv::launch_upload((int)n, a->h_x_dev, a->d_hx, a->hstream)
+                      : hipMemcpyAsync(a->d_hx, hx, nb, hipMemcpyHostToDevice, a->hstream);
+  if (e != hipSuccess)
     return hip_fail(e, "hmv_apply_host: copy x");
   if ((e = hmv::enqueue_apply(a, a->d_hx, a->h_y_dev, 0.0, nullptr, a->hstream)) != hipSuccess)
     return hip_fail(e, "hmv_apply_host: launch");

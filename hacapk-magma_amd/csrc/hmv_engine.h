@@ -62,10 +62,10 @@ struct hmv_arena_s {
   std::vector<int> seg;    // instance row offsets (ninst + 1) of a multi-instance arena
   int *d_winst1 = nullptr, *d_winst2 = nullptr;  // instance of each work item (multi only)
   hmv_tuning tuning{};     // the tuning the arena was built with
-  // hmv_apply_host: device x, pinned host staging of x and y, y's device
-  // address (the apply writes H zu there directly), its stream (made on the
+  // hmv_apply_host: device x, pinned host staging of x and y, their device
+  // addresses (the apply writes H zu there directly), its stream (made on the
   // first call)
-  double *d_hx = nullptr, *h_x = nullptr, *h_y = nullptr, *h_y_dev = nullptr;
+  double *d_hx = nullptr, *h_x = nullptr, *h_x_dev = nullptr, *h_y = nullptr, *h_y_dev = nullptr;
   hipStream_t hstream = nullptr;
   HmvSolveWork *solve = nullptr;             // solver workspace (lazy)
   struct HmvGcrWork *gcr = nullptr;          // GCR(m) workspace (lazy)
@@ -94,6 +94,8 @@ void fill_units(const hmv_arena_s *a, HmvUnits &u);
 // Enqueues Y = H X + beta*Y for k interleaved right-hand sides (1..128).
 hipError_t enqueue_apply_block(hmv_arena_s *a, int k, const double *x, double *y, double beta,
                                const int *skip, hipStream_t s);
+// dst[i] = src[i], src in pinned host memory.
+hipError_t launch_upload(int n, const double *src, double *dst, hipStream_t s);
 // Runs an arena's fill records on the device (image zeroed beforehand).
 hipError_t launch_fill(const FillOps &ops, char *arena);
 // Arena from leaves whose factors are in device memory (hmv_construct).

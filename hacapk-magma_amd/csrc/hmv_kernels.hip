@@ -395,3 +395,22 @@ extern "C" hipError_t hmv_launch_apply(const HmvLaunch *L, int phases, const dou
     launch_mode<float, HMV_DT_BF16, HMV_DT_BF16>(*L, phases, x, y, beta, skip, inst_done, stream);
   return hipGetLastError();
 }
+
+// x of a host product, read over PCIe from the pinned staging: 16 bytes a
+// thread, both arrays being allocations of their own.
+__global__ __launch_bounds__(256) void hmv_upload_kernel(int n, const double *__restrict__ src,
+                                                         double *__restrict__ dst) {
+  const int i = 2 * (blockIdx.x * 256 + threadIdx.x);
+  if (i + 1 < n)
+    *reinterpret_cast<double2 *>(dst + i) = *reinterpret_cast<const double2 *>(src + i);
+  else if (i < n)
+    dst[i] = src[i];
+}
+
+namespace hmv {
+hipError_t launch_upload(int n, const double *src, double *dst, hipStream_t s) {
+  if (n < 1) return hipSuccess;
+  hipLaunchKernelGGL(hmv_upload_kernel, dim3((n + 511) / 512), dim3(256), 0, s, n, src, dst);
+  return hipGetLastError();
+}
+}  // namespace hmv

@@ -305,3 +305,31 @@ def test_launches_around_the_longer_batches(gpu, O, prec, n):
     err = _rel(a.matvec(x), O.adot_body_lfmtx(hm, x))
     assert err <= {"f64": TOL64, "f32": 1e-5, "bf16": 2e-2, "bf16_all": 2e-2}[prec]
     a.free()
+
+
+# x read by a kernel up to 65,536 unknowns and copied above; the host's
+# passes on one thread below 131,072; odd lengths (the kernel reads pairs)
+@pytest.mark.parametrize("nd", [1, 3, 4097, 65535, 65536, 65537, 131071, 131073])
+def test_apply_host_lengths(gpu, nd):
+    """zau += H zu for a block-diagonal H (16 x 16 dense blocks) equals the
+    blocks' products on the host; every call sees its own zu.  At most 16
+    terms and the old zau are summed: 32 rounding errors of the sum of their
+    sizes."""
+    from synthetic_leaves import LeafSet
+    w = 16
+    sizes = [min(w, nd - r) for r in range(0, nd, w)]
+    lv = LeafSet(gpu, nd, [("dense", i * w, m, i * w, m, 0) for i, m in enumerate(sizes)], nd)
+    A = np.zeros((len(sizes), w, w))
+    for i, (buf, m) in enumerate(zip(lv._bufs, sizes)):
+        A[i, :m, :m] = buf.reshape(m, m)
+    a = gpu.Arena(lv, "f64")
+    for seed in (1, 2, 3):
+        zu, zau = gpu.uniform(seed, nd), gpu.uniform(10 + seed, nd)
+        x = np.zeros(len(sizes) * w)
+        x[:nd] = zu
+        x = x.reshape(-1, w, 1)
+        ref = zau + np.matmul(A, x).reshape(-1)[:nd]
+        size = np.abs(zau) + np.matmul(np.abs(A), np.abs(x)).reshape(-1)[:nd]
+        a.apply_host(zu, zau)
+        assert np.all(np.abs(zau - ref) <= 32 * 2.0 ** -53 * size)
+    a.free()
