@@ -124,15 +124,16 @@ constexpr int kPad = 32;    // zero-input entries past a window (one group of co
 // B source of columns past a window or part (never written)
 __device__ __attribute__((aligned(16))) double g_zero_inputs[128];
 
-// Right-hand side held by column j0 of RHS tile tt: 16 tt + j0 up to two
-// tiles; from four tiles on the tiles go in pairs, tile 2s + b holding
-// 32 s + 2 j0 + b, so that a lane's inputs of the two tiles of a pair are
-// adjacent and one 16-byte load brings both (for k = 128 five loads per
-// column quad instead of nine: one for A, four for B; 4.62 against 4.96 ms
-// at 327,680 unknowns, 2.53 against 2.72 at k = 64, products bit-equal).
+// Right-hand side held by column j0 of RHS tile tt: 16 tt + j0 for one tile;
+// from two on the tiles go in pairs, tile 2s + b holding 32 s + 2 j0 + b, so
+// that a lane's inputs of the two tiles of a pair are adjacent and one
+// 16-byte load brings both (for k = 128 five loads per column quad instead
+// of nine: one for A, four for B; 4.62 against 4.96 ms at 327,680 unknowns,
+// 2.53 against 2.72 at k = 64, products bit-equal; at k = 32 1.65 against
+// 1.69 ms, at k = 50 2.52 against 2.70, at k = 96 4.52 against 4.77).
 template <int KT>
 constexpr bool bpaired() {
-  return KT >= 4;
+  return KT >= 2;
 }
 template <int KT>
 __device__ inline int bcol(int tt, int j0) {
@@ -142,18 +143,23 @@ __device__ inline int bcol(int tt, int j0) {
 // Per-wave constants of the B loads.  Lane l (j0 = l%16) points at its
 // column's inputs + jl (jl = bcol(0, j0)); tile tt's input is jd[tt] =
 // bcol(tt, j0) - jl past it.  EXACT (k == 16 KT, inputs 16-byte aligned):
-// read at 16 tt, or paired tiles as 16-byte loads; otherwise each input is
-// read on its own at min(bcol, k - 1) (inputs j >= k only feed accumulator
-// columns that are not stored; the clamp keeps the read inside the
-// column's k values).
+// read at 16 tt, or paired tiles as aligned 16-byte loads; otherwise each
+// input (KT = 1) is read at min(bcol, k - 1), each pair as a 16-byte load of
+// 8-byte alignment at min(bcol, k - 2), where the pair that starts with the
+// column's last input takes it from the second half (inputs j >= k only feed
+// accumulator columns that are not stored; the clamps keep the reads inside
+// the column's k values; k > 16 where there are pairs).
 template <int KT>
 struct BLane {
   int j0;  // l % 16: the A row of the lane and its accumulator column
   int jl;
   int jd[KT];
+  int last;  // pair whose first input is the column's last one (k odd), or -1
 };
 typedef double gd2 __attribute__((ext_vector_type(2)));
 typedef const gd2 __attribute__((address_space(1))) ggd2;
+typedef gd2 gd2u __attribute__((aligned(8)));
+typedef const gd2u __attribute__((address_space(1))) ggd2u;
 
 // One prefetch group: U column quads of A (NT tiles) and B (KT RHS tiles),
 // as loaded (widened to Acc at the MFMA).
@@ -202,6 +208,13 @@ __device__ inline void load_group(Group<DT, KT, NT, U> &g, __amdgpu_buffer_rsrc_
       for (int tt = 0; tt < KT; tt += 2) {
         const gd2 v = *(ggd2 *)(p + 32 * (tt >> 1));
         g.b[u][tt] = v.x;
+        g.b[u][tt + 1] = v.y;
+      }
+    } else if constexpr (bpaired<KT>()) {
+#pragma unroll
+      for (int tt = 0; tt < KT; tt += 2) {
+        const gd2u v = *(ggd2u *)(p + bl.jd[tt]);
+        g.b[u][tt] = bl.last == (tt >> 1) ? v.y : v.x;
         g.b[u][tt + 1] = v.y;
       }
     } else {
@@ -339,7 +352,9 @@ __global__ __launch_bounds__(64 * NW) void hmv_matmat_kernel(
   bl.j0 = lane & 15;
   bl.jl = bcol<KT>(0, bl.j0);
 #pragma unroll
-  for (int tt = 0; tt < KT; ++tt) bl.jd[tt] = min(bcol<KT>(tt, bl.j0), k - 1) - bl.jl;
+  for (int tt = 0; tt < KT; ++tt)
+    bl.jd[tt] = min(bcol<KT>(tt, bl.j0), k - (bpaired<KT>() ? 2 : 1)) - bl.jl;
+  bl.last = (k & 1) && bl.j0 == ((k - 1) & 31) >> 1 ? (k - 1) >> 5 : -1;
   const Inputs in = load_inputs<64 * NW>(w, zsegs, runs);
   const __amdgpu_buffer_rsrc_t rs0 =
       rsrc(arena + w.off0, (uint32_t)((size_t)w.rows_p * w.ncol0 * Entry<DT0>::es));

@@ -243,3 +243,29 @@ def test_matmat_waves_sharing_a_unit(gpu, O, prec, k):
         assert np.linalg.norm(Y[:, j] - ref) / np.linalg.norm(ref) <= tol
     assert np.array_equal(a.matmat(X), Y)
     a.free()
+
+
+@pytest.fixture(scope="module")
+def sphere6_arenas(gpu):
+    nodes, faces = gpu.icosphere(6)  # more units than share waves
+    dm = gpu.DeviceHMatrix(nodes, faces, gpu.baseline_params(aca_eps=1e-4))
+    out = {p: dm.arena(p) for p in ("f64", "bf16")}
+    dm.free()
+    yield out
+    for a in out.values():
+        a.free()
+
+
+@pytest.mark.parametrize("prec", ["f64", "bf16"])
+@pytest.mark.parametrize("k", [17, 18, 31, 33, 47, 62, 63, 65, 97, 126, 127])
+def test_matmat_pairs_up_to_the_last_column(gpu, sphere4, sphere6_arenas, prec, k):
+    """A lane reads pairs of right-hand sides; with k odd the last pair starts
+    one column early.  Every column has the bits it has among a full tile
+    count of right-hand sides (the others' inputs do not enter its sums)."""
+    full = 32 if k <= 32 else 64 if k <= 64 else 128
+    small = gpu.Arena(sphere4, prec)
+    for a in (small, sphere6_arenas[prec]):
+        X = gpu.uniform(k, a.nd * full).reshape(a.nd, full)
+        ref = a.matmat(X)[:, :k]
+        assert np.array_equal(a.matmat(np.ascontiguousarray(X[:, :k])), ref)
+    small.free()
