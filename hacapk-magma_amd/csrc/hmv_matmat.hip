@@ -8,9 +8,10 @@
 // column groups in turn and add their accumulators in wave order at the end.
 //
 // The wave walks the item's columns four at a time.  Per column quad, one
-// 8-byte (or 4/2-byte) load per lane and tile gives the 16 x 4 A fragment
-// (lane l: row l%16 of column l/16 of the column-major block), and KT loads
-// per lane give the 4 x 16 B fragments x[column][16 tt + l%16] straight
+// 16-byte (or 8/4-byte) load per lane and two tiles gives two 16 x 4 A
+// fragments (lane l: rows 2 (l%16) and 2 (l%16) + 1 of column l/16 of the
+// column-major block; a tile on its own: one entry, row l%16), and one load
+// per lane and two RHS tiles gives two 4 x 16 B fragments (bcol) straight
 // from the interleaved inputs: phase 1 from its item's x run, phase 2
 // through a per-wave LDS table of the columns' input addresses (L2-resident
 // inputs: the units of an XCD are neighbouring items, so they share
@@ -34,6 +35,8 @@ namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef double gd2 __attribute__((ext_vector_type(2)));
+typedef float gf2 __attribute__((ext_vector_type(2)));
 
 constexpr int kNT = 2;                  // nontemporal cache policy
 
@@ -74,6 +77,11 @@ struct Entry<HMV_DT_F64> {
   __device__ static double load_raw(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kNT));
   }
+  __device__ static void load_pair(__amdgpu_buffer_rsrc_t r, uint32_t off, double &a, double &b) {
+    const gd2 v = __builtin_bit_cast(gd2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kNT));
+    a = v.x;
+    b = v.y;
+  }
   __device__ static double widen(double v) { return v; }
 };
 template <>
@@ -83,6 +91,11 @@ struct Entry<HMV_DT_F32> {
   __device__ static float load_raw(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kNT));
   }
+  __device__ static void load_pair(__amdgpu_buffer_rsrc_t r, uint32_t off, float &a, float &b) {
+    const gf2 v = __builtin_bit_cast(gf2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kNT));
+    a = v.x;
+    b = v.y;
+  }
   __device__ static float widen(float v) { return v; }
 };
 template <>
@@ -91,6 +104,11 @@ struct Entry<HMV_DT_BF16> {
   using raw = uint32_t;
   __device__ static uint32_t load_raw(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, kNT);
+  }
+  __device__ static void load_pair(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t &a,
+                                   uint32_t &b) {
+    a = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kNT);
+    b = a >> 16;  // widen() drops a's upper half
   }
   __device__ static float widen(uint32_t v) { return __uint_as_float(v << 16); }
 };
@@ -156,7 +174,6 @@ struct BLane {
   int jd[KT];
   int last;  // pair whose first input is the column's last one (k odd), or -1
 };
-typedef double gd2 __attribute__((ext_vector_type(2)));
 typedef const gd2 __attribute__((address_space(1))) ggd2;
 typedef gd2 gd2u __attribute__((aligned(8)));
 typedef const gd2u __attribute__((address_space(1))) ggd2u;
@@ -181,10 +198,24 @@ struct BSrc {
 
 // Loads the group of part columns [q0, q0 + 4U): lane l takes column
 // q0 + 4u + l/16.  A: row 16 (tile0 + m) + l%16 at byte offset
-// col * cs + r_es + 16 m es; a column past the part lies past the buffer
+// col * cs + r_es + 16 m es of a tile on its own, rows 2 (l%16) and one past
+// it of the 32 of a pair of tiles in one load (tile_row; its address is
+// 4-byte aligned, all that a buffer load needs, since blocks of BF16 have an
+// even number of padded rows; with an odd number of FP64 or FP32 rows the
+// pair of the last row of the last column ends past the range, which is
+// checked dword by dword: the row loads, what follows it is 0); a column past the part lies past the buffer
 // range and loads 0, and rows past the block only feed accumulator rows
 // that are not stored.  B: from the column's inputs as src gives them
 // (zeros past the window or the part).
+
+// Item row of accumulator row r of tile m of a unit of nt tiles: the tiles go
+// in pairs, the first of a pair holding the even and the second the odd rows
+// of its 32, so that a lane's entries of both are adjacent and one load brings
+// them (163,840 unknowns, k = 16 695 -> 663 us, k = 17 797 -> 768, k = 32
+// 877 -> 847, k = 64 1,351 -> 1,322; products bit-equal).
+__device__ inline int tile_row(int tile0, int m, int nt, int r) {
+  return m < (nt & ~1) ? (tile0 + (m & ~1)) * 16 + 2 * r + (m & 1) : (tile0 + m) * 16 + r;
+}
 
 template <bool EXACT, bool RUN, int DT, int KT, int NT, int U>
 __device__ inline void load_group(Group<DT, KT, NT, U> &g, __amdgpu_buffer_rsrc_t rs, uint32_t cs,
@@ -197,7 +228,10 @@ __device__ inline void load_group(Group<DT, KT, NT, U> &g, __amdgpu_buffer_rsrc_
     const int col = q0 + 4 * u + cq;
     const uint32_t cb = (uint32_t)col * cs + r_es;
 #pragma unroll
-    for (int m = 0; m < NT; ++m) g.a[u][m] = E::load_raw(rs, cb + (uint32_t)(m * 16 * E::es));
+    for (int m = 0; m + 1 < NT; m += 2)
+      E::load_pair(rs, cb + (uint32_t)((m * 16 + bl.j0) * E::es), g.a[u][m], g.a[u][m + 1]);
+    if constexpr (NT % 2 != 0)
+      g.a[u][NT - 1] = E::load_raw(rs, cb + (uint32_t)((NT - 1) * 16 * E::es));
     gdouble *p;
     if constexpr (RUN)
       p = col < src.hi ? src.xr + (size_t)col * k : src.zr;
@@ -412,7 +446,7 @@ __global__ __launch_bounds__(64 * NW) void hmv_matmat_kernel(
       if (j >= k) continue;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int row = (tile0 + m) * 16 + Mfma<Acc>::row(lane, i);
+        const int row = tile_row(tile0, m, min(nt, TW), Mfma<Acc>::row(lane, i));
         if (row >= w.rows) continue;
         const double v = (double)acc[m][tt][i];
         if constexpr (PHASE == 1) {

@@ -269,3 +269,40 @@ def test_matmat_pairs_up_to_the_last_column(gpu, sphere4, sphere6_arenas, prec, 
         ref = a.matmat(X)[:, :k]
         assert np.array_equal(a.matmat(np.ascontiguousarray(X[:, :k])), ref)
     small.free()
+
+
+# a pair of tiles reads rows in twos: row counts from one tile to beyond a
+# group of four, odd ones with a row on its own at the end of the block
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16", "bf16_all"])
+def test_matmat_pairs_of_rows(gpu, prec):
+    """Every row of every column within the rounding of its storage (2^-8 for
+    BF16 factors, twice for a low-rank product of two, 2^-23 and 2^-52 terms
+    for the others and for up to 130 summed columns) of sum |a| |x|: an entry
+    missed or read twice is a tenth of that sum and more."""
+    from synthetic_leaves import LeafSet
+    rows = [1, 15, 16, 17, 18, 19, 23, 31, 32, 33, 34, 47, 48, 49, 63, 64, 65, 79, 127, 129]
+    nd, lv, r = 2048, [], 0
+    for i, nr in enumerate(rows):
+        lv.append(("dense", r, nr, 30 * i, 1 + i % 9, 0))
+        # a rank of nr: the rows of a phase-1 item
+        lv.append(("lowrank", r, nr, 1000 + 40 * i, 1 + (5 * i) % 9, nr))
+        r += nr
+    lv.append(("dense", 2017, 31, 2000, 7, 0))  # the last block
+    hm = LeafSet(gpu, nd, lv, 4)
+    A, S = np.zeros((nd, nd)), np.zeros((nd, nd))
+    for (kind, r0, nr, c0, nc, q), buf in zip(lv, hm._bufs):
+        if kind == "dense":
+            M = buf.reshape(nr, nc)
+            A[r0:r0 + nr, c0:c0 + nc] += M
+            S[r0:r0 + nr, c0:c0 + nc] += np.abs(M)
+        else:
+            V, U = buf[:nc * q].reshape(q, nc), buf[nc * q:].reshape(q, nr)
+            A[r0:r0 + nr, c0:c0 + nc] += U.T @ V
+            S[r0:r0 + nr, c0:c0 + nc] += np.abs(U).T @ np.abs(V)
+    eps = {"f64": 140 * 2.0 ** -52, "f32": 140 * 2.0 ** -23}.get(prec, 2.0 ** -7 + 140 * 2.0 ** -23)
+    a = gpu.Arena(hm, prec)
+    for k in (9, 16, 19, 32, 50, 64, 128):
+        X = gpu.uniform(k, nd * k).reshape(nd, k)
+        Y = a.matmat(X)
+        assert np.all(np.abs(Y - A @ X) <= eps * (S @ np.abs(X))), k
+    a.free()
