@@ -247,9 +247,7 @@ __global__ __launch_bounds__(64) void hmv_yfinal_kernel(const HmvYFin *__restric
   const HmvYFin f = fin[blockIdx.x];
   if (inst_done && inst_done[f.inst]) return;
   for (int r = threadIdx.x; r < f.rows; r += 64) {
-    const double *p = yp + f.base + r;
-    double s = p[0];
-    for (int q = 1; q < f.np; ++q) s += p[(size_t)q * f.rows];
+    const double s = sum_pieces(yp + f.base + r, f.rows, f.np);
     y[f.row + r] = beta == 0.0 ? s : __builtin_fma(beta, y[f.row + r], s);
   }
 }

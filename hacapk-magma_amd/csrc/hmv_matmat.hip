@@ -480,7 +480,9 @@ __global__ __launch_bounds__(256) void hmv_tfinal_block_kernel(const HmvTFin *__
 }
 
 // Rows of the wide items: y = sum of the pieces' partial rows in piece order
-// + beta y (one workgroup per item, k columns interleaved).
+// + beta y (k columns interleaved; a workgroup per item and kYRhs of its
+// right-hand sides' worth of elements).
+constexpr int kYRhs = 4;
 __global__ __launch_bounds__(256) void hmv_yfinal_block_kernel(const HmvYFin *__restrict__ fin, int k,
                                                                const double *__restrict__ yp,
                                                                double *__restrict__ y, double beta,
@@ -489,10 +491,8 @@ __global__ __launch_bounds__(256) void hmv_yfinal_block_kernel(const HmvYFin *__
   const HmvYFin f = fin[blockIdx.x];
   const size_t n = (size_t)f.rows * k;
   double *py = y + (size_t)f.row * k;
-  for (size_t e = threadIdx.x; e < n; e += 256) {
-    const double *p = yp + (size_t)f.base * k + e;
-    double s = p[0];
-    for (int q = 1; q < f.np; ++q) s += p[(size_t)q * n];
+  for (size_t e = blockIdx.y * 256 + threadIdx.x; e < n; e += 256 * gridDim.y) {
+    const double s = sum_pieces(yp + (size_t)f.base * k + e, n, f.np);
     py[e] = beta == 0.0 ? s : __builtin_fma(beta, py[e], s);
   }
 }
@@ -590,8 +590,8 @@ void launch_block(const HmvLaunch &L, const HmvUnits &U, int k, const double *x,
   else
     launch_units<Acc, 2, DT0, DT1>(kt, L, U, L.work2, x, t, yp, y, k, beta, skip, s);
   if (L.nyfin > 0)
-    hipLaunchKernelGGL(hmv_yfinal_block_kernel, dim3(L.nyfin), dim3(256), 0, s, L.yfin, k, yp, y,
-                       beta, skip);
+    hipLaunchKernelGGL(hmv_yfinal_block_kernel, dim3(L.nyfin, (k + kYRhs - 1) / kYRhs), dim3(256),
+                       0, s, L.yfin, k, yp, y, beta, skip);
 }
 
 }  // namespace
