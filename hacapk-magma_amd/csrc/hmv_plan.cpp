@@ -109,12 +109,28 @@ bool build_plan_device(int nd, int nlf, const void *leaves, int stride, int prec
 }
 
 namespace {
-// Phase-1 bytes per workgroup of a problem whose V factors take `bytes`: 512
-// workgroups or more (two per CU), each of 32 to 96 KiB.  FP64 products: 5,120
-// unknowns (12 MB of V) 26.9 us at 96 KiB and 20.8 at 32; 20,480 (70 MB) 46.7
-// and 48.6.  All-BF16, 25,597 unknowns (22 MB): 31.9 and 25.4.
+// Phase-1 bytes per workgroup of a problem whose V factors take `bytes`: 32
+// to 96 KiB, 512 workgroups (two per CU) or more from 16 MiB on.  FP64
+// products: 1,280 unknowns (1.8 MB of V, 74 blocks and some 108) 11.8 us at 96
+// KiB and 10.7 at 32; 5,120 (12 MB) 26.9 and 20.8; 20,480 (70 MB) 46.7 and
+// 48.6.  All-BF16, 25,597 unknowns (22 MB): 31.9 and 25.4.
 int64_t target_bytes(int64_t bytes) {
   return std::min<int64_t>(96 << 10, std::max<int64_t>(32 << 10, bytes / 512));
+}
+
+// Rows of the next phase-1 block when `left` rank vectors of a column group
+// are left and a block holds at most rs: the last block but one gives rows to
+// a last one of fewer than 8.  A workgroup of 256 threads sums a block of r
+// rows in 256 / r column groups, and one thread a row adds their partials
+// one after the other: at 1,280 unknowns, whose whole phase 1 takes 6.8 to
+// 7.3 us, a block of one row makes it 8.5 (a product 12.3 us instead of 10.7).
+// What it gives keeps the number of 16-row tiles that the H-matmat makes of
+// both.
+int row_chunk(int left, int rs) {
+  const int rest = left - rs;
+  if (rest <= 0) return left;
+  if (rest >= 8) return rs;
+  return rs >= 32 ? rs - 16 : rs >= 16 ? rs - 8 : (left + 1) / 2;
 }
 
 // Small workgroups for a phase's short blocks (nt threads, the precision's
@@ -329,8 +345,8 @@ bool plan_impl(int nd, int nlf, const void *leaves, int stride, int prec, const 
       if (cw >= g.n) cw = g.n;
     }
     g.np = (int)((n + cw - 1) / cw);
-    for (int r0 = 0; r0 < g.r; r0 += rs) {
-      const int nr = std::min(rs, g.r - r0);
+    for (int r0 = 0, nr; r0 < g.r; r0 += nr) {
+      nr = row_chunk(g.r - r0, rs);
       for (int k = 0; k < g.np; ++k) {
         Piece p{c, r0, nr, k, k * cw, (int)std::min<int64_t>(cw, n - (int64_t)k * cw), 0, 0};
         pieces.push_back(p);

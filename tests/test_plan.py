@@ -157,3 +157,24 @@ def test_small_problems_take_more_and_whole_workgroups(H, O, sphere4, prec):
     g = G["work1"]
     assert (g["rows"] * g["ncol0"] * es).max() > 32 << 10
     assert G["nt1_small"] == max(0, H.default_tuning(prec)["p1_small_threads"])
+
+
+@pytest.mark.parametrize("prec,tune", [
+    ("f64", None), ("bf16", {"p1_target_bytes": 6 << 10}), ("f64", {"p1_target_bytes": 20 << 10}),
+    ("f32", {"p1_target_bytes": 8 << 10}), ("f64", {"p1_target_bytes": 96 << 10, "p1_row_tile": 17})])
+def test_no_block_of_a_few_leftover_rows(H, O, sphere3, prec, tune):
+    """The rank vectors of a column group run in blocks of at least 4 rows (one
+    row takes a workgroup a chain of 256 sums) unless the group has fewer."""
+    T = H.plan_tables(sphere3, prec, tune)
+    w, z = T["work1"], T["zseg"]
+    groups = {}
+    for it in w:
+        s = z[it["zseg_begin"]]
+        groups.setdefault((int(s["src"]), int(it["ncol0"])), []).append(int(it["rows"]))
+    assert any(len(g) > 1 for g in groups.values())
+    for g in groups.values():
+        assert min(g) >= min(sum(g), 4), g
+    x = H.uniform(8, sphere3.nd)
+    _, y = PE.run(T, x, sphere3.nd)
+    y_ref = O.adot_body_lfmtx(sphere3, x)
+    assert np.linalg.norm(y - y_ref) / np.linalg.norm(y_ref) < TOL[prec]
