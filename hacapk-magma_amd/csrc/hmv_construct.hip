@@ -10,9 +10,11 @@
 // workgroup per block, all of its lanes on the block's rows/columns, the
 // scalar steps of ACA+ in the same order and arithmetic as the host
 // restatement (the cross updates, the pivot searches with their first-index
-// ties; only the norms, which are compared with thresholds and enter no
-// factor, are summed in another order).  Floating-point contraction is off
-// in this file, so entries and updates round as the host's do.
+// ties).  Only the norms are summed in another order; they are compared with
+// thresholds, and a block with one too near its threshold for the order not to
+// matter runs again with all of them in the host's, so ranks and factors are
+// the host's on every mesh.  Floating-point contraction is off in this file,
+// so entries and updates round as the host's do.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -166,7 +168,7 @@ struct AcaParams {
   int kmax, kmin;
 };
 
-enum { kAcaOk = 0, kAcaOverflow = 1 };
+enum { kAcaOk = 0, kAcaOverflow = 1, kAcaNear = 2 };
 
 __global__ __launch_bounds__(kT) void k_dense(const CLeaf *__restrict__ lv, Geo g) {
   const CLeaf L = lv[blockIdx.x];
@@ -294,10 +296,9 @@ struct Aca {
     reduce(p, none, false);
   }
   // ||vec|| from its statistics.  The squares are safe up to 1e150; past
-  // that (or with an infinity) the entries are scaled by the largest.  The
-  // reference accumulates in entry order; here the order is the reduction's,
-  // which moves the last bits of a number that is only compared with
-  // thresholds (no factor entry depends on them).
+  // that the entries are scaled by the largest.  The reference accumulates in
+  // entry order; here the order is the reduction's, which moves the last bits
+  // of a number that is only compared with thresholds (see far).
   __device__ double norm(const VecStat &s, const double *vec, int n) {
     if (!(s.mx > 1.0e150)) return sqrt(s.ss);
     VecStat t;
@@ -306,6 +307,53 @@ struct Aca {
     return s.mx * sqrt(t.ss);
   }
 };
+
+// Two sums of n squares differ by less than n 2^-52 in their norm: 4e-9 at 16
+// million entries.  A norm at least kNear from a threshold (relative to it)
+// lies on the same side of it in every order of summation.
+constexpr double kNear = 1.0e-8;
+__device__ inline bool far(double v, double thr) {
+  // not with an infinity or a NaN
+  return fabs(v - thr) > kNear * thr || (v == 0.0 && thr == 0.0);
+}
+
+// HACApK_unrm_d, bit for bit, in one wave.  Its running scale zscl is the
+// prefix maximum of the |entries| (those below 1e-30 skipped): each lane forms
+// its entry's ratio zscl/zza or zza/zscl from a prefix maximum over the wave,
+// and only the accumulation of zzz runs entry by entry.
+__device__ double unrm(const double *vec, int n) {
+  const int lane = threadIdx.x;
+  double zscl = 0.0, zzz = 1.0;  // the same in every lane
+#pragma unroll 1
+  for (int c0 = 0; c0 < n; c0 += 64) {
+    const int nl = min(64, n - c0);
+    const double a = lane < nl ? fabs(vec[c0 + lane]) : 0.0;
+    const bool skip = lane >= nl || a < 1.0e-30;
+    double incl = skip ? 0.0 : a;
+#pragma unroll 1
+    for (int off = 1; off < 64; off <<= 1) {
+      const double o = __shfl_up(incl, off, 64);
+      if (lane >= off && o > incl) incl = o;
+    }
+    const double before = __shfl_up(incl, 1, 64);
+    const double m = lane > 0 && before > zscl ? before : zscl;  // zscl before the entry
+    const bool grows = !skip && m < a;
+    const double q = skip ? 0.0 : grows ? m / a : a / m;
+    const unsigned long long g = __ballot(grows), none = __ballot(skip);
+#pragma unroll 1
+    for (int l = 0; l < nl; ++l) {
+      if ((none >> l) & 1ull) continue;
+      const double ql = __shfl(q, l, 64);
+      if ((g >> l) & 1ull)
+        zzz = 1.0 + zzz * ql * ql;
+      else
+        zzz = zzz + ql * ql;
+    }
+    const double most = __shfl(incl, nl - 1, 64);
+    if (most > zscl) zscl = most;
+  }
+  return uniform(zscl * sqrt(zzz));
+}
 
 // Entry a of the residual column ip (col) or row ip of a block after k
 // crosses (HACApK_calc_vec): the matrix entry minus the cross products
@@ -372,8 +420,12 @@ __device__ inline VecStat residual_part(const CLeaf &L, const Geo &g, bool col, 
 
 // HACApK_acaplus (m_HACApK_base.f90:783-975) with param(61) = 1, for one
 // block per workgroup; restates the host fill's ACA+ step for step.  CENT:
-// the centroid kernel on blocks that hold no diagonal entry.
-template <int NT, bool CENT>
+// the centroid kernel on blocks that hold no diagonal entry.  HOST: norms in
+// the host's order (NT = 64); without it a block with a norm not far from its
+// threshold ends as kAcaNear, a matter of chance in 1e-8 per test.  (Forming
+// that norm here instead costs the others 5% (1,024 threads) to 36% (one
+// wave): registers held for a call that hardly ever comes.)
+template <int NT, bool CENT, bool HOST>
 __global__ __launch_bounds__(NT) void k_aca(const CLeaf *__restrict__ lv, Geo g, AcaParams p,
                                             int *__restrict__ kt_out, int *__restrict__ status) {
   __shared__ AcaShared<NT> shared;
@@ -418,9 +470,22 @@ __global__ __launch_bounds__(NT) void k_aca(const CLeaf *__restrict__ lv, Geo g,
     if (tid == 0) m[i1 - 1] = 1;
   };
 
+  auto norm = [&](const VecStat &s, const double *vec, int n) {
+    if constexpr (HOST)
+      return unrm(vec, n);
+    else
+      return R.norm(s, vec, n);
+  };
+  // whether a norm lies below thr
+  auto below = [&](double v, double thr) {
+    if constexpr (!HOST)
+      if (!far(v, thr)) st = kAcaNear;
+    return v < thr;
+  };
+
   int j_ref = 1;
   VecStat sa = calc(true, k, j_ref, pa_ref);  // of pa_ref, as it is now
-  double colnorm = R.norm(sa, pa_ref, ndl);
+  double colnorm = norm(sa, pa_ref, ndl);
   int i_ref;
   {
     // first index of the smallest |entry|: the largest of their negatives
@@ -436,7 +501,7 @@ __global__ __launch_bounds__(NT) void k_aca(const CLeaf *__restrict__ lv, Geo g,
     i_ref = s.ix + 1;
   }
   VecStat sb = calc(false, k, i_ref, pb_ref);  // of pb_ref, as it is now
-  double rownorm = R.norm(sb, pb_ref, ndt);
+  double rownorm = norm(sb, pb_ref, ndt);
 
   double apxnorm = 0.0;
   int lstop_aca = 0;
@@ -524,22 +589,22 @@ __global__ __launch_bounds__(NT) void k_aca(const CLeaf *__restrict__ lv, Geo g,
 
     if (i != i_ref) {
       if (!b_done) sb = axpy(pb_ref, prow, ndt, -uniform(pcol[i_ref - 1]));
-      rownorm = R.norm(sb, pb_ref, ndt);
+      rownorm = norm(sb, pb_ref, ndt);
     }
-    if (i == i_ref || rownorm < ACA_EPS) {
+    if (i == i_ref || below(rownorm, ACA_EPS)) {
       if (i == i_ref) ntries_row = ntries_row + 1;
       if (ntries_row > 0) {
         rownorm = 0.0;
         i = i_ref;
-        while (i != ((i_ref + ndl - 2) % ndl) + 1 && rownorm < za_ACA_EPS && ntries_row > 0) {
+        while (i != ((i_ref + ndl - 2) % ndl) + 1 && below(rownorm, za_ACA_EPS) && ntries_row > 0) {
           if (__builtin_amdgcn_readfirstlane(lrow_msk[i - 1]) == 0) {
             if (k + 1 > cap) {
               st = kAcaOverflow;
               break;
             }
             sb = calc(false, k + 1, i, pb_ref);
-            rownorm = R.norm(sb, pb_ref, ndt);
-            if (rownorm < ACA_EPS) set_mask(lrow_msk, i);
+            rownorm = norm(sb, pb_ref, ndt);
+            if (below(rownorm, ACA_EPS)) set_mask(lrow_msk, i);
             __syncthreads();
             ntries_row = ntries_row - 1;
           } else {
@@ -554,22 +619,22 @@ __global__ __launch_bounds__(NT) void k_aca(const CLeaf *__restrict__ lv, Geo g,
 
     if (j != j_ref) {
       if (!a_done) sa = axpy(pa_ref, pcol, ndl, -uniform(prow[j_ref - 1]));
-      colnorm = R.norm(sa, pa_ref, ndl);
+      colnorm = norm(sa, pa_ref, ndl);
     }
-    if (j == j_ref || colnorm < ACA_EPS) {
+    if (j == j_ref || below(colnorm, ACA_EPS)) {
       if (j == j_ref) ntries_col = ntries_col + 1;
       if (ntries_col > 0) {
         colnorm = 0.0;
         j = j_ref;
-        while (j != ((j_ref + ndt - 2) % ndt) + 1 && colnorm < za_ACA_EPS && ntries_col > 0) {
+        while (j != ((j_ref + ndt - 2) % ndt) + 1 && below(colnorm, za_ACA_EPS) && ntries_col > 0) {
           if (__builtin_amdgcn_readfirstlane(lcol_msk[j - 1]) == 0) {
             if (k + 1 > cap) {
               st = kAcaOverflow;
               break;
             }
             sa = calc(true, k + 1, j, pa_ref);
-            colnorm = R.norm(sa, pa_ref, ndl);
-            if (colnorm < ACA_EPS) set_mask(lcol_msk, j);
+            colnorm = norm(sa, pa_ref, ndl);
+            if (below(colnorm, ACA_EPS)) set_mask(lcol_msk, j);
             __syncthreads();
             ntries_col = ntries_col - 1;
           } else {
@@ -582,21 +647,21 @@ __global__ __launch_bounds__(NT) void k_aca(const CLeaf *__restrict__ lv, Geo g,
       }
     }
 
-    if (colnorm < ACA_EPS && rownorm < ACA_EPS && k >= p.kmin) {
+    if (below(colnorm, ACA_EPS) && below(rownorm, ACA_EPS) && k >= p.kmin) {
       lstop_aca = 1;
       k = k + 1;
     }
     if (lstop_aca == 0) {
-      const double blknorm = R.norm(q1, v1, n1) * R.norm(q2, v2, n2);
+      const double blknorm = norm(q1, v1, n1) * norm(q2, v2, n2);
       if (k == 0) {
         apxnorm = blknorm;
       } else {
-        if (blknorm < apxnorm * eps && rownorm < apxnorm * eps && colnorm < apxnorm * eps &&
-            k >= p.kmin)
-          lstop_aca = 1;
+        const double thr = apxnorm * eps;
+        const bool blk = below(blknorm, thr), row = below(rownorm, thr), col = below(colnorm, thr);
+        if (blk && row && col && k >= p.kmin) lstop_aca = 1;
       }
     }
-    if (lstop_aca == 1 && k >= p.kmin) break;
+    if (st != kAcaOk || (lstop_aca == 1 && k >= p.kmin)) break;
     k = k + 1;
   }
   if (st == kAcaOk && k > cap) st = kAcaOverflow;
@@ -705,11 +770,11 @@ hipError_t dalloc(hmv_dleaves_s *d, void **p, size_t bytes) {
 // 1024 (at 2,592 rows a block's 256 threads already make 11 trips a pass).
 constexpr int kAcaShort = 256, kAcaLong = 2048;
 
-template <int NT, bool CENT>
+template <int NT, bool CENT, bool HOST = false>
 void launch_aca_class(int n, const CLeaf *d_lv, const Geo &g, const AcaParams &p, int *d_kt,
                       int *d_st) {
   if (n > 0)
-    hipLaunchKernelGGL((k_aca<NT, CENT>), dim3((unsigned)n), dim3(NT), 0, nullptr, d_lv, g, p,
+    hipLaunchKernelGGL((k_aca<NT, CENT, HOST>), dim3((unsigned)n), dim3(NT), 0, nullptr, d_lv, g, p,
                        d_kt, d_st);
 }
 // The blocks of one batch, in the order of their classes (n of each).
@@ -730,9 +795,11 @@ int aca_class(const CLeaf &L) {
 // Runs ACA+ on the listed low-rank leaves (longest first) with at most
 // `columns` factor columns each, in batches; packs their factors into
 // allocations of d, and sets their records' base and cap and d->kt.  `again`
-// receives the leaves that need more columns.
+// receives the leaves that need more columns, `near` those with a norm at its
+// threshold (none with host_norms).
 hipError_t run_aca(hmv_dleaves_s *d, const std::vector<int> &ids, const Geo &g,
-                   const AcaParams &p, int columns, std::vector<int> &again) {
+                   const AcaParams &p, int columns, bool host_norms, std::vector<int> &again,
+                   std::vector<int> &near) {
   if (ids.empty()) return hipSuccess;
   // the analytic entry is needed with its kernel and on a diagonal
   bool cent = g.kernel == kKernelCentroid;
@@ -811,7 +878,9 @@ hipError_t run_aca(hmv_dleaves_s *d, const std::vector<int> &ids, const Geo &g,
     dst.assign(nb, nullptr);
     if ((e = hipMemcpy(d_lv, lv.data(), sizeof(CLeaf) * nb, hipMemcpyHostToDevice)) != hipSuccess)
       return e;
-    if (cent)
+    if (host_norms)
+      launch_aca_class<64, false, true>((int)nb, d_lv, g, p, d_kt, d_st);
+    else if (cent)
       launch_aca<true>(n, d_lv, g, p, d_kt, d_st);
     else
       launch_aca<false>(n, d_lv, g, p, d_kt, d_st);
@@ -827,7 +896,7 @@ hipError_t run_aca(hmv_dleaves_s *d, const std::vector<int> &ids, const Geo &g,
     size_t o = 0;
     for (size_t q = 0; q < nb; ++q) {
       if (st[q] != kAcaOk) {
-        again.push_back(batch[q]);
+        (st[q] == kAcaNear ? near : again).push_back(batch[q]);
         continue;
       }
       CLeaf &L = d->lv[batch[q]];
@@ -953,14 +1022,17 @@ int hmv_construct(int nnode, const double *nodes, int nface, const int *faces, c
     if ((e = hipGetLastError()) != hipSuccess)
       return hmv::hip_fail(e, "hmv_construct: dense fill");
   }
-  // low-rank leaves, largest first; then the ones that needed more columns
+  // low-rank leaves, largest first; then the ones that needed more columns, and
+  // the ones that hang on the order of a sum
   std::sort(lr_ids.begin(), lr_ids.end(), [&](int a, int b) {
     const int64_t sa = (int64_t)d->lv[a].ndl + d->lv[a].ndt, sb = (int64_t)d->lv[b].ndl + d->lv[b].ndt;
     return sa != sb ? sa > sb : a < b;
   });
-  std::vector<int> again, failed;
-  if ((e = run_aca(d.get(), lr_ids, g, ap, first_columns(cp->aca_eps), again)) != hipSuccess ||
-      (e = run_aca(d.get(), again, g, ap, INT_MAX, failed)) != hipSuccess ||
+  std::vector<int> again, failed, near, none;
+  if ((e = run_aca(d.get(), lr_ids, g, ap, first_columns(cp->aca_eps), false, again, near)) !=
+          hipSuccess ||
+      (e = run_aca(d.get(), again, g, ap, INT_MAX, false, failed, near)) != hipSuccess ||
+      (e = run_aca(d.get(), near, g, ap, INT_MAX, true, failed, none)) != hipSuccess ||
       (e = hipDeviceSynchronize()) != hipSuccess)  // the dense fill, if nothing followed it
     return hmv::hip_fail(e, "hmv_construct: ACA+");
   if (!failed.empty()) {

@@ -198,3 +198,33 @@ def test_aca_block_on_the_diagonal(gpu, H):
     A[np.arange(n), np.arange(n)] = self_term / (4 * np.pi)
     print("rank", k, "error %.2e" % (np.linalg.norm(uv - A) / np.linalg.norm(A)), flush=True)
     assert np.linalg.norm(uv - A) / np.linalg.norm(A) < 1e-10
+
+
+def test_ranks_at_the_stopping_test_itself(gpu, H):
+    """A block's rank changes where one of its norms crosses its threshold.
+    The two adjacent doubles aca_eps between which a rank of the host fill
+    changes, for blocks of several sizes: the norm is within rounding of the
+    threshold there, and the device takes the host's side on both."""
+    mesh = H.icosphere(3)
+
+    def table(eps):
+        hm = H.HMatrix(*mesh, H.baseline_params(aca_eps=eps))
+        t = hm.leaf_table()
+        hm.close()
+        return t
+
+    above, below = table(1e-4), table(1e-5)
+    change = np.nonzero(above[:, 1] != below[:, 1])[0]
+    longest = np.maximum(above[change, 3], above[change, 5])
+    for leaf in change[np.argsort(longest, kind="stable")][:: len(change) // 11]:
+        hi, lo, k_hi = 1e-4, 1e-5, above[leaf, 1]
+        while np.nextafter(lo, 1.0) < hi:
+            mid = 0.5 * (lo + hi)
+            if table(mid)[leaf, 1] == k_hi:
+                hi = mid
+            else:
+                lo = mid
+        for eps in (lo, hi):
+            dev = H.DeviceHMatrix(*mesh, H.baseline_params(aca_eps=eps))
+            assert np.array_equal(dev.table, table(eps)), (leaf, eps)
+            dev.free()
