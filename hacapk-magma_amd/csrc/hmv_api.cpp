@@ -361,7 +361,10 @@ int upload_plan(hmv::Plan &P, hmv_arena *out, std::chrono::steady_clock::time_po
       (e = upload(&a->d_codes, P.codes)) != hipSuccess ||
       (e = upload(&a->d_work2x, ws.work2)) != hipSuccess ||
       (e = upload(&a->d_yfin, ws.yfin)) != hipSuccess ||
-      (wide && (e = hipMalloc((void **)&a->d_yp, sizeof(double) * ws.nyp)) != hipSuccess)) {
+      (wide && (e = hipMalloc((void **)&a->d_yp,
+                              sizeof(double) * ws.nyp *
+                                  (1 + (size_t)hmv::static_max_rhs(P.tpart_size)))) !=
+                   hipSuccess)) {
     release(a);
     return hip_fail(e, "hmv_arena_build: upload");
   }

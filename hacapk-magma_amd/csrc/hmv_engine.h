@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -48,7 +49,8 @@ struct hmv_arena_s {
   double *d_t = nullptr;   // t slots + chunk partials (FP64 in every mode)
   // phase 2 as it is launched when the plan has wide items: the work list
   // with those in pieces (its input runs follow the plan's in d_zseg), and
-  // the pieces' partial rows
+  // the pieces' partial rows: of the single-vector product, then of
+  // hmv_apply_block_static (the H-matmat's are in d_tk)
   HmvWork *d_work2x = nullptr;
   HmvYFin *d_yfin = nullptr;
   double *d_yp = nullptr;
@@ -89,6 +91,11 @@ hipError_t enqueue_apply(hmv_arena_s *a, const double *x, double *y, double beta
 void free_solve_work(hmv_arena_s *a);
 void free_gcr_work(hmv_arena_s *a);
 void free_multi_work(hmv_arena_s *a);
+// Most right-hand sides of hmv_apply_block_static for tparts t entries.
+inline int static_max_rhs(int64_t tparts) {
+  const int64_t bytes = std::max<int64_t>(1, tparts) * (int64_t)sizeof(double);
+  return (int)std::min<int64_t>(HMV_MAX_RHS, (int64_t)HMV_STATIC_SCRATCH_BYTES / bytes);
+}
 // The arena's H-matmat unit lists and path choices.
 void fill_units(const hmv_arena_s *a, HmvUnits &u);
 // Enqueues Y = H X + beta*Y for k interleaved right-hand sides (1..128).

@@ -622,10 +622,9 @@ extern "C" hipError_t hmv_launch_block(const HmvLaunch *L, const HmvUnits *units
 // with that device current, and only that address reaches the kernels.
 // Nothing in it needs clearing between calls: phase 1 writes every t slot
 // and chunk partial that the finalize and phase 2 read.  Calls that overlap
-// on one device share the array and race.
-// Behind it, the partial rows of the wide items (at most HMV_PARTIAL_ROWS).
-constexpr size_t kStaticT = HMV_STATIC_SCRATCH_BYTES / sizeof(double);
-static __device__ __align__(256) double scratch[kStaticT + (size_t)HMV_PARTIAL_ROWS * HMV_MAX_RHS];
+// on one device share the array and race.  The partial rows of wide items
+// are in memory of their arena (d_yp), made with it.
+static __device__ __align__(256) double scratch[HMV_STATIC_SCRATCH_BYTES / sizeof(double)];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -668,7 +667,7 @@ extern "C" int hmv_apply_block_static(hmv_arena a, int k, const double *x, doubl
     return HMV_ERR_ARG;
   }
   const int64_t need = std::max<int64_t>(1, a->tpart_size) * k * (int64_t)sizeof(double);
-  if (need > (int64_t)HMV_STATIC_SCRATCH_BYTES) {
+  if (k > hmv::static_max_rhs(a->tpart_size)) {
     hmv::set_error("hmv_apply_block_static: the product needs " + std::to_string(need) +
                    " bytes of t buffer (k = " + std::to_string(k) +
                    "), the static scratch holds " + std::to_string(HMV_STATIC_SCRATCH_BYTES));
@@ -687,7 +686,8 @@ extern "C" int hmv_apply_block_static(hmv_arena a, int k, const double *x, doubl
   if (rc) return rc;
   HmvUnits u;
   hmv::fill_units(a, u);
-  e = hmv_launch_block(&a->launch, &u, k, x, t, t + kStaticT, y, beta, nullptr, (hipStream_t)stream);
+  e = hmv_launch_block(&a->launch, &u, k, x, t, a->d_yp + a->launch.nyp, y, beta, nullptr,
+                       (hipStream_t)stream);
   if (e != hipSuccess) return hmv::hip_fail(e, "hmv_apply_block_static: launch");
   return HMV_OK;
 }

@@ -3,6 +3,7 @@ without a GPU every compute entry point fails loudly (no CPU fallback)."""
 import ctypes as C
 import os
 import re
+import struct
 
 import numpy as np
 import pytest
@@ -108,3 +109,30 @@ def test_calibration_argument_checks(H):
     assert L.hmv_stream_test(2, None, buf, (1 << 27) + 8, 1, C.byref(ms)) == -1
     assert L.hmv_stream_test(2, None, None, 64, 1, C.byref(ms)) == -1
     assert b"hmv_stream_test" in L.hmv_last_error()
+
+
+def test_device_memory_of_the_library_itself():
+    """What every process holds on a device by loading the library: its code
+    (some MiB) and the static workspace that hmv.h declares, no more.  The
+    code objects' loaded segments, read from the ELF images in libhmv.so."""
+    with open(os.path.join(ROOT, "include", "hmv.h")) as f:
+        mib = int(re.search(r"define HMV_STATIC_SCRATCH_BYTES \(\(size_t\)(\d+) << 20\)", f.read())[1])
+    with open(os.path.join(ROOT, "hacapk-magma_amd", "lib", "libhmv.so"), "rb") as f:
+        b = f.read()
+    magic, at, held = b"__CLANG_OFFLOAD_BUNDLE__", 0, []
+    while (at := b.find(magic, at)) >= 0:
+        (count,), p = struct.unpack_from("<Q", b, at + 24), at + 32
+        for _ in range(count):
+            off, size, ln = struct.unpack_from("<QQQ", b, p)
+            triple = b[p + 24:p + 24 + ln]
+            p += 24 + ln
+            if b"amdgcn" not in triple or size == 0:
+                continue
+            elf = b[at + off:at + off + size]
+            assert elf[:4] == b"\x7fELF"
+            (phoff,), (phsize, phnum) = struct.unpack_from("<Q", elf, 32), struct.unpack_from("<HH", elf, 54)
+            heads = [struct.unpack_from("<IIQQQQQQ", elf, phoff + i * phsize) for i in range(phnum)]
+            held.append(sum(h[6] for h in heads if h[0] == 1))  # memory sizes of PT_LOAD
+        at = p
+    assert len(held) > 0
+    assert mib << 20 <= sum(held) <= (mib + 16) << 20, held

@@ -85,3 +85,32 @@ def test_partial_rows_are_bounded(gpu, O):
         x = gpu.uniform(4, s.nd)
         assert _err(a.matvec(x), O.adot_body_lfmtx(s, x)) <= 1e-12
         a.free()
+
+
+@pytest.fixture(scope="module")
+def tall(gpu):
+    """75,000 rows of wide items in three pieces each: more partial rows than
+    an arena may have."""
+    return LeafSet(gpu, 80000, [("dense", 250 * i, 250, 0, 3072, 0) for i in range(100)], 10)
+
+
+@pytest.mark.parametrize("name,prec,k", [
+    ("wide", "f64", 1), ("wide", "f64", 8), ("wide", "f64", 19), ("wide", "f64", 128),
+    ("wide", "bf16", 33), ("tall", "f64", 3), ("tall", "f64", 128)])
+def test_wide_items_without_allocation(gpu, request, name, prec, k):
+    """hmv_apply_block_static on wide items: the partial rows are the arena's
+    own; the same kernels and sums as hmv_apply_block, bit for bit, also with
+    the most partial rows."""
+    hm = request.getfixturevalue(name)
+    a = gpu.Arena(hm, prec)
+    X = np.stack([gpu.uniform(20 + j, hm.nd) for j in range(k)], axis=1)
+    want = a.matmat(X)
+    dx = gpu.DeviceBuffer.from_array(X.reshape(-1))
+    dy = gpu.DeviceBuffer.from_array(np.full(X.size, np.nan))
+    gpu._check(gpu.hmv_lib().hmv_apply_block_static(a.handle, k, dx.ptr, dy.ptr, 0.0, None),
+               "hmv_apply_block_static")
+    gpu.hmv_lib().hmv_device_synchronize()
+    assert np.array_equal(dy.download().reshape(hm.nd, k), want)
+    dx.free()
+    dy.free()
+    a.free()
