@@ -853,19 +853,14 @@ int seg_setup(hmv_arena_s *a, SegWork &w, const char *who) {
   bstart[w.nseg] = (int)tb.size();
   w.nblk = (int)tb.size();
   while (w.lanes < 64 && 4 * w.lanes < w.maxblk) w.lanes *= 2;
-  const size_t nbytes = sizeof(double) * (size_t)w.n;
   hipError_t e;
   if ((e = hipStreamCreateWithFlags(&w.s, hipStreamNonBlocking)) != hipSuccess ||
       (e = hipMalloc(&w.tb, sizeof(SegBlock) * tb.size())) != hipSuccess ||
       (e = hipMalloc(&w.bstart, sizeof(int) * bstart.size())) != hipSuccess ||
-      (e = hipMalloc(&w.r, nbytes)) != hipSuccess || (e = hipMalloc(&w.rhat, nbytes)) != hipSuccess ||
-      (e = hipMalloc(&w.p, nbytes)) != hipSuccess || (e = hipMalloc(&w.v, nbytes)) != hipSuccess ||
-      (e = hipMalloc(&w.t, nbytes)) != hipSuccess || (e = hipMalloc(&w.sv, nbytes)) != hipSuccess ||
       (e = hipMalloc(&w.part, sizeof(double) * 2 * tb.size())) != hipSuccess ||
       (e = hipMalloc(&w.cs, sizeof(ColState) * w.nseg)) != hipSuccess ||
       (e = hipMalloc(&w.bs, sizeof(BlockState))) != hipSuccess ||
       (e = hipMalloc(&w.flags, sizeof(int) * w.nseg)) != hipSuccess ||
-      (e = hipMalloc(&w.r2, nbytes)) != hipSuccess || (e = hipMalloc(&w.d, nbytes)) != hipSuccess ||
       (e = hipMemcpy(w.tb, tb.data(), sizeof(SegBlock) * tb.size(), hipMemcpyHostToDevice)) !=
           hipSuccess ||
       (e = hipMemcpy(w.bstart, bstart.data(), sizeof(int) * bstart.size(), hipMemcpyHostToDevice)) !=
@@ -877,20 +872,31 @@ int seg_setup(hmv_arena_s *a, SegWork &w, const char *who) {
 // Buffers of the GCR steps.
 int sg_setup(const SegWork &w, SegGcrWork &gw, int m, const char *who);
 
-// The arena's workspace, with the GCR part for m directions if m > 0.
-int multi_work(hmv_arena_s *a, int m, HmvMultiWork *&out, const char *who) {
+// The arena's workspace, with the vectors of a refinement if `refine`, and
+// with those of GCR for m directions (m > 0) or of BiCGSTAB (m = 0): a vector
+// is held from the first call that uses it on.
+int multi_work(hmv_arena_s *a, bool refine, int m, HmvMultiWork *&out, const char *who) {
   int rc = HMV_OK;
   if (!a->multi) {
     a->multi = new HmvMultiWork();
     rc = seg_setup(a, a->multi->w, who);
   }
+  SegWork &w = a->multi->w;
+  hipError_t e = hipSuccess;
+  auto vector = [&](double **v) {
+    if (rc == HMV_OK && !*v &&
+        (e = hipMalloc((void **)v, sizeof(double) * (size_t)w.n)) != hipSuccess)
+      rc = hmv::hip_fail(e, (std::string(who) + ": workspace").c_str());
+  };
+  if (refine)
+    for (double **v : {&w.r2, &w.d}) vector(v);
+  if (m == 0)
+    for (double **v : {&w.r, &w.rhat, &w.p, &w.v, &w.t, &w.sv}) vector(v);
   if (rc == HMV_OK && m > 0 && a->multi->gw.m != m) {
     a->multi->gw.free_all();
-    rc = sg_setup(a->multi->w, a->multi->gw, m, who);
+    rc = sg_setup(w, a->multi->gw, m, who);
   }
-  hipError_t e;
-  if (rc == HMV_OK &&
-      (e = hmv::solve_host(a, a->multi->w.s, a->multi->w.h)) != hipSuccess)
+  if (rc == HMV_OK && (e = hmv::solve_host(a, w.s, w.h)) != hipSuccess)
     rc = hmv::hip_fail(e, (std::string(who) + ": workspace").c_str());
   if (rc != HMV_OK) {
     hmv::free_multi_work(a);
@@ -1016,7 +1022,7 @@ extern "C" int hmv_multi_bicgstab(hmv_arena a, const double *b, double *u, doubl
   if (check_every < 1) check_every = 1;
   const char *who = "hmv_multi_bicgstab";
   HmvMultiWork *mw = nullptr;
-  int rc = multi_work(a, 0, mw, who);
+  int rc = multi_work(a, false, 0, mw, who);
   if (rc) return rc;
   SegWork &w = mw->w;
   const HmvInstHost *hi = hmv::inst_host(w.h);
@@ -1070,7 +1076,7 @@ extern "C" int hmv_multi_bicgstab_ir(hmv_arena a64, hmv_arena alow, const double
   }
   if (check_every < 1) check_every = 1;
   HmvMultiWork *mw = nullptr;  // inner solves over the low-precision arena
-  int rc = multi_work(alow, 0, mw, who);
+  int rc = multi_work(alow, true, 0, mw, who);
   if (rc) return rc;
   SegWork &w = mw->w;
   HmvInstHost *hi = hmv::inst_host(w.h);
@@ -1635,7 +1641,7 @@ extern "C" int hmv_multi_gcr_ir(hmv_arena a64, hmv_arena alow, const double *b, 
     return HMV_ERR_ARG;
   }
   HmvMultiWork *mw = nullptr;
-  int rc = multi_work(alow, m, mw, who);
+  int rc = multi_work(alow, true, m, mw, who);
   if (rc) return rc;
   SegWork &w = mw->w;  // block table, stream and FP64 residuals
   SegGcrWork &gw = mw->gw;

@@ -205,6 +205,18 @@ int hmv_apply_host(hmv_arena a, const double *zu, double *zau);
 /* Bytes of the device t-partial buffer owned by the arena. */
 int64_t hmv_arena_tbytes(hmv_arena a);
 
+/* ---- solvers ------------------------------------------------------------
+ * Workspace stays with the arena between calls, until hmv_arena_free: with
+ * the arena solved on (the low-precision one of a refinement) vectors of nd
+ * doubles from the first call that uses them on.  BiCGSTAB 8 (its refinement
+ * 8 with either arena); GCR(m) 2m + 2, its refinement 2 more; the per-instance solvers 6 for BiCGSTAB, 2m + 2 for
+ * GCR(m) (m of the last call) and 2 for their refinements.  The block solvers
+ * and the pipelined one free theirs on return.  Also some 8 KB of pinned host
+ * memory and 40 bytes per instance.
+ * The calling thread is busy for the whole solve: it launches the iterations
+ * and watches a word of host memory that the device writes; check_every does
+ * not make it look less often. */
+
 /* ---- BiCGSTAB ---------------------------------------------------------- */
 
 #define HMV_SOLVE_CONVERGED 0

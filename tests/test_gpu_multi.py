@@ -5,6 +5,8 @@ Bar: the concatenated apply and H-matmat equal each instance's own apply
 (FP64 <= 1e-13 relative per instance) and the oracle; each instance's solve
 reaches the true-residual bar and agrees with its single-instance solve.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -258,3 +260,46 @@ def test_multi_solvers_block_sizes(gpu, sizes):
         alow.free()
     m64.free()
     mlow.free()
+
+
+def test_solvers_hold_only_the_vectors_they_use(gpu):
+    """The per-instance solvers keep their workspace with the (low-precision)
+    arena.  GCR(1) refinement takes 6 vectors of all unknowns, BiCGSTAB 6, its
+    refinement 8, and their tables at most 3 allocations of 2 MiB (a vector of
+    this size takes one); freeing the arena gives all of it back."""
+    with open("/proc/self/maps") as f:  # the HIP runtime that the library uses
+        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    hm = gpu.HMatrix(*gpu.icosphere(5), gpu.baseline_params(aca_eps=1e-3))
+    m64, low = gpu.MultiArena([hm] * 8, "f64"), gpu.MultiArena([hm] * 8, "f32")
+    b = np.tile(gpu.uniform(3, hm.nd), 8)
+    unit = 2 << 20
+    assert unit / 2 < 8 * m64.nd <= unit
+
+    def solve(kind, a):
+        if kind == "gcr_ir":
+            gpu.multi_gcr_ir(m64, a, b, eps=1e-6, m=1, max_outer=1, max_inner=2)
+        elif kind == "bicgstab_ir":
+            gpu.multi_bicgstab_ir(m64, a, b, eps=1e-6, max_outer=1, max_inner=2)
+        else:
+            a.bicgstab_multi(b, eps=1e-6, maxit=2)
+
+    def free():
+        gpu.hmv_lib().hmv_device_synchronize()
+        left, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(left), C.byref(total)) == 0
+        return left.value
+
+    for kind in ("gcr_ir", "bicgstab_ir", "bicgstab"):
+        solve(kind, low)  # what a first launch of its kernels allocates is not the workspace
+    low.free()
+    for kind, vectors in (("gcr_ir", 6), ("bicgstab_ir", 8), ("bicgstab", 6)):
+        before = free()
+        low = gpu.MultiArena([hm] * 8, "f32")
+        built = free()
+        solve(kind, low)
+        held = (built - free()) / unit
+        print(kind, "allocations held %.2f" % held, flush=True)
+        assert held <= vectors + 3, kind
+        low.free()
+        assert before - free() <= unit, kind
+    m64.free()
