@@ -114,3 +114,58 @@ def test_wide_items_without_allocation(gpu, request, name, prec, k):
     dx.free()
     dy.free()
     a.free()
+
+
+class _Solvable(LeafSet):
+    """A well-conditioned matrix with wide items: 40 full rows among diagonal
+    blocks, and a low-rank block."""
+
+    def __init__(self, H, nd, seed):
+        at = [0, 700, nd - 40]  # first of the full rows: 40 at one of these
+        top = at[seed % 3]
+        lv = [("dense", top, 40, 0, nd, 0)]
+        for lo, hi in ((0, top), (top + 40, nd)):
+            lv += [("dense", r, min(60, hi - r), r, min(60, hi - r), 0) for r in range(lo, hi, 60)]
+        lv.append(("lowrank", 100, 300, nd - 900, 400, 3))
+        super().__init__(H, nd, lv, seed)
+        self.A = np.zeros((nd, nd))
+        for (kind, r0, nr, c0, nc, k), buf in zip(lv, self._bufs):
+            if kind == "dense":
+                block = buf.reshape(nr, nc)
+                block *= 0.05
+                i = np.arange(nr)
+                block[i, i + r0 - c0] += 3.0 + 0.01 * i
+                self.A[r0:r0 + nr, c0:c0 + nc] += block
+            else:
+                buf *= 0.1
+                v, u = buf[:nc * k].reshape(k, nc), buf[nc * k:].reshape(k, nr)
+                self.A[r0:r0 + nr, c0:c0 + nc] += u.T @ v
+
+
+@pytest.mark.parametrize("early", [0, 1, 2])
+def test_instances_with_wide_items_stop_on_their_own(gpu, O, early):
+    """Three instances with wide items, one of which starts at its solution:
+    its pieces and their sums are skipped from then on, the others' are not
+    (each instance's solution is that of its dense matrix)."""
+    hms = [_Solvable(gpu, nd, s) for s, nd in enumerate((3200, 3411, 3100))]
+    m64, low = gpu.MultiArena(hms, "f64"), gpu.MultiArena(hms, "f32")
+    off = np.cumsum([0] + [hm.nd for hm in hms])
+    b = gpu.uniform(30 + early, m64.nd)
+    want = np.concatenate([np.linalg.solve(hm.A, b[lo:hi])
+                           for hm, lo, hi in zip(hms, off, off[1:])])
+    assert _err(O.adot_body_lfmtx(hms[early], want[off[early]:off[early + 1]]),
+                b[off[early]:off[early + 1]]) < 1e-13
+    u0 = np.zeros(m64.nd)
+    u0[off[early]:off[early + 1]] = want[off[early]:off[early + 1]]
+    for name, (u, inst, *_) in (
+            ("bicgstab", m64.bicgstab_multi(b, u0, eps=1e-10)),
+            ("bicgstab_ir", gpu.multi_bicgstab_ir(m64, low, b, u0, eps=1e-10)),
+            ("gcr_ir", gpu.multi_gcr_ir(m64, low, b, u0, eps=1e-10))):
+        steps = [i["nstp"] for i in inst]
+        print(name, "steps", steps, flush=True)
+        assert [s == 0 for s in steps] == [i == early for i in range(3)]
+        for i, (lo, hi) in enumerate(zip(off, off[1:])):
+            assert inst[i]["status_name"] == "converged"
+            assert _err(u[lo:hi], want[lo:hi]) < 1e-8, (name, i)
+    m64.free()
+    low.free()
