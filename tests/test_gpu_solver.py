@@ -233,3 +233,23 @@ def test_fed_iterations(gpu, sphere3, maxit):
             assert np.array_equal(first[name][2], long[2][:maxit + 1]), name
     for a in (a64, alow, m64, mlow):
         a.free()
+
+
+@pytest.mark.parametrize("maxit,check_every", [(0, 4), (1, 4), (5, 4), (8, 4), (9, 2), (300, 7)])
+def test_reliable_updates_at_their_limits(gpu, sphere3, maxit, check_every):
+    """hmv_bicgstab_ru stops on the step limit wherever it falls in a burst,
+    reports the residual it stopped with, and takes no step from a solution."""
+    a64, alow = gpu.Arena(sphere3, "f64"), gpu.Arena(sphere3, "bf16")
+    b = gpu.uniform(17, sphere3.nd)
+    u, info = gpu.bicgstab_ru(a64, alow, b, eps=1e-9, maxit=maxit, check_every=check_every)
+    true = np.linalg.norm(b - a64.matvec(u)) / np.linalg.norm(b)
+    assert abs(info["true_relres"] - true) <= 1e-12 * max(1.0, true)
+    if maxit < 100:
+        assert info["nstp"] == maxit and info["status_name"] == "maxiter"
+    else:
+        assert info["status_name"] == "converged" and info["true_relres"] < 1e-9
+        u2, info2 = gpu.bicgstab_ru(a64, alow, b, u0=u, eps=1e-8, check_every=check_every)
+        assert info2["nstp"] == 0 and info2["status_name"] == "converged"
+        assert np.array_equal(u, u2)
+    a64.free()
+    alow.free()
