@@ -203,8 +203,8 @@ hmv_stream_kernel(
     double *__restrict__ yp, double *__restrict__ y, double beta, const int *__restrict__ skip,
     const int *__restrict__ winst, const int *__restrict__ inst_done) {
   // the flag and the work record are read together, one round trip instead of
-  // two (also the record's own start without a flag): 1,280 unknowns 11.5 ->
-  // 11.0 us a product, 20,480 42.0 -> 41.1 us
+  // two (also the record's own start without a flag): 1,280 unknowns 11.0 ->
+  // 10.5 us a repeated product, 5,120 17.6 -> 17.2, 20,480 39.7 -> 39.4
   const int stop = skip ? *skip : 0;
   const HmvWork w = works[blockIdx.x];
   asm volatile("" : : "s"(stop), "s"(w.off0), "s"(w.rows), "s"(w.ncol0), "s"(w.zseg_begin));
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(64) void hmv_yfinal_kernel(const HmvYFin *__restric
 // have too few columns for a longer batch (1,280 unknowns: 12.1 against
 // 11.0 us); above, the other workgroups cover the trips and the longer
 // batches only delay the ends (81,920: 182.4 against 182.2; 327,680: 1.4%
-// slower).
+// slower).  Both run 8 waves a SIMD (at most 64 VGPRs, no spill).
 constexpr int kDeepMin = 256, kDeepMax = 2560;
 
 template <typename Acc, int PHASE, int DT0, int DT1, int NT>
@@ -340,9 +340,11 @@ __global__ __launch_bounds__(HMV_WG_THREADS) void hmv_copy_kernel(const double2 
     dst[i] = src[i];
 }
 
-// FP64 MFMA rate: `rounds` x 8 independent 16x16x4 FP64 MFMAs per wave on
-// register operands (eight accumulator chains, so that no MFMA waits for
-// its predecessor's result).
+// FP64 MFMA calibration: `rounds` x 8 independent 16x16x4 FP64 MFMAs per wave
+// on register operands (eight accumulator chains, so that no MFMA waits for
+// its predecessor's result).  Its 47.5 TFLOP/s is this kernel's rate and no
+// ceiling: the H-matmat's phase 2 issues 50 at 76% of the pipe, and an FP64
+// library product of 8,192^3 reaches 73.0.
 typedef double hmv_d4 __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(64) void hmv_mfma_rate_kernel(int rounds, double *__restrict__ out) {
   hmv_d4 acc[8];
