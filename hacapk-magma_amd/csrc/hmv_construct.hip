@@ -12,9 +12,10 @@
 // restatement (the cross updates, the pivot searches with their first-index
 // ties).  Only the norms are summed in another order; they are compared with
 // thresholds, and a block with one too near its threshold for the order not to
-// matter runs again with all of them in the host's, so ranks and factors are
-// the host's on every mesh.  Floating-point contraction is off in this file,
-// so entries and updates round as the host's do.
+// matter runs again with all of them in the host's, so where the entries are
+// the host's (the centroid kernel off the diagonal) ranks and factors are too.
+// Floating-point contraction is off in this file, so entries and updates round
+// as the host's do.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -1,4 +1,4 @@
-"""GPU GCR(m) (hmv_gcrm, hipGraph per iteration) against the oracle's
+"""GPU GCR(m) (hmv_gcrm) against the oracle's
 restatement of HACApK_gcrm_lfmtx (m_HACApK_solve.f90:506-571)."""
 import numpy as np
 import pytest

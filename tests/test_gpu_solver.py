@@ -1,4 +1,4 @@
-"""GPU BiCGSTAB (hmv_bicgstab, hipGraph per iteration) against the oracle's
+"""GPU BiCGSTAB (hmv_bicgstab) against the oracle's
 restatement of HACApK_bicgstab_cax_lfmtx_hyp (m_HACApK_solve.f90:342-449)."""
 import json
 import os
